@@ -16,7 +16,8 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIBPATH = os.path.join(LIBDIR, "libcalibquant_hip.so")
-SOURCES = ["cq_core.hip", "cq_quantize.hip", "cq_lutvecmat.hip", "cq_decode.hip", "cq_rope.hip"]
+SOURCES = ["cq_core.hip", "cq_quantize.hip", "cq_lutvecmat.hip", "cq_decode.hip", "cq_decode_matrix_bf16.hip",
+           "cq_decode_matrix_fp16.hip", "cq_rope.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -34,7 +35,7 @@ EXTRA_FLAGS = {
 }
 
 
-def build(verbose: bool = True, jobs: int = 4) -> str:
+def build(verbose: bool = True, jobs: int = 8) -> str:
     os.makedirs(LIBDIR, exist_ok=True)
     objs, procs = [], []
     for src in SOURCES:
@@ -106,6 +107,8 @@ def build_phase_stops(verbose: bool = True) -> str:
     os.makedirs(LIBDIR, exist_ok=True)
     objs = []
     for src in SOURCES:
+        if "_matrix_" in src:   # the profiling build's one instantiation is part of its decode object
+            continue
         obj = os.path.join(LIBDIR, src.replace(".hip", ".phases.o" if src == "cq_decode.hip" else ".o"))
         if src == "cq_decode.hip" or not os.path.exists(obj):
             extra = EXTRA_FLAGS.get(src, []) + (["-DCQ_PHASE_STOPS"] if src == "cq_decode.hip" else [])

@@ -1,0 +1,1954 @@
+// Fused decode attention over bit-packed K/V for gfx950 (MI355X).
+//
+// One workgroup (1024 threads, or 512 threads with two workgroups resident per compute
+// unit when there are more units than compute units) owns one (batch, kv-head,
+// head-group, token-chunk) unit and runs the whole step for HPB query heads that share
+// the kv-head:
+//
+//   loads    the packed K rows are requested at kernel entry, the first block of
+//            packed V rows behind them (half before the logits, half as the K
+//            registers free up), the first tile of residual K/V rows when the
+//            packed-V phase ends: each stream is in flight while the phase before
+//            its consumer runs, and no phase starts behind a queue of requests
+//            it does not need.
+//   K side   q.s_k is folded into a byte-indexed partial-sum table in LDS
+//            (one entry per byte position and byte value, HPB floats wide,
+//            zero-point folded in).  A token's logits are NB table look-ups
+//            and adds; the fp16/bf16 K tensor is never materialised.
+//   stats    min / max of the image logits (calibration), then e = exp(w' - M)
+//            in place in LDS.
+//   V side   tokens are taken four at a time: a 16-entry table of subset sums
+//            of their e values is built once per group, every byte column of
+//            the packed V rows is staged byte-transposed (the 4 tokens' bytes of a
+//            column in one dword), a 4-byte dot product turns each bit lane of the
+//            column into a table offset, and the lane adds that table entry.  Scale /
+//            zero-point are applied once at the end.
+//   residual the full-precision rows run last as an online-softmax flash-decode in
+//            the same workgroup (packed dot2 for q.K) and are merged at the end.
+//
+// When the chunk does not cover all T tokens (long context or small batch)
+// a first launch computes every chunk's logits and publishes the per-chunk min / max;
+// the main launch recomputes its chunk's logits (or, where the packed K row is more
+// bytes than the logits - 2 bits, or fewer than four heads per unit - reads back what
+// the first launch left in a buffer, fp32, instead of building the table and doing the
+// look-ups again), exponentiates against the global min / max and writes an (m, l, acc)
+// partial; the last workgroup of a unit to get there combines the unit's partials.
+//
+// The matrix-core form (template flag MX: per-channel values, one launch) keeps this order of phases and replaces the
+// look-ups of both sides by 8-bit integer MFMAs; see matrix_query below.
+#pragma once
+#include "cq_common.h"
+
+// The kernels below lean on behaviour of this architecture family that the HIP memory model does not
+// promise (see the in-launch merge of the chunked step) and on its LDS size, DPP controls and
+// instruction set: refuse to build device code for anything else.
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "the decode kernels are written for gfx950"
+#endif
+
+#include <type_traits>
+
+namespace cq {
+
+constexpr int kD = 128;
+constexpr int kPF = 4;             // 16-byte loads kept in flight per thread and stream
+// matrix-core form: 16-byte pieces of packed K and V rows in flight per thread, and of the V rows how many are requested
+// ahead of the logits
+constexpr int kMatrixK = 4, kMatrixV = 4, kMatrixE = 2;
+constexpr int kLdsMax = 160 * 1024;
+constexpr int kDefaultUnits = 256; // compute units of a whole MI355X, assumed when no device can be asked
+constexpr int kRegPair = 8;        // rounds of logits a thread of a 512-thread workgroup keeps in registers (4 096 tokens)
+constexpr int kRegTwoBit = 4;      // ... of the 2-bit kernel with four heads per unit (4 096 tokens)
+constexpr int kRegLong = 10;       // ... of a 1024-thread workgroup that holds a long chunk in one launch (10 240 tokens)
+constexpr int kRegMost = 16;       // ... of the longest chunks a plan for fewer than four heads per unit can have (16 384 tokens)
+constexpr float kLog2e = 1.4426950408889634f;
+
+// Profiling build (-DCQ_PHASE_STOPS, `python -m calibquant_amd.build --phase-stops`; only the headline
+// instantiation is compiled): a launch can be told to end at a phase boundary (environment variable
+// CQ_DECODE_PHASE_STOP = k, read per call), so that whole-launch hardware counters of runs with successive
+// k give per-phase counts by subtraction.  The shipped library has none of this.
+#ifdef CQ_PHASE_STOPS
+#define CQ_PHASE(k) do { if (g.stop == (k)) return; } while (0)
+#else
+#define CQ_PHASE(k) do { } while (0)
+#endif
+
+
+template <int N> struct alignas(N * 4) Vec { float v[N]; };
+// native 16-byte vector: copies are single vector moves (HIP's uint4 struct copies lower to memcpy)
+typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+
+struct DecodeGeom {
+    const void* q;
+    const uint8_t* ck;
+    const uint8_t* cv;
+    const void *ks, *kz, *vs, *vz;
+    const void *kres, *vres;
+    int64_t rs_b, rs_h, rs_r;
+    const float* mask;
+    int64_t mask_sb;
+    void* out;
+    const int32_t* r_dev;   // optional: residual row count read at run time (R is then the capacity)
+    float* mm;    // [B][Hq][nsplit][2] chunk logit min / max
+    float* part;  // [B][Hq][nx][kD + 2] partials (m, l, acc)
+    float* lgt;   // chunked launch: [unit][T][HPB] logits, written by the min/max launch and read by the main
+                  // launch instead of its own K look-ups; NULL: the main launch recomputes them
+    int* cnt;     // chunked launch: [unit] count of the unit's chunks (+ residual unit) that have written their
+                  // partial; the one that finds all the others done merges them
+    // Chunked step in ONE launch (every chunk's workgroup resident at once): the chunks of a unit exchange their
+    // logit min / max inside the launch.  rec: [unit][head][chunk][2] 64-bit records, a float (min, then max)
+    // in the lower half and the call's epoch in the upper half - a record is valid by itself, so a chunk
+    // publishes with plain write-through stores and waits for nothing, and the others poll the records
+    // (whatever an earlier call or an uninitialised workspace left there has another epoch).  done64: [unit]
+    // partials written, tagged with the epoch the same way.  status: host-visible word that a workgroup sets
+    // when it gives up waiting (spin_limit polls); NULL: nowhere to report.
+    unsigned long long* rec;
+    unsigned long long* done64;
+    int* status;
+    uint32_t epoch;
+    int fused;
+    int spin_limit;
+#ifdef CQ_PHASE_STOPS
+    int stop;     // phase boundary at which the launch ends (-1: runs to the end)
+#endif
+    int B, Hq, Hkv, T, R, S;
+    int nsplit, chunk, nx;
+    int calib;
+    float off_max, off_min;
+    int cap;      // logits capacity of the LDS layout, tokens
+    FastDiv d_ng, d_nx, d_hkv;   // divisors of the unit decomposition: head groups, chunks (+ residual unit), kv heads
+    int G;        // query heads per kv head
+    int ncu;      // paired launch whose workgroups are all resident from the start (at most two per compute unit):
+                  // the number of compute units (the two workgroups of a unit are told apart by it); else 0
+    float one;    // 1.0f, opaque to the compiler: keeps f16 -> f32 accumulation in one mixed-precision FMA
+};
+
+constexpr int cmax(int a, int b) { return a > b ? a : b; }
+constexpr int cmin(int a, int b) { return a < b ? a : b; }
+
+// VTOK: values quantised per token and per group of 32 channels (scale * code + minimum,
+// codes in little-endian 32-bit words, first channel in the lowest bits) instead of per
+// channel.  A token slot then also carries the token's group scales, and every channel
+// group has its own subset-sum tables.
+// REGL > 0: a thread keeps the logits of its tokens (at most REGL rounds of kNT tokens) in registers
+// until the block's min / max are known and writes only e = exp(.) to the token slots, as packed fp16:
+// the slots take half the bytes, which is what lets two 512-thread workgroups share a compute unit's
+// LDS (with the K table built for half of the byte positions at a time), or one 1024-thread workgroup
+// hold a chunk of 9 984 tokens.
+// MX: the matrix-core form (see MatrixStep below).  No tables and no token slots: region A holds one 64-token tile
+// of weights and of packed V rows per wave, later the folds' partials.
+template <int BITS, int HPB, bool VTOK = false, int NT_ = 1024, int REGL = 0, bool MX = false> struct Lay {
+    static constexpr int kNT = NT_;                 // threads per workgroup
+    static constexpr int kNW = kNT / kWave;         // waves per workgroup
+    // residual window: tiles of 128 rows for either workgroup size - a 512-thread workgroup puts 4 lanes on a
+    // row (32 channels each), a 1024-thread one 8 (16 channels each)
+    static constexpr int LPR = kNT / 128;           // lanes per residual row
+    static constexpr int kResTile = kNT / LPR;      // residual rows per tile
+    static constexpr int NKP = 16 / LPR;            // 16-byte pieces of a row per lane
+    static constexpr int RPW = kResTile / kNW;      // rows of a tile whose values one wave multiplies
+    static constexpr int NB = 16 * BITS;            // bytes per packed row
+    static constexpr int PC = NB * 8;               // bit lanes per row
+    static constexpr int GPW = kWave / NB;          // 4-token groups per wave pass
+    static constexpr int MPL = 8 / GPW;             // bit lanes of a byte column handled by one lane
+    static constexpr int TPW = 4 * GPW;             // tokens per wave pass
+    static constexpr int ESZ = HPB * 4;             // bytes per fp32 table entry / logits slot
+    static constexpr int HW = HPB >= 2 ? HPB / 2 : 1;   // 32-bit words per packed-fp16 entry
+    static constexpr int ESZH = HW * 4;             // bytes per packed-fp16 table entry
+    // The byte-indexed K table covers NBP byte positions at a time: all of them when that fits the
+    // table's share of the LDS (64 KB; 32 KB for a 512-thread workgroup), else half of them in each of
+    // two (or a quarter in each of four) passes over the chunk's rows, the earlier passes' partial logits
+    // waiting in the token slots or, with REGL, in registers.
+    // INA (512-thread workgroup with the logits in registers): nothing else lives in LDS while the K table is
+    // in use, so the table takes all 64 KB of region A and the token slots, written only after the last
+    // look-up, sit in that region as well, behind the staged V block - one table pass at 1 bit (two at 2 bits)
+    // with 256-byte rows, i.e. single-permute look-up addresses, inside the 80 KB a paired workgroup may use.
+    // The table is then built straight from the per-bit weights (no nibble tables to find room for).
+    static constexpr bool INA = (NT_ == 512 && REGL > 0 && !MX);
+    static constexpr int KTMAX = ((NT_ == 512 && !INA) ? 32 : 64) * 1024;
+    static constexpr int KPASS = (NB * 256 * ESZ > 2 * KTMAX) ? 4 : (NB * 256 * ESZ > KTMAX) ? 2 : 1;
+    static constexpr int NBP = NB / KPASS;          // byte positions per pass
+    static constexpr int WPP = NBP / 4;             // 32-bit words of a row per pass
+    static constexpr int PCS = (WPP + 3) / 4;       // 16-byte pieces of a row a pass looks at
+    static constexpr int KT = NBP * 256 * ESZ;      // K table bytes
+    static_assert(NB * 256 * ESZ <= 4 * KTMAX, "at most four table passes");
+    static_assert(!(REGL > 0 && VTOK), "logits in registers: per-channel values only");
+    static constexpr int SLOT = MX ? 0 : VTOK ? 16 : (REGL > 0 ? ESZH : ESZ);   // bytes per token slot: logits, later e (+ 4 group scales)
+    static constexpr int NGRP = VTOK ? kD / 32 : 1; // channel groups with tables of their own
+    static constexpr int WTAB = kNW * NGRP * GPW * 16 * ESZH;
+    static constexpr int RW = cmax(3 * HPB, VTOK ? (NGRP + 1) * HPB : 0);   // per-wave partials: min/max + masked max, or the closing sums
+    static constexpr int VSUB = kNT * kPF / BITS;   // V tokens staged at a time
+    static constexpr int KR = (MX ? kMatrixK : kPF) / BITS;           // K token rounds in flight per thread
+    static constexpr int RED = kNW * PC * ESZ;
+    static constexpr int RED2 = kNW * kD * ESZ;
+    // fixed small region (floats)
+    static constexpr int F_WBIT = 0;                          // NB*8*HPB
+    static constexpr int F_QSZ = F_WBIT + NB * 8 * HPB;       // NB*HPB: zero-point sum per byte position and head
+    static constexpr int F_QRAW = F_QSZ + NB * HPB;           // HPB*kD raw 16-bit q
+    static constexpr int F_RED = F_QRAW + HPB * kD / 2;       // kNW*HPB
+    static constexpr int F_STAT = F_RED + kNW * RW;           // 8*HPB: per-head softmax state
+    static constexpr int F_VSZ = F_STAT + 8 * HPB;            // 2*kD: value scale, zero-point (VTOK: NGRP*HPB minimum terms)
+    static constexpr int F_NIB = F_VSZ + 2 * kD;              // NB*32*HPB: nibble tables
+    // (REGL: the nibble tables live in the token slots, which are first written after the last table pass;
+    // INA: there are none)
+    static constexpr int NIBF = NB * 32 * HPB;
+    static constexpr int F_SRES = F_NIB + (REGL > 0 ? 0 : NIBF);  // kResTile*HPB
+    static constexpr int F_PRES = F_SRES + kResTile * HPB;    // kResTile*HPB
+    static constexpr int F_END = F_PRES + kResTile * HPB;
+    static constexpr int FIXED = ((F_END * 4 + 255) / 256) * 256;
+    // byte offset of the token slots: behind the fixed region, or (INA) inside region A behind the staged V block
+    static constexpr int slots_in_a(int cap) { return WTAB + cmin(VSUB, cap) * NB; }
+    static constexpr int MXT = (1 + BITS) * 1024;   // MX: bytes of a wave's tile, weights then packed V rows
+    static constexpr int region_a(int cap) {
+        if (MX) return cmax(kNW * MXT, RED2);
+        return (cmax(cmax(KT, slots_in_a(cap) + (INA ? cap * SLOT : 0)), cmax(RED, RED2)) + 255) / 256 * 256;
+    }
+    static constexpr int lds_bytes(int cap) {
+        return region_a(cap) + FIXED + ((INA || MX) ? 0 : cmax(cap * SLOT, REGL > 0 ? NIBF * 4 : 0));
+    }
+    // largest chunk whose layout fits: the whole LDS for a 1024-thread workgroup, half of it for a
+    // 512-thread workgroup (two are meant to be resident per compute unit)
+    static constexpr int max_chunk() {
+        int best = 64;
+        for (int c = 64; c <= 16384; c += 64)
+            if (lds_bytes(c) <= (kNT == 512 ? kLdsMax / 2 : kLdsMax) && (REGL == 0 || c <= REGL * kNT)) best = c;
+        return best;
+    }
+};
+
+// One exchange step of an integer-key maximum, N values side by side: the N chains are
+// independent, so the cross-lane moves of one fill the wait states of the others.
+template <int N, int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ void max_step(int* k) {
+    constexpr int lo = static_cast<int>(0x80000000u);
+    int t[N];
+#pragma unroll
+    for (int h = 0; h < N; ++h) t[h] = dpp_move_i<CTRL, ROW_MASK>(k[h], lo);
+#pragma unroll
+    for (int h = 0; h < N; ++h) k[h] = max(k[h], t[h]);
+}
+
+// Block-wide maximum of N values (integer keys, see float_key); result wave-uniform.
+// One barrier; `red`: N words that hold the smallest key when the first wave gets here.
+template <int N, int kNW>
+__device__ __forceinline__ void block_max(float* v, float* red) {
+    const int lane = threadIdx.x & 63;
+    int* redi = reinterpret_cast<int*>(red);
+    int k[N];
+#pragma unroll
+    for (int h = 0; h < N; ++h) k[h] = float_key(v[h]);
+    max_step<N, 0xB1>(k);
+    max_step<N, 0x4E>(k);
+    max_step<N, 0x141>(k);
+    max_step<N, 0x140>(k);
+    max_step<N, 0x142, 0xa>(k);
+    max_step<N, 0x143, 0xc>(k);
+    // second stage: the waves' maxima meet in N words of LDS (set to the smallest key before the last barrier
+    // ahead of this call) through one atomic per wave and value
+    if (lane == 63) {   // the last lane holds the wave's maxima
+#pragma unroll
+        for (int h = 0; h < N; ++h) __hip_atomic_fetch_max(redi + h, k[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < N; ++h) v[h] = key_float(__builtin_amdgcn_readfirstlane(redi[h]));
+}
+
+// Unit decomposition of a 1-D grid.  Consecutive work ids share packed codes
+// (head groups of one kv-head), so when the grid is a multiple of the 8 XCDs
+// the hardware's round-robin placement is undone to keep them on one L2.
+__device__ __forceinline__ int virtual_block_id() {
+    const int n = gridDim.x;
+    const int l = blockIdx.x;
+    if ((n & 7) == 0) return (l & 7) * (n >> 3) + (l >> 3);
+    return l;
+}
+
+// Two-element dot product with fp32 accumulation on raw 16-bit pairs.
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+template <typename DT> __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c);
+template <> __device__ __forceinline__ float dot2<BF16>(uint32_t a, uint32_t b, float c) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
+}
+template <> __device__ __forceinline__ float dot2<FP16>(uint32_t a, uint32_t b, float c) {
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, a), __builtin_bit_cast(f16x2_t, b), c, false);
+}
+
+template <int N> struct alignas(N * 4) Words { uint32_t w[N]; };
+
+// N dwords at an absolute LDS byte address (N-dword aligned): one ds_read of that width.
+template <int N> __device__ __forceinline__ Words<N> lds_words(uint32_t addr) {
+    typedef uint32_t VT __attribute__((ext_vector_type(N)));
+    const VT v = *(const __attribute__((address_space(3))) VT*)(static_cast<uintptr_t>(addr));
+    Words<N> r;
+#pragma unroll
+    for (int k = 0; k < N; ++k) r.w[k] = v[k];
+    return r;
+}
+
+// N floats at an absolute LDS byte address.
+template <int N> __device__ __forceinline__ Vec<N> lds_floats(uint32_t addr) {
+    typedef float VT __attribute__((ext_vector_type(N)));
+    const VT v = *(const __attribute__((address_space(3))) VT*)(static_cast<uintptr_t>(addr));
+    Vec<N> r;
+#pragma unroll
+    for (int k = 0; k < N; ++k) r.v[k] = v[k];
+    return r;
+}
+
+// A float handed from one workgroup to another inside a launch: device-scope atomic store.
+__device__ __forceinline__ void publish(float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// One more arrival at an epoch-tagged counter; returns the arrivals of this epoch including this one.
+// Measured on this device: an atomic read-modify-write is executed at the memory side whatever scope it names
+// (about 2 us a round trip, those on one address one after the other), so such counters are for counting once
+// per workgroup, never for polling.
+// peek64: the current value of a 64-bit word as the memory side holds it, a compare-and-swap of 0 for 0.  (Not a
+// read-modify-write that changes nothing, such as OR 0: the compiler turns those into plain loads, which a
+// compute unit's own cache may answer with what it read earlier.)
+template <int SCOPE>
+__device__ __forceinline__ unsigned long long peek64(unsigned long long* c) {
+    unsigned long long v = 0ull;
+    __hip_atomic_compare_exchange_strong(c, &v, 0ull, __ATOMIC_RELAXED, __ATOMIC_RELAXED, SCOPE);
+    return v;
+}
+
+template <int SCOPE>
+__device__ __forceinline__ uint32_t arrive(unsigned long long* c, uint32_t epoch) {
+    unsigned long long old = peek64<SCOPE>(c);
+    for (;;) {   // every failed exchange is another workgroup's success: at most as many rounds as workgroups
+        const unsigned long long want = (static_cast<uint32_t>(old >> 32) == epoch)
+                                            ? old + 1 : ((static_cast<unsigned long long>(epoch) << 32) | 1u);
+        if (__hip_atomic_compare_exchange_strong(c, &old, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED, SCOPE))
+            return static_cast<uint32_t>(want);
+    }
+}
+
+// The single-launch chunked step's records and arrival counter of one unit back to empty: by the unit's last
+// workgroup, once every other one is past both.
+template <int HPB, int NT>
+__device__ __forceinline__ void clear_handover(const DecodeGeom& g, int64_t unit, int tid) {
+    for (int i = tid; i < HPB * g.nsplit * 2; i += NT)
+        __hip_atomic_store(g.rec + unit * HPB * g.nsplit * 2 + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) __hip_atomic_store(g.done64 + unit, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ uint32_t pack_f16(float a, float b) {
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    const f32x2_t v = {a, b};
+    const f16x2_t h = __builtin_convertvector(v, f16x2_t);   // one packed conversion, round to nearest even
+    return __builtin_bit_cast(uint32_t, h);
+}
+
+// ---- the step on the matrix cores (MX) --------------------------------------------------------------
+// The codes are small integers, so both contractions run exactly on 8-bit integer MFMAs (16 x 16 x 64): what is not
+// an integer - q.s_k, and the softmax weights - is put on a 32-bit fixed-point grid of its own maximum and split into
+// four signed byte digits.  16 rows of a tile are then four heads times four digits, the columns are tokens (logits)
+// or byte columns of the packed V rows (sums), and a lane of the result holds the four digits' sums of one head:
+// exact integers, put together in fp32.  A byte of packed codes is masked in place - one AND per 4 codes, bit i
+// counts 2^i (the sign bit -2^7), which the fixed-point operand (logits) or the closing fold (sums) takes back.
+// Measured, us per step, look-up form before and this one: batch 64 x 3 328 + 128, 1 bit 26.4 -> 19.4, 2 bits 47.8 -> 28.2;
+// batch 256 x 3 328 88 -> 55 (49 % of the rate of a large copy); 16 x 9 984, six heads 38.3 -> 23.5; 8 x 32 768 in
+// chunks 35.8 -> 29.0; batch 1 x 1 024 7.7 -> 6.4.  A 64-token tile of four heads takes about 140 vector instructions
+// (1 500 before) and 16 MFMAs; what bounds a launch now is the latency of its phases, then the memory.
+// Error against 64 bits: the grid's 2^-31 (2^-25 of the largest q.s_k at the top bit) and the fp32 roundings; the
+// look-up form added fp32 partial sums on the K side and held the weights as fp16 on the V side (fp16 outputs: 2.0e-4 away
+// from 64 bits here, which is their own rounding, 7e-4 to 1.3e-3 there).
+typedef int I4 __attribute__((ext_vector_type(4)));
+typedef int I2 __attribute__((ext_vector_type(2)));
+
+// four signed byte digits of x, |x| < 2^31 - 2^23 (digit 0 in the lowest byte)
+__device__ __forceinline__ uint32_t byte_digits(int x) {
+    return (static_cast<uint32_t>(x) + 0x00808080u) ^ 0x00808080u;
+}
+
+// One channel of one head of q.s_k into the K contraction's left operand: row (head, digit), in the byte that meets
+// the channel's code.  A wave holds one half of a head, the other half's values come along for the common scale and
+// the zero-point sum.  scale: [head][2] = (value of one grid step, zero-point sum).
+template <int BITS>
+__device__ __forceinline__ void matrix_query(float qs, float qsz, float qv2, float s2, float z2, int h, int d,
+                                             unsigned char* regA, float* scale) {
+    const float qs2 = qv2 * s2;
+    const int top = wave_max_key(max(__builtin_bit_cast(int, qs) & 0x7fffffff, __builtin_bit_cast(int, qs2) & 0x7fffffff));
+    const float zs = wave_sum(qsz + qs2 * z2);
+    // the largest value lies in [2^(e-1), 2^e); a head that is all but zero keeps a grid of 2^-90
+    const int e = max((top >> 23) - 126, -60);
+    // code field -> operand byte: 1 bit: the field is the bit, weight 2^i; 2 bits: fields 0..2 in place, field 3 moved
+    // down onto field 2 (a code in the sign bit would not be linear)
+    const int byte = BITS == 1 ? d >> 3 : d >> 2;                  // byte of the packed row
+    const int f = BITS == 1 ? 7 - (d & 7) : 3 - (d & 3);           // field of the byte, lowest first
+    const int sh = BITS == 1 ? f : 2 * min(f, 2);
+    float x = qs * __builtin_bit_cast(float, (30 - e + 127) << 23) * __builtin_bit_cast(float, (127 - sh) << 23);
+    if (BITS == 1 && f == 7) x = -x;
+    const uint32_t dg = byte_digits(__float2int_rn(x));
+    const int kg = (byte >> 2) & 3, b = byte & 3, i = BITS == 1 ? f : (byte >> 4) * 4 + f;   // operand dword i = 0 .. 7
+    unsigned char* o = regA + ((i >> 2) * 64 + kg * 16 + 4 * h) * 16 + (i & 3) * 4 + b;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) o[16 * p] = static_cast<unsigned char>(dg >> (8 * p));
+    if ((d & 127) == 0) {
+        // an infinity or a NaN anywhere in the head makes all its logits NaN, as a floating-point sum would
+        scale[2 * h] = top >= 0x7f800000 ? __builtin_nanf("") : __builtin_bit_cast(float, (e - 30 + 127) << 23);
+        scale[2 * h + 1] = zs;
+    }
+}
+
+// the right operand's dwords of one word of packed codes
+template <int BITS> __device__ __forceinline__ void code_fields(uint32_t w, int* o) {
+    if constexpr (BITS == 1) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = static_cast<int>(w & (0x01010101u << i));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) o[i] = static_cast<int>(w & (0x03030303u << (2 * i)));
+        o[3] = static_cast<int>((w >> 2) & 0x30303030u);
+    }
+}
+
+// Logits of 64 tokens, one row per lane: a 4 x 4 exchange of dwords between the four groups of 16 lanes gives lane
+// (x, k) dword k of the tokens x, 16 + x, 32 + x, 48 + x - the right operand of four 16-token tiles.
+template <int BITS>
+__device__ __forceinline__ void matrix_logits(const uint4* c, I4 a0, I4 a1, float inv, float zs, float* out) {
+    uint32_t w[BITS][4];
+#pragma unroll
+    for (int s = 0; s < BITS; ++s) {
+        const auto x01 = __builtin_amdgcn_permlane16_swap(c[s].x, c[s].y, false, false);
+        const auto x23 = __builtin_amdgcn_permlane16_swap(c[s].z, c[s].w, false, false);
+        const auto y02 = __builtin_amdgcn_permlane32_swap(x01[0], x23[0], false, false);
+        const auto y13 = __builtin_amdgcn_permlane32_swap(x01[1], x23[1], false, false);
+        w[s][0] = y02[0]; w[s][2] = y02[1]; w[s][1] = y13[0]; w[s][3] = y13[1];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        int f[8];
+        code_fields<BITS>(w[0][j], f);
+        if constexpr (BITS == 2) code_fields<BITS>(w[1][j], f + 4);
+        I4 acc = {0, 0, 0, 0};
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, I4{f[0], f[1], f[2], f[3]}, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, I4{f[4], f[5], f[6], f[7]}, acc, 0, 0, 0);
+        // digit sums are at most 128 * 128 * 128 in size: two of them meet as an integer
+        const float l = static_cast<float>(acc[0] + (acc[1] << 8)), u = static_cast<float>(acc[2] + (acc[3] << 8));
+        out[j] = __builtin_fmaf(__builtin_fmaf(u, 65536.f, l), inv, -zs);
+    }
+}
+
+// Eight rows of one byte column per lane: of a [row][16 bytes] tile in LDS, lane x of 16 gets byte x of eight rows
+__device__ __forceinline__ I2 column8(const unsigned char* p) {
+    return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) I2*)(p));
+}
+
+// Weighted code sums of 64 tokens.  The weights (lane: head lane / 16, tokens 16 j + x) go through the wave's LDS tile
+// as [token][head] words, i.e. rows of 16 digit bytes, the packed V rows as they are, [token][16 bytes]; both come
+// back by columns, 16 tokens of one column per lane.
+template <int BITS>
+__device__ __forceinline__ void matrix_values(unsigned char* tile, const float* e, const U4* v, I4* acc) {
+    const int lane = threadIdx.x & 63, x = lane & 15, k = lane >> 4;
+#pragma unroll
+    for (int s = 0; s < BITS; ++s) *reinterpret_cast<U4*>(tile + (1 + s) * 1024 + lane * 16) = v[s];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        // (a weight is at most 1 up to rounding; the cap keeps the digits in range whatever the rounding does)
+        const float xs = fminf(e[j] * 1073741824.f, 2130706432.f);
+        *reinterpret_cast<uint32_t*>(tile + (16 * j + x) * 16 + 4 * k) = byte_digits(__float2int_rn(xs));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const unsigned char* col = tile + (16 * k + (x >> 1)) * 16 + (x & 1) * 8;
+    const I2 e0 = column8(col), e1 = column8(col + 128);
+    const I4 a = {e0[0], e0[1], e1[0], e1[1]};
+#pragma unroll
+    for (int s = 0; s < BITS; ++s) {
+        const I2 v0 = column8(col + (1 + s) * 1024), v1 = column8(col + (1 + s) * 1024 + 128);
+        const int w[4] = {v0[0], v0[1], v1[0], v1[1]};
+        int f[4][8];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) code_fields<BITS>(static_cast<uint32_t>(w[r]), f[r]);
+        constexpr int NF = 8 / BITS;
+#pragma unroll
+        for (int i = 0; i < NF; ++i)
+            acc[s * NF + i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, I4{f[0][i], f[1][i], f[2][i], f[3][i]}, acc[s * NF + i], 0, 0, 0);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// the lane's sums (one head, byte column x) as floats in channel order
+template <int BITS> __device__ __forceinline__ void matrix_fold(const I4* acc, float* out, int x) {
+    constexpr int NF = 8 / BITS;
+#pragma unroll
+    for (int s = 0; s < BITS; ++s) {
+        Vec<4> o[NF / 4];
+#pragma unroll
+        for (int i = 0; i < NF; ++i) {
+            const I4 a = acc[s * NF + i];
+            float r = static_cast<float>(a[3]);
+#pragma unroll
+            for (int p = 2; p >= 0; --p) r = __builtin_fmaf(r, 256.f, static_cast<float>(a[p]));
+            const int sh = BITS == 1 ? i : 2 * cmin(i, 2);
+            const float unit = (BITS == 1 && i == 7 ? -1.f : 1.f) / (1073741824.f * static_cast<float>(1 << sh));
+            o[(NF - 1 - i) / 4].v[(NF - 1 - i) % 4] = r * unit;   // first channel of a byte in its top bits
+        }
+#pragma unroll
+        for (int q = 0; q < NF / 4; ++q) *reinterpret_cast<Vec<4>*>(out + (16 * s + x) * NF + 4 * q) = o[q];
+    }
+}
+
+// CHUNKED: the launch is one of the two of a chunked step (the min/max launch always is); a single launch carries
+// none of their code.  EXTRAS: an additive mask or a residual row count read from device memory may be present; a
+// call with neither runs an instantiation without their code (32.6-32.8 against 33.5-34.0 us at the benchmark shape:
+// the kernel sits at the register limit of its occupancy, and code that never runs still costs registers).
+// NH: query heads a unit serves, at most HPB.  Tables, slots and partials are laid out HPB heads wide either way
+// (16-byte entries at HPB = 4); with NH = 3 the fourth lane of every entry is dead and the arithmetic on it is
+// left out - six query heads per kv-head (InternLM2-20B) make two exact units of three instead of two units of
+// four that carry two padding heads between them.
+template <int BITS, int HPB, typename DT, bool MINMAX_ONLY, bool VTOK = false, int NT = 1024, int REGL = 0,
+          bool CHUNKED = MINMAX_ONLY, bool EXTRAS = !MINMAX_ONLY, int NH = HPB, bool MX = false>
+// (four waves per SIMD - at most 128 VGPRs - for either workgroup size: two 512-thread workgroups per compute
+// unit are only resident together within that)
+__global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
+    static_assert(!MX || (!VTOK && REGL > 0), "matrix-core form: per-channel values, logits in registers");
+    using L = Lay<BITS, HPB, VTOK, NT, REGL, MX>;
+    using V = Vec<HPB>;
+    constexpr int NB = L::NB;
+    constexpr int kNT = L::kNT, kNW = L::kNW, kResTile = L::kResTile;
+    extern __shared__ __attribute__((aligned(256))) unsigned char smem[];
+    const int reg_a = L::region_a(g.cap);
+    unsigned char* regA = smem;
+    float* fx = reinterpret_cast<float*>(smem + reg_a);
+    unsigned char* slots = L::INA ? smem + L::slots_in_a(g.cap) : smem + reg_a + L::FIXED;   // one slot per token of the chunk
+    auto slot = [&](int t) { return slots + t * L::SLOT; };
+    float* wbit = fx + L::F_WBIT;
+    float* qsz = fx + L::F_QSZ;
+    float* red = fx + L::F_RED;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wv = tid >> 6;
+    const int G = g.G;
+    // Wave priorities of the paired launch (two 512-thread workgroups per compute unit, all of them
+    // resident from the first cycle).  Left to the hardware's own arbitration the workgroup that was
+    // dispatched first gets most of the issue slots: it ends after about 56 K cycles and the other one
+    // after 77 K, the last 20 K alone on the unit with too few waves to hide its own latencies.  With the
+    // short, latency-bound phases (set-up, table build, reductions, staging, exp) above the throughput
+    // phases, the first workgroup ahead in the K look-ups and the second ahead in the packed-V loop,
+    // both end together (measured at the benchmark shape: 36.0 -> 33.8 us, same results).  Launches with
+    // more workgroups than fit at once start their later workgroups as earlier ones end, which staggers
+    // them by itself; there the priorities are left alone (with them: 66 -> 84 us at batch 128).
+    // `second`: the workgroup that shares its unit with an older one (workgroups are handed out unit by
+    // unit, g.ncu at a time).
+    const bool prio_on = NT == 512 && g.ncu > 0;
+    const bool second = prio_on && blockIdx.x >= static_cast<unsigned>(g.ncu);
+    auto phase_priority = [&](auto phase_c) {
+        constexpr int PH = decltype(phase_c)::value;   // 0 set-up and tables, 1 K look-ups, 2 min/max .. exp, 3 packed V, 4 folds, window, merge
+        if constexpr (NT == 512) {
+            if (prio_on) {
+                if constexpr (PH == 0 || PH == 2) __builtin_amdgcn_s_setprio(2);
+                else if constexpr (PH == 1) { if (second) __builtin_amdgcn_s_setprio(0); else __builtin_amdgcn_s_setprio(1); }
+                else if constexpr (PH == 3) { if (second) __builtin_amdgcn_s_setprio(2); else __builtin_amdgcn_s_setprio(1); }
+                else __builtin_amdgcn_s_setprio(0);
+            }
+        }
+    };
+    // (unconditional at entry - with no later change every wave simply runs at this priority - so that no branch
+    // on a kernel argument stands between the wave's start and the loads of the other arguments: all of them are
+    // then requested in one go instead of in two round trips)
+    if constexpr (NT == 512) __builtin_amdgcn_s_setprio(2);
+
+    uint32_t vb = static_cast<uint32_t>(virtual_block_id());
+    uint32_t qn = g.d_ng.quot(vb);
+    const int hg = static_cast<int>(vb - qn * g.d_ng.div); vb = qn;
+    qn = g.d_nx.quot(vb);
+    const int split = static_cast<int>(vb - qn * g.d_nx.div); vb = qn;
+    qn = g.d_hkv.quot(vb);
+    const int hkv = static_cast<int>(vb - qn * g.d_hkv.div);
+    const int b = static_cast<int>(qn);
+    static_assert(NH >= 1 && NH <= HPB, "heads per unit");
+    const int hq0 = hkv * G + hg * NH;
+    const int nh = min(NH, G - hg * NH);   // query heads of this unit; the rest of its NH heads are padding
+    const int64_t bh = static_cast<int64_t>(b) * g.Hkv + hkv;
+
+    const bool img_unit = split < g.nsplit && g.T > 0;
+    const int R = (EXTRAS && g.r_dev) ? min(*g.r_dev, g.R) : g.R;   // rows in the residual window
+    const bool do_res = !MINMAX_ONLY && R > 0 && (!CHUNKED || split == g.nsplit);
+    const int t0 = img_unit ? split * g.chunk : 0;
+    const int n = img_unit ? min(g.T, t0 + g.chunk) - t0 : 0;
+    const int npad = (n + L::TPW - 1) / L::TPW * L::TPW;
+    const float inv_sqrt_d = 0.08838834764831845f;  // 1/sqrt(128)
+
+    // ---- entry: the few elements phase 0 needs are requested first; the packed K rows follow
+    // phase 0, packed V rows and the residual tile later still (see the file header).
+    // Loads are unconditional with clamped (always valid) addresses: no divergent
+    // control flow around them, so the compiler can wait on exactly the counter value
+    // each consumer needs.
+    // A unit without packed tokens or without residual rows aims the unused streams
+    // at q (always mapped, at least 256 bytes) and never looks at what comes back.
+    const bool has_img = n > 0;
+    // chunked launch with a logits buffer: the min/max launch leaves this chunk's logits there and the main
+    // launch takes them from there - no packed K rows, no table, no look-ups of its own
+    const int64_t unit = bh * static_cast<int64_t>(g.d_ng.div) + hg;
+    V* gl = reinterpret_cast<V*>(g.lgt) + (unit * g.T + t0);
+    const bool from_gl = !MINMAX_ONLY && !MX && CHUNKED && g.lgt != nullptr && has_img;
+    const bool k_rows = has_img && !from_gl;
+    uint32_t q_raw, s_raw, z_raw;
+    constexpr bool kVSep = (HPB * kD > kNT - kD);
+    uint32_t vs_raw = 0, vz_raw = 0;
+    uint32_t q_raw2 = 0, s_raw2 = 0, z_raw2 = 0;   // MX: the head's other half, for a wave that needs the whole head
+    {
+        const int h = min(min(tid / kD, HPB - 1), nh - 1), d = tid % kD;   // a padding head repeats the last real one
+        const uint16_t* qp = static_cast<const uint16_t*>(g.q) + (static_cast<int64_t>(b) * g.Hq + hq0) * kD;
+        q_raw = qp[h * kD + d];
+        // the last kD threads fetch the value statistics, unless they are q threads as well
+        // (then the first kD threads fetch them with two loads of their own, below)
+        const bool vstat = tid >= kNT - kD && !kVSep;
+        const uint16_t* sp = has_img ? static_cast<const uint16_t*>((vstat && !VTOK) ? g.vs : g.ks) + bh * kD : qp;
+        const uint16_t* zp = has_img ? static_cast<const uint16_t*>((vstat && !VTOK) ? g.vz : g.kz) + bh * kD : qp;
+        s_raw = sp[d];
+        z_raw = zp[d];
+        if constexpr (MX) {
+            q_raw2 = qp[h * kD + (d ^ 64)];
+            s_raw2 = sp[d ^ 64];
+            z_raw2 = zp[d ^ 64];
+        }
+        if constexpr (kVSep && !VTOK) {
+            vs_raw = (has_img ? static_cast<const uint16_t*>(g.vs) + bh * kD : qp)[d];
+            vz_raw = (has_img ? static_cast<const uint16_t*>(g.vz) + bh * kD : qp)[d];
+        }
+    }
+    const int64_t code_off = has_img ? (bh * g.T + t0) * NB : 0;   // one offset for both code streams
+    const uint4* ckp = reinterpret_cast<const uint4*>(k_rows ? g.ck + code_off : static_cast<const uint8_t*>(g.q));
+    const uint4* cvp = reinterpret_cast<const uint4*>((has_img ? g.cv : static_cast<const uint8_t*>(g.q)) + code_off);
+    const U4* cvp4 = reinterpret_cast<const U4*>(cvp);
+    const int last_u = has_img ? n * NB / 16 - 1 : 0;   // last valid 16-byte unit of either stream
+    const int last_uk = k_rows ? last_u : 0;
+    const int last_row = k_rows ? n - 1 : 0;
+    // residual tile: K slice (row = tid / LPR, 128 / LPR elements); V: a wave owns RPW rows of the tile and a
+    // lane one channel pair of each of them, so the value products need no fold inside the wave
+    constexpr int LPR = L::LPR, NKP = L::NKP, RPW = L::RPW;
+    const int lq = tid % LPR, krow = tid / LPR;
+    const int wvr = __builtin_amdgcn_readfirstlane(wv);   // wave-uniform: scalar row arithmetic
+    // (the strides are read where the other kernel arguments are, not behind the branch that needs them: one
+    // round trip to the argument block instead of one more)
+    // (a single launch: every workgroup has a window; of a chunked launch only the residual units do)
+    int64_t arg_rs_b = g.rs_b, arg_rs_h = g.rs_h, arg_rs_r = g.rs_r;
+    if constexpr (!CHUNKED) asm volatile("" : "+s"(arg_rs_b), "+s"(arg_rs_h), "+s"(arg_rs_r));
+    const int64_t res_off = do_res ? b * arg_rs_b + hkv * arg_rs_h : 0;   // one offset for both windows
+    const uint16_t* kb = static_cast<const uint16_t*>(do_res ? g.kres : g.q) + res_off;
+    const uint16_t* vbp = static_cast<const uint16_t*>(do_res ? g.vres : g.q) + res_off;
+    const int last_r = do_res ? R - 1 : 0;
+    const int64_t rs_r = do_res ? arg_rs_r : 0;
+    uint4 rk[NKP];
+    uint32_t rv[RPW];
+    auto load_res_k = [&](int r0, uint4* k2) {   // rows past R re-read row R-1 (their logit is masked)
+        const uint16_t* kp = kb + min(r0 + krow, last_r) * rs_r + lq * 8;
+#pragma unroll
+        for (int i = 0; i < NKP; ++i) k2[i] = *reinterpret_cast<const uint4*>(kp + i * (LPR * 8));   // piece i * LPR + lq
+    };
+    auto load_res_v = [&](int r0, uint32_t* v8) {   // rows past R re-read row R-1 (their weight is 0)
+#pragma unroll
+        for (int i = 0; i < RPW; ++i) {
+            const int r2 = min(r0 + wvr * RPW + i, last_r);
+            v8[i] = *reinterpret_cast<const uint32_t*>(vbp + r2 * rs_r + 2 * lane);
+        }
+    };
+
+    CQ_PHASE(1);   // prologue, requests of q and the statistics
+    // ---- phase 0: q, per-bit weights ---------------------------------------------------
+    if (tid < HPB * kD) {
+        const int h = tid / kD, d = tid % kD;
+        const float qraw = Cvt<DT>::to_float(q_raw);
+        reinterpret_cast<uint16_t*>(fx + L::F_QRAW)[h * kD + d] = static_cast<uint16_t>(q_raw);
+        const float qv = qraw * inv_sqrt_d;
+        if (n > 0) {
+            const float s = Cvt<DT>::to_float(s_raw);
+            const float z = Cvt<DT>::to_float(z_raw);
+            const float qs = qv * s;
+            if constexpr (MX) {
+                matrix_query<BITS>(qs, qs * z, Cvt<DT>::to_float(q_raw2) * inv_sqrt_d, Cvt<DT>::to_float(s_raw2),
+                                   Cvt<DT>::to_float(z_raw2), h, d, regA, qsz);
+            } else {
+            // zero-point term of the byte position: sum of q s z over the channels of one byte
+            // (consecutive lanes), kept [byte position][head]
+            constexpr int cpb0 = 8 / BITS;
+            const float zsum = (cpb0 == 8) ? oct_reduce(qs * z, OpSum(), 0.f) : quad_reduce(qs * z, OpSum(), 0.f);
+            if (d % cpb0 == 0) qsz[(d / cpb0) * HPB + h] = zsum;
+            if constexpr (BITS == 1) {
+                wbit[((7 - (d & 7)) * NB + (d >> 3)) * HPB + h] = qs;   // [bit][byte position][head]
+            } else {
+                const int sh = 6 - 2 * (d & 3);
+                wbit[(sh * NB + (d >> 2)) * HPB + h] = qs;
+                wbit[((sh + 1) * NB + (d >> 2)) * HPB + h] = 2.0f * qs;
+            }
+            }
+        }
+    }
+    if constexpr (kVSep) {
+        if (!VTOK && n > 0 && tid < kD) {
+            fx[L::F_VSZ + tid] = Cvt<DT>::to_float(vs_raw);
+            fx[L::F_VSZ + kD + tid] = Cvt<DT>::to_float(vz_raw);
+        }
+    } else if (!VTOK && n > 0 && tid >= kNT - kD) {
+        const int d = tid - (kNT - kD);
+        fx[L::F_VSZ + d] = Cvt<DT>::to_float(s_raw);
+        fx[L::F_VSZ + kD + d] = Cvt<DT>::to_float(z_raw);
+    }
+    if (tid < 3 * HPB) reinterpret_cast<int*>(red)[tid] = static_cast<int>(0x80000000u);   // block_max's meeting words
+    // The packed K rows are requested only now: a wave that has to queue 64 KB of requests
+    // first gets to phase 0 thousands of cycles later, and the table build below covers
+    // their latency anyway.
+    // (requested any later - after the table build, or all but the first round - the launch is slower;
+    // requested at kernel entry, ahead of q, as well)
+    uint4 kc[L::KR][BITS];
+#pragma unroll
+    for (int r = 0; r < L::KR; ++r) {
+#pragma unroll
+        for (int i = 0; i < BITS; ++i)
+            kc[r][i] = MX ? ckp[min(tid + r * kNT, last_row) * BITS + i] : ckp[min((tid + r * kNT) * BITS + i, last_uk)];
+    }
+    // Chunked launch: the chunks' logit min / max, lane s the pair of chunk s for every head (all in flight
+    // together; they are folded across the wave where the calibration needs them), and - with a logits
+    // buffer and the logits in registers - this thread's logits.
+    struct alignas(8) MinMax { float lo, hi; };
+    MinMax mraw[HPB];
+    // REGL: the logits of this thread's tokens, round r = token tid + r * kNT
+    V lg[REGL > 0 && !MX ? REGL : 1];
+    // MX: round rd's 64 tokens of a wave start at 64 * wv + rd * kNT; lane (x, h) = (lane & 15, lane >> 4) has the
+    // logits of head h for the tokens 16 j + x of them
+    float lx[MX ? REGL : 1][4];
+    if constexpr (!MINMAX_ONLY) {
+        if (CHUNKED && has_img && !g.fused) {
+#pragma unroll
+            for (int h = 0; h < HPB; ++h) {
+                const MinMax* p = reinterpret_cast<const MinMax*>(g.mm) +
+                                  (static_cast<int64_t>(b) * g.Hq + hq0 + min(h, nh - 1)) * g.nsplit;
+                mraw[h] = p[min(lane, g.nsplit - 1)];
+            }
+        }
+        if constexpr (REGL > 0 && !MX) {
+            if (from_gl) {
+#pragma unroll
+                for (int rd = 0; rd < REGL; ++rd) lg[rd] = gl[min(tid + rd * kNT, n - 1)];
+            }
+        }
+    }
+    __syncthreads();
+
+    float* stat = fx + L::F_STAT;   // [alpha | m_res | l_res | m_img | l_img][HPB]
+    float o_res = 0.f;
+    float mn[HPB], mx[HPB];
+#pragma unroll
+    for (int h = 0; h < HPB; ++h) { mn[h] = h < NH ? INFINITY : 0.f; mx[h] = h < NH ? -INFINITY : 0.f; }
+    // logits (later: calibrated, masked logits) of a token: in its slot, or in the thread's registers
+    auto load_logits = [&](int rd, int tt) {
+        if constexpr (REGL > 0 && !MX) return lg[rd];
+        else return *reinterpret_cast<const V*>(slot(tt));
+    };
+    auto store_logits = [&](int rd, int tt, const V& w) {
+        if constexpr (REGL > 0 && !MX) lg[rd] = w;
+        else *reinterpret_cast<V*>(slot(tt)) = w;
+    };
+    // f(round, token) for the thread's tokens below lim; with REGL the rounds are unrolled so that
+    // lg[] is indexed by constants
+    auto for_my_tokens = [&](int lim, auto&& f) {
+        if constexpr (REGL > 0) {
+#pragma unroll
+            for (int rd = 0; rd < REGL; ++rd) {
+                const int tt = tid + rd * kNT;
+                if (tt < lim) f(rd, tt);
+            }
+        } else {
+            for (int tt = tid; tt < lim; tt += kNT) f(0, tt);
+        }
+    };
+    // First block of packed V rows: half of it is requested here, behind the packed K rows, the
+    // rest as the K registers free up, so it has arrived when the logits are done.
+    constexpr int kVF = MX ? kMatrixV : kPF;   // 16-byte pieces of packed V rows in flight per thread
+    U4 vc[kVF];
+    auto request_v = [&](int r) { vc[r] = cvp4[min((tid + (r / BITS) * kNT) * BITS + r % BITS, last_u)]; };
+    constexpr int kVEarly = MX ? kMatrixE : kPF / 2;
+    if constexpr (!MINMAX_ONLY) {
+#pragma unroll
+        for (int r = 0; r < kVEarly; ++r) request_v(r);
+    }
+
+    if (from_gl) {
+        // (the look-up rounds, which request the rest of the first packed V block as they go, do not run)
+#pragma unroll
+        for (int r = kVEarly; r < kPF; ++r) request_v(r);
+        if constexpr (REGL == 0) for_my_tokens(n, [&](int rd, int tt) { store_logits(rd, tt, gl[tt]); });
+    }
+    CQ_PHASE(2);   // q, per-bit weights, first packed K rows requested
+    // MX: the wave's first token, and the head whose results this lane holds (lanes beyond the unit's heads repeat
+    // the last one)
+    const int wt0 = __builtin_amdgcn_readfirstlane(tid);
+    const int hl = min(lane >> 4, HPB - 1);
+    if constexpr (MX) {
+        if (k_rows) {
+            const I4* aq = reinterpret_cast<const I4*>(regA);
+            const I4 a0 = aq[lane], a1 = aq[64 + lane];
+            const float inv = qsz[2 * hl], zs = qsz[2 * hl + 1];
+            float lo = INFINITY, hi = -INFINITY;
+            phase_priority(std::integral_constant<int, 1>{});
+#pragma unroll
+            for (int rd = 0; rd < REGL; ++rd) {
+                if (wt0 + rd * kNT < n) {
+                    matrix_logits<BITS>(kc[rd % L::KR], a0, a1, inv, zs, lx[rd]);
+                    if (rd + L::KR < REGL) {
+#pragma unroll
+                        for (int i = 0; i < BITS; ++i) kc[rd % L::KR][i] = ckp[min(tid + (rd + L::KR) * kNT, last_row) * BITS + i];
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) { lo = fminf(lo, lx[rd][j]); hi = fmaxf(hi, lx[rd][j]); }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (!MINMAX_ONLY && rd < kVF - kVEarly) request_v(kVEarly + rd);   // the rest of the first packed V rows
+            }
+            phase_priority(std::integral_constant<int, 2>{});
+            // the waves' minima and maxima meet in LDS, as in block_max, from one lane per head
+            const int klo = row_max_key(float_key(-lo)), khi = row_max_key(float_key(hi));
+            int* redi = reinterpret_cast<int*>(red);
+            if ((lane & 15) == 0 && (lane >> 4) < HPB) {
+                __hip_atomic_fetch_max(redi + hl, klo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_fetch_max(redi + HPB + hl, khi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int h = 0; h < HPB; ++h) {
+                mn[h] = -key_float(__builtin_amdgcn_readfirstlane(redi[h]));
+                mx[h] = key_float(__builtin_amdgcn_readfirstlane(redi[HPB + h]));
+            }
+        }
+    } else {
+    if (k_rows) {
+        // ---- phase 2: byte table = high-nibble table + low-nibble table ----------------
+        // nibble tables: entry (j, half, v) = sum of the per-bit weights v selects; the
+        // zero-point sum of the byte position is folded into the high half.
+        V* nib = REGL > 0 ? reinterpret_cast<V*>(slots) : reinterpret_cast<V*>(fx + L::F_NIB);   // [half*16 + value][byte position]
+        V* ktab = reinterpret_cast<V*>(regA);           // [byte value][byte position]
+        if constexpr (!L::INA)
+        for (int e = tid; e < NB * 32; e += kNT) {
+            const int j = e % NB, half = (e / NB) >> 4, v = (e / NB) & 15;
+            // position-fastest: the lanes of a wave read consecutive entries
+            const V* wb = reinterpret_cast<const V*>(wbit) + half * 4 * NB + j;
+            V acc;
+            const V zs = reinterpret_cast<const V*>(qsz)[j];
+#pragma unroll
+            for (int h = 0; h < HPB; ++h) acc.v[h] = half ? -zs.v[h] : 0.f;
+#pragma unroll
+            for (int bt = 0; bt < 4; ++bt) {
+                const V w4 = wb[bt * NB];
+                const float f = static_cast<float>((v >> bt) & 1);
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) acc.v[h] += f * w4.v[h];
+            }
+            nib[e] = acc;
+        }
+        if constexpr (!L::INA) __syncthreads();
+
+        phase_priority(std::integral_constant<int, 1>{});
+        // ---- phase 3: logits of the chunk ------------------------------------------------
+        // Lane l walks the byte positions of a pass in the order k ^ (l mod NBP): in every step
+        // the lanes that the LDS serves together read NBP distinct positions of the
+        // position-fastest table, i.e. distinct banks whatever the byte values are.  The
+        // row is permuted by the same XOR once, so step k finds its byte at a fixed place.
+        // The NBP terms are added as a balanced binary tree over k; an XOR of the leaf index
+        // only swaps the two children of some tree levels, so every lane gets bit-identical
+        // logits for identical rows.
+        constexpr int NBP = L::NBP;
+        constexpr int NW32 = NBP / 4;
+        const int skew = lane % NBP;
+        // byte i of a word <- byte i ^ (skew & 3)
+        const uint32_t bsel = (0x03020100u ^ (0x01010101u * (skew & 3)));
+        uint32_t pofs[NBP];   // byte offset of position k ^ skew inside a table row
+#pragma unroll
+        for (int k = 0; k < NBP; ++k) pofs[k] = (k ^ skew) * L::ESZ;
+        const unsigned char* ktab_b = regA;
+        // With 256-byte table rows the address of a look-up is two bytes side by side, the
+        // byte value above the position offset: one byte permute builds it from the row word
+        // and a word holding four position offsets.
+        constexpr bool kPermAddr = (NBP * L::ESZ == 256);
+        uint32_t pofs4[NBP / 4];
+#pragma unroll
+        for (int i = 0; i < NBP / 4; ++i)
+            pofs4[i] = pofs[4 * i] | (pofs[4 * i + 1] << 8) | (pofs[4 * i + 2] << 16) | (pofs[4 * i + 3] << 24);
+        // c: the L::PCS 16-byte pieces of the row that pass P looks at; rd: the token's round (REGL)
+        // kLateMM (one table pass, logits in registers): a wave works out a round's logits for all its lanes as soon
+        // as its first lane has a token - the lanes past the chunk's end hold a copy of its last row (clamped
+        // request) and get that token's logits - so the min / max can be taken afterwards over the registers, two
+        // rounds per instruction, with no lane left out.
+        constexpr bool kLateMM = L::KPASS == 1 && REGL > 0 && !MINMAX_ONLY;
+        // a table entry: the NH live floats of it (12 bytes at three heads)
+        auto lds_entry = [&](uint32_t addr) {
+            V r;
+            if constexpr (NH == HPB) {
+                r = lds_floats<HPB>(addr);
+            } else {
+                typedef float VT __attribute__((ext_vector_type(NH)));
+                const VT v = *(const __attribute__((address_space(3))) VT*)(static_cast<uintptr_t>(addr));
+#pragma unroll
+                for (int k = 0; k < HPB; ++k) r.v[k] = k < NH ? v[k < NH ? k : 0] : 0.f;
+            }
+            return r;
+        };
+        auto token_logits = [&](auto pass_c, int rd, int tt, const uint4* c) {
+            constexpr int P = decltype(pass_c)::value;
+            if (kLateMM ? (__builtin_amdgcn_readfirstlane(tt) < n) : (tt < n)) {
+                constexpr int WO = (P * L::WPP) % 4;   // the pass's first word inside its first piece
+                uint32_t w[NW32];
+#pragma unroll
+                for (int i = 0; i < NW32; ++i) {
+                    const uint4& pc = c[(WO + i) / 4];
+                    const int k4 = (WO + i) % 4;
+                    w[i] = k4 == 0 ? pc.x : k4 == 1 ? pc.y : k4 == 2 ? pc.z : pc.w;
+                }
+#pragma unroll
+                for (int st = 0; (1 << st) < NW32; ++st) {   // word i <- word i ^ (skew / 4)
+                    const bool on = ((skew >> 2) >> st) & 1;
+                    uint32_t t[NW32];
+#pragma unroll
+                    for (int i = 0; i < NW32; ++i) t[i] = w[i ^ (1 << st)];
+#pragma unroll
+                    for (int i = 0; i < NW32; ++i) w[i] = on ? t[i] : w[i];
+                }
+                uint32_t wds[NW32];
+#pragma unroll
+                for (int i = 0; i < NW32; ++i) wds[i] = __builtin_amdgcn_perm(w[i], w[i], bsel);
+                // balanced-tree sum with a small stack of partial sums (level l holds 2^l terms)
+                V part[6];
+#pragma unroll
+                for (int k = 0; k < NBP; ++k) {
+                    V cur;
+                    if constexpr (kPermAddr) {
+                        const uint32_t sel = static_cast<uint32_t>(k & 3) | (static_cast<uint32_t>(4 + (k & 3)) << 8) | 0x0c0c0000u;
+                        // The kernel's only LDS object is the dynamic array, so it starts at LDS
+                        // address 0 and the K table with it (the host checks that the kernel has no
+                        // static LDS before the first launch): the permute result is the address.
+                        cur = lds_entry(__builtin_amdgcn_perm(wds[k >> 2], pofs4[k >> 2], sel));
+                    } else {
+                        const uint32_t byte = (wds[k >> 2] >> (8 * (k & 3))) & 0xffu;
+                        cur = *reinterpret_cast<const V*>(ktab_b + byte * (NBP * L::ESZ) + pofs[k]);
+                    }
+#pragma unroll
+                    for (int l = 0; l < 6; ++l) {
+                        if ((k >> l) & 1) {
+#pragma unroll
+                            for (int h = 0; h < NH; ++h) cur.v[h] += part[l].v[h];
+                        } else {
+                            part[l] = cur;
+                            break;
+                        }
+                    }
+                    if (k == NBP - 1) part[5] = cur;
+                    // keep at most 8 look-ups in flight: bounds the registers this loop needs
+                    if ((k & 7) == 7) __builtin_amdgcn_sched_barrier(0);
+                }
+                V acc = part[5];
+                if constexpr (P > 0) {   // add the earlier pass's partial
+                    const V prev = load_logits(rd, tt);
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) acc.v[h] += prev.v[h];
+                }
+#pragma unroll
+                for (int h = NH; h < HPB; ++h) acc.v[h] = 0.f;   // dead lanes of the entry
+                if constexpr (!MINMAX_ONLY || P + 1 < L::KPASS) store_logits(rd, tt, acc);
+                if constexpr (MINMAX_ONLY && P + 1 == L::KPASS) {
+                    if (g.lgt) gl[tt] = acc;   // for the main launch
+                }
+                if constexpr (P + 1 == L::KPASS && !kLateMM) {
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) { mn[h] = fminf(mn[h], acc.v[h]); mx[h] = fmaxf(mx[h], acc.v[h]); }
+                }
+            }
+        };
+        // The min/max launch has no value rows, tables or sums to keep: with the logits in registers it also keeps
+        // the packed K rows of all its tokens there across the table passes instead of requesting, in every pass, the
+        // 16-byte piece that pass looks at (at 2 bits, four passes: 214 MB fetched for 67 MB of rows at batch 8 x
+        // 32 768 - the rows of the 512 workgroups in flight do not fit the L2s between two passes).
+        constexpr bool kKeepRows = MINMAX_ONLY && REGL > 0 && L::KPASS > 1;
+        uint4 kall[kKeepRows ? REGL : 1][BITS];
+        // Two table passes in a paired workgroup (2 bits): the first pass requests whole rows and keeps the
+        // 16-byte piece the second pass looks at in registers - requested one piece per pass, every 32-byte row
+        // would cross the memory system twice (a piece is half a row, and memory is fetched by the row or more).
+        constexpr bool kKeepHalf = !MINMAX_ONLY && L::INA && L::KPASS == 2 && BITS == 2 && !kKeepRows;
+        uint4 khalf[kKeepHalf ? REGL : 1];
+        auto k_pass = [&](auto pass_c) {
+            constexpr int P = decltype(pass_c)::value;
+            constexpr int kP0 = (P * L::WPP) / 4;   // first 16-byte piece of a row the pass looks at
+            if constexpr (L::INA) {
+                // Straight from the per-bit weights: a thread owns (position, high nibble, bit 3) and writes the
+                // eight entries of the low three bits - the part common to all eight first, then one or two adds
+                // per entry; a wave writes four whole 256-byte rows at a time.
+                static_assert(!L::INA || (NBP == 16 && kNT == 512), "thread mapping of the direct table build");
+                const int pos = tid & 15, hv = (tid >> 4) & 15, b3 = tid >> 8;
+                const V* wb = reinterpret_cast<const V*>(wbit) + P * NBP + pos;
+                const V zs = reinterpret_cast<const V*>(qsz)[P * NBP + pos];
+                V base;
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) base.v[h] = -zs.v[h];
+#pragma unroll
+                for (int bt = 3; bt < 8; ++bt) {
+                    const V w4 = wb[bt * NB];
+                    const float f = static_cast<float>(bt == 3 ? b3 : (hv >> (bt - 4)) & 1);
+#pragma unroll
+                    for (int h = 0; h < HPB; ++h) base.v[h] += f * w4.v[h];
+                }
+                const V w0 = wb[0], w1 = wb[NB], w2 = wb[2 * NB];
+                V hp[2], p01;
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) {
+                    hp[0].v[h] = base.v[h];
+                    hp[1].v[h] = base.v[h] + w2.v[h];
+                    p01.v[h] = w0.v[h] + w1.v[h];
+                }
+                V* row = ktab + (hv * 16 + b3 * 8) * NBP + pos;
+#pragma unroll
+                for (int l = 0; l < 8; ++l) {
+                    V o = hp[l >> 2];
+                    if ((l & 3) != 0) {
+                        const V& ad = (l & 3) == 1 ? w0 : (l & 3) == 2 ? w1 : p01;
+#pragma unroll
+                        for (int h = 0; h < HPB; ++h) o.v[h] += ad.v[h];
+                    }
+                    row[l * NBP] = o;
+                }
+            } else {
+            // byte table of the pass's positions = high-nibble table + low-nibble table
+            for (int e = tid; e < NBP * 256; e += kNT) {
+                const int j = P * NBP + e % NBP, v = e / NBP;
+                const V hi = nib[(16 + (v >> 4)) * NB + j];
+                const V lo = nib[(v & 15) * NB + j];
+                V o;
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) o.v[h] = hi.v[h] + lo.v[h];
+                ktab[e] = o;
+            }
+            }
+            __syncthreads();
+            // One table pass, logits in registers: the rows stream through the KR row registers - when a
+            // round's row has been looked up its registers take the row of KR rounds later, so KR rounds
+            // are in flight while one is worked on and no batch of rows is waited for as a whole.
+            constexpr bool kRotate = L::KPASS == 1 && REGL > 0;
+            if constexpr (kRotate) {
+                static_assert(!kRotate || BITS == 1, "one 16-byte piece per row");
+#pragma unroll
+                for (int rd = 0; rd < REGL; ++rd) {
+                    token_logits(pass_c, rd, tid + rd * kNT, kc[rd % L::KR]);
+                    if (rd + L::KR < REGL) kc[rd % L::KR][0] = ckp[min(tid + (rd + L::KR) * kNT, last_uk)];
+                    if constexpr (!MINMAX_ONLY) {
+                        if (rd < kPF - kVEarly) request_v(kVEarly + rd);   // the rest of the first packed V block
+                    }
+                }
+                if constexpr (kLateMM) {
+                    const int t0w = __builtin_amdgcn_readfirstlane(tid);   // the wave's first token of round 0
+#pragma unroll
+                    for (int rd = 0; rd < REGL; rd += 2) {
+                        if (rd + 1 < REGL && t0w + (rd + 1) * kNT < n) {
+#pragma unroll
+                            for (int h = 0; h < NH; ++h) {
+                                mn[h] = fminf(mn[h], fminf(lg[rd].v[h], lg[rd + 1].v[h]));
+                                mx[h] = fmaxf(mx[h], fmaxf(lg[rd].v[h], lg[rd + 1].v[h]));
+                            }
+                        } else if (t0w + rd * kNT < n) {
+#pragma unroll
+                            for (int h = 0; h < NH; ++h) { mn[h] = fminf(mn[h], lg[rd].v[h]); mx[h] = fmaxf(mx[h], lg[rd].v[h]); }
+                        }
+                    }
+                }
+                return;
+            }
+            // first batch: rows already in registers; each consumed round of the last pass frees
+            // registers that take the first block of packed V rows
+            // (written out round by round with constant indices so vc stays in registers)
+#define CQ_K_ROUND(R)                                                                         \
+            if constexpr (L::KR > (R)) {                                                      \
+                token_logits(pass_c, (R), tid + (R) * kNT, kc[(R)] + kP0);                    \
+                if constexpr (!MINMAX_ONLY && P + 1 == L::KPASS) {                            \
+                    if constexpr (kVEarly + (R) * BITS < kPF) request_v(kVEarly + (R) * BITS);    \
+                    if constexpr (BITS == 2 && kVEarly + (R) * BITS + 1 < kPF) request_v(kVEarly + (R) * BITS + 1); \
+                }                                                                             \
+            }
+            CQ_K_ROUND(0)
+            CQ_K_ROUND(1)
+            CQ_K_ROUND(2)
+            CQ_K_ROUND(3)
+#undef CQ_K_ROUND
+            static_assert(L::KR <= 4, "rounds are written out up to 4");
+            uint4 kx[L::KR][L::PCS];   // rows beyond the first batch: this pass's pieces only
+            if constexpr (kKeepRows) {
+                // whole rows, requested in the first pass and kept for the later ones
+#pragma unroll
+                for (int ob = 1; ob < (REGL + L::KR - 1) / L::KR; ++ob) {
+                    const int tb = ob * kNT * L::KR;
+                    if (tb < n) {
+                        if constexpr (P == 0) {
+#pragma unroll
+                            for (int r = 0; r < L::KR; ++r) {
+                                const int tt = min(tb + tid + r * kNT, n - 1);
+#pragma unroll
+                                for (int i = 0; i < BITS; ++i)
+                                    if (ob * L::KR + r < REGL) kall[ob * L::KR + r][i] = ckp[static_cast<int64_t>(tt) * BITS + i];
+                            }
+                        }
+#pragma unroll
+                        for (int r = 0; r < L::KR; ++r)
+                            if (ob * L::KR + r < REGL)
+                                token_logits(pass_c, ob * L::KR + r, tb + tid + r * kNT, kall[ob * L::KR + r] + kP0);
+                    }
+                }
+            } else if constexpr (REGL > 0) {
+                // batches written out, so that the logits' registers are indexed by constants
+#pragma unroll
+                for (int ob = 1; ob < (REGL + L::KR - 1) / L::KR; ++ob) {
+                    const int tb = ob * kNT * L::KR;
+                    if (tb < n) {
+#pragma unroll
+                        for (int r = 0; r < L::KR; ++r) {
+                            const int tt = min(tb + tid + r * kNT, n - 1);
+                            if constexpr (kKeepHalf) {
+                                static_assert(!kKeepHalf || L::PCS == 1, "a pass looks at one piece of the row");
+                                if constexpr (P == 0) {
+                                    kx[r][0] = ckp[static_cast<int64_t>(tt) * BITS];
+                                    if (ob * L::KR + r < REGL) khalf[ob * L::KR + r] = ckp[static_cast<int64_t>(tt) * BITS + 1];
+                                } else {
+                                    if (ob * L::KR + r < REGL) kx[r][0] = khalf[ob * L::KR + r];
+                                }
+                                continue;
+                            }
+#pragma unroll
+                            for (int i = 0; i < L::PCS; ++i) kx[r][i] = ckp[static_cast<int64_t>(tt) * BITS + kP0 + i];
+                        }
+#pragma unroll
+                        for (int r = 0; r < L::KR; ++r)
+                            if (ob * L::KR + r < REGL) token_logits(pass_c, ob * L::KR + r, tb + tid + r * kNT, kx[r]);
+                    }
+                }
+            } else {
+                for (int tb = kNT * L::KR; tb < n; tb += kNT * L::KR) {
+#pragma unroll
+                    for (int r = 0; r < L::KR; ++r) {
+                        const int tt = min(tb + tid + r * kNT, n - 1);
+#pragma unroll
+                        for (int i = 0; i < L::PCS; ++i) kx[r][i] = ckp[static_cast<int64_t>(tt) * BITS + kP0 + i];
+                    }
+#pragma unroll
+                    for (int r = 0; r < L::KR; ++r) token_logits(pass_c, 0, tb + tid + r * kNT, kx[r]);
+                }
+            }
+        };
+        k_pass(std::integral_constant<int, 0>{});
+        if constexpr (L::KPASS >= 2) {
+            __syncthreads();   // every wave is done with the previous pass's table
+            k_pass(std::integral_constant<int, 1>{});
+        }
+        if constexpr (L::KPASS == 4) {
+            __syncthreads();
+            k_pass(std::integral_constant<int, 2>{});
+            __syncthreads();
+            k_pass(std::integral_constant<int, 3>{});
+        }
+    }
+    CQ_PHASE(3);   // K table and look-ups
+    phase_priority(std::integral_constant<int, 2>{});
+    if (k_rows) {   // one reduction for both: max of (-min, max)
+        float mm2[2 * HPB];
+#pragma unroll
+        for (int h = 0; h < HPB; ++h) { mm2[h] = -mn[h]; mm2[HPB + h] = mx[h]; }
+        block_max<2 * HPB, kNW>(mm2, red);
+#pragma unroll
+        for (int h = 0; h < HPB; ++h) { mn[h] = -mm2[h]; mx[h] = mm2[HPB + h]; }
+    }
+    }
+
+    CQ_PHASE(4);   // block min / max
+    if constexpr (MINMAX_ONLY) {
+#pragma unroll
+        for (int h = 0; h < HPB; ++h) {
+            if (n > 0 && tid == h && h < nh) {
+                float* o = g.mm + ((static_cast<int64_t>(b) * g.Hq + hq0 + h) * g.nsplit + split) * 2;
+                o[0] = mn[h];
+                o[1] = mx[h];
+            }
+        }
+        if (split == 0 && tid == 0) g.cnt[unit] = 0;   // the main launch counts the unit's partials from 0
+        return;
+    } else {
+        float m_img[HPB];
+#pragma unroll
+        for (int h = 0; h < HPB; ++h) m_img[h] = -INFINITY;
+        float o_img = 0.f;  // thread (h, d) = (tid / kD, tid % kD) for tid < HPB*kD
+
+        if constexpr (CHUNKED) {
+            // One launch: this chunk's min / max go out now (write-through stores, waited for, then the arrival
+            // count); the other chunks' are collected further down, after the staging of the first V block.
+            if (g.fused && k_rows && tid == 0) {
+                unsigned long long* o = g.rec + ((unit * HPB) * g.nsplit + split) * 2;
+                const unsigned long long tag = static_cast<unsigned long long>(g.epoch) << 32;
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) {
+                    __hip_atomic_store(o + h * g.nsplit * 2, tag | __float_as_uint(mn[h]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(o + h * g.nsplit * 2 + 1, tag | __float_as_uint(mx[h]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+        }
+
+        if (n > 0) {
+            // The K table is dead: stage the first block of packed V rows in its place
+            // (ordered by the barrier of block_max).  Layout: [unit of TPW tokens]
+            // [byte column][token], so the 4 bytes that the 4 tokens of a group have in one
+            // column form one dword.  A quad of lanes holds a group (tokens are
+            // lane-consecutive): per dword of its 16-byte piece the quad transposes a 4 x 4 byte
+            // block in two exchange steps (lane ^ 1, then lane ^ 2), a byte permute after each,
+            // and lane i ends up with the 4 tokens' bytes of column 4 q + i.
+            unsigned char* vst = regA + L::WTAB;
+            const int qi = lane & 3;
+            // step 1, operands (partner, own): bytes qi and qi ^ 2 of the even and of the odd lane
+            const uint32_t b0 = static_cast<uint32_t>(qi), b2 = static_cast<uint32_t>(qi ^ 2);
+            const uint32_t sel1 = (qi & 1) ? ((4 + b0) | (b0 << 8) | ((4 + b2) << 16) | (b2 << 24))
+                                           : (b0 | ((4 + b0) << 8) | (b2 << 16) | ((4 + b2) << 24));
+            // step 2, operands (partner, own): own low half and the partner's high half, pair 0 first
+            const uint32_t sel2 = (qi & 2) ? 0x01000706u : 0x07060100u;
+            auto stage_piece = [&](U4 c, int tok, int piece, bool write) {
+                const uint32_t w[4] = {c.x, c.y, c.z, c.w};
+                const int base = ((tok / L::TPW) * NB + 16 * piece + qi) * L::TPW + ((tok % L::TPW) & ~3);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t p1 = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w[q]), 0xB1, 0xf, 0xf, true));
+                    const uint32_t a = __builtin_amdgcn_perm(p1, w[q], sel1);
+                    const uint32_t p2 = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(a), 0x4E, 0xf, 0xf, true));
+                    const uint32_t t4 = __builtin_amdgcn_perm(p2, a, sel2);
+                    if (write) *reinterpret_cast<uint32_t*>(vst + base + 4 * q * L::TPW) = t4;
+                }
+            };
+            if constexpr (!MX) {
+                const int vn0 = min(L::VSUB, npad);
+#pragma unroll
+                for (int r = 0; r < kPF; ++r) {
+                    const int tok = tid + (r / BITS) * kNT;
+                    stage_piece(vc[r], tok, r % BITS, tok < vn0);
+                }
+            }
+            // The registers of a staged block take the next block's rows (clamped addresses when there is none):
+            // the block is in flight while the current one is multiplied, instead of being asked for behind a
+            // barrier when the loop gets there.  (The first residual tile requested here as well measured slower.)
+            constexpr bool kVAhead = L::INA;
+            auto request_v_block = [&](int vs0) {
+#pragma unroll
+                for (int r = 0; r < kPF; ++r) vc[r] = cvp4[min((vs0 + tid + (r / BITS) * kNT) * BITS + r % BITS, last_u)];
+            };
+
+            CQ_PHASE(5);   // staging of the first packed V block
+            // ---- phase 4: calibration + exp ---------------------------------------------
+            if constexpr (CHUNKED) {
+                if (g.fused) {
+                    // Wait until every chunk of the unit has published: the first wave polls the records, lane s
+                    // those of chunk s, a bounded number of times (workgroups that are not all resident together -
+                    // a smaller device than planned for - must not spin for ever; giving up ends this workgroup
+                    // without a result and tells the host), folds them and leaves the unit's min / max in LDS.
+                    float* fold = red + 4 * HPB;           // 2 * HPB floats, then whether the wait succeeded
+                    int* flag = reinterpret_cast<int*>(fold + 2 * HPB);
+                    if (wv == 0) {
+                        const unsigned long long* pr = g.rec + ((unit * HPB) * g.nsplit + min(lane, g.nsplit - 1)) * 2;
+                        float mm2[2 * HPB];
+                        bool ok = false;
+                        for (int it = 0; it < g.spin_limit && !ok; ++it) {
+                            bool valid = true;
+#pragma unroll
+                            for (int h = 0; h < HPB; ++h) {
+                                const unsigned long long lo = __hip_atomic_load(pr + h * g.nsplit * 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                const unsigned long long hi = __hip_atomic_load(pr + h * g.nsplit * 2 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                valid = valid && static_cast<uint32_t>(lo >> 32) == g.epoch && static_cast<uint32_t>(hi >> 32) == g.epoch;
+                                mm2[h] = -__uint_as_float(static_cast<uint32_t>(lo));
+                                mm2[HPB + h] = __uint_as_float(static_cast<uint32_t>(hi));
+                            }
+                            ok = __builtin_amdgcn_ballot_w64(!valid) == 0;
+                            if (!ok) __builtin_amdgcn_s_sleep(2);
+                        }
+                        wave_reduce_n<2 * HPB>(mm2, OpMax(), -INFINITY);
+                        if (lane == 0) {
+#pragma unroll
+                            for (int i = 0; i < 2 * HPB; ++i) fold[i] = mm2[i];
+                            *flag = ok ? 1 : 0;
+                            if (!ok && g.status) __hip_atomic_store(g.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        }
+                    }
+                    __syncthreads();
+                    if (!*flag) {
+                        // Given up: no result from this workgroup, but it is still counted, so that the unit's
+                        // last workgroup - this one or another - leaves the records and the counter empty and a
+                        // replay of this very launch (same epoch) does not take this launch's records for its own.
+                        int* last = reinterpret_cast<int*>(red);
+                        if (tid == 0) *last = arrive<__HIP_MEMORY_SCOPE_AGENT>(g.done64 + unit, g.epoch) == static_cast<uint32_t>(g.nx);
+                        __syncthreads();
+                        if (*last) clear_handover<HPB, kNT>(g, unit, tid);
+                        return;
+                    }
+#pragma unroll
+                    for (int h = 0; h < HPB; ++h) { mn[h] = -fold[h]; mx[h] = fold[HPB + h]; }
+                } else {
+                // one fold for both: max of (-min, max) over the chunks
+                float mm2[2 * HPB];
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) {
+                    mm2[h] = -mraw[h].lo;
+                    mm2[HPB + h] = mraw[h].hi;
+                    const MinMax* p = reinterpret_cast<const MinMax*>(g.mm) +
+                                      (static_cast<int64_t>(b) * g.Hq + hq0 + min(h, nh - 1)) * g.nsplit;
+                    for (int s = lane + 64; s < g.nsplit; s += 64) {   // (more than 64 chunks)
+                        const MinMax v = p[s];
+                        mm2[h] = fmaxf(mm2[h], -v.lo);
+                        mm2[HPB + h] = fmaxf(mm2[HPB + h], v.hi);
+                    }
+                }
+                wave_reduce_n<2 * HPB>(mm2, OpMax(), -INFINITY);
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) { mn[h] = -mm2[h]; mx[h] = mm2[HPB + h]; }
+                }
+            }
+            float slope[HPB], tmin[HPB];
+#pragma unroll
+            for (int h = 0; h < HPB; ++h) {
+                if (g.calib) {
+                    const float tgt_max = mx[h] + g.off_max;
+                    tmin[h] = mn[h] + g.off_min;
+                    // (the hardware reciprocal, one unit in the last place: far inside the tolerance of the map)
+                    slope[h] = (tgt_max - tmin[h]) * __builtin_amdgcn_rcpf(mx[h] - mn[h] + 1e-8f);
+                } else {
+                    tmin[h] = mn[h];
+                    slope[h] = 1.0f;
+                }
+            }
+            // a value of the lane's head (MX)
+            auto mine = [&](const float* v) {
+                auto uni = [](float f) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f))); };
+                float r = uni(v[0]);   // (wave-uniform: scalar operands, and no array that would be indexed by the lane)
+#pragma unroll
+                for (int h = 1; h < HPB; ++h) r = hl == h ? uni(v[h]) : r;
+                return r;
+            };
+            if (MX && EXTRAS && g.mask) {
+                const float* mk = g.mask + b * g.mask_sb + g.S + t0;
+                const float mnl = mine(mn), sl = mine(slope), tl = mine(tmin);
+                float top = -INFINITY;
+#pragma unroll
+                for (int rd = 0; rd < (MX ? REGL : 1); ++rd) {
+                    if (wt0 + rd * kNT < n) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const float mv = mk[min(wt0 + rd * kNT + 16 * j + (lane & 15), n - 1)];
+                            lx[rd][j] = (lx[rd][j] - mnl) * sl + tl + mv;
+                            top = fmaxf(top, lx[rd][j]);
+                        }
+                    }
+                }
+                const int kt = row_max_key(float_key(top));
+                int* redi = reinterpret_cast<int*>(red + 2 * HPB);
+                if ((lane & 15) == 0 && (lane >> 4) < HPB)
+                    __hip_atomic_fetch_max(redi + hl, kt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __syncthreads();
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) {
+                    m_img[h] = key_float(__builtin_amdgcn_readfirstlane(redi[h]));
+                    slope[h] = 1.0f; tmin[h] = 0.f; mn[h] = 0.f;
+                }
+            } else if (EXTRAS && g.mask) {
+                const float* mk = g.mask + b * g.mask_sb + g.S + t0;
+                float lm[HPB];
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) lm[h] = -INFINITY;
+                for_my_tokens(n, [&](int rd, int tt) {
+                    V w = load_logits(rd, tt);
+                    const float mv = mk[tt];
+#pragma unroll
+                    for (int h = 0; h < HPB; ++h) {
+                        w.v[h] = (w.v[h] - mn[h]) * slope[h] + tmin[h] + mv;
+                        lm[h] = fmaxf(lm[h], w.v[h]);
+                    }
+                    store_logits(rd, tt, w);
+                });
+                block_max<HPB, kNW>(lm, red + 2 * HPB);   // words of its own
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) { m_img[h] = lm[h]; slope[h] = 1.0f; tmin[h] = 0.f; mn[h] = 0.f; }
+            } else {
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) m_img[h] = fmaxf(tmin[h], (mx[h] - mn[h]) * slope[h] + tmin[h]);
+            }
+            float ls[HPB];
+#pragma unroll
+            for (int h = 0; h < HPB; ++h) ls[h] = 0.f;
+            // e = exp(x - M) with x = (w - mn) * slope + tmin, as exp2((w - mn) * ea + ec)
+            float ea[HPB], ec[HPB];
+#pragma unroll
+            for (int h = 0; h < HPB; ++h) {
+                const bool dead = (m_img[h] == -INFINITY);   // every position masked out
+                ea[h] = dead ? 0.f : slope[h] * kLog2e;
+                ec[h] = dead ? -INFINITY : (tmin[h] - m_img[h]) * kLog2e;
+            }
+            using HWv = Words<L::HW>;
+            // per-token value statistics (VTOK): (T, NGRP) scales and minima of this kv-head
+            const uint16_t* tsc = static_cast<const uint16_t*>(g.vs) + (bh * g.T + t0) * L::NGRP;
+            const uint16_t* tmn = static_cast<const uint16_t*>(g.vz) + (bh * g.T + t0) * L::NGRP;
+            float cma[VTOK ? L::NGRP * HPB : 1];   // sum_t e[t][h] * minimum[t][group], kept [group][head]
+#pragma unroll
+            for (int i = 0; i < (VTOK ? L::NGRP * HPB : 1); ++i) cma[i] = 0.f;
+            // With a slope of ordinary size the subtraction folds into the constant: exp2(w * ea + (ec - mn * ea)), one
+            // FMA per logit.  A degenerate logit range makes the slope ~1e8, and only the exact zero of (w - mn)
+            // keeps the product finite: those units take the two-step form.
+            float ec2[HPB];
+            bool plain = true;
+#pragma unroll
+            for (int h = 0; h < HPB; ++h) {
+                ec2[h] = ec[h] - mn[h] * ea[h];
+                if (h < NH) plain = plain && fabsf(ea[h]) <= 4.0f;
+            }
+            if constexpr (MX) {
+                float ec3[HPB], mn3[HPB];
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) { ec3[h] = plain ? ec2[h] : ec[h]; mn3[h] = plain ? 0.f : mn[h]; }
+                const float eal = mine(ea), ecl = mine(ec3), mnl = mine(mn3);
+                float lsum = 0.f;
+                I4 acc[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc[i] = I4{0, 0, 0, 0};
+                unsigned char* et = regA + wv * L::MXT;
+                constexpr int KV = kVF / BITS;   // rounds of packed V rows in flight
+                phase_priority(std::integral_constant<int, 3>{});
+#pragma unroll
+                for (int rd = 0; rd < REGL; ++rd) {
+                    const int tw = wt0 + rd * kNT;
+                    if (tw < n) {
+                        float e[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(lx[rd][j] - mnl, eal, ecl));
+                        if (tw + kWave > n) {   // the chunk's last tile: what is past the end weighs nothing
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) e[j] = tw + 16 * j + (lane & 15) < n ? e[j] : 0.f;
+                        }
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) lsum += e[j];
+                        matrix_values<BITS>(et, e, vc + (rd % KV) * BITS, acc);
+                        __builtin_amdgcn_sched_barrier(0);   // one round at a time: interleaved, they do not fit the registers
+                        if (rd + KV < REGL) {
+#pragma unroll
+                            for (int i = 0; i < BITS; ++i)
+                                vc[(rd % KV) * BITS + i] = cvp4[min((tid + (rd + KV) * kNT) * BITS + i, last_u)];
+                        }
+                    }
+                }
+                phase_priority(std::integral_constant<int, 4>{});
+                load_res_k(0, rk);   // first residual tile's K rows: in flight during the fold below
+                float* lpart = fx + L::F_PRES;   // the waves' sums of e (not in `red`, which a slower wave may still read)
+                lsum = row_reduce(lsum, OpSum(), 0.f);
+                if ((lane & 15) == 0 && (lane >> 4) < HPB) lpart[wv * HPB + hl] = lsum;
+                __syncthreads();
+                float* redv = reinterpret_cast<float*>(regA);   // [wave][head][channel]
+                if ((lane >> 4) < HPB) matrix_fold<BITS>(acc, redv + (wv * HPB + hl) * kD, lane & 15);
+                __syncthreads();
+                if (tid < HPB * kD) {
+                    const int h = tid / kD, d = tid % kD;
+                    float a = 0.f, lh = 0.f;
+#pragma unroll
+                    for (int w = 0; w < kNW; ++w) { a += redv[(w * HPB + h) * kD + d]; lh += lpart[w * HPB + h]; }
+                    o_img = fx[L::F_VSZ + d] * (a - fx[L::F_VSZ + kD + d] * lh);
+                    if (d == 0) stat[4 * HPB + h] = lh;
+                }
+                __syncthreads();
+            } else {
+            auto exp_tokens = [&](auto fused_c) {
+            constexpr bool kFused = decltype(fused_c)::value;
+            for_my_tokens(npad, [&](int rd, int tt) {
+                float e[4] = {0.f, 0.f, 0.f, 0.f};
+                uint32_t sc2[2] = {0u, 0u};   // the token's group scales as fp16
+                if (tt < n) {
+                    const V w = load_logits(rd, tt);
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) {
+                        if constexpr (kFused) e[h] = __builtin_amdgcn_exp2f(__builtin_fmaf(w.v[h], ea[h], ec2[h]));
+                        else e[h] = __builtin_amdgcn_exp2f((w.v[h] - mn[h]) * ea[h] + ec[h]);
+                        ls[h] += e[h];
+                    }
+                    if constexpr (VTOK) {
+                        const uint2 sr = *reinterpret_cast<const uint2*>(tsc + tt * L::NGRP);
+                        const uint2 mr = *reinterpret_cast<const uint2*>(tmn + tt * L::NGRP);
+                        sc2[0] = pack_f16(Cvt<DT>::lo(sr.x), Cvt<DT>::hi(sr.x));
+                        sc2[1] = pack_f16(Cvt<DT>::lo(sr.y), Cvt<DT>::hi(sr.y));
+                        const float mg[4] = {Cvt<DT>::lo(mr.x), Cvt<DT>::hi(mr.x), Cvt<DT>::lo(mr.y), Cvt<DT>::hi(mr.y)};
+#pragma unroll
+                        for (int gi = 0; gi < L::NGRP; ++gi)
+#pragma unroll
+                            for (int h = 0; h < HPB; ++h) cma[gi * HPB + h] += e[h] * mg[gi];
+                    }
+                }
+                // e as packed fp16 in the first bytes of the token's slot (read by the V tables)
+                HWv hw;
+                hw.w[0] = pack_f16(e[0], e[1]);
+                if constexpr (L::HW == 2) hw.w[1] = pack_f16(e[2], e[3]);
+                *reinterpret_cast<HWv*>(slot(tt)) = hw;
+                if constexpr (VTOK) *reinterpret_cast<uint2*>(slot(tt) + 8) = make_uint2(sc2[0], sc2[1]);
+            });
+            };
+            if (plain) exp_tokens(std::true_type{});
+            else exp_tokens(std::false_type{});
+            // The sums of e (and of e * minimum) are only needed at the very end: each thread
+            // keeps its partial through the packed-V phase and the fold rides on that phase's
+            // closing barriers.
+            __syncthreads();   // publishes e and vst
+            CQ_PHASE(6);   // calibration and exponentials
+            // (requested here, not right after the staging: the logits' registers are free now)
+            if constexpr (kVAhead) request_v_block(L::VSUB);
+
+            // ---- phase 5: packed V ----------------------------------------------------------
+            // lane = (byte column j, slice c of its 8 bit lanes); a wave pass covers TPW tokens
+            unsigned char* wtab = regA + wv * (L::NGRP * L::GPW * 16 * L::ESZH);   // [channel group][token group][16]
+            const int j = lane / L::GPW, cs = lane % L::GPW;
+            const int wvu = __builtin_amdgcn_readfirstlane(wv);
+            const int bg = lane >> 4, be = lane & 15;   // table build: group, entry
+            f16x2_t bsel[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const _Float16 f = static_cast<_Float16>(static_cast<float>((be >> i) & 1));
+                bsel[i] = f16x2_t{f, f};
+            }
+            float acc[L::MPL][HPB];
+#pragma unroll
+            for (int m = 0; m < L::MPL; ++m)
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) acc[m][h] = 0.f;
+            const float one = g.one;
+            // Bit lane m of a byte is bit 7 - m; table offset = sum_i bit(token i) * ESZH * 2^i.
+            // The lane's MPL bit lanes sit in one nibble: the dword is shifted by 4 * (m < 4) once,
+            // each lane masks its bit in place (value 2^s per byte) and the dot-product
+            // multiplier carries the 2^-s: ESZH * 2^i >> s stays integral for s <= 3, ESZH = 8;
+            // with 4-byte entries the multiplier is kept whole and s = 0 (bit moved down first).
+            constexpr bool kInPlace = (L::ESZH == 8);
+            const uint32_t nib_shift = (cs * L::MPL < 4) ? 4u : 0u;
+            uint32_t bmask[L::MPL], bmult[L::MPL], bshr[L::MPL];
+#pragma unroll
+            for (int m = 0; m < L::MPL; ++m) {
+                const uint32_t sft = 3 - ((cs * L::MPL + m) & 3);   // bit position inside the nibble
+                bmask[m] = kInPlace ? (0x01010101u << sft) : 0x01010101u;
+                bmult[m] = kInPlace ? ((L::ESZH * 0x08040201u) >> sft) & 0x7f7f7f7fu : L::ESZH * 0x08040201u;
+                bshr[m] = kInPlace ? 0u : sft;
+            }
+            using WG = Words<L::GPW>;   // the GPW dwords of one (unit, column)
+            // channel group of the lane's byte column (32 channels = 4*BITS columns): lane / 16 for both widths
+            const int cgrp = VTOK ? (lane >> 4) : 0;
+            // absolute LDS address of the wave's tables (the dot product's addend)
+            const uint32_t wtab_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+                (__attribute__((address_space(3))) unsigned char*)wtab));
+
+            phase_priority(std::integral_constant<int, 3>{});
+            for (int vs0 = 0; vs0 < npad; vs0 += L::VSUB) {
+                const int vn = min(L::VSUB, npad - vs0);
+                if (vs0 > 0) {
+                    __syncthreads();  // previous block consumed
+                    if constexpr (!kVAhead) request_v_block(vs0);
+#pragma unroll
+                    for (int r = 0; r < kPF; ++r) {
+                        const int tok = tid + (r / BITS) * kNT;
+                        stage_piece(vc[r], tok, r % BITS, tok < vn);
+                    }
+                    if constexpr (kVAhead) request_v_block(vs0 + L::VSUB);
+                    __syncthreads();
+                }
+                // One pass over the TPW tokens of unit u: the sum of the entries each of the lane's bit lanes picks,
+                // as packed fp16 (GPW entries of at most 4 terms each, added pairwise).
+                struct PreV { HWv e[4]; WG cw; };
+                auto load_pre = [&](int u, PreV& p) {
+                    const int tl = u * L::TPW;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) p.e[i] = *reinterpret_cast<const HWv*>(slot(vs0 + tl + 4 * bg + i));
+                    p.cw = *reinterpret_cast<const WG*>(vst + (u * NB + j) * L::TPW);
+                };
+                // A pass in three steps, so that two passes can be woven together: the table of the second is built and
+                // written while the look-ups of the first are in flight (the LDS executes a wave's instructions in
+                // order: the second table's write lands after the first pass's reads).
+                auto v_build = [&](int u, const PreV& pre) {
+                    const int tl = u * L::TPW;        // token offset inside the block
+                    (void)tl;
+                    if (bg < L::GPW) {
+                        f16x2_t val[L::NGRP][L::HW];
+#pragma unroll
+                        for (int gi = 0; gi < L::NGRP; ++gi)
+#pragma unroll
+                            for (int k = 0; k < L::HW; ++k) val[gi][k] = f16x2_t{0, 0};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const unsigned char* sl = slot(vs0 + tl + 4 * bg + i);
+                            const HWv e = VTOK ? *reinterpret_cast<const HWv*>(sl) : pre.e[i];
+                            if constexpr (VTOK) {
+                                const uint2 sc = *reinterpret_cast<const uint2*>(sl + 8);
+                                const f16x2_t s01 = __builtin_bit_cast(f16x2_t, sc.x), s23 = __builtin_bit_cast(f16x2_t, sc.y);
+                                const _Float16 sg[4] = {s01.x, s01.y, s23.x, s23.y};
+#pragma unroll
+                                for (int gi = 0; gi < L::NGRP; ++gi) {
+                                    const f16x2_t w2 = bsel[i] * f16x2_t{sg[gi], sg[gi]};
+#pragma unroll
+                                    for (int k = 0; k < L::HW; ++k) val[gi][k] += __builtin_bit_cast(f16x2_t, e.w[k]) * w2;
+                                }
+                            } else {
+#pragma unroll
+                                for (int k = 0; k < L::HW; ++k) val[0][k] += __builtin_bit_cast(f16x2_t, e.w[k]) * bsel[i];
+                            }
+                        }
+#pragma unroll
+                        for (int gi = 0; gi < L::NGRP; ++gi) {
+                            HWv o;
+#pragma unroll
+                            for (int k = 0; k < L::HW; ++k) o.w[k] = __builtin_bit_cast(uint32_t, val[gi][k]);
+                            reinterpret_cast<HWv*>(wtab)[(gi * L::GPW + bg) * 16 + be] = o;
+                        }
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                };
+                auto v_lookups = [&](const WG& cw, f16x2_t (&pk)[L::MPL][L::GPW][L::HW]) {
+#pragma unroll
+                    for (int gq = 0; gq < L::GPW; ++gq) {
+                        const uint32_t tbase = wtab_addr + static_cast<uint32_t>((cgrp * L::GPW + gq) * 16 * L::ESZH);
+                        const uint32_t wsh = cw.w[gq] >> nib_shift;
+#pragma unroll
+                        for (int m = 0; m < L::MPL; ++m) {
+                            const uint32_t bits = (kInPlace ? wsh : (wsh >> bshr[m])) & bmask[m];
+                            const uint32_t off = __builtin_amdgcn_udot4(bits, bmult[m], tbase, false);
+                            const HWv e = lds_words<L::HW>(off);
+#pragma unroll
+                            for (int k = 0; k < L::HW; ++k) pk[m][gq][k] = __builtin_bit_cast(f16x2_t, e.w[k]);
+                        }
+                    }
+                };
+                auto v_reduce = [&](f16x2_t (&pk)[L::MPL][L::GPW][L::HW], f16x2_t (&sum)[L::MPL][L::HW]) {
+#pragma unroll
+                    for (int m = 0; m < L::MPL; ++m) {
+#pragma unroll
+                        for (int st = 1; st < L::GPW; st *= 2)
+#pragma unroll
+                            for (int gq = 0; gq + st < L::GPW; gq += 2 * st)
+#pragma unroll
+                                for (int k = 0; k < L::HW; ++k) pk[m][gq][k] += pk[m][gq + st][k];
+#pragma unroll
+                        for (int k = 0; k < L::HW; ++k) sum[m][k] = pk[m][0][k];
+                    }
+                };
+                auto v_pass = [&](int u, f16x2_t (&sum)[L::MPL][L::HW], const PreV& pre, auto&& after_lookups) {
+                    f16x2_t pk[L::MPL][L::GPW][L::HW];
+                    v_build(u, pre);
+                    v_lookups(pre.cw, pk);
+                    after_lookups();
+                    v_reduce(pk, sum);
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                };
+                // one mixed-precision FMA per head moves a packed sum into the fp32 accumulators
+                auto v_flush = [&](const f16x2_t (&sum)[L::MPL][L::HW]) {
+#pragma unroll
+                    for (int m = 0; m < L::MPL; ++m)
+#pragma unroll
+                        for (int h = 0; h < NH; ++h) {
+                            const f16x2_t pr = sum[m][h >> 1];
+                            const _Float16 hv = (h & 1) ? pr.y : pr.x;
+                            acc[m][h] = __builtin_fmaf(static_cast<float>(hv), one, acc[m][h]);
+                        }
+                };
+                int u = wvu;   // wave-uniform loop control
+                // the slot entries and code words of a pass are read while the pass before it waits for its look-ups
+                PreV cur, nxt;
+                if (u * L::TPW < vn) load_pre(u, cur);
+                {
+                    // two passes per fp32 accumulation: the sums of 2 * TPW tokens meet as packed fp16 first
+                    for (; (u + kNW) * L::TPW < vn; u += 2 * kNW) {
+                        f16x2_t s0[L::MPL][L::HW], s1[L::MPL][L::HW];
+                        f16x2_t pk0[L::MPL][L::GPW][L::HW], pk1[L::MPL][L::GPW][L::HW];
+                        v_build(u, cur);
+                        v_lookups(cur.cw, pk0);
+                        load_pre(u + kNW, nxt);
+                        v_build(u + kNW, nxt);           // (its table write queues behind the look-ups above)
+                        v_lookups(nxt.cw, pk1);
+                        if ((u + 2 * kNW) * L::TPW < vn) load_pre(u + 2 * kNW, cur);
+                        v_reduce(pk0, s0);
+                        v_reduce(pk1, s1);
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                        for (int m = 0; m < L::MPL; ++m)
+#pragma unroll
+                            for (int k = 0; k < L::HW; ++k) s0[m][k] += s1[m][k];
+                        v_flush(s0);
+                    }
+                }
+                for (; u * L::TPW < vn; u += kNW) {
+                    f16x2_t s0[L::MPL][L::HW];
+                    v_pass(u, s0, cur, [&]() { if ((u + kNW) * L::TPW < vn) load_pre(u + kNW, cur); });
+                    v_flush(s0);
+                }
+            }
+            CQ_PHASE(7);   // packed-V loop (tables, look-ups, sums; staging of the later blocks)
+            phase_priority(std::integral_constant<int, 4>{});
+            load_res_k(0, rk);   // first residual tile's K rows: in flight during the fold below
+            // per-wave partial sums of e (and of e * minimum), folded by the output threads below
+            constexpr int kSums = VTOK ? (L::NGRP + 1) * HPB : HPB;
+            wave_reduce_n<HPB>(ls, OpSum(), 0.f);
+            if constexpr (VTOK) {
+#pragma unroll
+                for (int gi = 0; gi < L::NGRP; ++gi) wave_reduce_n<HPB>(cma + gi * HPB, OpSum(), 0.f);
+            }
+            if (lane == 0) {
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) red[wv * kSums + h] = ls[h];
+                if constexpr (VTOK) {
+#pragma unroll
+                    for (int i = 0; i < L::NGRP * HPB; ++i) red[wv * kSums + HPB + i] = cma[i];
+                }
+            }
+            __syncthreads();
+            // head-major, so that the fold below reads consecutive words with consecutive lanes
+            float* redv = reinterpret_cast<float*>(regA);  // [wave][head][bit lane]
+#pragma unroll
+            for (int h = 0; h < HPB; ++h) {
+                Vec<L::MPL> a4;
+#pragma unroll
+                for (int m = 0; m < L::MPL; ++m) a4.v[m] = acc[m][h];
+                *reinterpret_cast<Vec<L::MPL>*>(redv + (wv * HPB + h) * L::PC + j * 8 + cs * L::MPL) = a4;
+            }
+            __syncthreads();
+            if (tid < HPB * kD) {
+                const int h = tid / kD, d = tid % kD;
+                float a = 0.f;
+                // bit lanes of channel d.  Per-channel codes: first channel of a byte in its top
+                // bits; per-token codes: first channel in the lowest bits.
+                const int per = 8 / BITS;                       // channels per byte
+                const int cb = d / per * 8, c = d % per;
+                const int lane_hi = VTOK ? cb + 8 - BITS * (c + 1) : cb + BITS * c;   // bit lane of the code's top bit
+                if constexpr (BITS == 1) {
+#pragma unroll
+                    for (int w = 0; w < kNW; ++w) a += redv[(w * HPB + h) * L::PC + lane_hi];
+                } else {
+#pragma unroll
+                    for (int w = 0; w < kNW; ++w)
+                        a += 2.0f * redv[(w * HPB + h) * L::PC + lane_hi] + redv[(w * HPB + h) * L::PC + lane_hi + 1];
+                }
+                float lh = 0.f;   // sum of e of this thread's head
+#pragma unroll
+                for (int w = 0; w < kNW; ++w) lh += red[w * kSums + h];
+                if constexpr (VTOK) {
+                    float cm = 0.f;   // sum_t e * minimum of the channel's group
+#pragma unroll
+                    for (int w = 0; w < kNW; ++w) cm += red[w * kSums + HPB + (d >> 5) * HPB + h];
+                    o_img = a + cm;
+                } else {
+                    const float s = fx[L::F_VSZ + d];
+                    const float z = fx[L::F_VSZ + kD + d];
+                    o_img = s * (a - z * lh);
+                }
+                if (d == 0) stat[4 * HPB + h] = lh;
+            }
+            __syncthreads();
+            }
+        }
+
+        if (n == 0) load_res_k(0, rk);
+        CQ_PHASE(8);   // fold of the packed part
+        // ---- phase 6: full-precision residual rows, online softmax.  Runs last: its first
+        // tile is requested when the packed-V phase ends and arrives during that phase's fold.
+#pragma unroll
+        for (int h = 0; h < HPB; ++h) {
+            if (tid == h) {
+                stat[HPB + h] = -INFINITY;
+                stat[2 * HPB + h] = 0.f;
+            }
+        }
+        if (do_res) {
+            float m_run = -INFINITY, l_run = 0.f;
+            float* sres = fx + L::F_SRES;
+            float* pres = fx + L::F_PRES;
+            // raw 16-bit q, [head][kD], read per head as two 16-byte LDS loads
+            const uint4* q128 = reinterpret_cast<const uint4*>(fx + L::F_QRAW);
+            float accv[2][HPB];   // the lane's channel pair
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) accv[k][h] = 0.f;
+            const float* mk = (EXTRAS && g.mask) ? g.mask + b * g.mask_sb : nullptr;
+
+            for (int r0 = 0; r0 < R; r0 += kResTile) {
+                const bool more = r0 + kResTile < R;
+                const int r = r0 + krow;
+                load_res_v(r0, rv);   // the tile's value words: in flight while its logits and weights are worked out
+                float dot[HPB];
+#pragma unroll
+                for (int h = NH; h < HPB; ++h) dot[h] = 0.f;
+#pragma unroll
+                for (int h = 0; h < NH; ++h) {
+                    float a = 0.f;
+#pragma unroll
+                    for (int i = 0; i < NKP; ++i) {
+                        const uint4 qa = q128[h * (kD / 8) + i * LPR + lq];
+                        a = dot2<DT>(qa.x, rk[i].x, a); a = dot2<DT>(qa.y, rk[i].y, a);
+                        a = dot2<DT>(qa.z, rk[i].z, a); a = dot2<DT>(qa.w, rk[i].w, a);
+                    }
+                    dot[h] = (LPR == 4 ? quad_reduce(a, OpSum(), 0.f) : oct_reduce(a, OpSum(), 0.f)) * inv_sqrt_d;
+                    // one head's q pieces at a time: all of them side by side would not fit the registers
+                    if constexpr (NKP > 2) __builtin_amdgcn_sched_barrier(0);
+                }
+                if (more) load_res_k(r0 + kResTile, rk);   // next tile's K slice, in place
+                if (lq == 0) {
+                    float mv = 0.f;
+                    if (mk && r < R) mv = mk[r < g.S ? r : g.T + r];
+#pragma unroll
+                    for (int h = 0; h < HPB; ++h) sres[krow * HPB + h] = (r < R) ? dot[h] + mv : -INFINITY;
+                }
+                __syncthreads();
+                if (wv < NH) {   // wave h keeps the running softmax state of head h
+                    const int h = wv;
+                    constexpr int kRL = kResTile / kWave;   // tile rows per lane
+                    float sv[kRL], smax = -INFINITY;
+#pragma unroll
+                    for (int i = 0; i < kRL; ++i) {
+                        sv[i] = sres[(lane + i * kWave) * HPB + h];
+                        smax = fmaxf(smax, sv[i]);
+                    }
+                    const float mnew = fmaxf(m_run, wave_max(smax));
+                    const bool dead = (mnew == -INFINITY);
+                    float psum = 0.f;
+#pragma unroll
+                    for (int i = 0; i < kRL; ++i) {
+                        const float pi = dead ? 0.f : __expf(sv[i] - mnew);
+                        pres[(lane + i * kWave) * HPB + h] = pi;
+                        psum += pi;
+                    }
+                    const float al = dead ? 1.0f : __expf(m_run - mnew);
+                    l_run = l_run * al + wave_sum(psum);
+                    m_run = mnew;
+                    if (lane == 0) { stat[h] = al; stat[HPB + h] = m_run; stat[2 * HPB + h] = l_run; }
+                }
+                __syncthreads();
+                if (r0 > 0) {
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) {
+                        const float al = stat[h];
+                        accv[0][h] *= al;
+                        accv[1][h] *= al;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < RPW; ++i) {
+                    const float f0 = Cvt<DT>::lo(rv[i]), f1 = Cvt<DT>::hi(rv[i]);
+                    const V p = reinterpret_cast<const V*>(pres)[wvr * RPW + i];   // the row's weights (0 past R), one address per wave
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) {
+                        accv[0][h] = __builtin_fmaf(p.v[h], f0, accv[0][h]);
+                        accv[1][h] = __builtin_fmaf(p.v[h], f1, accv[1][h]);
+                    }
+                }
+            }
+            __syncthreads();
+            float* red2 = reinterpret_cast<float*>(regA);  // [wave][head][kD]: the fold reads consecutive words
+#pragma unroll
+            for (int h = 0; h < HPB; ++h) {
+                Vec<2> a2;
+                a2.v[0] = accv[0][h]; a2.v[1] = accv[1][h];
+                *reinterpret_cast<Vec<2>*>(red2 + (wv * HPB + h) * kD + 2 * lane) = a2;
+            }
+            __syncthreads();
+            if (tid < HPB * kD) {
+                const int h = tid / kD, d = tid % kD;
+#pragma unroll
+                for (int w = 0; w < kNW; ++w) o_res += red2[(w * HPB + h) * kD + d];
+            }
+        }
+
+#pragma unroll
+        for (int h = 0; h < HPB; ++h) {
+            if (tid == h) {
+                stat[3 * HPB + h] = m_img[h];
+                if (n == 0) stat[4 * HPB + h] = 0.f;
+            }
+        }
+        CQ_PHASE(9);   // residual window
+        // ---- phase 7: merge / write ---------------------------------------------------------
+        __syncthreads();
+        if (tid < nh * kD) {
+            const int h = tid / kD, d = tid % kD;
+            const float mr = stat[HPB + h], lr = stat[2 * HPB + h];
+            const float mi = stat[3 * HPB + h], li = stat[4 * HPB + h];
+            const int64_t row = static_cast<int64_t>(b) * g.Hq + hq0 + h;
+            if constexpr (!CHUNKED) {
+                const float mf = fmaxf(mi, mr);
+                const float wi = (mi == -INFINITY) ? 0.f : __expf(mi - mf);
+                const float wr = (mr == -INFINITY) ? 0.f : __expf(mr - mf);
+                const float num = o_img * wi + o_res * wr;
+                const float den = li * wi + lr * wr;
+                store_elem<DT>(g.out, row * kD + d, num * __builtin_amdgcn_rcpf(den));
+            } else {
+                float* p = g.part + (row * g.nx + split) * (kD + 2);
+                const bool is_img = split < g.nsplit;
+                if (d == 0) { publish(p, is_img ? mi : mr); publish(p + 1, is_img ? li : lr); }
+                publish(p + 2 + d, is_img ? o_img : o_res);
+            }
+        }
+        if constexpr (CHUNKED) {
+            // The unit's chunks (and its residual unit) each leave an (m, l, acc) partial; the workgroup that
+            // finds all the others' already counted combines them.  The partials are device-scope atomic stores
+            // (written through to the level all compute units share, so no cache has to be written back as a
+            // whole): every thread waits for its own stores to complete, the barrier collects the workgroup,
+            // then one thread counts.
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            int* last = reinterpret_cast<int*>(red);
+            if (tid == 0) {
+                if (g.fused) *last = arrive<__HIP_MEMORY_SCOPE_AGENT>(g.done64 + unit, g.epoch) == static_cast<uint32_t>(g.nx);
+                else *last = __hip_atomic_fetch_add(g.cnt + unit, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.nx - 1;
+            }
+            __syncthreads();
+            if (*last) {
+                // the reader: one acquire drops this compute unit's and this die's cached copies of what other
+                // dies wrote, after which ordinary loads (issued together, unlike atomic ones) see the partials
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                if (tid < nh * kD) {
+                    const int h = tid / kD, d = tid % kD;
+                    const int64_t row = static_cast<int64_t>(b) * g.Hq + hq0 + h;
+                    const float* p = g.part + row * g.nx * (kD + 2);
+                    // eight partials at a time, their loads in flight together; running (m, num, den)
+                    float m = -INFINITY, num = 0.f, den = 0.f;
+                    for (int s0 = 0; s0 < g.nx; s0 += 8) {
+                        float ms[8], ls[8], as[8];
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) {
+                            const float* q = p + min(s0 + k, g.nx - 1) * (kD + 2);
+                            ms[k] = q[0]; ls[k] = q[1]; as[k] = q[2 + d];
+                        }
+                        float mb = m;
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) mb = fmaxf(mb, (s0 + k < g.nx) ? ms[k] : -INFINITY);
+                        const float keep = (m == -INFINITY) ? 0.f : __expf(m - mb);
+                        num *= keep; den *= keep;
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) {
+                            const float w = (s0 + k < g.nx && ms[k] != -INFINITY) ? __expf(ms[k] - mb) : 0.f;
+                            den += ls[k] * w;
+                            num += as[k] * w;
+                        }
+                        m = mb;
+                    }
+                    store_elem<DT>(g.out, row * kD + d, num / den);
+                }
+                // every other workgroup of the unit is past both counters: leave them empty for a replay of this
+                // very launch (a recorded step comes back with the same epoch)
+                if (g.fused) clear_handover<HPB, kNT>(g, unit, tid);
+            }
+        }
+    }
+}
+
+// The min/max launch of a two-launch chunked step: no residual unit, and `cap` tokens' worth of slots.
+static inline DecodeGeom minmax_geometry(const DecodeGeom& g, int cap) {
+    DecodeGeom g1 = g;
+    g1.nx = g.nsplit;
+    g1.d_nx.set(static_cast<uint32_t>(g.nsplit));
+    g1.cap = cap;
+    return g1;
+}
+
+}  // namespace cq

@@ -1,0 +1,68 @@
+"""The matrix-core form of the decode step at the edges of its tiling: 64-token tiles, 512- and 1 024-token rounds of a
+workgroup, and the fixed-point operands' range."""
+import numpy as np
+import pytest
+
+from oracle import cq_oracle as O
+from tests.test_gpu_decode import _oracle, _run
+from tests.util import make_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from calibquant_amd import ops
+    return ops
+
+
+def _close(got, want):
+    # fp16 results: one rounding (2^-11 of the value) on sums kept in 32 bits (a few 1e-6 of the largest, times the
+    # logits' size in the exponent: logits of about 10)
+    assert np.isfinite(got).all()
+    bound = 2.0 ** -11 * np.abs(want) + 1e-4 * np.abs(want).max()
+    assert (np.abs(got - want) <= bound).all(), float((np.abs(got - want) / bound).max())
+
+
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("case", [
+    # B, Hq, Hkv, T: few units (1 024 threads) around a tile, a round and two rounds; one, two, three, four heads
+    (1, 8, 8, 2), (1, 4, 4, 63), (1, 8, 4, 64), (1, 12, 4, 65), (2, 32, 8, 1023), (2, 32, 8, 1025), (1, 24, 4, 2049),
+    # more units than compute units (512 threads): below and above a tile and a round
+    (33, 32, 8, 63), (33, 32, 8, 129), (33, 32, 8, 513), (65, 24, 4, 577),
+])
+def test_tile_edges(ops, case, bits):
+    B, Hq, Hkv, T = case
+    print(f"case matrix {case} bits={bits}", flush=True)
+    c = make_case(B, Hq, Hkv, 128, T, 0, bits, "fp16", seed=T)
+    _close(_run(ops, c, "fp16", 0, bits), _oracle(c, 0, bits))
+
+
+@pytest.mark.parametrize("bits", [1, 2])
+def test_masked_tiles(ops, bits):
+    """A mask that leaves out whole tiles, single tokens and the ragged end."""
+    B, T = 3, 331
+    c = make_case(B, 32, 8, 128, T, 0, bits, "fp16", seed=5)
+    mask = np.zeros((B, T), np.float32)
+    mask[0, :130] = mask[1, 1::2] = mask[2, 300:] = -1e4
+    _close(_run(ops, c, "fp16", 0, bits, mask=mask), _oracle(c, 0, bits, mask=mask))
+
+
+def test_query_of_any_scale(ops):
+    """Queries far from 1 move the fixed-point grid; a query of zeros has no largest value to take it from."""
+    for scale in (0.0, 2.0 ** -12, 2.0 ** 4):
+        c = make_case(1, 32, 8, 128, 200, 0, 1, "fp16", seed=11)
+        c["q"] = O.round_to(c["q"] * np.float32(scale), "fp16")
+        _close(_run(ops, c, "fp16", 0, 1, calibrate=False), _oracle(c, 0, 1, calibrate_logits=False))
+
+
+def test_infinity_in_one_head_stays_there(ops):
+    c = make_case(1, 32, 8, 128, 200, 0, 1, "fp16", seed=12)
+    want = _oracle(c, 0, 1)
+    c["q"][0, 5, 17] = np.inf
+    c["q"][0, 9, 3] = np.nan
+    got = _run(ops, c, "fp16", 0, 1)
+    hit = np.zeros(32, bool)
+    hit[[5, 9]] = True
+    assert np.isnan(got[0, hit]).all()
+    _close(got[0, ~hit], want[0, ~hit])
