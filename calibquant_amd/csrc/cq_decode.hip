@@ -13,6 +13,9 @@ namespace cq {
 // Launches the matrix-core form (one source file per storage type: cq_decode_matrix_*.hip).
 template <typename DT>
 int launch_matrix(const DecodeGeom& g, int bits, int hpb, int nh, int nt, unsigned units, hipStream_t st);
+// ... with per-token values (cq_decode_matrix_token_*.hip)
+template <typename DT>
+int launch_matrix_token(const DecodeGeom& g, int bits, int hpb, int nt, unsigned units, hipStream_t st);
 
 // ---- the chunked step in one launch: host side ------------------------------------------------------
 // A word of pinned host memory per device that a workgroup sets when it gives up waiting for the other
@@ -206,71 +209,17 @@ static DecodeGeom unit_geometry(const DecodeGeom& g, int nh, int nt) {
     return gm;
 }
 
-// Per-token values: the look-up form.
-template <int BITS, int HPB, typename DT>
-static int launch(const DecodeGeom& g, const Plan& p, hipStream_t st) {
-    constexpr int NT = 1024;
-    const unsigned units = static_cast<unsigned>(g.B) * g.Hkv * ngroups(g.Hq / g.Hkv, HPB);
-    const bool extras = g.mask != nullptr || g.r_dev != nullptr;
-    auto kmain = g.nsplit > 1 ? (extras ? decode_kernel<BITS, HPB, DT, false, true, NT, 0, true, true>
-                                        : decode_kernel<BITS, HPB, DT, false, true, NT, 0, true, false>)
-                              : (extras ? decode_kernel<BITS, HPB, DT, false, true, NT, 0, false, true>
-                                        : decode_kernel<BITS, HPB, DT, false, true, NT, 0, false, false>);
-    auto kmm = decode_kernel<BITS, HPB, DT, true, false, NT, 0>;   // the min/max pass never looks at values
-    // raise the dynamic-LDS limit once per device for this instantiation
-    static std::atomic<uint32_t> attr_done{0};
-    int dev = 0;
-    CQ_HIP_CHECK(hipGetDevice(&dev));
-    const uint32_t bit = 1u << (dev & 31);
-    if (!(attr_done.load(std::memory_order_acquire) & bit)) {
-        // the K look-ups address the table absolutely: the dynamic LDS array must start at 0
-        const void* kernels[5] = {reinterpret_cast<const void*>(decode_kernel<BITS, HPB, DT, false, true, NT, 0, false, false>),
-                                  reinterpret_cast<const void*>(decode_kernel<BITS, HPB, DT, false, true, NT, 0, false, true>),
-                                  reinterpret_cast<const void*>(decode_kernel<BITS, HPB, DT, false, true, NT, 0, true, false>),
-                                  reinterpret_cast<const void*>(decode_kernel<BITS, HPB, DT, false, true, NT, 0, true, true>),
-                                  reinterpret_cast<const void*>(kmm)};
-        for (const void* k : kernels) {
-            hipFuncAttributes fa;
-            CQ_HIP_CHECK(hipFuncGetAttributes(&fa, k));
-            if (fa.sharedSizeBytes != 0) return CQ_ERR_LAUNCH;
-            CQ_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax));
-        }
-        attr_done.fetch_or(bit, std::memory_order_release);
-    }
-    const DecodeGeom gm = unit_geometry(g, HPB, NT);
-    if (g.nsplit > 1 && !g.fused) {
-        const DecodeGeom g1 = minmax_geometry(gm, Lay<BITS, HPB, false, NT, 0>::KPASS > 1 ? p.cap : 0);
-        hipLaunchKernelGGL(kmm, dim3(units * g.nsplit), dim3(NT), (Lay<BITS, HPB, false, NT, 0>::lds_bytes(g1.cap)), st, g1);
-        CQ_LAUNCH_CHECK();
-    }
-    hipLaunchKernelGGL(kmain, dim3(units * g.nx), dim3(NT), p.lds, st, gm);
-    CQ_LAUNCH_CHECK();
-    return CQ_OK;
-}
-
-// Per-channel values run on the matrix cores at every size, per-token values (a weight per channel group) through
-// the look-up tables.
 template <typename DT>
 static int dispatch(const DecodeGeom& g, const Plan& p, int bits, bool vtok, hipStream_t st) {
-    if (!vtok) {
-        const DecodeGeom gm = unit_geometry(g, p.nh, p.nt);
-        const unsigned units = static_cast<unsigned>(g.B) * g.Hkv * ngroups(gm.G, p.nh);
+    const DecodeGeom gm = unit_geometry(g, p.nh, p.nt);
+    const unsigned units = static_cast<unsigned>(g.B) * g.Hkv * ngroups(gm.G, p.nh);
 #ifdef CQ_PHASE_STOPS
-        if (!std::is_same<DT, BF16>::value || bits != 1 || p.hpb != 4 || p.nh != 4 || p.nt != 512 || g.nsplit > 1)
-            return CQ_ERR_UNSUPPORTED;
-        return launch_matrix_one<1, 4, BF16, 512, kRegPair, false, false, 4>(gm, units, st);
+    if (vtok || !std::is_same<DT, BF16>::value || bits != 1 || p.hpb != 4 || p.nh != 4 || p.nt != 512 || g.nsplit > 1)
+        return CQ_ERR_UNSUPPORTED;
+    return launch_matrix_one<1, 4, BF16, false, 512, kRegPair, false, false, 4>(gm, units, st);
 #else
-        return launch_matrix<DT>(gm, bits, p.hpb, p.nh, p.nt, units, st);
-#endif
-    }
-#ifdef CQ_PHASE_STOPS
-    return CQ_ERR_UNSUPPORTED;
-#else
-    if (bits == 1) {
-        if (p.hpb == 4) return launch<1, 4, DT>(g, p, st);
-        return p.hpb == 2 ? launch<1, 2, DT>(g, p, st) : launch<1, 1, DT>(g, p, st);
-    }
-    return p.hpb == 2 ? launch<2, 2, DT>(g, p, st) : launch<2, 1, DT>(g, p, st);
+    return vtok ? launch_matrix_token<DT>(gm, bits, p.hpb, p.nt, units, st)
+                : launch_matrix<DT>(gm, bits, p.hpb, p.nh, p.nt, units, st);
 #endif
 }
 

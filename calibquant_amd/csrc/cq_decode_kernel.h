@@ -171,7 +171,7 @@ template <int BITS, int HPB, bool VTOK = false, int NT_ = 1024, int REGL = 0, bo
     static constexpr int PCS = (WPP + 3) / 4;       // 16-byte pieces of a row a pass looks at
     static constexpr int KT = NBP * 256 * ESZ;      // K table bytes
     static_assert(NB * 256 * ESZ <= 4 * KTMAX, "at most four table passes");
-    static_assert(!(REGL > 0 && VTOK), "logits in registers: per-channel values only");
+    static_assert(!(REGL > 0 && VTOK && !MX), "look-ups with logits in registers: per-channel values only");
     static constexpr int SLOT = MX ? 0 : VTOK ? 16 : (REGL > 0 ? ESZH : ESZ);   // bytes per token slot: logits, later e (+ 4 group scales)
     static constexpr int NGRP = VTOK ? kD / 32 : 1; // channel groups with tables of their own
     static constexpr int WTAB = kNW * NGRP * GPW * 16 * ESZH;
@@ -197,7 +197,8 @@ template <int BITS, int HPB, bool VTOK = false, int NT_ = 1024, int REGL = 0, bo
     static constexpr int FIXED = ((F_END * 4 + 255) / 256) * 256;
     // byte offset of the token slots: behind the fixed region, or (INA) inside region A behind the staged V block
     static constexpr int slots_in_a(int cap) { return WTAB + cmin(VSUB, cap) * NB; }
-    static constexpr int MXT = (1 + BITS) * 1024;   // MX: bytes of a wave's tile, weights then packed V rows
+    // MX: bytes of a wave's tile: weights, then packed V rows (VTOK: weights and rows of one channel group, statistics)
+    static constexpr int MXT = VTOK ? 2560 : (1 + BITS) * 1024;
     static constexpr int region_a(int cap) {
         if (MX) return cmax(kNW * MXT, RED2);
         return (cmax(cmax(KT, slots_in_a(cap) + (INA ? cap * SLOT : 0)), cmax(RED, RED2)) + 255) / 256 * 256;
@@ -358,6 +359,7 @@ __device__ __forceinline__ uint32_t pack_f16(float a, float b) {
 // from 64 bits here, which is their own rounding, 7e-4 to 1.3e-3 there).
 typedef int I4 __attribute__((ext_vector_type(4)));
 typedef int I2 __attribute__((ext_vector_type(2)));
+typedef uint32_t U2 __attribute__((ext_vector_type(2)));
 
 // four signed byte digits of x, |x| < 2^31 - 2^23 (digit 0 in the lowest byte)
 __device__ __forceinline__ uint32_t byte_digits(int x) {
@@ -495,6 +497,83 @@ template <int BITS> __device__ __forceinline__ void matrix_fold(const I4* acc, f
     }
 }
 
+// Per-token values: a weight is e * scale[token][group of 32 channels], so every group has a left operand of its own.
+// The right operand is arranged for it: a group's 4 (8) bytes of a row, read back by columns as 8 rows x 8 bytes (at 1 bit
+// the four bytes twice), meet in lane x as byte x mod 4 (8), and the lane keeps the field x / 4 (x / 8) of it and, from the
+// byte shifted by four, the one half a byte higher: 16 columns of the result are 16 channels, two MFMAs are a group.
+// The grid is the wave's largest scale of the group; sums of e * minimum stay in fp32.
+// Measured at batch 64 x 3 328 + 128, 1 bit, us per step: look-up form 58.1, this one 38.3 (1 024 threads, one workgroup per
+// compute unit: the four groups' operands, converted and read back one after the other, are what bounds it).
+// Weights and scales have 32 bits here, the look-up tables held their products and short sums as fp16.
+// st: the lane's own token's scales and minima (layout of `stats` below); pw: the wave's grid, 2^(30 - e) per group.
+template <int BITS, typename DT>
+__device__ __forceinline__ void matrix_values_token(unsigned char* tile, const float* e, const U4* v, U4 st, const float* pw,
+                                                    float* cm, I4* acc) {
+    const int lane = threadIdx.x & 63, x = lane & 15, k = lane >> 4;
+    unsigned char* rows = tile + 1024;    // [token][8 bytes]
+    unsigned char* stats = tile + 1536;   // [token][scales 0 1, minima 0 1, scales 2 3, minima 2 3]
+    *reinterpret_cast<U4*>(stats + lane * 16) = st;
+    const uint32_t mask = BITS == 1 ? 0x01010101u << (x >> 2) : 0x03030303u << (2 * (x >> 3));
+    const unsigned char* col = tile + (16 * k + (x >> 1)) * 16 + (x & 1) * 8;
+    const unsigned char* rcol = rows + (16 * k + (x >> 1)) * 8;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float sc[4][2];                       // [16 j + x][group of the pair]: e * scale
+#pragma unroll
+    for (int gi = 0; gi < 4; ++gi) {
+        if (gi % 2 == 0) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const U2 t = *reinterpret_cast<const U2*>(stats + (16 * j + x) * 16 + 4 * gi);
+                sc[j][0] = e[j] * Cvt<DT>::lo(t.x);
+                sc[j][1] = e[j] * Cvt<DT>::hi(t.x);
+                cm[gi] = __builtin_fmaf(e[j], Cvt<DT>::lo(t.y), cm[gi]);
+                cm[gi + 1] = __builtin_fmaf(e[j], Cvt<DT>::hi(t.y), cm[gi + 1]);
+            }
+        }
+        U2 w2;
+        if constexpr (BITS == 1) { w2.x = v[0][gi]; w2.y = v[0][gi]; }
+        else { w2.x = v[gi >> 1][2 * (gi & 1)]; w2.y = v[gi >> 1][2 * (gi & 1) + 1]; }
+        *reinterpret_cast<U2*>(rows + lane * 8) = w2;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float xs = __builtin_amdgcn_fmed3f(sc[j][gi % 2] * pw[gi], -2130706432.f, 2130706432.f);
+            *reinterpret_cast<uint32_t*>(tile + (16 * j + x) * 16 + 4 * k) = byte_digits(__float2int_rn(xs));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const I2 e0 = column8(col), e1 = column8(col + 128), v0 = column8(rcol), v1 = column8(rcol + 64);
+        const I4 a = {e0[0], e0[1], e1[0], e1[1]};
+        const uint32_t w[4] = {static_cast<uint32_t>(v0[0]), static_cast<uint32_t>(v0[1]), static_cast<uint32_t>(v1[0]), static_cast<uint32_t>(v1[1])};
+        I4 f0, f1;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) { f0[r] = static_cast<int>(w[r] & mask); f1[r] = static_cast<int>((w[r] >> 4) & mask); }
+        acc[2 * gi] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, f0, acc[2 * gi], 0, 0, 0);
+        acc[2 * gi + 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, f1, acc[2 * gi + 1], 0, 0, 0);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// its sums as floats in channel order; unit: the value of one grid step per group
+template <int BITS> __device__ __forceinline__ void matrix_fold_token(const I4* acc, const float* unit, float* out, int x) {
+    const int byte = BITS == 1 ? x & 3 : x & 7, f = BITS == 1 ? x >> 2 : x >> 3;
+    const float field = __builtin_bit_cast(float, (127 - BITS * f) << 23);   // the field counts 2^(BITS f)
+#pragma unroll
+    for (int gi = 0; gi < 4; ++gi) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const I4 a = acc[2 * gi + q];
+            float r = static_cast<float>(a[3]);
+#pragma unroll
+            for (int p = 2; p >= 0; --p) r = __builtin_fmaf(r, 256.f, static_cast<float>(a[p]));
+            out[32 * gi + byte * (8 / BITS) + f + q * (4 / BITS)] = r * field * unit[gi];
+        }
+    }
+}
+
 // CHUNKED: the launch is one of the two of a chunked step (the min/max launch always is); a single launch carries
 // none of their code.  EXTRAS: an additive mask or a residual row count read from device memory may be present; a
 // call with neither runs an instantiation without their code (32.6-32.8 against 33.5-34.0 us at the benchmark shape:
@@ -508,7 +587,7 @@ template <int BITS, int HPB, typename DT, bool MINMAX_ONLY, bool VTOK = false, i
 // (four waves per SIMD - at most 128 VGPRs - for either workgroup size: two 512-thread workgroups per compute
 // unit are only resident together within that)
 __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
-    static_assert(!MX || (!VTOK && REGL > 0), "matrix-core form: per-channel values, logits in registers");
+    static_assert(!MX || REGL > 0, "matrix-core form: logits in registers");
     using L = Lay<BITS, HPB, VTOK, NT, REGL, MX>;
     using V = Vec<HPB>;
     constexpr int NB = L::NB;
@@ -763,10 +842,10 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     };
     // First block of packed V rows: half of it is requested here, behind the packed K rows, the
     // rest as the K registers free up, so it has arrived when the logits are done.
-    constexpr int kVF = MX ? kMatrixV : kPF;   // 16-byte pieces of packed V rows in flight per thread
+    constexpr int kVF = MX ? (VTOK ? (REGL > 4 ? 1 : 2) * BITS : kMatrixV) : kPF;   // 16-byte pieces of packed V rows in flight per thread
     U4 vc[kVF];
     auto request_v = [&](int r) { vc[r] = cvp4[min((tid + (r / BITS) * kNT) * BITS + r % BITS, last_u)]; };
-    constexpr int kVEarly = MX ? kMatrixE : kPF / 2;
+    constexpr int kVEarly = MX ? (VTOK ? BITS : kMatrixE) : kPF / 2;
     if constexpr (!MINMAX_ONLY) {
 #pragma unroll
         for (int r = 0; r < kVEarly; ++r) request_v(r);
@@ -783,6 +862,10 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     // the last one)
     const int wt0 = __builtin_amdgcn_readfirstlane(tid);
     const int hl = min(lane >> 4, HPB - 1);
+    // MX with per-token values: the chunk's scales and minima, four 16-bit values a token; the wave's grids
+    const U2* vsp = reinterpret_cast<const U2*>(has_img ? static_cast<const uint16_t*>(g.vs) + (bh * g.T + t0) * 4 : static_cast<const uint16_t*>(g.q));
+    const U2* vmp = reinterpret_cast<const U2*>(has_img ? static_cast<const uint16_t*>(g.vz) + (bh * g.T + t0) * 4 : static_cast<const uint16_t*>(g.q));
+    float vpw[4] = {0.f, 0.f, 0.f, 0.f}, vunit[4] = {0.f, 0.f, 0.f, 0.f};
     if constexpr (MX) {
         if (k_rows) {
             const I4* aq = reinterpret_cast<const I4*>(regA);
@@ -805,6 +888,28 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 if (!MINMAX_ONLY && rd < kVF - kVEarly) request_v(kVEarly + rd);   // the rest of the first packed V rows
             }
             phase_priority(std::integral_constant<int, 2>{});
+            if constexpr (VTOK && !MINMAX_ONLY) {
+                // the largest scale of every group among the wave's tokens (bit patterns: the sign cleared)
+                uint32_t t0s = 0, t1s = 0, t2s = 0, t3s = 0;
+#pragma unroll
+                for (int rd = 0; rd < REGL; ++rd) {
+                    if (wt0 + rd * kNT < n) {
+                        const U2 t = vsp[min(tid + rd * kNT, n - 1)];
+                        t0s = max(t0s, t.x & 0x7fffu); t1s = max(t1s, (t.x >> 16) & 0x7fffu);
+                        t2s = max(t2s, t.y & 0x7fffu); t3s = max(t3s, (t.y >> 16) & 0x7fffu);
+                    }
+                }
+                const uint32_t ts[4] = {t0s, t1s, t2s, t3s};
+#pragma unroll
+                for (int gi = 0; gi < 4; ++gi) {
+                    const float f = Cvt<DT>::to_float(static_cast<uint16_t>(wave_max_key(static_cast<int>(ts[gi]))));
+                    const int bits = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f));
+                    const int e = max((bits >> 23) - 126, -90);   // the largest lies in [2^(e-1), 2^e)
+                    vpw[gi] = __builtin_bit_cast(float, (30 - e + 127) << 23);
+                    // an infinity or a NaN among them makes the group's sums NaN
+                    vunit[gi] = bits >= 0x7f800000 ? __builtin_nanf("") : __builtin_bit_cast(float, (e - 30 + 127) << 23);
+                }
+            }
             // the waves' minima and maxima meet in LDS, as in block_max, from one lane per head
             const int klo = row_max_key(float_key(-lo)), khi = row_max_key(float_key(hi));
             int* redi = reinterpret_cast<int*>(red);
@@ -1412,6 +1517,15 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 for (int i = 0; i < 8; ++i) acc[i] = I4{0, 0, 0, 0};
                 unsigned char* et = regA + wv * L::MXT;
                 constexpr int KV = kVF / BITS;   // rounds of packed V rows in flight
+                U2 ssc[VTOK ? KV : 1], smin[VTOK ? KV : 1];   // VTOK: the statistics of the lane's own tokens, as many rounds ahead
+                float cm[4] = {0.f, 0.f, 0.f, 0.f};
+                if constexpr (VTOK) {
+#pragma unroll
+                    for (int r = 0; r < KV; ++r) {
+                        ssc[r] = vsp[min(tid + r * kNT, n - 1)];
+                        smin[r] = vmp[min(tid + r * kNT, n - 1)];
+                    }
+                }
                 phase_priority(std::integral_constant<int, 3>{});
 #pragma unroll
                 for (int rd = 0; rd < REGL; ++rd) {
@@ -1426,12 +1540,21 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                         }
 #pragma unroll
                         for (int j = 0; j < 4; ++j) lsum += e[j];
-                        matrix_values<BITS>(et, e, vc + (rd % KV) * BITS, acc);
+                        if constexpr (VTOK) {
+                            const U2 a = ssc[rd % KV], m = smin[rd % KV];
+                            matrix_values_token<BITS, DT>(et, e, vc + (rd % KV) * BITS, U4{a.x, m.x, a.y, m.y}, vpw, cm, acc);
+                        } else {
+                            matrix_values<BITS>(et, e, vc + (rd % KV) * BITS, acc);
+                        }
                         __builtin_amdgcn_sched_barrier(0);   // one round at a time: interleaved, they do not fit the registers
                         if (rd + KV < REGL) {
 #pragma unroll
                             for (int i = 0; i < BITS; ++i)
                                 vc[(rd % KV) * BITS + i] = cvp4[min((tid + (rd + KV) * kNT) * BITS + i, last_u)];
+                            if constexpr (VTOK) {
+                                ssc[rd % KV] = vsp[min(tid + (rd + KV) * kNT, n - 1)];
+                                smin[rd % KV] = vmp[min(tid + (rd + KV) * kNT, n - 1)];
+                            }
                         }
                     }
                 }
@@ -1439,17 +1562,39 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 load_res_k(0, rk);   // first residual tile's K rows: in flight during the fold below
                 float* lpart = fx + L::F_PRES;   // the waves' sums of e (not in `red`, which a slower wave may still read)
                 lsum = row_reduce(lsum, OpSum(), 0.f);
-                if ((lane & 15) == 0 && (lane >> 4) < HPB) lpart[wv * HPB + hl] = lsum;
+                constexpr int kParts = VTOK ? 5 : 1;     // VTOK: and of e * minimum per channel group
+                if constexpr (VTOK) {
+#pragma unroll
+                    for (int gi = 0; gi < 4; ++gi) cm[gi] = row_reduce(cm[gi], OpSum(), 0.f);
+                }
+                if ((lane & 15) == 0 && (lane >> 4) < HPB) {
+                    lpart[wv * kParts * HPB + hl] = lsum;
+                    if constexpr (VTOK) {
+#pragma unroll
+                        for (int gi = 0; gi < 4; ++gi) lpart[(wv * kParts + 1 + gi) * HPB + hl] = cm[gi];
+                    }
+                }
                 __syncthreads();
                 float* redv = reinterpret_cast<float*>(regA);   // [wave][head][channel]
-                if ((lane >> 4) < HPB) matrix_fold<BITS>(acc, redv + (wv * HPB + hl) * kD, lane & 15);
+                if ((lane >> 4) < HPB) {
+                    float* o = redv + (wv * HPB + hl) * kD;
+                    if constexpr (VTOK) matrix_fold_token<BITS>(acc, vunit, o, lane & 15);
+                    else matrix_fold<BITS>(acc, o, lane & 15);
+                }
                 __syncthreads();
                 if (tid < HPB * kD) {
                     const int h = tid / kD, d = tid % kD;
                     float a = 0.f, lh = 0.f;
 #pragma unroll
-                    for (int w = 0; w < kNW; ++w) { a += redv[(w * HPB + h) * kD + d]; lh += lpart[w * HPB + h]; }
-                    o_img = fx[L::F_VSZ + d] * (a - fx[L::F_VSZ + kD + d] * lh);
+                    for (int w = 0; w < kNW; ++w) { a += redv[(w * HPB + h) * kD + d]; lh += lpart[w * kParts * HPB + h]; }
+                    if constexpr (VTOK) {
+                        float cmin = 0.f;
+#pragma unroll
+                        for (int w = 0; w < kNW; ++w) cmin += lpart[(w * kParts + 1 + (d >> 5)) * HPB + h];
+                        o_img = a + cmin;
+                    } else {
+                        o_img = fx[L::F_VSZ + d] * (a - fx[L::F_VSZ + kD + d] * lh);
+                    }
                     if (d == 0) stat[4 * HPB + h] = lh;
                 }
                 __syncthreads();

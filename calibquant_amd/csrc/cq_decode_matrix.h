@@ -6,30 +6,31 @@
 
 namespace cq {
 
-template <int BITS, int HPB, typename DT, int NT, int REGL, bool CHUNKED, bool EXTRAS, int NH>
+template <int BITS, int HPB, typename DT, bool VTOK, int NT, int REGL, bool CHUNKED, bool EXTRAS, int NH>
 static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st) {
-    constexpr int lds = Lay<BITS, HPB, false, NT, REGL, true>::lds_bytes(0);
+    constexpr int lds = Lay<BITS, HPB, VTOK, NT, REGL, true>::lds_bytes(0);
     static_assert(lds <= 64 * 1024, "no raised dynamic-LDS limit needed; two 512-thread workgroups share a compute unit");
     if constexpr (CHUNKED) {
         if (!g.fused) {
-            const DecodeGeom g1 = minmax_geometry(g, 0);
+            const DecodeGeom g1 = minmax_geometry(g, 0);   // (this launch never looks at values)
+            constexpr int lds1 = Lay<BITS, HPB, false, NT, REGL, true>::lds_bytes(0);
             hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, true, false, NT, REGL, true, false, NH, true>),
-                               dim3(units * g.nsplit), dim3(NT), lds, st, g1);
+                               dim3(units * g.nsplit), dim3(NT), lds1, st, g1);
             CQ_LAUNCH_CHECK();
         }
     }
-    hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, false, false, NT, REGL, CHUNKED, EXTRAS, NH, true>), dim3(units * g.nx),
+    hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, false, VTOK, NT, REGL, CHUNKED, EXTRAS, NH, true>), dim3(units * g.nx),
                        dim3(NT), lds, st, g);
     CQ_LAUNCH_CHECK();
     return CQ_OK;
 }
 
 // A chunked launch has one instantiation: what the mask and the row count cost it in registers, it has to spare.
-template <int BITS, int HPB, typename DT, int NT, int REGL, int NH = HPB>
+template <int BITS, int HPB, typename DT, int NT, int REGL, int NH = HPB, bool VTOK = false>
 static int launch_matrix_unit(const DecodeGeom& g, unsigned units, hipStream_t st) {
-    if (g.nsplit > 1) return launch_matrix_one<BITS, HPB, DT, NT, REGL, true, true, NH>(g, units, st);
-    if (g.mask || g.r_dev) return launch_matrix_one<BITS, HPB, DT, NT, REGL, false, true, NH>(g, units, st);
-    return launch_matrix_one<BITS, HPB, DT, NT, REGL, false, false, NH>(g, units, st);
+    if (g.nsplit > 1) return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, true, true, NH>(g, units, st);
+    if (g.mask || g.r_dev) return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, false, true, NH>(g, units, st);
+    return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, false, false, NH>(g, units, st);
 }
 
 template <int BITS, typename DT>
@@ -56,6 +57,23 @@ int launch_matrix(const DecodeGeom& g, int bits, int hpb, int nh, int nt, unsign
     const int rounds = hpb == 4 ? (nt == 512 ? kRegPair : kRegLong) : kRegMost;
     if (g.chunk > rounds * nt || (nt == 512 && hpb == 1)) return CQ_ERR_UNSUPPORTED;
     return bits == 1 ? launch_matrix_bits<1, DT>(g, hpb, nh, nt, units, st) : launch_matrix_bits<2, DT>(g, hpb, nh, nt, units, st);
+}
+
+// Per-token values: 1 024 threads, four heads at 1 bit at most, two at 2 bits.  Four rounds of logits for chunks of up to
+// 4 096 tokens (the sixteen registers more of eight rounds do not fit beside the statistics of the values), eight above.
+template <int BITS, int HPB, typename DT>
+static int launch_token_unit(const DecodeGeom& g, unsigned units, hipStream_t st) {
+    static_assert(Lay<BITS, HPB, true, 1024, 0>::max_chunk() <= kRegPair * 1024, "the plan's chunks fit eight rounds");
+    if (g.chunk <= kRegTwoBit * 1024) return launch_matrix_unit<BITS, HPB, DT, 1024, kRegTwoBit, HPB, true>(g, units, st);
+    return launch_matrix_unit<BITS, HPB, DT, 1024, kRegPair, HPB, true>(g, units, st);
+}
+
+template <typename DT>
+int launch_matrix_token(const DecodeGeom& g, int bits, int hpb, int nt, unsigned units, hipStream_t st) {
+    if (g.chunk > kRegPair * 1024 || nt != 1024 || (bits == 2 && hpb == 4)) return CQ_ERR_UNSUPPORTED;
+    if (bits == 2) return hpb == 2 ? launch_token_unit<2, 2, DT>(g, units, st) : launch_token_unit<2, 1, DT>(g, units, st);
+    if (hpb == 4) return launch_token_unit<1, 4, DT>(g, units, st);
+    return hpb == 2 ? launch_token_unit<1, 2, DT>(g, units, st) : launch_token_unit<1, 1, DT>(g, units, st);
 }
 
 }  // namespace cq

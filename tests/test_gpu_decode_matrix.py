@@ -5,6 +5,7 @@ import pytest
 
 from oracle import cq_oracle as O
 from tests.test_gpu_decode import _oracle, _run
+from tests.test_gpu_token_mode import _token_case
 from tests.util import make_case
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +67,43 @@ def test_infinity_in_one_head_stays_there(ops):
     hit[[5, 9]] = True
     assert np.isnan(got[0, hit]).all()
     _close(got[0, ~hit], want[0, ~hit])
+
+
+def _token_run(ops, c, bits):
+    from tests.util import case_to_gpu, to_np
+    g = case_to_gpu(c, "fp16")
+    out = ops.decode_attn(g["q"], g["ck"], g["cv"], g["sk"], g["zk"], g["sv"], g["zv"], None, None, bits=bits, v_mode="token")
+    want = O.decode_attention(c["q"], c["ck"], c["cv"], c["sk"], c["zk"], c["sv"], c["zv"], None, None, 0, bits, v_token_group=32)
+    return to_np(out), want
+
+
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("case", [
+    # one, two, three, four heads per unit; around a tile, a round (1 024 tokens), four rounds and, beyond, eight
+    (1, 8, 8, 2), (1, 4, 4, 63), (1, 8, 4, 65), (1, 12, 4, 64), (2, 32, 8, 1023), (33, 32, 8, 1025), (1, 8, 2, 4095), (1, 8, 2, 4097), (1, 2, 1, 5001),
+])
+def test_token_values_tile_edges(ops, case, bits):
+    B, Hq, Hkv, T = case
+    print(f"case token matrix {case} bits={bits}", flush=True)
+    _close(*_token_run(ops, _token_case(B, Hq, Hkv, T, 0, bits, "fp16", seed=T), bits))
+
+
+def test_token_values_scales_far_apart(ops):
+    """Every wave takes its grid from the largest scale of a group among its tokens; a group of zero scales has none."""
+    c = _token_case(1, 32, 8, 300, 0, 1, "fp16", seed=3)
+    c["sv"][:, :, 64:128] *= np.float32(2.0 ** -8)
+    c["sv"][:, :, :, 1] = 0.0
+    c["sv"][:, :, 5, 2] *= np.float32(2.0 ** 6)
+    c["sv"] = O.round_to(c["sv"], "fp16")
+    _close(*_token_run(ops, c, 1))
+
+
+def test_token_values_infinite_scale_stays_in_its_group(ops):
+    c = _token_case(1, 32, 8, 200, 0, 1, "fp16", seed=4)
+    got, want = _token_run(ops, c, 1)
+    c["sv"][0, 3, 17, 2] = np.inf
+    hit, _ = _token_run(ops, c, 1)
+    assert not np.isfinite(hit[0, 12:16, 64:96]).any()
+    rest = np.ones(hit.shape, bool)
+    rest[0, 12:16, 64:96] = False
+    assert np.array_equal(hit[rest], got[rest])
