@@ -95,9 +95,8 @@ static void plan_for(const cq_decode_args* a, Plan* p, int nh = HPB) {
     p->ws_cnt = nsplit > 1 ? (static_cast<size_t>(units) * sizeof(unsigned long long) + 255) / 256 * 256 +
                                  static_cast<size_t>(units) * HPB * nsplit * 16 : 0;
     p->fused = false;
-    // The logits go through a buffer where that is less traffic than the main launch reading the packed K rows
-    // again (4 bytes per head and token against the row's 16 or 32 bytes).  Measured at batch 8 x 32 768 tokens,
-    // four heads per unit: 2 bits 108.6 -> 90.9 us with the buffer, 1 bit (equal bytes) 52.3 -> 54.0 us.
+    // (room for the logits, which a two-launch step once handed over here: the kernel recomputes them, callers'
+    // workspaces keep their size)
     const bool hand_over = nsplit > 1 && 16 * BITS > 4 * HPB;
     p->ws_lgt = hand_over ? static_cast<size_t>(units) * a->T * HPB * sizeof(float) : 0;
 }
@@ -200,9 +199,7 @@ static DecodeGeom unit_geometry(const DecodeGeom& g, int nh, int nt) {
     DecodeGeom gm = g;
     gm.G = g.Hq / g.Hkv;
     const int64_t blocks = static_cast<int64_t>(g.B) * g.Hkv * ngroups(gm.G, nh) * g.nx;
-    // (a main launch that reads its logits back has no look-up phase for the first workgroup to get ahead in:
-    // with the priorities the second one would hold the packed-V loop to itself)
-    gm.ncu = (nt == 512 && !g.lgt && !g.fused && blocks <= 2 * static_cast<int64_t>(pair_units())) ? pair_units() : 0;
+    gm.ncu = (nt == 512 && !g.fused && blocks <= 2 * static_cast<int64_t>(pair_units())) ? pair_units() : 0;
     gm.d_ng.set(static_cast<uint32_t>(ngroups(gm.G, nh)));
     gm.d_nx.set(static_cast<uint32_t>(g.nx));
     gm.d_hkv.set(static_cast<uint32_t>(g.Hkv));
@@ -288,9 +285,8 @@ static int decode_entry(const cq_decode_args* a, void* workspace, size_t workspa
     if (a->R > 0 && (!aligned16(a->k_res) || !aligned16(a->v_res) || (a->res_stride_b % 8) ||
                      (a->res_stride_h % 8) || (a->res_stride_r % 8)))
         return CQ_ERR_ALIGN;
-    // the logits buffer is the last part of the workspace; the static scratch does without it when it
-    // does not fit (the main launch then recomputes the logits)
-    const size_t need_min = p.ws_mm + p.ws_part + p.ws_cnt;
+    // (a caller's own workspace for two launches is as large as cq_decode_attn_workspace says)
+    const size_t need = p.ws_mm + p.ws_part + p.ws_cnt + (static_scratch || p.fused ? 0 : p.ws_lgt);
     // One launch when the plan allows it, the caller's own workspace is used (the static entry point allocates
     // nothing, not even the status word) and no earlier launch of this process gave up waiting.
     int* status = nullptr;
@@ -305,11 +301,6 @@ static int decode_entry(const cq_decode_args* a, void* workspace, size_t workspa
             return CQ_ERR_LAUNCH;   // an earlier single-launch step did not complete: its output is not valid
         }
     }
-    bool with_logits = !fused && p.ws_lgt > 0;
-    if (static_scratch && need_min + p.ws_lgt > kScratchBytes) with_logits = false;
-    // (a plan for one launch sizes the caller's workspace without the logits buffer)
-    if (!static_scratch && p.fused && workspace_bytes < need_min + p.ws_lgt) with_logits = false;
-    const size_t need = need_min + (with_logits ? p.ws_lgt : 0);
     if (static_scratch) {
         if (need > kScratchBytes) return CQ_ERR_SCRATCH_LIMIT;
         workspace = nullptr;
@@ -350,12 +341,10 @@ static int decode_entry(const cq_decode_args* a, void* workspace, size_t workspa
     g.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
     uint32_t ep = g_epoch.fetch_add(1, std::memory_order_relaxed) + 1;
     g.epoch = ep ? ep : g_epoch.fetch_add(1, std::memory_order_relaxed) + 1;   // 0 marks an empty counter
-    g.lgt = with_logits ? reinterpret_cast<float*>(static_cast<char*>(workspace) + need_min) : nullptr;
     g.B = a->B; g.Hq = a->Hq; g.Hkv = a->Hkv; g.T = a->T; g.R = a->R; g.S = a->sprompt_len;
     g.nsplit = p.nsplit; g.chunk = p.chunk; g.nx = p.nx;
     g.calib = a->calibrate; g.off_max = a->calib_off_max; g.off_min = a->calib_off_min;
     g.cap = p.cap;
-    g.one = 1.0f;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool vtok = a->v_mode == CQ_V_PER_TOKEN;
     if (a->dtype == CQ_BF16) return dispatch<BF16>(g, p, a->bits, vtok, st);

@@ -11,31 +11,19 @@
 //            packed-V phase ends: each stream is in flight while the phase before
 //            its consumer runs, and no phase starts behind a queue of requests
 //            it does not need.
-//   K side   q.s_k is folded into a byte-indexed partial-sum table in LDS
-//            (one entry per byte position and byte value, HPB floats wide,
-//            zero-point folded in).  A token's logits are NB table look-ups
-//            and adds; the fp16/bf16 K tensor is never materialised.
-//   stats    min / max of the image logits (calibration), then e = exp(w' - M)
-//            in place in LDS.
-//   V side   tokens are taken four at a time: a 16-entry table of subset sums
-//            of their e values is built once per group, every byte column of
-//            the packed V rows is staged byte-transposed (the 4 tokens' bytes of a
-//            column in one dword), a 4-byte dot product turns each bit lane of the
-//            column into a table offset, and the lane adds that table entry.  Scale /
-//            zero-point are applied once at the end.
+//   K side   the codes are small integers: q.s_k goes onto a fixed-point grid, four signed byte digits a value, and a
+//            tile's logits are 8-bit integer MFMAs (see "the step on the matrix cores" below); the fp16/bf16 K tensor
+//            is never materialised.  A thread keeps its logits in registers.
+//   stats    min / max of the image logits (calibration), then e = exp(w' - M).
+//   V side   e (times the token's group scale, for per-token values) as four byte digits against the packed V rows,
+//            on the same MFMAs.  Per-channel scale / zero-point are applied once at the end.
 //   residual the full-precision rows run last as an online-softmax flash-decode in
 //            the same workgroup (packed dot2 for q.K) and are merged at the end.
 //
 // When the chunk does not cover all T tokens (long context or small batch)
 // a first launch computes every chunk's logits and publishes the per-chunk min / max;
-// the main launch recomputes its chunk's logits (or, where the packed K row is more
-// bytes than the logits - 2 bits, or fewer than four heads per unit - reads back what
-// the first launch left in a buffer, fp32, instead of building the table and doing the
-// look-ups again), exponentiates against the global min / max and writes an (m, l, acc)
+// the main launch recomputes its chunk's logits, exponentiates against the global min / max and writes an (m, l, acc)
 // partial; the last workgroup of a unit to get there combines the unit's partials.
-//
-// The matrix-core form (template flag MX: per-channel values, one launch) keeps this order of phases and replaces the
-// look-ups of both sides by 8-bit integer MFMAs; see matrix_query below.
 #pragma once
 #include "cq_common.h"
 
@@ -91,8 +79,6 @@ struct DecodeGeom {
     const int32_t* r_dev;   // optional: residual row count read at run time (R is then the capacity)
     float* mm;    // [B][Hq][nsplit][2] chunk logit min / max
     float* part;  // [B][Hq][nx][kD + 2] partials (m, l, acc)
-    float* lgt;   // chunked launch: [unit][T][HPB] logits, written by the min/max launch and read by the main
-                  // launch instead of its own K look-ups; NULL: the main launch recomputes them
     int* cnt;     // chunked launch: [unit] count of the unit's chunks (+ residual unit) that have written their
                   // partial; the one that finds all the others done merges them
     // Chunked step in ONE launch (every chunk's workgroup resident at once): the chunks of a unit exchange their
@@ -120,23 +106,18 @@ struct DecodeGeom {
     int G;        // query heads per kv head
     int ncu;      // paired launch whose workgroups are all resident from the start (at most two per compute unit):
                   // the number of compute units (the two workgroups of a unit are told apart by it); else 0
-    float one;    // 1.0f, opaque to the compiler: keeps f16 -> f32 accumulation in one mixed-precision FMA
 };
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 constexpr int cmin(int a, int b) { return a < b ? a : b; }
 
-// VTOK: values quantised per token and per group of 32 channels (scale * code + minimum,
-// codes in little-endian 32-bit words, first channel in the lowest bits) instead of per
-// channel.  A token slot then also carries the token's group scales, and every channel
-// group has its own subset-sum tables.
-// REGL > 0: a thread keeps the logits of its tokens (at most REGL rounds of kNT tokens) in registers
-// until the block's min / max are known and writes only e = exp(.) to the token slots, as packed fp16:
-// the slots take half the bytes, which is what lets two 512-thread workgroups share a compute unit's
-// LDS (with the K table built for half of the byte positions at a time), or one 1024-thread workgroup
-// hold a chunk of 9 984 tokens.
-// MX: the matrix-core form (see MatrixStep below).  No tables and no token slots: region A holds one 64-token tile
-// of weights and of packed V rows per wave, later the folds' partials.
+// VTOK: values quantised per token and per group of 32 channels (scale * code + minimum, codes in little-endian
+// 32-bit words, first channel in the lowest bits) instead of per channel.
+// REGL: rounds of kNT tokens whose logits a thread keeps in registers.
+// MX: the layout the kernel runs with: region A holds one 64-token tile of weights and of packed V rows per wave,
+// later the folds' partials.  Without it the struct describes the table layout of the look-up form this kernel had before;
+// plans are still cut with it (max_chunk, and the LDS a plan reports), so that chunks and workspace sizes are the ones
+// callers have laid out: its fields are sizes only.
 template <int BITS, int HPB, bool VTOK = false, int NT_ = 1024, int REGL = 0, bool MX = false> struct Lay {
     static constexpr int kNT = NT_;                 // threads per workgroup
     static constexpr int kNW = kNT / kWave;         // waves per workgroup
@@ -216,44 +197,6 @@ template <int BITS, int HPB, bool VTOK = false, int NT_ = 1024, int REGL = 0, bo
     }
 };
 
-// One exchange step of an integer-key maximum, N values side by side: the N chains are
-// independent, so the cross-lane moves of one fill the wait states of the others.
-template <int N, int CTRL, int ROW_MASK = 0xf>
-__device__ __forceinline__ void max_step(int* k) {
-    constexpr int lo = static_cast<int>(0x80000000u);
-    int t[N];
-#pragma unroll
-    for (int h = 0; h < N; ++h) t[h] = dpp_move_i<CTRL, ROW_MASK>(k[h], lo);
-#pragma unroll
-    for (int h = 0; h < N; ++h) k[h] = max(k[h], t[h]);
-}
-
-// Block-wide maximum of N values (integer keys, see float_key); result wave-uniform.
-// One barrier; `red`: N words that hold the smallest key when the first wave gets here.
-template <int N, int kNW>
-__device__ __forceinline__ void block_max(float* v, float* red) {
-    const int lane = threadIdx.x & 63;
-    int* redi = reinterpret_cast<int*>(red);
-    int k[N];
-#pragma unroll
-    for (int h = 0; h < N; ++h) k[h] = float_key(v[h]);
-    max_step<N, 0xB1>(k);
-    max_step<N, 0x4E>(k);
-    max_step<N, 0x141>(k);
-    max_step<N, 0x140>(k);
-    max_step<N, 0x142, 0xa>(k);
-    max_step<N, 0x143, 0xc>(k);
-    // second stage: the waves' maxima meet in N words of LDS (set to the smallest key before the last barrier
-    // ahead of this call) through one atomic per wave and value
-    if (lane == 63) {   // the last lane holds the wave's maxima
-#pragma unroll
-        for (int h = 0; h < N; ++h) __hip_atomic_fetch_max(redi + h, k[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int h = 0; h < N; ++h) v[h] = key_float(__builtin_amdgcn_readfirstlane(redi[h]));
-}
-
 // Unit decomposition of a 1-D grid.  Consecutive work ids share packed codes
 // (head groups of one kv-head), so when the grid is a multiple of the 8 XCDs
 // the hardware's round-robin placement is undone to keep them on one L2.
@@ -273,28 +216,6 @@ template <> __device__ __forceinline__ float dot2<BF16>(uint32_t a, uint32_t b, 
 }
 template <> __device__ __forceinline__ float dot2<FP16>(uint32_t a, uint32_t b, float c) {
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, a), __builtin_bit_cast(f16x2_t, b), c, false);
-}
-
-template <int N> struct alignas(N * 4) Words { uint32_t w[N]; };
-
-// N dwords at an absolute LDS byte address (N-dword aligned): one ds_read of that width.
-template <int N> __device__ __forceinline__ Words<N> lds_words(uint32_t addr) {
-    typedef uint32_t VT __attribute__((ext_vector_type(N)));
-    const VT v = *(const __attribute__((address_space(3))) VT*)(static_cast<uintptr_t>(addr));
-    Words<N> r;
-#pragma unroll
-    for (int k = 0; k < N; ++k) r.w[k] = v[k];
-    return r;
-}
-
-// N floats at an absolute LDS byte address.
-template <int N> __device__ __forceinline__ Vec<N> lds_floats(uint32_t addr) {
-    typedef float VT __attribute__((ext_vector_type(N)));
-    const VT v = *(const __attribute__((address_space(3))) VT*)(static_cast<uintptr_t>(addr));
-    Vec<N> r;
-#pragma unroll
-    for (int k = 0; k < N; ++k) r.v[k] = v[k];
-    return r;
 }
 
 // A float handed from one workgroup to another inside a launch: device-scope atomic store.
@@ -336,14 +257,7 @@ __device__ __forceinline__ void clear_handover(const DecodeGeom& g, int64_t unit
     if (tid == 0) __hip_atomic_store(g.done64 + unit, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ uint32_t pack_f16(float a, float b) {
-    typedef float f32x2_t __attribute__((ext_vector_type(2)));
-    const f32x2_t v = {a, b};
-    const f16x2_t h = __builtin_convertvector(v, f16x2_t);   // one packed conversion, round to nearest even
-    return __builtin_bit_cast(uint32_t, h);
-}
-
-// ---- the step on the matrix cores (MX) --------------------------------------------------------------
+// ---- the step on the matrix cores --------------------------------------------------------------
 // The codes are small integers, so both contractions run exactly on 8-bit integer MFMAs (16 x 16 x 64): what is not
 // an integer - q.s_k, and the softmax weights - is put on a 32-bit fixed-point grid of its own maximum and split into
 // four signed byte digits.  16 rows of a tile are then four heads times four digits, the columns are tokens (logits)
@@ -583,12 +497,11 @@ template <int BITS> __device__ __forceinline__ void matrix_fold_token(const I4* 
 // left out - six query heads per kv-head (InternLM2-20B) make two exact units of three instead of two units of
 // four that carry two padding heads between them.
 template <int BITS, int HPB, typename DT, bool MINMAX_ONLY, bool VTOK = false, int NT = 1024, int REGL = 0,
-          bool CHUNKED = MINMAX_ONLY, bool EXTRAS = !MINMAX_ONLY, int NH = HPB, bool MX = false>
+          bool CHUNKED = MINMAX_ONLY, bool EXTRAS = !MINMAX_ONLY, int NH = HPB>
 // (four waves per SIMD - at most 128 VGPRs - for either workgroup size: two 512-thread workgroups per compute
 // unit are only resident together within that)
 __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
-    static_assert(!MX || REGL > 0, "matrix-core form: logits in registers");
-    using L = Lay<BITS, HPB, VTOK, NT, REGL, MX>;
+    using L = Lay<BITS, HPB, VTOK, NT, REGL, true>;
     using V = Vec<HPB>;
     constexpr int NB = L::NB;
     constexpr int kNT = L::kNT, kNW = L::kNW, kResTile = L::kResTile;
@@ -596,9 +509,6 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     const int reg_a = L::region_a(g.cap);
     unsigned char* regA = smem;
     float* fx = reinterpret_cast<float*>(smem + reg_a);
-    unsigned char* slots = L::INA ? smem + L::slots_in_a(g.cap) : smem + reg_a + L::FIXED;   // one slot per token of the chunk
-    auto slot = [&](int t) { return slots + t * L::SLOT; };
-    float* wbit = fx + L::F_WBIT;
     float* qsz = fx + L::F_QSZ;
     float* red = fx + L::F_RED;
 
@@ -653,7 +563,6 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     const bool do_res = !MINMAX_ONLY && R > 0 && (!CHUNKED || split == g.nsplit);
     const int t0 = img_unit ? split * g.chunk : 0;
     const int n = img_unit ? min(g.T, t0 + g.chunk) - t0 : 0;
-    const int npad = (n + L::TPW - 1) / L::TPW * L::TPW;
     const float inv_sqrt_d = 0.08838834764831845f;  // 1/sqrt(128)
 
     // ---- entry: the few elements phase 0 needs are requested first; the packed K rows follow
@@ -664,16 +573,11 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     // A unit without packed tokens or without residual rows aims the unused streams
     // at q (always mapped, at least 256 bytes) and never looks at what comes back.
     const bool has_img = n > 0;
-    // chunked launch with a logits buffer: the min/max launch leaves this chunk's logits there and the main
-    // launch takes them from there - no packed K rows, no table, no look-ups of its own
     const int64_t unit = bh * static_cast<int64_t>(g.d_ng.div) + hg;
-    V* gl = reinterpret_cast<V*>(g.lgt) + (unit * g.T + t0);
-    const bool from_gl = !MINMAX_ONLY && !MX && CHUNKED && g.lgt != nullptr && has_img;
-    const bool k_rows = has_img && !from_gl;
     uint32_t q_raw, s_raw, z_raw;
     constexpr bool kVSep = (HPB * kD > kNT - kD);
     uint32_t vs_raw = 0, vz_raw = 0;
-    uint32_t q_raw2 = 0, s_raw2 = 0, z_raw2 = 0;   // MX: the head's other half, for a wave that needs the whole head
+    uint32_t q_raw2, s_raw2, z_raw2;   // the head's other half, for a wave that needs the whole head
     {
         const int h = min(min(tid / kD, HPB - 1), nh - 1), d = tid % kD;   // a padding head repeats the last real one
         const uint16_t* qp = static_cast<const uint16_t*>(g.q) + (static_cast<int64_t>(b) * g.Hq + hq0) * kD;
@@ -685,23 +589,20 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         const uint16_t* zp = has_img ? static_cast<const uint16_t*>((vstat && !VTOK) ? g.vz : g.kz) + bh * kD : qp;
         s_raw = sp[d];
         z_raw = zp[d];
-        if constexpr (MX) {
-            q_raw2 = qp[h * kD + (d ^ 64)];
-            s_raw2 = sp[d ^ 64];
-            z_raw2 = zp[d ^ 64];
-        }
+        q_raw2 = qp[h * kD + (d ^ 64)];
+        s_raw2 = sp[d ^ 64];
+        z_raw2 = zp[d ^ 64];
         if constexpr (kVSep && !VTOK) {
             vs_raw = (has_img ? static_cast<const uint16_t*>(g.vs) + bh * kD : qp)[d];
             vz_raw = (has_img ? static_cast<const uint16_t*>(g.vz) + bh * kD : qp)[d];
         }
     }
     const int64_t code_off = has_img ? (bh * g.T + t0) * NB : 0;   // one offset for both code streams
-    const uint4* ckp = reinterpret_cast<const uint4*>(k_rows ? g.ck + code_off : static_cast<const uint8_t*>(g.q));
+    const uint4* ckp = reinterpret_cast<const uint4*>(has_img ? g.ck + code_off : static_cast<const uint8_t*>(g.q));
     const uint4* cvp = reinterpret_cast<const uint4*>((has_img ? g.cv : static_cast<const uint8_t*>(g.q)) + code_off);
     const U4* cvp4 = reinterpret_cast<const U4*>(cvp);
     const int last_u = has_img ? n * NB / 16 - 1 : 0;   // last valid 16-byte unit of either stream
-    const int last_uk = k_rows ? last_u : 0;
-    const int last_row = k_rows ? n - 1 : 0;
+    const int last_row = has_img ? n - 1 : 0;
     // residual tile: K slice (row = tid / LPR, 128 / LPR elements); V: a wave owns RPW rows of the tile and a
     // lane one channel pair of each of them, so the value products need no fold inside the wave
     constexpr int LPR = L::LPR, NKP = L::NKP, RPW = L::RPW;
@@ -743,23 +644,8 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             const float s = Cvt<DT>::to_float(s_raw);
             const float z = Cvt<DT>::to_float(z_raw);
             const float qs = qv * s;
-            if constexpr (MX) {
-                matrix_query<BITS>(qs, qs * z, Cvt<DT>::to_float(q_raw2) * inv_sqrt_d, Cvt<DT>::to_float(s_raw2),
-                                   Cvt<DT>::to_float(z_raw2), h, d, regA, qsz);
-            } else {
-            // zero-point term of the byte position: sum of q s z over the channels of one byte
-            // (consecutive lanes), kept [byte position][head]
-            constexpr int cpb0 = 8 / BITS;
-            const float zsum = (cpb0 == 8) ? oct_reduce(qs * z, OpSum(), 0.f) : quad_reduce(qs * z, OpSum(), 0.f);
-            if (d % cpb0 == 0) qsz[(d / cpb0) * HPB + h] = zsum;
-            if constexpr (BITS == 1) {
-                wbit[((7 - (d & 7)) * NB + (d >> 3)) * HPB + h] = qs;   // [bit][byte position][head]
-            } else {
-                const int sh = 6 - 2 * (d & 3);
-                wbit[(sh * NB + (d >> 2)) * HPB + h] = qs;
-                wbit[((sh + 1) * NB + (d >> 2)) * HPB + h] = 2.0f * qs;
-            }
-            }
+            matrix_query<BITS>(qs, qs * z, Cvt<DT>::to_float(q_raw2) * inv_sqrt_d, Cvt<DT>::to_float(s_raw2),
+                               Cvt<DT>::to_float(z_raw2), h, d, regA, qsz);
         }
     }
     if constexpr (kVSep) {
@@ -783,18 +669,15 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     for (int r = 0; r < L::KR; ++r) {
 #pragma unroll
         for (int i = 0; i < BITS; ++i)
-            kc[r][i] = MX ? ckp[min(tid + r * kNT, last_row) * BITS + i] : ckp[min((tid + r * kNT) * BITS + i, last_uk)];
+            kc[r][i] = ckp[min(tid + r * kNT, last_row) * BITS + i];
     }
     // Chunked launch: the chunks' logit min / max, lane s the pair of chunk s for every head (all in flight
-    // together; they are folded across the wave where the calibration needs them), and - with a logits
-    // buffer and the logits in registers - this thread's logits.
+    // together; they are folded across the wave where the calibration needs them).
     struct alignas(8) MinMax { float lo, hi; };
     MinMax mraw[HPB];
-    // REGL: the logits of this thread's tokens, round r = token tid + r * kNT
-    V lg[REGL > 0 && !MX ? REGL : 1];
-    // MX: round rd's 64 tokens of a wave start at 64 * wv + rd * kNT; lane (x, h) = (lane & 15, lane >> 4) has the
+    // Logits: round rd's 64 tokens of a wave start at 64 * wv + rd * kNT; lane (x, h) = (lane & 15, lane >> 4) has the
     // logits of head h for the tokens 16 j + x of them
-    float lx[MX ? REGL : 1][4];
+    float lx[REGL][4];
     if constexpr (!MINMAX_ONLY) {
         if (CHUNKED && has_img && !g.fused) {
 #pragma unroll
@@ -802,12 +685,6 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 const MinMax* p = reinterpret_cast<const MinMax*>(g.mm) +
                                   (static_cast<int64_t>(b) * g.Hq + hq0 + min(h, nh - 1)) * g.nsplit;
                 mraw[h] = p[min(lane, g.nsplit - 1)];
-            }
-        }
-        if constexpr (REGL > 0 && !MX) {
-            if (from_gl) {
-#pragma unroll
-                for (int rd = 0; rd < REGL; ++rd) lg[rd] = gl[min(tid + rd * kNT, n - 1)];
             }
         }
     }
@@ -818,451 +695,82 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     float mn[HPB], mx[HPB];
 #pragma unroll
     for (int h = 0; h < HPB; ++h) { mn[h] = h < NH ? INFINITY : 0.f; mx[h] = h < NH ? -INFINITY : 0.f; }
-    // logits (later: calibrated, masked logits) of a token: in its slot, or in the thread's registers
-    auto load_logits = [&](int rd, int tt) {
-        if constexpr (REGL > 0 && !MX) return lg[rd];
-        else return *reinterpret_cast<const V*>(slot(tt));
-    };
-    auto store_logits = [&](int rd, int tt, const V& w) {
-        if constexpr (REGL > 0 && !MX) lg[rd] = w;
-        else *reinterpret_cast<V*>(slot(tt)) = w;
-    };
-    // f(round, token) for the thread's tokens below lim; with REGL the rounds are unrolled so that
-    // lg[] is indexed by constants
-    auto for_my_tokens = [&](int lim, auto&& f) {
-        if constexpr (REGL > 0) {
-#pragma unroll
-            for (int rd = 0; rd < REGL; ++rd) {
-                const int tt = tid + rd * kNT;
-                if (tt < lim) f(rd, tt);
-            }
-        } else {
-            for (int tt = tid; tt < lim; tt += kNT) f(0, tt);
-        }
-    };
     // First block of packed V rows: half of it is requested here, behind the packed K rows, the
     // rest as the K registers free up, so it has arrived when the logits are done.
-    constexpr int kVF = MX ? (VTOK ? (REGL > 4 ? 1 : 2) * BITS : kMatrixV) : kPF;   // 16-byte pieces of packed V rows in flight per thread
+    constexpr int kVF = VTOK ? (REGL > 4 ? 1 : 2) * BITS : kMatrixV;   // 16-byte pieces of packed V rows in flight per thread
     U4 vc[kVF];
     auto request_v = [&](int r) { vc[r] = cvp4[min((tid + (r / BITS) * kNT) * BITS + r % BITS, last_u)]; };
-    constexpr int kVEarly = MX ? (VTOK ? BITS : kMatrixE) : kPF / 2;
+    constexpr int kVEarly = VTOK ? BITS : kMatrixE;
     if constexpr (!MINMAX_ONLY) {
 #pragma unroll
         for (int r = 0; r < kVEarly; ++r) request_v(r);
     }
 
-    if (from_gl) {
-        // (the look-up rounds, which request the rest of the first packed V block as they go, do not run)
-#pragma unroll
-        for (int r = kVEarly; r < kPF; ++r) request_v(r);
-        if constexpr (REGL == 0) for_my_tokens(n, [&](int rd, int tt) { store_logits(rd, tt, gl[tt]); });
-    }
     CQ_PHASE(2);   // q, per-bit weights, first packed K rows requested
-    // MX: the wave's first token, and the head whose results this lane holds (lanes beyond the unit's heads repeat
+    // the wave's first token, and the head whose results this lane holds (lanes beyond the unit's heads repeat
     // the last one)
     const int wt0 = __builtin_amdgcn_readfirstlane(tid);
     const int hl = min(lane >> 4, HPB - 1);
-    // MX with per-token values: the chunk's scales and minima, four 16-bit values a token; the wave's grids
+    // per-token values: the chunk's scales and minima, four 16-bit values a token; the wave's grids
     const U2* vsp = reinterpret_cast<const U2*>(has_img ? static_cast<const uint16_t*>(g.vs) + (bh * g.T + t0) * 4 : static_cast<const uint16_t*>(g.q));
     const U2* vmp = reinterpret_cast<const U2*>(has_img ? static_cast<const uint16_t*>(g.vz) + (bh * g.T + t0) * 4 : static_cast<const uint16_t*>(g.q));
     float vpw[4] = {0.f, 0.f, 0.f, 0.f}, vunit[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (MX) {
-        if (k_rows) {
-            const I4* aq = reinterpret_cast<const I4*>(regA);
-            const I4 a0 = aq[lane], a1 = aq[64 + lane];
-            const float inv = qsz[2 * hl], zs = qsz[2 * hl + 1];
-            float lo = INFINITY, hi = -INFINITY;
-            phase_priority(std::integral_constant<int, 1>{});
+    if (has_img) {
+        const I4* aq = reinterpret_cast<const I4*>(regA);
+        const I4 a0 = aq[lane], a1 = aq[64 + lane];
+        const float inv = qsz[2 * hl], zs = qsz[2 * hl + 1];
+        float lo = INFINITY, hi = -INFINITY;
+        phase_priority(std::integral_constant<int, 1>{});
+#pragma unroll
+        for (int rd = 0; rd < REGL; ++rd) {
+            if (wt0 + rd * kNT < n) {
+                matrix_logits<BITS>(kc[rd % L::KR], a0, a1, inv, zs, lx[rd]);
+                if (rd + L::KR < REGL) {
+#pragma unroll
+                    for (int i = 0; i < BITS; ++i) kc[rd % L::KR][i] = ckp[min(tid + (rd + L::KR) * kNT, last_row) * BITS + i];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) { lo = fminf(lo, lx[rd][j]); hi = fmaxf(hi, lx[rd][j]); }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (!MINMAX_ONLY && rd < kVF - kVEarly) request_v(kVEarly + rd);   // the rest of the first packed V rows
+        }
+        phase_priority(std::integral_constant<int, 2>{});
+        if constexpr (VTOK && !MINMAX_ONLY) {
+            // the largest scale of every group among the wave's tokens (bit patterns: the sign cleared)
+            uint32_t t0s = 0, t1s = 0, t2s = 0, t3s = 0;
 #pragma unroll
             for (int rd = 0; rd < REGL; ++rd) {
                 if (wt0 + rd * kNT < n) {
-                    matrix_logits<BITS>(kc[rd % L::KR], a0, a1, inv, zs, lx[rd]);
-                    if (rd + L::KR < REGL) {
-#pragma unroll
-                        for (int i = 0; i < BITS; ++i) kc[rd % L::KR][i] = ckp[min(tid + (rd + L::KR) * kNT, last_row) * BITS + i];
-                    }
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) { lo = fminf(lo, lx[rd][j]); hi = fmaxf(hi, lx[rd][j]); }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                if (!MINMAX_ONLY && rd < kVF - kVEarly) request_v(kVEarly + rd);   // the rest of the first packed V rows
-            }
-            phase_priority(std::integral_constant<int, 2>{});
-            if constexpr (VTOK && !MINMAX_ONLY) {
-                // the largest scale of every group among the wave's tokens (bit patterns: the sign cleared)
-                uint32_t t0s = 0, t1s = 0, t2s = 0, t3s = 0;
-#pragma unroll
-                for (int rd = 0; rd < REGL; ++rd) {
-                    if (wt0 + rd * kNT < n) {
-                        const U2 t = vsp[min(tid + rd * kNT, n - 1)];
-                        t0s = max(t0s, t.x & 0x7fffu); t1s = max(t1s, (t.x >> 16) & 0x7fffu);
-                        t2s = max(t2s, t.y & 0x7fffu); t3s = max(t3s, (t.y >> 16) & 0x7fffu);
-                    }
-                }
-                const uint32_t ts[4] = {t0s, t1s, t2s, t3s};
-#pragma unroll
-                for (int gi = 0; gi < 4; ++gi) {
-                    const float f = Cvt<DT>::to_float(static_cast<uint16_t>(wave_max_key(static_cast<int>(ts[gi]))));
-                    const int bits = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f));
-                    const int e = max((bits >> 23) - 126, -90);   // the largest lies in [2^(e-1), 2^e)
-                    vpw[gi] = __builtin_bit_cast(float, (30 - e + 127) << 23);
-                    // an infinity or a NaN among them makes the group's sums NaN
-                    vunit[gi] = bits >= 0x7f800000 ? __builtin_nanf("") : __builtin_bit_cast(float, (e - 30 + 127) << 23);
+                    const U2 t = vsp[min(tid + rd * kNT, n - 1)];
+                    t0s = max(t0s, t.x & 0x7fffu); t1s = max(t1s, (t.x >> 16) & 0x7fffu);
+                    t2s = max(t2s, t.y & 0x7fffu); t3s = max(t3s, (t.y >> 16) & 0x7fffu);
                 }
             }
-            // the waves' minima and maxima meet in LDS, as in block_max, from one lane per head
-            const int klo = row_max_key(float_key(-lo)), khi = row_max_key(float_key(hi));
-            int* redi = reinterpret_cast<int*>(red);
-            if ((lane & 15) == 0 && (lane >> 4) < HPB) {
-                __hip_atomic_fetch_max(redi + hl, klo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_max(redi + HPB + hl, khi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
-            __syncthreads();
+            const uint32_t ts[4] = {t0s, t1s, t2s, t3s};
 #pragma unroll
-            for (int h = 0; h < HPB; ++h) {
-                mn[h] = -key_float(__builtin_amdgcn_readfirstlane(redi[h]));
-                mx[h] = key_float(__builtin_amdgcn_readfirstlane(redi[HPB + h]));
+            for (int gi = 0; gi < 4; ++gi) {
+                const float f = Cvt<DT>::to_float(static_cast<uint16_t>(wave_max_key(static_cast<int>(ts[gi]))));
+                const int bits = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f));
+                const int e = max((bits >> 23) - 126, -90);   // the largest lies in [2^(e-1), 2^e)
+                vpw[gi] = __builtin_bit_cast(float, (30 - e + 127) << 23);
+                // an infinity or a NaN among them makes the group's sums NaN
+                vunit[gi] = bits >= 0x7f800000 ? __builtin_nanf("") : __builtin_bit_cast(float, (e - 30 + 127) << 23);
             }
         }
-    } else {
-    if (k_rows) {
-        // ---- phase 2: byte table = high-nibble table + low-nibble table ----------------
-        // nibble tables: entry (j, half, v) = sum of the per-bit weights v selects; the
-        // zero-point sum of the byte position is folded into the high half.
-        V* nib = REGL > 0 ? reinterpret_cast<V*>(slots) : reinterpret_cast<V*>(fx + L::F_NIB);   // [half*16 + value][byte position]
-        V* ktab = reinterpret_cast<V*>(regA);           // [byte value][byte position]
-        if constexpr (!L::INA)
-        for (int e = tid; e < NB * 32; e += kNT) {
-            const int j = e % NB, half = (e / NB) >> 4, v = (e / NB) & 15;
-            // position-fastest: the lanes of a wave read consecutive entries
-            const V* wb = reinterpret_cast<const V*>(wbit) + half * 4 * NB + j;
-            V acc;
-            const V zs = reinterpret_cast<const V*>(qsz)[j];
-#pragma unroll
-            for (int h = 0; h < HPB; ++h) acc.v[h] = half ? -zs.v[h] : 0.f;
-#pragma unroll
-            for (int bt = 0; bt < 4; ++bt) {
-                const V w4 = wb[bt * NB];
-                const float f = static_cast<float>((v >> bt) & 1);
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) acc.v[h] += f * w4.v[h];
-            }
-            nib[e] = acc;
+        // the waves' minima and maxima meet in LDS, as in block_max, from one lane per head
+        const int klo = row_max_key(float_key(-lo)), khi = row_max_key(float_key(hi));
+        int* redi = reinterpret_cast<int*>(red);
+        if ((lane & 15) == 0 && (lane >> 4) < HPB) {
+            __hip_atomic_fetch_max(redi + hl, klo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_fetch_max(redi + HPB + hl, khi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
-        if constexpr (!L::INA) __syncthreads();
-
-        phase_priority(std::integral_constant<int, 1>{});
-        // ---- phase 3: logits of the chunk ------------------------------------------------
-        // Lane l walks the byte positions of a pass in the order k ^ (l mod NBP): in every step
-        // the lanes that the LDS serves together read NBP distinct positions of the
-        // position-fastest table, i.e. distinct banks whatever the byte values are.  The
-        // row is permuted by the same XOR once, so step k finds its byte at a fixed place.
-        // The NBP terms are added as a balanced binary tree over k; an XOR of the leaf index
-        // only swaps the two children of some tree levels, so every lane gets bit-identical
-        // logits for identical rows.
-        constexpr int NBP = L::NBP;
-        constexpr int NW32 = NBP / 4;
-        const int skew = lane % NBP;
-        // byte i of a word <- byte i ^ (skew & 3)
-        const uint32_t bsel = (0x03020100u ^ (0x01010101u * (skew & 3)));
-        uint32_t pofs[NBP];   // byte offset of position k ^ skew inside a table row
+        __syncthreads();
 #pragma unroll
-        for (int k = 0; k < NBP; ++k) pofs[k] = (k ^ skew) * L::ESZ;
-        const unsigned char* ktab_b = regA;
-        // With 256-byte table rows the address of a look-up is two bytes side by side, the
-        // byte value above the position offset: one byte permute builds it from the row word
-        // and a word holding four position offsets.
-        constexpr bool kPermAddr = (NBP * L::ESZ == 256);
-        uint32_t pofs4[NBP / 4];
-#pragma unroll
-        for (int i = 0; i < NBP / 4; ++i)
-            pofs4[i] = pofs[4 * i] | (pofs[4 * i + 1] << 8) | (pofs[4 * i + 2] << 16) | (pofs[4 * i + 3] << 24);
-        // c: the L::PCS 16-byte pieces of the row that pass P looks at; rd: the token's round (REGL)
-        // kLateMM (one table pass, logits in registers): a wave works out a round's logits for all its lanes as soon
-        // as its first lane has a token - the lanes past the chunk's end hold a copy of its last row (clamped
-        // request) and get that token's logits - so the min / max can be taken afterwards over the registers, two
-        // rounds per instruction, with no lane left out.
-        constexpr bool kLateMM = L::KPASS == 1 && REGL > 0 && !MINMAX_ONLY;
-        // a table entry: the NH live floats of it (12 bytes at three heads)
-        auto lds_entry = [&](uint32_t addr) {
-            V r;
-            if constexpr (NH == HPB) {
-                r = lds_floats<HPB>(addr);
-            } else {
-                typedef float VT __attribute__((ext_vector_type(NH)));
-                const VT v = *(const __attribute__((address_space(3))) VT*)(static_cast<uintptr_t>(addr));
-#pragma unroll
-                for (int k = 0; k < HPB; ++k) r.v[k] = k < NH ? v[k < NH ? k : 0] : 0.f;
-            }
-            return r;
-        };
-        auto token_logits = [&](auto pass_c, int rd, int tt, const uint4* c) {
-            constexpr int P = decltype(pass_c)::value;
-            if (kLateMM ? (__builtin_amdgcn_readfirstlane(tt) < n) : (tt < n)) {
-                constexpr int WO = (P * L::WPP) % 4;   // the pass's first word inside its first piece
-                uint32_t w[NW32];
-#pragma unroll
-                for (int i = 0; i < NW32; ++i) {
-                    const uint4& pc = c[(WO + i) / 4];
-                    const int k4 = (WO + i) % 4;
-                    w[i] = k4 == 0 ? pc.x : k4 == 1 ? pc.y : k4 == 2 ? pc.z : pc.w;
-                }
-#pragma unroll
-                for (int st = 0; (1 << st) < NW32; ++st) {   // word i <- word i ^ (skew / 4)
-                    const bool on = ((skew >> 2) >> st) & 1;
-                    uint32_t t[NW32];
-#pragma unroll
-                    for (int i = 0; i < NW32; ++i) t[i] = w[i ^ (1 << st)];
-#pragma unroll
-                    for (int i = 0; i < NW32; ++i) w[i] = on ? t[i] : w[i];
-                }
-                uint32_t wds[NW32];
-#pragma unroll
-                for (int i = 0; i < NW32; ++i) wds[i] = __builtin_amdgcn_perm(w[i], w[i], bsel);
-                // balanced-tree sum with a small stack of partial sums (level l holds 2^l terms)
-                V part[6];
-#pragma unroll
-                for (int k = 0; k < NBP; ++k) {
-                    V cur;
-                    if constexpr (kPermAddr) {
-                        const uint32_t sel = static_cast<uint32_t>(k & 3) | (static_cast<uint32_t>(4 + (k & 3)) << 8) | 0x0c0c0000u;
-                        // The kernel's only LDS object is the dynamic array, so it starts at LDS
-                        // address 0 and the K table with it (the host checks that the kernel has no
-                        // static LDS before the first launch): the permute result is the address.
-                        cur = lds_entry(__builtin_amdgcn_perm(wds[k >> 2], pofs4[k >> 2], sel));
-                    } else {
-                        const uint32_t byte = (wds[k >> 2] >> (8 * (k & 3))) & 0xffu;
-                        cur = *reinterpret_cast<const V*>(ktab_b + byte * (NBP * L::ESZ) + pofs[k]);
-                    }
-#pragma unroll
-                    for (int l = 0; l < 6; ++l) {
-                        if ((k >> l) & 1) {
-#pragma unroll
-                            for (int h = 0; h < NH; ++h) cur.v[h] += part[l].v[h];
-                        } else {
-                            part[l] = cur;
-                            break;
-                        }
-                    }
-                    if (k == NBP - 1) part[5] = cur;
-                    // keep at most 8 look-ups in flight: bounds the registers this loop needs
-                    if ((k & 7) == 7) __builtin_amdgcn_sched_barrier(0);
-                }
-                V acc = part[5];
-                if constexpr (P > 0) {   // add the earlier pass's partial
-                    const V prev = load_logits(rd, tt);
-#pragma unroll
-                    for (int h = 0; h < NH; ++h) acc.v[h] += prev.v[h];
-                }
-#pragma unroll
-                for (int h = NH; h < HPB; ++h) acc.v[h] = 0.f;   // dead lanes of the entry
-                if constexpr (!MINMAX_ONLY || P + 1 < L::KPASS) store_logits(rd, tt, acc);
-                if constexpr (MINMAX_ONLY && P + 1 == L::KPASS) {
-                    if (g.lgt) gl[tt] = acc;   // for the main launch
-                }
-                if constexpr (P + 1 == L::KPASS && !kLateMM) {
-#pragma unroll
-                    for (int h = 0; h < NH; ++h) { mn[h] = fminf(mn[h], acc.v[h]); mx[h] = fmaxf(mx[h], acc.v[h]); }
-                }
-            }
-        };
-        // The min/max launch has no value rows, tables or sums to keep: with the logits in registers it also keeps
-        // the packed K rows of all its tokens there across the table passes instead of requesting, in every pass, the
-        // 16-byte piece that pass looks at (at 2 bits, four passes: 214 MB fetched for 67 MB of rows at batch 8 x
-        // 32 768 - the rows of the 512 workgroups in flight do not fit the L2s between two passes).
-        constexpr bool kKeepRows = MINMAX_ONLY && REGL > 0 && L::KPASS > 1;
-        uint4 kall[kKeepRows ? REGL : 1][BITS];
-        // Two table passes in a paired workgroup (2 bits): the first pass requests whole rows and keeps the
-        // 16-byte piece the second pass looks at in registers - requested one piece per pass, every 32-byte row
-        // would cross the memory system twice (a piece is half a row, and memory is fetched by the row or more).
-        constexpr bool kKeepHalf = !MINMAX_ONLY && L::INA && L::KPASS == 2 && BITS == 2 && !kKeepRows;
-        uint4 khalf[kKeepHalf ? REGL : 1];
-        auto k_pass = [&](auto pass_c) {
-            constexpr int P = decltype(pass_c)::value;
-            constexpr int kP0 = (P * L::WPP) / 4;   // first 16-byte piece of a row the pass looks at
-            if constexpr (L::INA) {
-                // Straight from the per-bit weights: a thread owns (position, high nibble, bit 3) and writes the
-                // eight entries of the low three bits - the part common to all eight first, then one or two adds
-                // per entry; a wave writes four whole 256-byte rows at a time.
-                static_assert(!L::INA || (NBP == 16 && kNT == 512), "thread mapping of the direct table build");
-                const int pos = tid & 15, hv = (tid >> 4) & 15, b3 = tid >> 8;
-                const V* wb = reinterpret_cast<const V*>(wbit) + P * NBP + pos;
-                const V zs = reinterpret_cast<const V*>(qsz)[P * NBP + pos];
-                V base;
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) base.v[h] = -zs.v[h];
-#pragma unroll
-                for (int bt = 3; bt < 8; ++bt) {
-                    const V w4 = wb[bt * NB];
-                    const float f = static_cast<float>(bt == 3 ? b3 : (hv >> (bt - 4)) & 1);
-#pragma unroll
-                    for (int h = 0; h < HPB; ++h) base.v[h] += f * w4.v[h];
-                }
-                const V w0 = wb[0], w1 = wb[NB], w2 = wb[2 * NB];
-                V hp[2], p01;
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) {
-                    hp[0].v[h] = base.v[h];
-                    hp[1].v[h] = base.v[h] + w2.v[h];
-                    p01.v[h] = w0.v[h] + w1.v[h];
-                }
-                V* row = ktab + (hv * 16 + b3 * 8) * NBP + pos;
-#pragma unroll
-                for (int l = 0; l < 8; ++l) {
-                    V o = hp[l >> 2];
-                    if ((l & 3) != 0) {
-                        const V& ad = (l & 3) == 1 ? w0 : (l & 3) == 2 ? w1 : p01;
-#pragma unroll
-                        for (int h = 0; h < HPB; ++h) o.v[h] += ad.v[h];
-                    }
-                    row[l * NBP] = o;
-                }
-            } else {
-            // byte table of the pass's positions = high-nibble table + low-nibble table
-            for (int e = tid; e < NBP * 256; e += kNT) {
-                const int j = P * NBP + e % NBP, v = e / NBP;
-                const V hi = nib[(16 + (v >> 4)) * NB + j];
-                const V lo = nib[(v & 15) * NB + j];
-                V o;
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) o.v[h] = hi.v[h] + lo.v[h];
-                ktab[e] = o;
-            }
-            }
-            __syncthreads();
-            // One table pass, logits in registers: the rows stream through the KR row registers - when a
-            // round's row has been looked up its registers take the row of KR rounds later, so KR rounds
-            // are in flight while one is worked on and no batch of rows is waited for as a whole.
-            constexpr bool kRotate = L::KPASS == 1 && REGL > 0;
-            if constexpr (kRotate) {
-                static_assert(!kRotate || BITS == 1, "one 16-byte piece per row");
-#pragma unroll
-                for (int rd = 0; rd < REGL; ++rd) {
-                    token_logits(pass_c, rd, tid + rd * kNT, kc[rd % L::KR]);
-                    if (rd + L::KR < REGL) kc[rd % L::KR][0] = ckp[min(tid + (rd + L::KR) * kNT, last_uk)];
-                    if constexpr (!MINMAX_ONLY) {
-                        if (rd < kPF - kVEarly) request_v(kVEarly + rd);   // the rest of the first packed V block
-                    }
-                }
-                if constexpr (kLateMM) {
-                    const int t0w = __builtin_amdgcn_readfirstlane(tid);   // the wave's first token of round 0
-#pragma unroll
-                    for (int rd = 0; rd < REGL; rd += 2) {
-                        if (rd + 1 < REGL && t0w + (rd + 1) * kNT < n) {
-#pragma unroll
-                            for (int h = 0; h < NH; ++h) {
-                                mn[h] = fminf(mn[h], fminf(lg[rd].v[h], lg[rd + 1].v[h]));
-                                mx[h] = fmaxf(mx[h], fmaxf(lg[rd].v[h], lg[rd + 1].v[h]));
-                            }
-                        } else if (t0w + rd * kNT < n) {
-#pragma unroll
-                            for (int h = 0; h < NH; ++h) { mn[h] = fminf(mn[h], lg[rd].v[h]); mx[h] = fmaxf(mx[h], lg[rd].v[h]); }
-                        }
-                    }
-                }
-                return;
-            }
-            // first batch: rows already in registers; each consumed round of the last pass frees
-            // registers that take the first block of packed V rows
-            // (written out round by round with constant indices so vc stays in registers)
-#define CQ_K_ROUND(R)                                                                         \
-            if constexpr (L::KR > (R)) {                                                      \
-                token_logits(pass_c, (R), tid + (R) * kNT, kc[(R)] + kP0);                    \
-                if constexpr (!MINMAX_ONLY && P + 1 == L::KPASS) {                            \
-                    if constexpr (kVEarly + (R) * BITS < kPF) request_v(kVEarly + (R) * BITS);    \
-                    if constexpr (BITS == 2 && kVEarly + (R) * BITS + 1 < kPF) request_v(kVEarly + (R) * BITS + 1); \
-                }                                                                             \
-            }
-            CQ_K_ROUND(0)
-            CQ_K_ROUND(1)
-            CQ_K_ROUND(2)
-            CQ_K_ROUND(3)
-#undef CQ_K_ROUND
-            static_assert(L::KR <= 4, "rounds are written out up to 4");
-            uint4 kx[L::KR][L::PCS];   // rows beyond the first batch: this pass's pieces only
-            if constexpr (kKeepRows) {
-                // whole rows, requested in the first pass and kept for the later ones
-#pragma unroll
-                for (int ob = 1; ob < (REGL + L::KR - 1) / L::KR; ++ob) {
-                    const int tb = ob * kNT * L::KR;
-                    if (tb < n) {
-                        if constexpr (P == 0) {
-#pragma unroll
-                            for (int r = 0; r < L::KR; ++r) {
-                                const int tt = min(tb + tid + r * kNT, n - 1);
-#pragma unroll
-                                for (int i = 0; i < BITS; ++i)
-                                    if (ob * L::KR + r < REGL) kall[ob * L::KR + r][i] = ckp[static_cast<int64_t>(tt) * BITS + i];
-                            }
-                        }
-#pragma unroll
-                        for (int r = 0; r < L::KR; ++r)
-                            if (ob * L::KR + r < REGL)
-                                token_logits(pass_c, ob * L::KR + r, tb + tid + r * kNT, kall[ob * L::KR + r] + kP0);
-                    }
-                }
-            } else if constexpr (REGL > 0) {
-                // batches written out, so that the logits' registers are indexed by constants
-#pragma unroll
-                for (int ob = 1; ob < (REGL + L::KR - 1) / L::KR; ++ob) {
-                    const int tb = ob * kNT * L::KR;
-                    if (tb < n) {
-#pragma unroll
-                        for (int r = 0; r < L::KR; ++r) {
-                            const int tt = min(tb + tid + r * kNT, n - 1);
-                            if constexpr (kKeepHalf) {
-                                static_assert(!kKeepHalf || L::PCS == 1, "a pass looks at one piece of the row");
-                                if constexpr (P == 0) {
-                                    kx[r][0] = ckp[static_cast<int64_t>(tt) * BITS];
-                                    if (ob * L::KR + r < REGL) khalf[ob * L::KR + r] = ckp[static_cast<int64_t>(tt) * BITS + 1];
-                                } else {
-                                    if (ob * L::KR + r < REGL) kx[r][0] = khalf[ob * L::KR + r];
-                                }
-                                continue;
-                            }
-#pragma unroll
-                            for (int i = 0; i < L::PCS; ++i) kx[r][i] = ckp[static_cast<int64_t>(tt) * BITS + kP0 + i];
-                        }
-#pragma unroll
-                        for (int r = 0; r < L::KR; ++r)
-                            if (ob * L::KR + r < REGL) token_logits(pass_c, ob * L::KR + r, tb + tid + r * kNT, kx[r]);
-                    }
-                }
-            } else {
-                for (int tb = kNT * L::KR; tb < n; tb += kNT * L::KR) {
-#pragma unroll
-                    for (int r = 0; r < L::KR; ++r) {
-                        const int tt = min(tb + tid + r * kNT, n - 1);
-#pragma unroll
-                        for (int i = 0; i < L::PCS; ++i) kx[r][i] = ckp[static_cast<int64_t>(tt) * BITS + kP0 + i];
-                    }
-#pragma unroll
-                    for (int r = 0; r < L::KR; ++r) token_logits(pass_c, 0, tb + tid + r * kNT, kx[r]);
-                }
-            }
-        };
-        k_pass(std::integral_constant<int, 0>{});
-        if constexpr (L::KPASS >= 2) {
-            __syncthreads();   // every wave is done with the previous pass's table
-            k_pass(std::integral_constant<int, 1>{});
+        for (int h = 0; h < HPB; ++h) {
+            mn[h] = -key_float(__builtin_amdgcn_readfirstlane(redi[h]));
+            mx[h] = key_float(__builtin_amdgcn_readfirstlane(redi[HPB + h]));
         }
-        if constexpr (L::KPASS == 4) {
-            __syncthreads();
-            k_pass(std::integral_constant<int, 2>{});
-            __syncthreads();
-            k_pass(std::integral_constant<int, 3>{});
-        }
-    }
-    CQ_PHASE(3);   // K table and look-ups
-    phase_priority(std::integral_constant<int, 2>{});
-    if (k_rows) {   // one reduction for both: max of (-min, max)
-        float mm2[2 * HPB];
-#pragma unroll
-        for (int h = 0; h < HPB; ++h) { mm2[h] = -mn[h]; mm2[HPB + h] = mx[h]; }
-        block_max<2 * HPB, kNW>(mm2, red);
-#pragma unroll
-        for (int h = 0; h < HPB; ++h) { mn[h] = -mm2[h]; mx[h] = mm2[HPB + h]; }
-    }
     }
 
     CQ_PHASE(4);   // block min / max
@@ -1286,7 +794,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         if constexpr (CHUNKED) {
             // One launch: this chunk's min / max go out now (write-through stores, waited for, then the arrival
             // count); the other chunks' are collected further down, after the staging of the first V block.
-            if (g.fused && k_rows && tid == 0) {
+            if (g.fused && has_img && tid == 0) {
                 unsigned long long* o = g.rec + ((unit * HPB) * g.nsplit + split) * 2;
                 const unsigned long long tag = static_cast<unsigned long long>(g.epoch) << 32;
 #pragma unroll
@@ -1298,51 +806,6 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         }
 
         if (n > 0) {
-            // The K table is dead: stage the first block of packed V rows in its place
-            // (ordered by the barrier of block_max).  Layout: [unit of TPW tokens]
-            // [byte column][token], so the 4 bytes that the 4 tokens of a group have in one
-            // column form one dword.  A quad of lanes holds a group (tokens are
-            // lane-consecutive): per dword of its 16-byte piece the quad transposes a 4 x 4 byte
-            // block in two exchange steps (lane ^ 1, then lane ^ 2), a byte permute after each,
-            // and lane i ends up with the 4 tokens' bytes of column 4 q + i.
-            unsigned char* vst = regA + L::WTAB;
-            const int qi = lane & 3;
-            // step 1, operands (partner, own): bytes qi and qi ^ 2 of the even and of the odd lane
-            const uint32_t b0 = static_cast<uint32_t>(qi), b2 = static_cast<uint32_t>(qi ^ 2);
-            const uint32_t sel1 = (qi & 1) ? ((4 + b0) | (b0 << 8) | ((4 + b2) << 16) | (b2 << 24))
-                                           : (b0 | ((4 + b0) << 8) | (b2 << 16) | ((4 + b2) << 24));
-            // step 2, operands (partner, own): own low half and the partner's high half, pair 0 first
-            const uint32_t sel2 = (qi & 2) ? 0x01000706u : 0x07060100u;
-            auto stage_piece = [&](U4 c, int tok, int piece, bool write) {
-                const uint32_t w[4] = {c.x, c.y, c.z, c.w};
-                const int base = ((tok / L::TPW) * NB + 16 * piece + qi) * L::TPW + ((tok % L::TPW) & ~3);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t p1 = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w[q]), 0xB1, 0xf, 0xf, true));
-                    const uint32_t a = __builtin_amdgcn_perm(p1, w[q], sel1);
-                    const uint32_t p2 = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(a), 0x4E, 0xf, 0xf, true));
-                    const uint32_t t4 = __builtin_amdgcn_perm(p2, a, sel2);
-                    if (write) *reinterpret_cast<uint32_t*>(vst + base + 4 * q * L::TPW) = t4;
-                }
-            };
-            if constexpr (!MX) {
-                const int vn0 = min(L::VSUB, npad);
-#pragma unroll
-                for (int r = 0; r < kPF; ++r) {
-                    const int tok = tid + (r / BITS) * kNT;
-                    stage_piece(vc[r], tok, r % BITS, tok < vn0);
-                }
-            }
-            // The registers of a staged block take the next block's rows (clamped addresses when there is none):
-            // the block is in flight while the current one is multiplied, instead of being asked for behind a
-            // barrier when the loop gets there.  (The first residual tile requested here as well measured slower.)
-            constexpr bool kVAhead = L::INA;
-            auto request_v_block = [&](int vs0) {
-#pragma unroll
-                for (int r = 0; r < kPF; ++r) vc[r] = cvp4[min((vs0 + tid + (r / BITS) * kNT) * BITS + r % BITS, last_u)];
-            };
-
-            CQ_PHASE(5);   // staging of the first packed V block
             // ---- phase 4: calibration + exp ---------------------------------------------
             if constexpr (CHUNKED) {
                 if (g.fused) {
@@ -1423,7 +886,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     slope[h] = 1.0f;
                 }
             }
-            // a value of the lane's head (MX)
+            // a value of the lane's head
             auto mine = [&](const float* v) {
                 auto uni = [](float f) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f))); };
                 float r = uni(v[0]);   // (wave-uniform: scalar operands, and no array that would be indexed by the lane)
@@ -1431,12 +894,12 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 for (int h = 1; h < HPB; ++h) r = hl == h ? uni(v[h]) : r;
                 return r;
             };
-            if (MX && EXTRAS && g.mask) {
+            if (EXTRAS && g.mask) {
                 const float* mk = g.mask + b * g.mask_sb + g.S + t0;
                 const float mnl = mine(mn), sl = mine(slope), tl = mine(tmin);
                 float top = -INFINITY;
 #pragma unroll
-                for (int rd = 0; rd < (MX ? REGL : 1); ++rd) {
+                for (int rd = 0; rd < REGL; ++rd) {
                     if (wt0 + rd * kNT < n) {
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
@@ -1456,31 +919,10 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     m_img[h] = key_float(__builtin_amdgcn_readfirstlane(redi[h]));
                     slope[h] = 1.0f; tmin[h] = 0.f; mn[h] = 0.f;
                 }
-            } else if (EXTRAS && g.mask) {
-                const float* mk = g.mask + b * g.mask_sb + g.S + t0;
-                float lm[HPB];
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) lm[h] = -INFINITY;
-                for_my_tokens(n, [&](int rd, int tt) {
-                    V w = load_logits(rd, tt);
-                    const float mv = mk[tt];
-#pragma unroll
-                    for (int h = 0; h < HPB; ++h) {
-                        w.v[h] = (w.v[h] - mn[h]) * slope[h] + tmin[h] + mv;
-                        lm[h] = fmaxf(lm[h], w.v[h]);
-                    }
-                    store_logits(rd, tt, w);
-                });
-                block_max<HPB, kNW>(lm, red + 2 * HPB);   // words of its own
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) { m_img[h] = lm[h]; slope[h] = 1.0f; tmin[h] = 0.f; mn[h] = 0.f; }
             } else {
 #pragma unroll
                 for (int h = 0; h < HPB; ++h) m_img[h] = fmaxf(tmin[h], (mx[h] - mn[h]) * slope[h] + tmin[h]);
             }
-            float ls[HPB];
-#pragma unroll
-            for (int h = 0; h < HPB; ++h) ls[h] = 0.f;
             // e = exp(x - M) with x = (w - mn) * slope + tmin, as exp2((w - mn) * ea + ec)
             float ea[HPB], ec[HPB];
 #pragma unroll
@@ -1489,13 +931,6 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 ea[h] = dead ? 0.f : slope[h] * kLog2e;
                 ec[h] = dead ? -INFINITY : (tmin[h] - m_img[h]) * kLog2e;
             }
-            using HWv = Words<L::HW>;
-            // per-token value statistics (VTOK): (T, NGRP) scales and minima of this kv-head
-            const uint16_t* tsc = static_cast<const uint16_t*>(g.vs) + (bh * g.T + t0) * L::NGRP;
-            const uint16_t* tmn = static_cast<const uint16_t*>(g.vz) + (bh * g.T + t0) * L::NGRP;
-            float cma[VTOK ? L::NGRP * HPB : 1];   // sum_t e[t][h] * minimum[t][group], kept [group][head]
-#pragma unroll
-            for (int i = 0; i < (VTOK ? L::NGRP * HPB : 1); ++i) cma[i] = 0.f;
             // With a slope of ordinary size the subtraction folds into the constant: exp2(w * ea + (ec - mn * ea)), one
             // FMA per logit.  A degenerate logit range makes the slope ~1e8, and only the exact zero of (w - mn)
             // keeps the product finite: those units take the two-step form.
@@ -1506,390 +941,97 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 ec2[h] = ec[h] - mn[h] * ea[h];
                 if (h < NH) plain = plain && fabsf(ea[h]) <= 4.0f;
             }
-            if constexpr (MX) {
-                float ec3[HPB], mn3[HPB];
+            float ec3[HPB], mn3[HPB];
 #pragma unroll
-                for (int h = 0; h < HPB; ++h) { ec3[h] = plain ? ec2[h] : ec[h]; mn3[h] = plain ? 0.f : mn[h]; }
-                const float eal = mine(ea), ecl = mine(ec3), mnl = mine(mn3);
-                float lsum = 0.f;
-                I4 acc[8];
+            for (int h = 0; h < HPB; ++h) { ec3[h] = plain ? ec2[h] : ec[h]; mn3[h] = plain ? 0.f : mn[h]; }
+            const float eal = mine(ea), ecl = mine(ec3), mnl = mine(mn3);
+            float lsum = 0.f;
+            I4 acc[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) acc[i] = I4{0, 0, 0, 0};
-                unsigned char* et = regA + wv * L::MXT;
-                constexpr int KV = kVF / BITS;   // rounds of packed V rows in flight
-                U2 ssc[VTOK ? KV : 1], smin[VTOK ? KV : 1];   // VTOK: the statistics of the lane's own tokens, as many rounds ahead
-                float cm[4] = {0.f, 0.f, 0.f, 0.f};
-                if constexpr (VTOK) {
-#pragma unroll
-                    for (int r = 0; r < KV; ++r) {
-                        ssc[r] = vsp[min(tid + r * kNT, n - 1)];
-                        smin[r] = vmp[min(tid + r * kNT, n - 1)];
-                    }
-                }
-                phase_priority(std::integral_constant<int, 3>{});
-#pragma unroll
-                for (int rd = 0; rd < REGL; ++rd) {
-                    const int tw = wt0 + rd * kNT;
-                    if (tw < n) {
-                        float e[4];
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(lx[rd][j] - mnl, eal, ecl));
-                        if (tw + kWave > n) {   // the chunk's last tile: what is past the end weighs nothing
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) e[j] = tw + 16 * j + (lane & 15) < n ? e[j] : 0.f;
-                        }
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) lsum += e[j];
-                        if constexpr (VTOK) {
-                            const U2 a = ssc[rd % KV], m = smin[rd % KV];
-                            matrix_values_token<BITS, DT>(et, e, vc + (rd % KV) * BITS, U4{a.x, m.x, a.y, m.y}, vpw, cm, acc);
-                        } else {
-                            matrix_values<BITS>(et, e, vc + (rd % KV) * BITS, acc);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);   // one round at a time: interleaved, they do not fit the registers
-                        if (rd + KV < REGL) {
-#pragma unroll
-                            for (int i = 0; i < BITS; ++i)
-                                vc[(rd % KV) * BITS + i] = cvp4[min((tid + (rd + KV) * kNT) * BITS + i, last_u)];
-                            if constexpr (VTOK) {
-                                ssc[rd % KV] = vsp[min(tid + (rd + KV) * kNT, n - 1)];
-                                smin[rd % KV] = vmp[min(tid + (rd + KV) * kNT, n - 1)];
-                            }
-                        }
-                    }
-                }
-                phase_priority(std::integral_constant<int, 4>{});
-                load_res_k(0, rk);   // first residual tile's K rows: in flight during the fold below
-                float* lpart = fx + L::F_PRES;   // the waves' sums of e (not in `red`, which a slower wave may still read)
-                lsum = row_reduce(lsum, OpSum(), 0.f);
-                constexpr int kParts = VTOK ? 5 : 1;     // VTOK: and of e * minimum per channel group
-                if constexpr (VTOK) {
-#pragma unroll
-                    for (int gi = 0; gi < 4; ++gi) cm[gi] = row_reduce(cm[gi], OpSum(), 0.f);
-                }
-                if ((lane & 15) == 0 && (lane >> 4) < HPB) {
-                    lpart[wv * kParts * HPB + hl] = lsum;
-                    if constexpr (VTOK) {
-#pragma unroll
-                        for (int gi = 0; gi < 4; ++gi) lpart[(wv * kParts + 1 + gi) * HPB + hl] = cm[gi];
-                    }
-                }
-                __syncthreads();
-                float* redv = reinterpret_cast<float*>(regA);   // [wave][head][channel]
-                if ((lane >> 4) < HPB) {
-                    float* o = redv + (wv * HPB + hl) * kD;
-                    if constexpr (VTOK) matrix_fold_token<BITS>(acc, vunit, o, lane & 15);
-                    else matrix_fold<BITS>(acc, o, lane & 15);
-                }
-                __syncthreads();
-                if (tid < HPB * kD) {
-                    const int h = tid / kD, d = tid % kD;
-                    float a = 0.f, lh = 0.f;
-#pragma unroll
-                    for (int w = 0; w < kNW; ++w) { a += redv[(w * HPB + h) * kD + d]; lh += lpart[w * kParts * HPB + h]; }
-                    if constexpr (VTOK) {
-                        float cmin = 0.f;
-#pragma unroll
-                        for (int w = 0; w < kNW; ++w) cmin += lpart[(w * kParts + 1 + (d >> 5)) * HPB + h];
-                        o_img = a + cmin;
-                    } else {
-                        o_img = fx[L::F_VSZ + d] * (a - fx[L::F_VSZ + kD + d] * lh);
-                    }
-                    if (d == 0) stat[4 * HPB + h] = lh;
-                }
-                __syncthreads();
-            } else {
-            auto exp_tokens = [&](auto fused_c) {
-            constexpr bool kFused = decltype(fused_c)::value;
-            for_my_tokens(npad, [&](int rd, int tt) {
-                float e[4] = {0.f, 0.f, 0.f, 0.f};
-                uint32_t sc2[2] = {0u, 0u};   // the token's group scales as fp16
-                if (tt < n) {
-                    const V w = load_logits(rd, tt);
-#pragma unroll
-                    for (int h = 0; h < NH; ++h) {
-                        if constexpr (kFused) e[h] = __builtin_amdgcn_exp2f(__builtin_fmaf(w.v[h], ea[h], ec2[h]));
-                        else e[h] = __builtin_amdgcn_exp2f((w.v[h] - mn[h]) * ea[h] + ec[h]);
-                        ls[h] += e[h];
-                    }
-                    if constexpr (VTOK) {
-                        const uint2 sr = *reinterpret_cast<const uint2*>(tsc + tt * L::NGRP);
-                        const uint2 mr = *reinterpret_cast<const uint2*>(tmn + tt * L::NGRP);
-                        sc2[0] = pack_f16(Cvt<DT>::lo(sr.x), Cvt<DT>::hi(sr.x));
-                        sc2[1] = pack_f16(Cvt<DT>::lo(sr.y), Cvt<DT>::hi(sr.y));
-                        const float mg[4] = {Cvt<DT>::lo(mr.x), Cvt<DT>::hi(mr.x), Cvt<DT>::lo(mr.y), Cvt<DT>::hi(mr.y)};
-#pragma unroll
-                        for (int gi = 0; gi < L::NGRP; ++gi)
-#pragma unroll
-                            for (int h = 0; h < HPB; ++h) cma[gi * HPB + h] += e[h] * mg[gi];
-                    }
-                }
-                // e as packed fp16 in the first bytes of the token's slot (read by the V tables)
-                HWv hw;
-                hw.w[0] = pack_f16(e[0], e[1]);
-                if constexpr (L::HW == 2) hw.w[1] = pack_f16(e[2], e[3]);
-                *reinterpret_cast<HWv*>(slot(tt)) = hw;
-                if constexpr (VTOK) *reinterpret_cast<uint2*>(slot(tt) + 8) = make_uint2(sc2[0], sc2[1]);
-            });
-            };
-            if (plain) exp_tokens(std::true_type{});
-            else exp_tokens(std::false_type{});
-            // The sums of e (and of e * minimum) are only needed at the very end: each thread
-            // keeps its partial through the packed-V phase and the fold rides on that phase's
-            // closing barriers.
-            __syncthreads();   // publishes e and vst
-            CQ_PHASE(6);   // calibration and exponentials
-            // (requested here, not right after the staging: the logits' registers are free now)
-            if constexpr (kVAhead) request_v_block(L::VSUB);
-
-            // ---- phase 5: packed V ----------------------------------------------------------
-            // lane = (byte column j, slice c of its 8 bit lanes); a wave pass covers TPW tokens
-            unsigned char* wtab = regA + wv * (L::NGRP * L::GPW * 16 * L::ESZH);   // [channel group][token group][16]
-            const int j = lane / L::GPW, cs = lane % L::GPW;
-            const int wvu = __builtin_amdgcn_readfirstlane(wv);
-            const int bg = lane >> 4, be = lane & 15;   // table build: group, entry
-            f16x2_t bsel[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const _Float16 f = static_cast<_Float16>(static_cast<float>((be >> i) & 1));
-                bsel[i] = f16x2_t{f, f};
-            }
-            float acc[L::MPL][HPB];
-#pragma unroll
-            for (int m = 0; m < L::MPL; ++m)
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) acc[m][h] = 0.f;
-            const float one = g.one;
-            // Bit lane m of a byte is bit 7 - m; table offset = sum_i bit(token i) * ESZH * 2^i.
-            // The lane's MPL bit lanes sit in one nibble: the dword is shifted by 4 * (m < 4) once,
-            // each lane masks its bit in place (value 2^s per byte) and the dot-product
-            // multiplier carries the 2^-s: ESZH * 2^i >> s stays integral for s <= 3, ESZH = 8;
-            // with 4-byte entries the multiplier is kept whole and s = 0 (bit moved down first).
-            constexpr bool kInPlace = (L::ESZH == 8);
-            const uint32_t nib_shift = (cs * L::MPL < 4) ? 4u : 0u;
-            uint32_t bmask[L::MPL], bmult[L::MPL], bshr[L::MPL];
-#pragma unroll
-            for (int m = 0; m < L::MPL; ++m) {
-                const uint32_t sft = 3 - ((cs * L::MPL + m) & 3);   // bit position inside the nibble
-                bmask[m] = kInPlace ? (0x01010101u << sft) : 0x01010101u;
-                bmult[m] = kInPlace ? ((L::ESZH * 0x08040201u) >> sft) & 0x7f7f7f7fu : L::ESZH * 0x08040201u;
-                bshr[m] = kInPlace ? 0u : sft;
-            }
-            using WG = Words<L::GPW>;   // the GPW dwords of one (unit, column)
-            // channel group of the lane's byte column (32 channels = 4*BITS columns): lane / 16 for both widths
-            const int cgrp = VTOK ? (lane >> 4) : 0;
-            // absolute LDS address of the wave's tables (the dot product's addend)
-            const uint32_t wtab_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-                (__attribute__((address_space(3))) unsigned char*)wtab));
-
-            phase_priority(std::integral_constant<int, 3>{});
-            for (int vs0 = 0; vs0 < npad; vs0 += L::VSUB) {
-                const int vn = min(L::VSUB, npad - vs0);
-                if (vs0 > 0) {
-                    __syncthreads();  // previous block consumed
-                    if constexpr (!kVAhead) request_v_block(vs0);
-#pragma unroll
-                    for (int r = 0; r < kPF; ++r) {
-                        const int tok = tid + (r / BITS) * kNT;
-                        stage_piece(vc[r], tok, r % BITS, tok < vn);
-                    }
-                    if constexpr (kVAhead) request_v_block(vs0 + L::VSUB);
-                    __syncthreads();
-                }
-                // One pass over the TPW tokens of unit u: the sum of the entries each of the lane's bit lanes picks,
-                // as packed fp16 (GPW entries of at most 4 terms each, added pairwise).
-                struct PreV { HWv e[4]; WG cw; };
-                auto load_pre = [&](int u, PreV& p) {
-                    const int tl = u * L::TPW;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) p.e[i] = *reinterpret_cast<const HWv*>(slot(vs0 + tl + 4 * bg + i));
-                    p.cw = *reinterpret_cast<const WG*>(vst + (u * NB + j) * L::TPW);
-                };
-                // A pass in three steps, so that two passes can be woven together: the table of the second is built and
-                // written while the look-ups of the first are in flight (the LDS executes a wave's instructions in
-                // order: the second table's write lands after the first pass's reads).
-                auto v_build = [&](int u, const PreV& pre) {
-                    const int tl = u * L::TPW;        // token offset inside the block
-                    (void)tl;
-                    if (bg < L::GPW) {
-                        f16x2_t val[L::NGRP][L::HW];
-#pragma unroll
-                        for (int gi = 0; gi < L::NGRP; ++gi)
-#pragma unroll
-                            for (int k = 0; k < L::HW; ++k) val[gi][k] = f16x2_t{0, 0};
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const unsigned char* sl = slot(vs0 + tl + 4 * bg + i);
-                            const HWv e = VTOK ? *reinterpret_cast<const HWv*>(sl) : pre.e[i];
-                            if constexpr (VTOK) {
-                                const uint2 sc = *reinterpret_cast<const uint2*>(sl + 8);
-                                const f16x2_t s01 = __builtin_bit_cast(f16x2_t, sc.x), s23 = __builtin_bit_cast(f16x2_t, sc.y);
-                                const _Float16 sg[4] = {s01.x, s01.y, s23.x, s23.y};
-#pragma unroll
-                                for (int gi = 0; gi < L::NGRP; ++gi) {
-                                    const f16x2_t w2 = bsel[i] * f16x2_t{sg[gi], sg[gi]};
-#pragma unroll
-                                    for (int k = 0; k < L::HW; ++k) val[gi][k] += __builtin_bit_cast(f16x2_t, e.w[k]) * w2;
-                                }
-                            } else {
-#pragma unroll
-                                for (int k = 0; k < L::HW; ++k) val[0][k] += __builtin_bit_cast(f16x2_t, e.w[k]) * bsel[i];
-                            }
-                        }
-#pragma unroll
-                        for (int gi = 0; gi < L::NGRP; ++gi) {
-                            HWv o;
-#pragma unroll
-                            for (int k = 0; k < L::HW; ++k) o.w[k] = __builtin_bit_cast(uint32_t, val[gi][k]);
-                            reinterpret_cast<HWv*>(wtab)[(gi * L::GPW + bg) * 16 + be] = o;
-                        }
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                };
-                auto v_lookups = [&](const WG& cw, f16x2_t (&pk)[L::MPL][L::GPW][L::HW]) {
-#pragma unroll
-                    for (int gq = 0; gq < L::GPW; ++gq) {
-                        const uint32_t tbase = wtab_addr + static_cast<uint32_t>((cgrp * L::GPW + gq) * 16 * L::ESZH);
-                        const uint32_t wsh = cw.w[gq] >> nib_shift;
-#pragma unroll
-                        for (int m = 0; m < L::MPL; ++m) {
-                            const uint32_t bits = (kInPlace ? wsh : (wsh >> bshr[m])) & bmask[m];
-                            const uint32_t off = __builtin_amdgcn_udot4(bits, bmult[m], tbase, false);
-                            const HWv e = lds_words<L::HW>(off);
-#pragma unroll
-                            for (int k = 0; k < L::HW; ++k) pk[m][gq][k] = __builtin_bit_cast(f16x2_t, e.w[k]);
-                        }
-                    }
-                };
-                auto v_reduce = [&](f16x2_t (&pk)[L::MPL][L::GPW][L::HW], f16x2_t (&sum)[L::MPL][L::HW]) {
-#pragma unroll
-                    for (int m = 0; m < L::MPL; ++m) {
-#pragma unroll
-                        for (int st = 1; st < L::GPW; st *= 2)
-#pragma unroll
-                            for (int gq = 0; gq + st < L::GPW; gq += 2 * st)
-#pragma unroll
-                                for (int k = 0; k < L::HW; ++k) pk[m][gq][k] += pk[m][gq + st][k];
-#pragma unroll
-                        for (int k = 0; k < L::HW; ++k) sum[m][k] = pk[m][0][k];
-                    }
-                };
-                auto v_pass = [&](int u, f16x2_t (&sum)[L::MPL][L::HW], const PreV& pre, auto&& after_lookups) {
-                    f16x2_t pk[L::MPL][L::GPW][L::HW];
-                    v_build(u, pre);
-                    v_lookups(pre.cw, pk);
-                    after_lookups();
-                    v_reduce(pk, sum);
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                };
-                // one mixed-precision FMA per head moves a packed sum into the fp32 accumulators
-                auto v_flush = [&](const f16x2_t (&sum)[L::MPL][L::HW]) {
-#pragma unroll
-                    for (int m = 0; m < L::MPL; ++m)
-#pragma unroll
-                        for (int h = 0; h < NH; ++h) {
-                            const f16x2_t pr = sum[m][h >> 1];
-                            const _Float16 hv = (h & 1) ? pr.y : pr.x;
-                            acc[m][h] = __builtin_fmaf(static_cast<float>(hv), one, acc[m][h]);
-                        }
-                };
-                int u = wvu;   // wave-uniform loop control
-                // the slot entries and code words of a pass are read while the pass before it waits for its look-ups
-                PreV cur, nxt;
-                if (u * L::TPW < vn) load_pre(u, cur);
-                {
-                    // two passes per fp32 accumulation: the sums of 2 * TPW tokens meet as packed fp16 first
-                    for (; (u + kNW) * L::TPW < vn; u += 2 * kNW) {
-                        f16x2_t s0[L::MPL][L::HW], s1[L::MPL][L::HW];
-                        f16x2_t pk0[L::MPL][L::GPW][L::HW], pk1[L::MPL][L::GPW][L::HW];
-                        v_build(u, cur);
-                        v_lookups(cur.cw, pk0);
-                        load_pre(u + kNW, nxt);
-                        v_build(u + kNW, nxt);           // (its table write queues behind the look-ups above)
-                        v_lookups(nxt.cw, pk1);
-                        if ((u + 2 * kNW) * L::TPW < vn) load_pre(u + 2 * kNW, cur);
-                        v_reduce(pk0, s0);
-                        v_reduce(pk1, s1);
-                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                        for (int m = 0; m < L::MPL; ++m)
-#pragma unroll
-                            for (int k = 0; k < L::HW; ++k) s0[m][k] += s1[m][k];
-                        v_flush(s0);
-                    }
-                }
-                for (; u * L::TPW < vn; u += kNW) {
-                    f16x2_t s0[L::MPL][L::HW];
-                    v_pass(u, s0, cur, [&]() { if ((u + kNW) * L::TPW < vn) load_pre(u + kNW, cur); });
-                    v_flush(s0);
-                }
-            }
-            CQ_PHASE(7);   // packed-V loop (tables, look-ups, sums; staging of the later blocks)
-            phase_priority(std::integral_constant<int, 4>{});
-            load_res_k(0, rk);   // first residual tile's K rows: in flight during the fold below
-            // per-wave partial sums of e (and of e * minimum), folded by the output threads below
-            constexpr int kSums = VTOK ? (L::NGRP + 1) * HPB : HPB;
-            wave_reduce_n<HPB>(ls, OpSum(), 0.f);
+            for (int i = 0; i < 8; ++i) acc[i] = I4{0, 0, 0, 0};
+            unsigned char* et = regA + wv * L::MXT;
+            constexpr int KV = kVF / BITS;   // rounds of packed V rows in flight
+            U2 ssc[VTOK ? KV : 1], smin[VTOK ? KV : 1];   // VTOK: the statistics of the lane's own tokens, as many rounds ahead
+            float cm[4] = {0.f, 0.f, 0.f, 0.f};
             if constexpr (VTOK) {
 #pragma unroll
-                for (int gi = 0; gi < L::NGRP; ++gi) wave_reduce_n<HPB>(cma + gi * HPB, OpSum(), 0.f);
+                for (int r = 0; r < KV; ++r) {
+                    ssc[r] = vsp[min(tid + r * kNT, n - 1)];
+                    smin[r] = vmp[min(tid + r * kNT, n - 1)];
+                }
             }
-            if (lane == 0) {
+            phase_priority(std::integral_constant<int, 3>{});
 #pragma unroll
-                for (int h = 0; h < HPB; ++h) red[wv * kSums + h] = ls[h];
+            for (int rd = 0; rd < REGL; ++rd) {
+                const int tw = wt0 + rd * kNT;
+                if (tw < n) {
+                    float e[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(lx[rd][j] - mnl, eal, ecl));
+                    if (tw + kWave > n) {   // the chunk's last tile: what is past the end weighs nothing
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) e[j] = tw + 16 * j + (lane & 15) < n ? e[j] : 0.f;
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) lsum += e[j];
+                    if constexpr (VTOK) {
+                        const U2 a = ssc[rd % KV], m = smin[rd % KV];
+                        matrix_values_token<BITS, DT>(et, e, vc + (rd % KV) * BITS, U4{a.x, m.x, a.y, m.y}, vpw, cm, acc);
+                    } else {
+                        matrix_values<BITS>(et, e, vc + (rd % KV) * BITS, acc);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);   // one round at a time: interleaved, they do not fit the registers
+                    if (rd + KV < REGL) {
+#pragma unroll
+                        for (int i = 0; i < BITS; ++i)
+                            vc[(rd % KV) * BITS + i] = cvp4[min((tid + (rd + KV) * kNT) * BITS + i, last_u)];
+                        if constexpr (VTOK) {
+                            ssc[rd % KV] = vsp[min(tid + (rd + KV) * kNT, n - 1)];
+                            smin[rd % KV] = vmp[min(tid + (rd + KV) * kNT, n - 1)];
+                        }
+                    }
+                }
+            }
+            phase_priority(std::integral_constant<int, 4>{});
+            load_res_k(0, rk);   // first residual tile's K rows: in flight during the fold below
+            float* lpart = fx + L::F_PRES;   // the waves' sums of e (not in `red`, which a slower wave may still read)
+            lsum = row_reduce(lsum, OpSum(), 0.f);
+            constexpr int kParts = VTOK ? 5 : 1;     // VTOK: and of e * minimum per channel group
+            if constexpr (VTOK) {
+#pragma unroll
+                for (int gi = 0; gi < 4; ++gi) cm[gi] = row_reduce(cm[gi], OpSum(), 0.f);
+            }
+            if ((lane & 15) == 0 && (lane >> 4) < HPB) {
+                lpart[wv * kParts * HPB + hl] = lsum;
                 if constexpr (VTOK) {
 #pragma unroll
-                    for (int i = 0; i < L::NGRP * HPB; ++i) red[wv * kSums + HPB + i] = cma[i];
+                    for (int gi = 0; gi < 4; ++gi) lpart[(wv * kParts + 1 + gi) * HPB + hl] = cm[gi];
                 }
             }
             __syncthreads();
-            // head-major, so that the fold below reads consecutive words with consecutive lanes
-            float* redv = reinterpret_cast<float*>(regA);  // [wave][head][bit lane]
-#pragma unroll
-            for (int h = 0; h < HPB; ++h) {
-                Vec<L::MPL> a4;
-#pragma unroll
-                for (int m = 0; m < L::MPL; ++m) a4.v[m] = acc[m][h];
-                *reinterpret_cast<Vec<L::MPL>*>(redv + (wv * HPB + h) * L::PC + j * 8 + cs * L::MPL) = a4;
+            float* redv = reinterpret_cast<float*>(regA);   // [wave][head][channel]
+            if ((lane >> 4) < HPB) {
+                float* o = redv + (wv * HPB + hl) * kD;
+                if constexpr (VTOK) matrix_fold_token<BITS>(acc, vunit, o, lane & 15);
+                else matrix_fold<BITS>(acc, o, lane & 15);
             }
             __syncthreads();
             if (tid < HPB * kD) {
                 const int h = tid / kD, d = tid % kD;
-                float a = 0.f;
-                // bit lanes of channel d.  Per-channel codes: first channel of a byte in its top
-                // bits; per-token codes: first channel in the lowest bits.
-                const int per = 8 / BITS;                       // channels per byte
-                const int cb = d / per * 8, c = d % per;
-                const int lane_hi = VTOK ? cb + 8 - BITS * (c + 1) : cb + BITS * c;   // bit lane of the code's top bit
-                if constexpr (BITS == 1) {
+                float a = 0.f, lh = 0.f;
 #pragma unroll
-                    for (int w = 0; w < kNW; ++w) a += redv[(w * HPB + h) * L::PC + lane_hi];
-                } else {
-#pragma unroll
-                    for (int w = 0; w < kNW; ++w)
-                        a += 2.0f * redv[(w * HPB + h) * L::PC + lane_hi] + redv[(w * HPB + h) * L::PC + lane_hi + 1];
-                }
-                float lh = 0.f;   // sum of e of this thread's head
-#pragma unroll
-                for (int w = 0; w < kNW; ++w) lh += red[w * kSums + h];
+                for (int w = 0; w < kNW; ++w) { a += redv[(w * HPB + h) * kD + d]; lh += lpart[w * kParts * HPB + h]; }
                 if constexpr (VTOK) {
-                    float cm = 0.f;   // sum_t e * minimum of the channel's group
+                    float cmin = 0.f;
 #pragma unroll
-                    for (int w = 0; w < kNW; ++w) cm += red[w * kSums + HPB + (d >> 5) * HPB + h];
-                    o_img = a + cm;
+                    for (int w = 0; w < kNW; ++w) cmin += lpart[(w * kParts + 1 + (d >> 5)) * HPB + h];
+                    o_img = a + cmin;
                 } else {
-                    const float s = fx[L::F_VSZ + d];
-                    const float z = fx[L::F_VSZ + kD + d];
-                    o_img = s * (a - z * lh);
+                    o_img = fx[L::F_VSZ + d] * (a - fx[L::F_VSZ + kD + d] * lh);
                 }
                 if (d == 0) stat[4 * HPB + h] = lh;
             }
             __syncthreads();
-            }
         }
 
         if (n == 0) load_res_k(0, rk);

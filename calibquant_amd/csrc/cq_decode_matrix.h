@@ -14,12 +14,12 @@ static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st
         if (!g.fused) {
             const DecodeGeom g1 = minmax_geometry(g, 0);   // (this launch never looks at values)
             constexpr int lds1 = Lay<BITS, HPB, false, NT, REGL, true>::lds_bytes(0);
-            hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, true, false, NT, REGL, true, false, NH, true>),
+            hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, true, false, NT, REGL, true, false, NH>),
                                dim3(units * g.nsplit), dim3(NT), lds1, st, g1);
             CQ_LAUNCH_CHECK();
         }
     }
-    hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, false, VTOK, NT, REGL, CHUNKED, EXTRAS, NH, true>), dim3(units * g.nx),
+    hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, false, VTOK, NT, REGL, CHUNKED, EXTRAS, NH>), dim3(units * g.nx),
                        dim3(NT), lds, st, g);
     CQ_LAUNCH_CHECK();
     return CQ_OK;
