@@ -28,8 +28,8 @@ FLAGS = [
     "-Wall", "-Wno-unused-command-line-argument",
     "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
 ]
-# per-source additions.  The decode kernels are bound by vector-instruction issue: the
-# ILP-first machine scheduler measures 1-3 % faster there (same register counts, no scratch).
+# per-source additions (the profiling build's decode kernel is part of cq_decode.hip; the shipped ones, in
+# cq_decode_matrix*.hip, are scheduled by default)
 EXTRA_FLAGS = {
     "cq_decode.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
 }
