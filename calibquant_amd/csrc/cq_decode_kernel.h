@@ -490,12 +490,11 @@ template <int BITS> __device__ __forceinline__ void matrix_fold_token(const I4* 
 
 // CHUNKED: the launch is one of the two of a chunked step (the min/max launch always is); a single launch carries
 // none of their code.  EXTRAS: an additive mask or a residual row count read from device memory may be present; a
-// call with neither runs an instantiation without their code (32.6-32.8 against 33.5-34.0 us at the benchmark shape:
-// the kernel sits at the register limit of its occupancy, and code that never runs still costs registers).
-// NH: query heads a unit serves, at most HPB.  Tables, slots and partials are laid out HPB heads wide either way
-// (16-byte entries at HPB = 4); with NH = 3 the fourth lane of every entry is dead and the arithmetic on it is
-// left out - six query heads per kv-head (InternLM2-20B) make two exact units of three instead of two units of
-// four that carry two padding heads between them.
+// call with neither runs an instantiation without their code (the kernel sits at the register limit of its occupancy,
+// and code that never runs still costs registers).
+// NH: query heads a unit serves, at most HPB.  Operands and partials are laid out HPB heads wide either way; with
+// NH = 3 the fourth head's rows are padding - six query heads per kv-head (InternLM2-20B) make two exact units of
+// three instead of two units of four that carry two padding heads between them.
 template <int BITS, int HPB, typename DT, bool MINMAX_ONLY, bool VTOK = false, int NT = 1024, int REGL = 0,
           bool CHUNKED = MINMAX_ONLY, bool EXTRAS = !MINMAX_ONLY, int NH = HPB>
 // (four waves per SIMD - at most 128 VGPRs - for either workgroup size: two 512-thread workgroups per compute
@@ -530,7 +529,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     const bool prio_on = NT == 512 && g.ncu > 0;
     const bool second = prio_on && blockIdx.x >= static_cast<unsigned>(g.ncu);
     auto phase_priority = [&](auto phase_c) {
-        constexpr int PH = decltype(phase_c)::value;   // 0 set-up and tables, 1 K look-ups, 2 min/max .. exp, 3 packed V, 4 folds, window, merge
+        constexpr int PH = decltype(phase_c)::value;   // 0 set-up, 1 logits, 2 min/max .. mask, 3 exp and packed V, 4 folds, window, merge
         if constexpr (NT == 512) {
             if (prio_on) {
                 if constexpr (PH == 0 || PH == 2) __builtin_amdgcn_s_setprio(2);
@@ -1229,7 +1228,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     }
 }
 
-// The min/max launch of a two-launch chunked step: no residual unit, and `cap` tokens' worth of slots.
+// The min/max launch of a two-launch chunked step: no residual unit.
 static inline DecodeGeom minmax_geometry(const DecodeGeom& g, int cap) {
     DecodeGeom g1 = g;
     g1.nx = g.nsplit;
