@@ -262,15 +262,20 @@ __device__ __forceinline__ void clear_handover(const DecodeGeom& g, int64_t unit
 // an integer - q.s_k, and the softmax weights - is put on a 32-bit fixed-point grid of its own maximum and split into
 // four signed byte digits.  16 rows of a tile are then four heads times four digits, the columns are tokens (logits)
 // or byte columns of the packed V rows (sums), and a lane of the result holds the four digits' sums of one head:
-// exact integers, put together in fp32.  A byte of packed codes is masked in place - one AND per 4 codes, bit i
-// counts 2^i (the sign bit -2^7), which the fixed-point operand (logits) or the closing fold (sums) takes back.
+// exact integers, put together in fp32.  Packed codes are masked in place, the upper half of a byte after one shift of
+// the word - one AND per 4 codes; a code then counts 2^s, s = 0 .. 3, which the fixed-point operand (logits) or the
+// closing fold (sums) takes back.
 // Measured, us per step, look-up form before and this one: batch 64 x 3 328 + 128, 1 bit 26.4 -> 19.4, 2 bits 47.8 -> 28.2;
 // batch 256 x 3 328 88 -> 55 (49 % of the rate of a large copy); 16 x 9 984, six heads 38.3 -> 23.5; 8 x 32 768 in
 // chunks 35.8 -> 29.0; batch 1 x 1 024 7.7 -> 6.4.  A 64-token tile of four heads takes about 140 vector instructions
 // (1 500 before) and 16 MFMAs; what bounds a launch now is the latency of its phases, then the memory.
-// Error against 64 bits: the grid's 2^-31 (2^-25 of the largest q.s_k at the top bit) and the fp32 roundings; the
-// look-up form added fp32 partial sums on the K side and held the weights as fp16 on the V side (fp16 outputs: 2.0e-4 away
-// from 64 bits here, which is their own rounding, 7e-4 to 1.3e-3 there).
+// Error against 64 bits: a weight is off by 2^-31 at most, a channel's q.s_k by 2^-27 of the head's largest (s = 3 costs
+// three of the grid's bits; masked in place all through, the top bit of a byte would cost seven), then the fp32 roundings.
+// The look-up form added fp32 partial sums on the K side and held the weights as fp16 on the V side.  Root-mean-square
+// logit error over its own (a model of both on the CPU, keys with outlier channels of 1, 10, 100 and 1 000 times the
+// others): 0.59, 0.57, 0.56, 0.55 at 1 bit - 0.93, 1.4, 2.2, 2.8 masked in place -, 0.55, 0.52, 0.56, 0.53 at 2 bits.
+// (The shift costs batch 64 x 3 328 0.25 us at 1 bit and nothing at 2 bits.)
+// fp16 outputs lie 2.0e-4 from 64 bits, which is their own rounding, 7e-4 to 1.3e-3 there.
 typedef int I4 __attribute__((ext_vector_type(4)));
 typedef int I2 __attribute__((ext_vector_type(2)));
 typedef uint32_t U2 __attribute__((ext_vector_type(2)));
@@ -279,6 +284,9 @@ typedef uint32_t U2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t byte_digits(int x) {
     return (static_cast<uint32_t>(x) + 0x00808080u) ^ 0x00808080u;
 }
+
+// what field f (lowest first) of a masked byte of codes counts, as a shift: the upper half-byte's fields are moved down
+template <int BITS> __device__ __forceinline__ constexpr int field_shift(int f) { return (BITS * f) & 3; }
 
 // One channel of one head of q.s_k into the K contraction's left operand: row (head, digit), in the byte that meets
 // the channel's code.  A wave holds one half of a head, the other half's values come along for the common scale and
@@ -291,13 +299,9 @@ __device__ __forceinline__ void matrix_query(float qs, float qsz, float qv2, flo
     const float zs = wave_sum(qsz + qs2 * z2);
     // the largest value lies in [2^(e-1), 2^e); a head that is all but zero keeps a grid of 2^-90
     const int e = max((top >> 23) - 126, -60);
-    // code field -> operand byte: 1 bit: the field is the bit, weight 2^i; 2 bits: fields 0..2 in place, field 3 moved
-    // down onto field 2 (a code in the sign bit would not be linear)
     const int byte = BITS == 1 ? d >> 3 : d >> 2;                  // byte of the packed row
     const int f = BITS == 1 ? 7 - (d & 7) : 3 - (d & 3);           // field of the byte, lowest first
-    const int sh = BITS == 1 ? f : 2 * min(f, 2);
-    float x = qs * __builtin_bit_cast(float, (30 - e + 127) << 23) * __builtin_bit_cast(float, (127 - sh) << 23);
-    if (BITS == 1 && f == 7) x = -x;
+    const float x = qs * __builtin_bit_cast(float, (30 - e + 127) << 23) * __builtin_bit_cast(float, (127 - field_shift<BITS>(f)) << 23);
     const uint32_t dg = byte_digits(__float2int_rn(x));
     const int kg = (byte >> 2) & 3, b = byte & 3, i = BITS == 1 ? f : (byte >> 4) * 4 + f;   // operand dword i = 0 .. 7
     unsigned char* o = regA + ((i >> 2) * 64 + kg * 16 + 4 * h) * 16 + (i & 3) * 4 + b;
@@ -312,13 +316,13 @@ __device__ __forceinline__ void matrix_query(float qs, float qsz, float qv2, flo
 
 // the right operand's dwords of one word of packed codes
 template <int BITS> __device__ __forceinline__ void code_fields(uint32_t w, int* o) {
-    if constexpr (BITS == 1) {
+    constexpr uint32_t kCode = BITS == 1 ? 0x01010101u : 0x03030303u;
+    constexpr int kHalf = 4 / BITS;   // codes of half a byte
+    const uint32_t up = w >> 4;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = static_cast<int>(w & (0x01010101u << i));
-    } else {
-#pragma unroll
-        for (int i = 0; i < 3; ++i) o[i] = static_cast<int>(w & (0x03030303u << (2 * i)));
-        o[3] = static_cast<int>((w >> 2) & 0x30303030u);
+    for (int i = 0; i < kHalf; ++i) {
+        o[i] = static_cast<int>(w & (kCode << (BITS * i)));
+        o[kHalf + i] = static_cast<int>(up & (kCode << (BITS * i)));
     }
 }
 
@@ -343,7 +347,7 @@ __device__ __forceinline__ void matrix_logits(const uint4* c, I4 a0, I4 a1, floa
         I4 acc = {0, 0, 0, 0};
         acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, I4{f[0], f[1], f[2], f[3]}, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, I4{f[4], f[5], f[6], f[7]}, acc, 0, 0, 0);
-        // digit sums are at most 128 * 128 * 128 in size: two of them meet as an integer
+        // digit sums are at most 128 * 128 * 12 in size: two of them meet as an integer
         const float l = static_cast<float>(acc[0] + (acc[1] << 8)), u = static_cast<float>(acc[2] + (acc[3] << 8));
         out[j] = __builtin_fmaf(__builtin_fmaf(u, 65536.f, l), inv, -zs);
     }
@@ -402,8 +406,7 @@ template <int BITS> __device__ __forceinline__ void matrix_fold(const I4* acc, f
             float r = static_cast<float>(a[3]);
 #pragma unroll
             for (int p = 2; p >= 0; --p) r = __builtin_fmaf(r, 256.f, static_cast<float>(a[p]));
-            const int sh = BITS == 1 ? i : 2 * cmin(i, 2);
-            const float unit = (BITS == 1 && i == 7 ? -1.f : 1.f) / (1073741824.f * static_cast<float>(1 << sh));
+            const float unit = 1.f / (1073741824.f * static_cast<float>(1 << field_shift<BITS>(i)));
             o[(NF - 1 - i) / 4].v[(NF - 1 - i) % 4] = r * unit;   // first channel of a byte in its top bits
         }
 #pragma unroll

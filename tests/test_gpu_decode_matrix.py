@@ -69,6 +69,37 @@ def test_infinity_in_one_head_stays_there(ops):
     _close(got[0, ~hit], want[0, ~hit])
 
 
+@pytest.mark.parametrize("bits", [1, 2])
+def test_logits_keep_small_channels_beside_a_large_one(ops, bits):
+    """One channel's q.s_k is about 2^16 (its codes are 0, it adds nothing to any logit), the others' are 7/16 of 2^-6,
+    once for every position a channel can have in a byte.  Odd tokens have all small codes, even tokens none."""
+    cpb = 8 // bits                                 # channels per byte
+    T, big = 200, 3
+    odd = np.arange(T) % 2 == 1
+    for pos in range(cpb):
+        c = make_case(1, 32, 8, 128, T, 0, bits, "fp16", seed=13)
+        small = np.arange(128) % cpb == pos
+        small[big] = False
+        q = np.where(small, 0.4375 * 2.0 ** -6 * 128 ** 0.5, 0.0)[None, :] * (1 + np.arange(32)[:, None] / 64)
+        q[:, big] = 512.0
+        c["q"] = O.round_to(q[None].astype(np.float32), "fp16")
+        c["sk"][:], c["zk"][:] = 1.0, 0.0
+        c["sk"][..., big] = 2048.0
+        code = np.where(odd[:, None] & small[None, :], 1, 0)
+        c["ck"][:] = O.encode(np.broadcast_to(code, (1, 8, T, 128)), bits)
+        c["cv"][:] = O.encode(np.broadcast_to(odd[:, None], (1, 8, T, 128)), bits)
+        c["sv"][:], c["zv"][:] = 1.0, 0.5
+        got = _run(ops, c, "fp16", 0, bits, calibrate=False)
+        k = code.astype(np.float64)
+        w = (c["q"][0].astype(np.float64) / 128 ** 0.5) @ k.T
+        p = np.exp(w - w.max(-1, keepdims=True))
+        want = (p[:, odd].sum(-1) / p.sum(-1) - 0.5)[None, :, None]
+        # fp32's own step at the large value is 2^-7; a channel may be off by half of 1/8 of that at most.  The weight of
+        # the odd tokens moves by a quarter of a logit's change; then one rounding of the result.
+        bound = small.sum() * 2.0 ** -11 / 4 + 2.0 ** -11 * np.abs(want) + 1e-6
+        assert (np.abs(got - want) <= bound).all(), (pos, float((np.abs(got - want) / bound).max()))
+
+
 def _token_run(ops, c, bits):
     from tests.util import case_to_gpu, to_np
     g = case_to_gpu(c, "fp16")
