@@ -418,11 +418,13 @@ template <int BITS> __device__ __forceinline__ void matrix_fold(const I4* acc, f
 // The right operand is arranged for it: a group's 4 (8) bytes of a row, read back by columns as 8 rows x 8 bytes (at 1 bit
 // the four bytes twice), meet in lane x as byte x mod 4 (8), and the lane keeps the field x / 4 (x / 8) of it and, from the
 // byte shifted by four, the one half a byte higher: 16 columns of the result are 16 channels, two MFMAs are a group.
-// The grid is the wave's largest scale of the group; sums of e * minimum stay in fp32.
-// Measured at batch 64 x 3 328 + 128, 1 bit, us per step: look-up form 58.1, this one 38.3 (1 024 threads, one workgroup per
-// compute unit: the four groups' operands, converted and read back one after the other, are what bounds it).
+// The grid is a head's own largest e * scale of the group among the wave's tokens - the weighted scale, because a token
+// without weight (masked, or out of this head's sight) may have a scale of any size; sums of e * minimum stay in fp32.
+// Measured at batch 64 x 3 328 + 128, 1 bit, us per step: look-up form 58.1, this one 36.7 (1 024 threads, one workgroup per
+// compute unit: the four groups' operands, converted and read back one after the other, are what bounds it).  Grids of the
+// scales alone, as wide as the least weighted token makes them, were 36.9 there and 2.5 % faster in the middle of 60 shapes.
 // Weights and scales have 32 bits here, the look-up tables held their products and short sums as fp16.
-// st: the lane's own token's scales and minima (layout of `stats` below); pw: the wave's grid, 2^(30 - e) per group.
+// st: the lane's own token's scales and minima (layout of `stats` below); pw: the head's grid, 2^(30 - e) per group.
 template <int BITS, typename DT>
 __device__ __forceinline__ void matrix_values_token(unsigned char* tile, const float* e, const U4* v, U4 st, const float* pw,
                                                     float* cm, I4* acc) {
@@ -455,8 +457,8 @@ __device__ __forceinline__ void matrix_values_token(unsigned char* tile, const f
         *reinterpret_cast<U2*>(rows + lane * 8) = w2;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const float xs = __builtin_amdgcn_fmed3f(sc[j][gi % 2] * pw[gi], -2130706432.f, 2130706432.f);
-            *reinterpret_cast<uint32_t*>(tile + (16 * j + x) * 16 + 4 * k) = byte_digits(__float2int_rn(xs));
+            // (at most 2^30: the grid comes from this very product)
+            *reinterpret_cast<uint32_t*>(tile + (16 * j + x) * 16 + 4 * k) = byte_digits(__float2int_rn(sc[j][gi % 2] * pw[gi]));
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -474,19 +476,43 @@ __device__ __forceinline__ void matrix_values_token(unsigned char* tile, const f
     }
 }
 
-// its sums as floats in channel order; unit: the value of one grid step per group
-template <int BITS> __device__ __forceinline__ void matrix_fold_token(const I4* acc, const float* unit, float* out, int x) {
+// A dword of every lane's own token to the lanes that hold the token's weights: o[j] is that of token 16 j + x
+__device__ __forceinline__ void token_rows(uint32_t v, uint32_t* o) {
+    const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    const auto a = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false), b = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
+    o[0] = a[0]; o[1] = a[1]; o[2] = b[0]; o[3] = b[1];
+}
+
+// The largest |e * scale| of every group so far, as bit patterns (unsigned: a NaN is larger than any number).
+// scales: the lane's own token's
+template <typename DT> __device__ __forceinline__ void token_tops(const float* e, U2 scales, uint32_t* top) {
+    uint32_t s01[4], s23[4];
+    token_rows(scales.x & 0x7fff7fffu, s01);
+    token_rows(scales.y & 0x7fff7fffu, s23);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        top[0] = max(top[0], __builtin_bit_cast(uint32_t, e[j] * Cvt<DT>::lo(s01[j])));
+        top[1] = max(top[1], __builtin_bit_cast(uint32_t, e[j] * Cvt<DT>::hi(s01[j])));
+        top[2] = max(top[2], __builtin_bit_cast(uint32_t, e[j] * Cvt<DT>::lo(s23[j])));
+        top[3] = max(top[3], __builtin_bit_cast(uint32_t, e[j] * Cvt<DT>::hi(s23[j])));
+    }
+}
+
+// its sums as floats in channel order; pw: the grids
+template <int BITS> __device__ __forceinline__ void matrix_fold_token(const I4* acc, const float* pw, float* out, int x) {
     const int byte = BITS == 1 ? x & 3 : x & 7, f = BITS == 1 ? x >> 2 : x >> 3;
     const float field = __builtin_bit_cast(float, (127 - BITS * f) << 23);   // the field counts 2^(BITS f)
 #pragma unroll
     for (int gi = 0; gi < 4; ++gi) {
+        // the value of one grid step: 1 / pw, or the NaN that stands for a group with an infinity or a NaN in it
+        const float unit = pw[gi] != pw[gi] ? pw[gi] : __builtin_bit_cast(float, (254 << 23) - __builtin_bit_cast(int, pw[gi]));
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const I4 a = acc[2 * gi + q];
             float r = static_cast<float>(a[3]);
 #pragma unroll
             for (int p = 2; p >= 0; --p) r = __builtin_fmaf(r, 256.f, static_cast<float>(a[p]));
-            out[32 * gi + byte * (8 / BITS) + f + q * (4 / BITS)] = r * field * unit[gi];
+            out[32 * gi + byte * (8 / BITS) + f + q * (4 / BITS)] = r * field * unit;
         }
     }
 }
@@ -713,10 +739,10 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     // the last one)
     const int wt0 = __builtin_amdgcn_readfirstlane(tid);
     const int hl = min(lane >> 4, HPB - 1);
-    // per-token values: the chunk's scales and minima, four 16-bit values a token; the wave's grids
+    // per-token values: the chunk's scales and minima, four 16-bit values a token
     const U2* vsp = reinterpret_cast<const U2*>(has_img ? static_cast<const uint16_t*>(g.vs) + (bh * g.T + t0) * 4 : static_cast<const uint16_t*>(g.q));
     const U2* vmp = reinterpret_cast<const U2*>(has_img ? static_cast<const uint16_t*>(g.vz) + (bh * g.T + t0) * 4 : static_cast<const uint16_t*>(g.q));
-    float vpw[4] = {0.f, 0.f, 0.f, 0.f}, vunit[4] = {0.f, 0.f, 0.f, 0.f};
+    U2 ts[VTOK && !MINMAX_ONLY ? REGL : 1];   // the scales of the lane's own tokens
     if (has_img) {
         const I4* aq = reinterpret_cast<const I4*>(regA);
         const I4 a0 = aq[lane], a1 = aq[64 + lane];
@@ -738,27 +764,9 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             if (!MINMAX_ONLY && rd < kVF - kVEarly) request_v(kVEarly + rd);   // the rest of the first packed V rows
         }
         phase_priority(std::integral_constant<int, 2>{});
-        if constexpr (VTOK && !MINMAX_ONLY) {
-            // the largest scale of every group among the wave's tokens (bit patterns: the sign cleared)
-            uint32_t t0s = 0, t1s = 0, t2s = 0, t3s = 0;
+        if constexpr (VTOK && !MINMAX_ONLY) {   // they arrive during the min / max and the calibration
 #pragma unroll
-            for (int rd = 0; rd < REGL; ++rd) {
-                if (wt0 + rd * kNT < n) {
-                    const U2 t = vsp[min(tid + rd * kNT, n - 1)];
-                    t0s = max(t0s, t.x & 0x7fffu); t1s = max(t1s, (t.x >> 16) & 0x7fffu);
-                    t2s = max(t2s, t.y & 0x7fffu); t3s = max(t3s, (t.y >> 16) & 0x7fffu);
-                }
-            }
-            const uint32_t ts[4] = {t0s, t1s, t2s, t3s};
-#pragma unroll
-            for (int gi = 0; gi < 4; ++gi) {
-                const float f = Cvt<DT>::to_float(static_cast<uint16_t>(wave_max_key(static_cast<int>(ts[gi]))));
-                const int bits = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f));
-                const int e = max((bits >> 23) - 126, -90);   // the largest lies in [2^(e-1), 2^e)
-                vpw[gi] = __builtin_bit_cast(float, (30 - e + 127) << 23);
-                // an infinity or a NaN among them makes the group's sums NaN
-                vunit[gi] = bits >= 0x7f800000 ? __builtin_nanf("") : __builtin_bit_cast(float, (e - 30 + 127) << 23);
-            }
+            for (int rd = 0; rd < REGL; ++rd) ts[rd] = vsp[min(tid + rd * kNT, n - 1)];
         }
         // the waves' minima and maxima meet in LDS, as in block_max, from one lane per head
         const int klo = row_max_key(float_key(-lo)), khi = row_max_key(float_key(hi));
@@ -958,21 +966,48 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             if constexpr (VTOK) {
 #pragma unroll
                 for (int r = 0; r < KV; ++r) {
-                    ssc[r] = vsp[min(tid + r * kNT, n - 1)];
+                    ssc[r] = ts[r];
                     smin[r] = vmp[min(tid + r * kNT, n - 1)];
                 }
             }
             phase_priority(std::integral_constant<int, 3>{});
+            auto weights = [&](int rd, float* e) {   // of round rd's tile
+                const int tw = wt0 + rd * kNT;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(lx[rd][j] - mnl, eal, ecl));
+                if (tw + kWave > n) {   // the chunk's last tile: what is past the end weighs nothing
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) e[j] = tw + 16 * j + (lane & 15) < n ? e[j] : 0.f;
+                }
+            };
+            float vpw[4] = {0.f, 0.f, 0.f, 0.f};   // VTOK: the grids of the lane's head
+            if constexpr (VTOK) {
+                uint32_t top[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int rd = 0; rd < REGL; ++rd) {
+                    if (wt0 + rd * kNT < n) {
+                        weights(rd, lx[rd]);   // (in place: the logits are not needed any more)
+                        token_tops<DT>(lx[rd], ts[rd], top);
+                    }
+                }
+#pragma unroll
+                for (int gi = 0; gi < 4; ++gi) {
+                    const int bits = row_max_key(static_cast<int>(top[gi] & 0x7fffffffu));
+                    const int e = max((bits >> 23) - 126, -90);   // the largest lies in [2^(e-1), 2^e)
+                    // an infinity or a NaN among them makes the head's sums of the group NaN
+                    vpw[gi] = bits >= 0x7f800000 ? __builtin_nanf("") : __builtin_bit_cast(float, (30 - e + 127) << 23);
+                }
+            }
 #pragma unroll
             for (int rd = 0; rd < REGL; ++rd) {
                 const int tw = wt0 + rd * kNT;
                 if (tw < n) {
                     float e[4];
+                    if constexpr (VTOK) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(lx[rd][j] - mnl, eal, ecl));
-                    if (tw + kWave > n) {   // the chunk's last tile: what is past the end weighs nothing
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) e[j] = tw + 16 * j + (lane & 15) < n ? e[j] : 0.f;
+                        for (int j = 0; j < 4; ++j) e[j] = lx[rd][j];
+                    } else {
+                        weights(rd, e);
                     }
 #pragma unroll
                     for (int j = 0; j < 4; ++j) lsum += e[j];
@@ -1014,7 +1049,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             float* redv = reinterpret_cast<float*>(regA);   // [wave][head][channel]
             if ((lane >> 4) < HPB) {
                 float* o = redv + (wv * HPB + hl) * kD;
-                if constexpr (VTOK) matrix_fold_token<BITS>(acc, vunit, o, lane & 15);
+                if constexpr (VTOK) matrix_fold_token<BITS>(acc, vpw, o, lane & 15);
                 else matrix_fold<BITS>(acc, o, lane & 15);
             }
             __syncthreads();

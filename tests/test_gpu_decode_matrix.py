@@ -17,11 +17,11 @@ def ops():
     return ops
 
 
-def _close(got, want):
-    # fp16 results: one rounding (2^-11 of the value) on sums kept in 32 bits (a few 1e-6 of the largest, times the
+def _close(got, want, rounding=2.0 ** -11):
+    # fp16 results: one rounding (2^-11 of the value; bf16: 2^-8) on sums kept in 32 bits (a few 1e-6 of the largest, times the
     # logits' size in the exponent: logits of about 10)
     assert np.isfinite(got).all()
-    bound = 2.0 ** -11 * np.abs(want) + 1e-4 * np.abs(want).max()
+    bound = rounding * np.abs(want) + 1e-4 * np.abs(want).max()
     assert (np.abs(got - want) <= bound).all(), float((np.abs(got - want) / bound).max())
 
 
@@ -100,11 +100,14 @@ def test_logits_keep_small_channels_beside_a_large_one(ops, bits):
         assert (np.abs(got - want) <= bound).all(), (pos, float((np.abs(got - want) / bound).max()))
 
 
-def _token_run(ops, c, bits):
+def _token_run(ops, c, bits, dtype="fp16", mask=None, calibrate=True):
+    import torch
     from tests.util import case_to_gpu, to_np
-    g = case_to_gpu(c, "fp16")
-    out = ops.decode_attn(g["q"], g["ck"], g["cv"], g["sk"], g["zk"], g["sv"], g["zv"], None, None, bits=bits, v_mode="token")
-    want = O.decode_attention(c["q"], c["ck"], c["cv"], c["sk"], c["zk"], c["sv"], c["zv"], None, None, 0, bits, v_token_group=32)
+    g = case_to_gpu(c, dtype)
+    out = ops.decode_attn(g["q"], g["ck"], g["cv"], g["sk"], g["zk"], g["sv"], g["zv"], None, None, bits=bits, v_mode="token",
+                          mask=None if mask is None else torch.from_numpy(mask).cuda(), calibrate=calibrate)
+    want = O.decode_attention(c["q"], c["ck"], c["cv"], c["sk"], c["zk"], c["sv"], c["zv"], None, None, 0, bits, v_token_group=32,
+                              mask=mask, calibrate_logits=calibrate)
     return to_np(out), want
 
 
@@ -138,3 +141,28 @@ def test_token_values_infinite_scale_stays_in_its_group(ops):
     rest = np.ones(hit.shape, bool)
     rest[0, 12:16, 64:96] = False
     assert np.array_equal(hit[rest], got[rest])
+
+
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("dtype, far", [("fp16", 2.0 ** 15), ("bf16", 2.0 ** 40)])
+def test_token_values_large_scale_of_a_token_without_weight(ops, dtype, far, bits):
+    """A token's value scale may be of any size where its weight is zero: in the first sample it is masked (left padding),
+    in the second one head of the unit gives it weight and the others give it none."""
+    T = 200
+    c = _token_case(2, 32, 8, T, 0, bits, dtype, seed=6)
+    c["sv"] = O.round_to(c["sv"] * np.float32(2.0 ** -8), dtype)
+    c["zv"] = O.round_to(c["zv"] * np.float32(2.0 ** -8), dtype)
+    c["sv"][:, :, 7, 1] = far
+    mask = np.zeros((2, T), np.float32)
+    mask[0, :9] = -1e4
+    # second sample: channel 0 tells token 7 from the others, exp(-100 * 16 / sqrt(128)) is 0 in fp32
+    first = 1 << (8 - bits)                      # code 1 of a byte's first channel
+    c["ck"][1, :, :, 0] &= first - 1
+    c["ck"][1, :, 7, 0] |= first
+    c["sk"][1, :, 0], c["zk"][1, :, 0] = 16.0, 0.0
+    c["q"][1, :, 0] = -100.0
+    c["q"][1, ::4, 0] = 0.0
+    got, want = _token_run(ops, c, bits, dtype, mask, calibrate=False)
+    for b in range(2):
+        for h in range(32):
+            _close(got[b, h], want[b, h], 2.0 ** -11 if dtype == "fp16" else 2.0 ** -8)
