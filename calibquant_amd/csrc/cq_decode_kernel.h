@@ -368,7 +368,7 @@ __device__ __forceinline__ void matrix_values(unsigned char* tile, const float* 
     for (int s = 0; s < BITS; ++s) *reinterpret_cast<U4*>(tile + (1 + s) * 1024 + lane * 16) = v[s];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        // (a weight is at most 1 up to rounding; the cap keeps the digits in range whatever the rounding does)
+        // (a weight is at most 1; the cap keeps the digits in range whatever comes)
         const float xs = fminf(e[j] * 1073741824.f, 2130706432.f);
         *reinterpret_cast<uint32_t*>(tile + (16 * j + x) * 16 + 4 * k) = byte_digits(__float2int_rn(xs));
     }
@@ -927,34 +927,24 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
 #pragma unroll
                 for (int h = 0; h < HPB; ++h) {
                     m_img[h] = key_float(__builtin_amdgcn_readfirstlane(redi[h]));
-                    slope[h] = 1.0f; tmin[h] = 0.f; mn[h] = 0.f;
+                    slope[h] = 1.0f;
                 }
             } else {
 #pragma unroll
                 for (int h = 0; h < HPB; ++h) m_img[h] = fmaxf(tmin[h], (mx[h] - mn[h]) * slope[h] + tmin[h]);
             }
-            // e = exp(x - M) with x = (w - mn) * slope + tmin, as exp2((w - mn) * ea + ec)
-            float ea[HPB], ec[HPB];
+            // e = exp(x - M) with x = (w - mn) * slope + tmin, as exp2((w - peak) * ea): `peak` is the logit whose x is M, so no
+            // weight is above 1 - which the fixed-point weights rely on - however large the logits are or far from 0 they lie
+            // (a constant that takes M back is off by M's own rounding), and a degenerate logit range, whose slope is
+            // ~1e8, meets the exact zero of (w - peak).
+            float ea[HPB], peak[HPB];
 #pragma unroll
             for (int h = 0; h < HPB; ++h) {
                 const bool dead = (m_img[h] == -INFINITY);   // every position masked out
-                ea[h] = dead ? 0.f : slope[h] * kLog2e;
-                ec[h] = dead ? -INFINITY : (tmin[h] - m_img[h]) * kLog2e;
+                ea[h] = dead ? 1.f : slope[h] * kLog2e;
+                peak[h] = dead ? INFINITY : (EXTRAS && g.mask) ? m_img[h] : slope[h] < 0.f ? mn[h] : mx[h];
             }
-            // With a slope of ordinary size the subtraction folds into the constant: exp2(w * ea + (ec - mn * ea)), one
-            // FMA per logit.  A degenerate logit range makes the slope ~1e8, and only the exact zero of (w - mn)
-            // keeps the product finite: those units take the two-step form.
-            float ec2[HPB];
-            bool plain = true;
-#pragma unroll
-            for (int h = 0; h < HPB; ++h) {
-                ec2[h] = ec[h] - mn[h] * ea[h];
-                if (h < NH) plain = plain && fabsf(ea[h]) <= 4.0f;
-            }
-            float ec3[HPB], mn3[HPB];
-#pragma unroll
-            for (int h = 0; h < HPB; ++h) { ec3[h] = plain ? ec2[h] : ec[h]; mn3[h] = plain ? 0.f : mn[h]; }
-            const float eal = mine(ea), ecl = mine(ec3), mnl = mine(mn3);
+            const float eal = mine(ea), pkl = mine(peak);
             float lsum = 0.f;
             I4 acc[8];
 #pragma unroll
@@ -974,7 +964,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             auto weights = [&](int rd, float* e) {   // of round rd's tile
                 const int tw = wt0 + rd * kNT;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(lx[rd][j] - mnl, eal, ecl));
+                for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f((lx[rd][j] - pkl) * eal);
                 if (tw + kWave > n) {   // the chunk's last tile: what is past the end weighs nothing
 #pragma unroll
                     for (int j = 0; j < 4; ++j) e[j] = tw + 16 * j + (lane & 15) < n ? e[j] : 0.f;

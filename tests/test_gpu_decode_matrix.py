@@ -122,6 +122,43 @@ def test_token_values_tile_edges(ops, case, bits):
     _close(*_token_run(ops, _token_case(B, Hq, Hkv, T, 0, bits, "fp16", seed=T), bits))
 
 
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("values", ["channel", "token"])
+def test_logits_far_from_zero(ops, values, bits):
+    """A channel with the same code in every token moves all logits of a head by 2^25 to 2^27, where fp32 has steps of 4
+    and 8: the largest weight is 1 all the same, and a constant in the exponent would be off by powers of two."""
+    T, odd = 200, np.arange(200) % 2 == 1
+    c = _token_case(1, 32, 8, T, 0, bits, "fp16", seed=14) if values == "token" else make_case(1, 32, 8, 128, T, 0, bits, "fp16", seed=14)
+    q = np.zeros((32, 128))
+    q[:, 3] = 2.0 ** 14 * (1 + np.arange(32) / 16)        # times 2^15: the same for all tokens
+    q[:, 40:44] = 512.0                                   # odd tokens: about 181 more
+    c["q"] = O.round_to(q[None].astype(np.float32), "fp16")
+    c["sk"][:], c["zk"][:] = 1.0, 0.0
+    c["sk"][..., 3] = 2.0 ** 15
+    code = np.zeros((T, 128), np.int64)
+    code[:, 3] = 1
+    code[odd, 40:44] = 1
+    c["ck"][:] = O.encode(np.broadcast_to(code, (1, 8, T, 128)), bits)
+    if values == "token":
+        c["cv"][:] = np.where(odd, -1 if bits == 1 else 0x55555555, 0)[:, None]
+        c["sv"][:], c["zv"][:] = 1.0, -0.5
+        got, _ = _token_run(ops, c, bits, calibrate=False)
+    else:
+        c["cv"][:] = O.encode(np.broadcast_to(odd[:, None], (1, 8, T, 128)), bits)
+        c["sv"][:], c["zv"][:] = 1.0, 0.5
+        got = _run(ops, c, "fp16", 0, bits, calibrate=False)
+    assert np.abs(got - 0.5).max() <= 2.0 ** -11          # the odd tokens' value: one rounding
+
+
+@pytest.mark.parametrize("T", [200, 5000])
+def test_mask_of_the_lowest_value_over_every_packed_token(ops, T):
+    """fp32's lowest value on all packed tokens of the first sample (a padded prompt): its window alone counts."""
+    c = make_case(2, 32, 8, 128, T, 40, 1, "fp16", seed=15)
+    mask = np.zeros((2, T + 40), np.float32)
+    mask[0, 8:8 + T] = np.finfo(np.float32).min
+    _close(_run(ops, c, "fp16", 8, 1, mask=mask), _oracle(c, 8, 1, mask=mask))
+
+
 def test_token_values_scales_far_apart(ops):
     """Every wave takes its grid from the largest scale of a group among its tokens; a group of zero scales has none."""
     c = _token_case(1, 32, 8, 300, 0, 1, "fp16", seed=3)
