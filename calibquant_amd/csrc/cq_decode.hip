@@ -49,7 +49,7 @@ static int pair_units() {
 static inline int ngroups(int G, int hpb) { return (G + hpb - 1) / hpb; }
 
 struct Plan {
-    int hpb, nh, nt, regl, nsplit, chunk, nx, cap, lds;   // hpb: heads an entry is wide; nh: heads a unit serves
+    int hpb, nh, nt, nsplit, chunk, nx, cap;   // hpb: heads an entry is wide; nh: heads a unit serves
     bool fused;   // chunked step in one launch: every chunk's workgroup fits the device at once
     size_t ws_mm, ws_part, ws_cnt, ws_lgt;   // chunked launch: min / max, partials, counters; logits (optional)
 };
@@ -82,12 +82,10 @@ static void plan_for(const cq_decode_args* a, Plan* p, int nh = HPB) {
     p->hpb = HPB;
     p->nh = nh;
     p->nt = NT;
-    p->regl = REGL;
     p->nsplit = nsplit;
     p->chunk = chunk;
     p->nx = nsplit + ((nsplit > 1 && a->R > 0) ? 1 : 0);
     p->cap = a->T > 0 ? chunk : 64;
-    p->lds = L::lds_bytes(p->cap);
     const size_t rows = static_cast<size_t>(a->B) * a->Hq;
     p->ws_mm = nsplit > 1 ? ((rows * nsplit * 2 * sizeof(float) + 255) / 256 * 256) : 0;
     p->ws_part = nsplit > 1 ? (rows * p->nx * (kD + 2) * sizeof(float) + 255) / 256 * 256 : 0;
@@ -143,7 +141,7 @@ static int make_plan(const cq_decode_args* a, Plan* p) {
             if (p->hpb == 4) plan_for<1, 4, false, 512, kRegPair>(a, &q, nh4); else plan_for<1, 2, false, 512, 0>(a, &q);
             const bool single = p->nsplit == 1 && q.nsplit == 1 && units > kPairUnits;
             const bool chunked = p->hpb == 4 && p->nsplit > 1 && q.nsplit > 1 && units * q.nsplit > kPairUnits;
-            if ((single || chunked) && q.lds <= kLdsMax / 2) *p = q;
+            if (single || chunked) *p = q;
         }
     } else {
         // four heads per unit need the two-pass K table; with per-token values their LDS layout
@@ -158,7 +156,7 @@ static int make_plan(const cq_decode_args* a, Plan* p) {
                 plan_for<2, 4, false, 512, kRegPair>(a, &q, nh4);
                 const bool single = p->nsplit == 1 && q.nsplit == 1 && units > kPairUnits;
                 const bool chunked = p->nsplit > 1 && q.nsplit > 1 && units * q.nsplit > kPairUnits;
-                if ((single || chunked) && q.lds <= kLdsMax / 2) *p = q;
+                if (single || chunked) *p = q;
             }
         }
         else if (G >= 2) vtok ? plan_for<2, 2, true>(a, p) : plan_for<2, 2, false>(a, p);   // (per-token values: two heads per unit, padded for odd G)
@@ -187,7 +185,7 @@ static int make_plan(const cq_decode_args* a, Plan* p) {
     // the packed K rows, no logits buffer.  (The residual units wait for nobody and make room as they end.)
     if (p->nsplit > 1) {
         const int64_t waiting = static_cast<int64_t>(a->B) * a->Hkv * ngroups(G, p->nh) * p->nsplit;
-        const int64_t room = static_cast<int64_t>(kPairUnits) * ((p->nt == 512 && p->lds <= kLdsMax / 2) ? 2 : 1);
+        const int64_t room = static_cast<int64_t>(kPairUnits) * (p->nt == 512 && launch_lds(a->bits, vtok, p->hpb, p->nt) <= kLdsMax / 2 ? 2 : 1);
         // (one lane per chunk polls)
         if (waiting <= room && p->nsplit <= 64 && g_fused_wanted.load(std::memory_order_relaxed)) p->fused = true;
     }
@@ -394,8 +392,9 @@ int cq_decode_attn_plan(const cq_decode_args* args, cq_decode_plan* plan) {
     plan->chunks = p.nsplit;
     plan->chunk_tokens = args->T > 0 ? p.chunk : 0;
     plan->launches = (p.nsplit > 1 && !p.fused) ? 2 : 1;
-    plan->lds_bytes = p.lds;
-    plan->register_logits = p.regl;
+    const bool vtok = args->v_mode == CQ_V_PER_TOKEN;
+    plan->lds_bytes = cq::launch_lds(args->bits, vtok, p.hpb, p.nt);
+    plan->register_logits = cq::launch_rounds(vtok, p.hpb, p.nt, p.chunk);
     return CQ_OK;
 }
 

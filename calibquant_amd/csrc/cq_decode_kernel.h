@@ -197,6 +197,25 @@ template <int BITS, int HPB, bool VTOK = false, int NT_ = 1024, int REGL = 0, bo
     }
 };
 
+// What a launch of units of hpb heads in nt threads runs with: the rounds of logits its instantiation keeps in
+// registers for chunks of at most `chunk` tokens, and its dynamic LDS.  Launches pick by the first and check themselves
+// against both (cq_decode_matrix.h); cq_decode_attn_plan reports them.
+constexpr int launch_rounds(bool vtok, int hpb, int nt, int chunk) {
+    if (vtok) return chunk <= kRegTwoBit * nt ? kRegTwoBit : kRegPair;
+    if (hpb == 4) return nt == 512 ? kRegPair : kRegLong;
+    const int few = nt == 512 ? kRegPair : kRegLong;
+    return chunk <= few * nt ? few : kRegMost;
+}
+template <int BITS, bool VTOK, int NT> constexpr int launch_lds(int hpb) {
+    return hpb == 4 ? Lay<BITS, 4, VTOK, NT, kRegPair, true>::lds_bytes(0)
+         : hpb == 2 ? Lay<BITS, 2, VTOK, NT, kRegPair, true>::lds_bytes(0) : Lay<BITS, 1, VTOK, NT, kRegPair, true>::lds_bytes(0);
+}
+inline int launch_lds(int bits, bool vtok, int hpb, int nt) {
+    if (vtok) return bits == 1 ? launch_lds<1, true, 1024>(hpb) : launch_lds<2, true, 1024>(hpb);
+    if (nt == 512) return bits == 1 ? launch_lds<1, false, 512>(hpb) : launch_lds<2, false, 512>(hpb);
+    return bits == 1 ? launch_lds<1, false, 1024>(hpb) : launch_lds<2, false, 1024>(hpb);
+}
+
 // Unit decomposition of a 1-D grid.  Consecutive work ids share packed codes
 // (head groups of one kv-head), so when the grid is a multiple of the 8 XCDs
 // the hardware's round-robin placement is undone to keep them on one L2.

@@ -10,6 +10,8 @@ template <int BITS, int HPB, typename DT, bool VTOK, int NT, int REGL, bool CHUN
 static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st) {
     constexpr int lds = Lay<BITS, HPB, VTOK, NT, REGL, true>::lds_bytes(0);
     static_assert(lds <= 64 * 1024, "no raised dynamic-LDS limit needed; two 512-thread workgroups share a compute unit");
+    static_assert(lds == launch_lds<BITS, VTOK, NT>(HPB), "the LDS that plans report");
+    if (launch_rounds(VTOK, HPB, NT, g.chunk) != REGL || g.chunk > REGL * NT) return CQ_ERR_UNSUPPORTED;   // (a token too many would be left out of the sum)
     if constexpr (CHUNKED) {
         if (!g.fused) {
             const DecodeGeom g1 = minmax_geometry(g, 0);   // (this launch never looks at values)
@@ -35,27 +37,25 @@ static int launch_matrix_unit(const DecodeGeom& g, unsigned units, hipStream_t s
 
 template <int BITS, typename DT>
 static int launch_matrix_bits(const DecodeGeom& g, int hpb, int nh, int nt, unsigned units, hipStream_t st) {
+    const bool most = launch_rounds(false, hpb, nt, g.chunk) == kRegMost;
     if (nt == 512) {
         if (hpb == 4 && nh == 3) return launch_matrix_unit<BITS, 4, DT, 512, kRegPair, 3>(g, units, st);
         if (hpb == 4) return launch_matrix_unit<BITS, 4, DT, 512, kRegPair>(g, units, st);
-        if (g.chunk <= kRegPair * 512) return launch_matrix_unit<BITS, 2, DT, 512, kRegPair>(g, units, st);
-        return launch_matrix_unit<BITS, 2, DT, 512, kRegMost>(g, units, st);
+        return most ? launch_matrix_unit<BITS, 2, DT, 512, kRegMost>(g, units, st)
+                    : launch_matrix_unit<BITS, 2, DT, 512, kRegPair>(g, units, st);
     }
     if (hpb == 4 && nh == 3) return launch_matrix_unit<BITS, 4, DT, 1024, kRegLong, 3>(g, units, st);
     if (hpb == 4) return launch_matrix_unit<BITS, 4, DT, 1024, kRegLong>(g, units, st);
-    if (g.chunk <= kRegLong * 1024)
-        return hpb == 2 ? launch_matrix_unit<BITS, 2, DT, 1024, kRegLong>(g, units, st)
-                        : launch_matrix_unit<BITS, 1, DT, 1024, kRegLong>(g, units, st);
-    return hpb == 2 ? launch_matrix_unit<BITS, 2, DT, 1024, kRegMost>(g, units, st)
-                    : launch_matrix_unit<BITS, 1, DT, 1024, kRegMost>(g, units, st);
+    if (hpb == 2) return most ? launch_matrix_unit<BITS, 2, DT, 1024, kRegMost>(g, units, st)
+                              : launch_matrix_unit<BITS, 2, DT, 1024, kRegLong>(g, units, st);
+    return most ? launch_matrix_unit<BITS, 1, DT, 1024, kRegMost>(g, units, st)
+                : launch_matrix_unit<BITS, 1, DT, 1024, kRegLong>(g, units, st);
 }
 
-// nt threads per workgroup, g.chunk tokens at most: the plan's (cq_decode.hip: make_plan), whose layouts hold no more
-// tokens than the instantiation picked here - checked, because a token too many would be left out of the sum
+// nt threads per workgroup, g.chunk tokens at most: the plan's (cq_decode.hip: make_plan)
 template <typename DT>
 int launch_matrix(const DecodeGeom& g, int bits, int hpb, int nh, int nt, unsigned units, hipStream_t st) {
-    const int rounds = hpb == 4 ? (nt == 512 ? kRegPair : kRegLong) : kRegMost;
-    if (g.chunk > rounds * nt || (nt == 512 && hpb == 1)) return CQ_ERR_UNSUPPORTED;
+    if (nt == 512 && hpb == 1) return CQ_ERR_UNSUPPORTED;
     return bits == 1 ? launch_matrix_bits<1, DT>(g, hpb, nh, nt, units, st) : launch_matrix_bits<2, DT>(g, hpb, nh, nt, units, st);
 }
 
@@ -64,13 +64,14 @@ int launch_matrix(const DecodeGeom& g, int bits, int hpb, int nh, int nt, unsign
 template <int BITS, int HPB, typename DT>
 static int launch_token_unit(const DecodeGeom& g, unsigned units, hipStream_t st) {
     static_assert(Lay<BITS, HPB, true, 1024, 0>::max_chunk() <= kRegPair * 1024, "the plan's chunks fit eight rounds");
-    if (g.chunk <= kRegTwoBit * 1024) return launch_matrix_unit<BITS, HPB, DT, 1024, kRegTwoBit, HPB, true>(g, units, st);
+    if (launch_rounds(true, HPB, 1024, g.chunk) == kRegTwoBit)
+        return launch_matrix_unit<BITS, HPB, DT, 1024, kRegTwoBit, HPB, true>(g, units, st);
     return launch_matrix_unit<BITS, HPB, DT, 1024, kRegPair, HPB, true>(g, units, st);
 }
 
 template <typename DT>
 int launch_matrix_token(const DecodeGeom& g, int bits, int hpb, int nt, unsigned units, hipStream_t st) {
-    if (g.chunk > kRegPair * 1024 || nt != 1024 || (bits == 2 && hpb == 4)) return CQ_ERR_UNSUPPORTED;
+    if (nt != 1024 || (bits == 2 && hpb == 4)) return CQ_ERR_UNSUPPORTED;
     if (bits == 2) return hpb == 2 ? launch_token_unit<2, 2, DT>(g, units, st) : launch_token_unit<2, 1, DT>(g, units, st);
     if (hpb == 4) return launch_token_unit<1, 4, DT>(g, units, st);
     return hpb == 2 ? launch_token_unit<1, 2, DT>(g, units, st) : launch_token_unit<1, 1, DT>(g, units, st);

@@ -300,8 +300,8 @@ typedef struct cq_decode_plan {
     int chunk_tokens;     /* packed tokens per chunk */
     int launches;         /* 1 or 2 (what the plan asks for; see cq_decode_attn_wait_polls for when one becomes two) */
     int lds_bytes;        /* dynamic LDS of the main launch */
-    int register_logits;  /* > 0: a thread keeps the logits of up to this many of its tokens in registers (fp32)
-                           * and the token slots in LDS hold only exp(.) as fp16; 0: fp32 logits wait in the slots */
+    int register_logits;  /* a thread keeps the fp32 logits of this many rounds of `threads` tokens in registers;
+                           * chunk_tokens <= register_logits * threads */
 } cq_decode_plan;
 int cq_decode_attn_plan(const cq_decode_args* args, cq_decode_plan* plan);
 

@@ -28,8 +28,8 @@ def test_library_loads_and_exports_every_declared_symbol():
 def test_decode_launch_plan_is_a_function_of_the_shape():
     """`cq_decode_attn_plan` (host only): which launch a shape gets.  Two 512-thread workgroups per compute
     unit need a layout within half of the 160 KB LDS and more units of work than the 256 compute units;
-    logits kept in registers only at 1 bit with four heads per unit; chunked shapes take two launches, or one
-    when all their workgroups fit the device at once."""
+    logits are kept in registers, for as many rounds of the workgroup as the launched kernel has; chunked shapes
+    take two launches, or one when all their workgroups fit the device at once."""
     from calibquant_amd import _lib
     lib = _lib.load()
 
@@ -44,14 +44,14 @@ def test_decode_launch_plan_is_a_function_of_the_shape():
     assert (bench["threads"], bench["heads_per_unit"], bench["launches"], bench["register_logits"]) == (512, 4, 1, 8)
     assert bench["lds_bytes"] <= 80 * 1024 and bench["chunk_tokens"] == 3328
     small = plan(32, 32, 8, 3328, 128)                       # 256 units: one 1024-thread workgroup per compute unit
-    assert (small["threads"], small["register_logits"], small["launches"]) == (1024, 0, 1)
+    assert (small["threads"], small["register_logits"], small["launches"]) == (1024, 10, 1)
     two_bit = plan(64, 32, 8, 3328, 128, bits=2)            # 2 bits: paired as well, K table in two passes
     assert (two_bit["threads"], two_bit["register_logits"]) == (512, 8) and two_bit["lds_bytes"] <= 80 * 1024
     assert plan(32, 32, 8, 3328, 128, bits=2)["threads"] == 1024
     assert plan(64, 32, 8, 3328, 128, v_mode=1)["threads"] == 1024
     assert plan(64, 32, 8, 3328, 128, force_splits=2) == dict(plan(64, 32, 8, 3328, 128, force_splits=2), threads=1024, launches=2)
-    two = plan(128, 16, 8, 3328, 128)                        # two heads per unit: paired, fp32 logits
-    assert (two["threads"], two["heads_per_unit"], two["register_logits"]) == (512, 2, 0)
+    two = plan(128, 16, 8, 3328, 128)                        # two heads per unit: paired
+    assert (two["threads"], two["heads_per_unit"], two["register_logits"]) == (512, 2, 8)
     long = plan(8, 32, 8, 32768, 0)                          # chunked: the chunks are the units; all 512 resident: one launch
     assert long["launches"] == 1 and long["threads"] == 512 and long["chunks"] * long["chunk_tokens"] >= 32768
     assert long["lds_bytes"] <= 80 * 1024
@@ -67,17 +67,22 @@ def test_decode_launch_plan_is_a_function_of_the_shape():
     assert plan(64, 24, 8, 3328, 128, bits=2)["heads_per_unit"] == 3      # three heads per kv head: one exact unit
     assert plan(64, 40, 8, 3328, 128)["heads_per_unit"] == 4              # five: units of 4 + 1
     assert big["lds_bytes"] <= 160 * 1024
-    tok = plan(16, 48, 8, 9984, 64, v_mode=1)               # per-token values: padded four-head units too, chunked (16-byte slots)
-    assert (tok["heads_per_unit"], tok["threads"], tok["register_logits"]) == (4, 1024, 0) and tok["launches"] == 2
+    tok = plan(16, 48, 8, 9984, 64, v_mode=1)               # per-token values: padded four-head units too, chunked
+    assert (tok["heads_per_unit"], tok["threads"], tok["register_logits"]) == (4, 1024, 4) and tok["launches"] == 2
+    # the dynamic LDS of the launch: a tile per wave (a row and its weights, 1 + bits times 64 x 16 bytes; 2 560 bytes with
+    # per-token values), or the fold's fp32 partials where those are more, and the per-unit words behind them
+    assert bench["lds_bytes"] == 8 * 2048 + 8960 and big["lds_bytes"] == 16 * 4 * 128 * 4 + 9472
+    assert plan(64, 32, 8, 3328, 128, v_mode=1)["lds_bytes"] == 16 * 2560 + 9984
+    assert plan(1, 32, 8, 1024, 0)["lds_bytes"] == 16 * 2048 + 3328
     a = _lib.DecodeArgs()
     assert lib.cq_decode_attn_plan(ctypes.byref(a), None) < 0
     assert lib.cq_decode_attn_plan(ctypes.byref(a), ctypes.byref(_lib.DecodePlan())) < 0   # all-zero arguments
 
 
 def test_decode_launch_plan_invariants_over_random_shapes():
-    """Whatever the shape, the plan stays inside what the kernels assume: LDS within the device's 160 KB (half of
-    it for a 512-thread workgroup), chunks that cover T, register-resident logits only for chunks that fit the
-    rounds a thread keeps, two launches and a workspace exactly when T is chunked."""
+    """Whatever the shape, the plan stays inside what the kernels assume: LDS that needs no raised limit
+    and lets two 512-thread workgroups share a compute unit, chunks that cover T and fit the rounds of logits a
+    thread keeps, two launches and a workspace exactly when T is chunked."""
     from calibquant_amd import _lib
     lib = _lib.load()
     rng = np.random.default_rng(11)
@@ -98,17 +103,17 @@ def test_decode_launch_plan_invariants_over_random_shapes():
         assert p.threads in (512, 1024) and p.heads_per_unit in (1, 2, 3, 4), shape
         G_ = a.Hq // a.Hkv
         assert (p.heads_per_unit == 3) <= (G_ % 3 == 0 and G_ % 4 != 0 and a.v_mode == 0), shape   # three only for exact units
-        assert 0 < p.lds_bytes <= (80 if p.threads == 512 else 160) * 1024, shape
+        assert 0 < p.lds_bytes <= 64 * 1024, shape
         assert p.chunks >= 1 and p.chunks * p.chunk_tokens >= a.T, shape
         assert p.chunk_tokens % 64 == 0, shape
-        assert p.register_logits == 0 or p.chunk_tokens <= p.register_logits * p.threads, shape
+        assert p.register_logits > 0 and p.chunk_tokens <= p.register_logits * p.threads, shape
         assert p.launches in (1, 2) and (p.launches == 1 or p.chunks > 1), shape
         if p.launches == 1 and p.chunks > 1:      # one launch: every chunk's workgroup resident at once
             units_ = a.B * a.Hkv * -(-G_ // p.heads_per_unit)
             assert units_ * p.chunks <= 256 * (2 if p.threads == 512 else 1) and p.chunks <= 64, shape
         assert (lib.cq_decode_attn_workspace(ctypes.byref(a)) > 0) == (p.chunks > 1), shape
         if a.v_mode == 1:
-            assert p.threads == 1024 and p.register_logits == 0, shape
+            assert p.threads == 1024 and p.register_logits in (4, 8), shape
 
 
 def test_c_abi_rejects_bad_arguments_without_touching_the_gpu():
