@@ -51,7 +51,7 @@ static inline int ngroups(int G, int hpb) { return (G + hpb - 1) / hpb; }
 struct Plan {
     int hpb, nh, nt, nsplit, chunk, nx, cap;   // hpb: heads an entry is wide; nh: heads a unit serves
     bool fused;   // chunked step in one launch: every chunk's workgroup fits the device at once
-    size_t ws_mm, ws_part, ws_cnt, ws_lgt;   // chunked launch: min / max, partials, counters; logits (optional)
+    size_t ws_mm, ws_part, ws_cnt;   // chunked launch: min / max, partials, counters
 };
 
 template <int BITS, int HPB, bool VTOK, int NT = 1024, int REGL = 0>
@@ -93,10 +93,6 @@ static void plan_for(const cq_decode_args* a, Plan* p, int nh = HPB) {
     p->ws_cnt = nsplit > 1 ? (static_cast<size_t>(units) * sizeof(unsigned long long) + 255) / 256 * 256 +
                                  static_cast<size_t>(units) * HPB * nsplit * 16 : 0;
     p->fused = false;
-    // (room for the logits, which a two-launch step once handed over here: the kernel recomputes them, callers'
-    // workspaces keep their size)
-    const bool hand_over = nsplit > 1 && 16 * BITS > 4 * HPB;
-    p->ws_lgt = hand_over ? static_cast<size_t>(units) * a->T * HPB * sizeof(float) : 0;
 }
 
 static int make_plan(const cq_decode_args* a, Plan* p) {
@@ -283,8 +279,7 @@ static int decode_entry(const cq_decode_args* a, void* workspace, size_t workspa
     if (a->R > 0 && (!aligned16(a->k_res) || !aligned16(a->v_res) || (a->res_stride_b % 8) ||
                      (a->res_stride_h % 8) || (a->res_stride_r % 8)))
         return CQ_ERR_ALIGN;
-    // (a caller's own workspace for two launches is as large as cq_decode_attn_workspace says)
-    const size_t need = p.ws_mm + p.ws_part + p.ws_cnt + (static_scratch || p.fused ? 0 : p.ws_lgt);
+    const size_t need = p.ws_mm + p.ws_part + p.ws_cnt;
     // One launch when the plan allows it, the caller's own workspace is used (the static entry point allocates
     // nothing, not even the status word) and no earlier launch of this process gave up waiting.
     int* status = nullptr;
@@ -356,7 +351,7 @@ extern "C" {
 size_t cq_decode_attn_workspace(const cq_decode_args* args) {
     cq::Plan p;
     if (cq::make_plan(args, &p) != CQ_OK) return 0;
-    return p.ws_mm + p.ws_part + p.ws_cnt + (p.fused ? 0 : p.ws_lgt);
+    return p.ws_mm + p.ws_part + p.ws_cnt;
 }
 
 int cq_decode_attn_single_launch(int enable) {

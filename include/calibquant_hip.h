@@ -267,21 +267,19 @@ int cq_decode_attn(const cq_decode_args* args, cq_stream_t stream);
  * outputs and temporaries with torch on every call.  Same arguments and the
  * same kernels as cq_decode_attn, except that args->workspace /
  * workspace_bytes are ignored: the scratch of the chunked path (per-chunk
- * logit min / max, the flash-decoding partials and their counters, and - where
- * the plan hands the first launch's logits to the second through a buffer
- * (2 bits, or fewer than four heads per unit) and it fits beside them - those)
- * lives in a static device array of cq_decode_attn_static_limit() bytes
- * (8 MiB) inside the library; every GPU the library runs on holds its own
- * copy until the process ends.  When the logits do not fit, the second launch
- * recomputes them (same results, more work).  A request whose plan needs more
- * than the limit even so returns CQ_ERR_SCRATCH_LIMIT and launches nothing
- * (batch 8 x 32 768 tokens needs 1.2 MiB; at 2 bits 33 MiB more with the logits).
+ * logit min / max, the flash-decoding partials and their counters) lives in a
+ * static device array of cq_decode_attn_static_limit() bytes (8 MiB) inside
+ * the library; every GPU the library runs on holds its own copy until the
+ * process ends.  A request whose plan needs more than the limit returns
+ * CQ_ERR_SCRATCH_LIMIT and launches nothing (batch 8 x 32 768 tokens needs
+ * 1.2 MiB).
  * The call allocates and frees nothing and does not synchronise.  Nothing in
  * the scratch has to start at zero: every word a launch reads was written by
- * an earlier launch of the same call (the first launch clears the counters).  All calls on one GPU share that GPU's array, so two calls that
- * may overlap on one GPU (different streams, or one stream per host thread)
- * race on it: keep them on one stream, or give the overlapping ones
- * cq_decode_attn with workspaces of their own. */
+ * an earlier launch of the same call (the first launch clears the counters).
+ * All calls on one GPU share that GPU's array, so two calls that may overlap
+ * on one GPU (different streams, or one stream per host thread) race on it:
+ * keep them on one stream, or give the overlapping ones cq_decode_attn with
+ * workspaces of their own. */
 size_t cq_decode_attn_static_limit(void);
 int cq_decode_attn_static(const cq_decode_args* args, cq_stream_t stream);
 

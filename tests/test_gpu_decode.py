@@ -400,10 +400,9 @@ def two_launches():
 
 @pytest.mark.parametrize("case", [(2, 16, 8, 20000, 50, 3, 1), (2, 8, 8, 20000, 0, 0, 1), (1, 32, 8, 20000, 33, 5, 2),
                                   (1, 16, 8, 20000, 33, 0, 2)], ids=lambda c: "-".join(str(x) for x in c))
-def test_decode_attn_chunked_with_the_logits_buffer(ops, case, two_launches):
-    """Chunked launches whose first launch hands the logits to the second through the workspace (a packed K row
-    of more bytes than the logits: 2 bits, or fewer than four heads per unit), against the oracle.  (Four-head
-    units at 1 bit recompute their logits: `test_long_context_batch_8_kv_32768` and the chunked cases above.)"""
+def test_decode_attn_chunked_without_a_logits_buffer(ops, case, two_launches):
+    """Two launches per step at 2 bits or with fewer than four heads per unit, against the oracle: the second
+    recomputes the logits from the packed K rows, so the workspace has no room for them."""
     B, Hq, Hkv, T, R, S, bits = case
     c = make_case(B, Hq, Hkv, 128, T, max(R, 1), bits, "bf16", seed=500 + Hq + bits, outlier_kind="student")
     g = case_to_gpu(c, "bf16")
@@ -412,7 +411,7 @@ def test_decode_attn_chunked_with_the_logits_buffer(ops, case, two_launches):
     plan = call.plan()
     assert plan["chunks"] > 1 and plan["launches"] == 2
     units = B * Hkv * ((Hq // Hkv + plan["heads_per_unit"] - 1) // plan["heads_per_unit"])
-    assert call.workspace_bytes >= units * T * plan["heads_per_unit"] * 4      # the logits are part of it
+    assert call.workspace_bytes < units * T * plan["heads_per_unit"] * 4       # the logits are no part of it
     out = call.run()
     torch.cuda.synchronize()
     want = O.decode_attention(c["q"], c["ck"], c["cv"], c["sk"], c["zk"], c["sv"], c["zv"],
@@ -429,7 +428,7 @@ def test_decode_attn_chunked_with_the_logits_buffer(ops, case, two_launches):
                          ids=lambda c: "-".join(str(x) for x in c))
 def test_decode_attn_chunked_launches_replayed_from_a_graph(ops, case, single, request):
     """The chunked step - two launches (counters cleared by the first, partials merged by the last workgroup of a
-    unit in the second; logits through the workspace or recomputed), or one launch whose chunks exchange their
+    unit in the second, which recomputes the logits), or one launch whose chunks exchange their
     min / max inside it (the records and counters it leaves are emptied by the merging workgroup, so a replay
     with the same epoch starts clean) - recorded into a HIP graph: every replay, with eager work and
     synchronisations in between, gives the bits of the eager call."""

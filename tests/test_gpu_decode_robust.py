@@ -58,7 +58,7 @@ LARGE = {
     "chunked-one-launch": (1, 8, 32, 8, 20000, 70, 1, False, dict(launches=1)),
     "chunked-one-launch-2bit": (1, 8, 32, 8, 12000, 70, 2, False, dict(launches=1)),
     "chunked-recompute": (1, 12, 32, 8, 20000, 70, 1, False, dict(launches=2)),       # 96 units x 6 chunks: too many to wait
-    "chunked-logits-buffer": (1, 12, 32, 8, 20000, 70, 2, False, dict(launches=2)),
+    "chunked-recompute-2bit": (1, 12, 32, 8, 20000, 70, 2, False, dict(launches=2)),
     "token-values": (2, 20, 32, 8, 3328, 128, 1, True, dict(chunks=1)),
     "token-values-2bit": (1, 8, 32, 8, 2000, 40, 2, True, dict(chunks=1)),
 }

@@ -112,6 +112,12 @@ def test_decode_launch_plan_invariants_over_random_shapes():
             units_ = a.B * a.Hkv * -(-G_ // p.heads_per_unit)
             assert units_ * p.chunks <= 256 * (2 if p.threads == 512 else 1) and p.chunks <= 64, shape
         assert (lib.cq_decode_attn_workspace(ctypes.byref(a)) > 0) == (p.chunks > 1), shape
+        if p.chunks > 1:    # min / max, partials (a chunk's and the window's), counters and records: nothing the size of T
+            rows, units_ = a.B * a.Hq, a.B * a.Hkv * -(-G_ // p.heads_per_unit)
+            up = lambda n: (n + 255) // 256 * 256
+            want = up(rows * p.chunks * 8) + up(rows * (p.chunks + (a.R > 0)) * 130 * 4) + up(units_ * 8)
+            want += units_ * {3: 4}.get(p.heads_per_unit, p.heads_per_unit) * p.chunks * 16
+            assert lib.cq_decode_attn_workspace(ctypes.byref(a)) == want, shape
         if a.v_mode == 1:
             assert p.threads == 1024 and p.register_logits in (4, 8), shape
 
