@@ -27,10 +27,14 @@ static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st
     return CQ_OK;
 }
 
-// A chunked launch has one instantiation: what the mask and the row count cost it in registers, it has to spare.
-template <int BITS, int HPB, typename DT, int NT, int REGL, int NH = HPB, bool VTOK = false>
+// A chunked launch has one instantiation, with the mask and the row count.  Of the kernels that chunked plans ask for,
+// those of 512 threads and of per-token values keep within the 128 registers; those of ten rounds spill up to 22 (48 B of
+// scratch per lane), those of sixteen 78 to 126 (152 to 224 B; 9 to 24 in single launches without mask and row count).
+// SINGLE: no plan chunks such units.
+template <int BITS, int HPB, typename DT, int NT, int REGL, int NH = HPB, bool VTOK = false, bool SINGLE = false>
 static int launch_matrix_unit(const DecodeGeom& g, unsigned units, hipStream_t st) {
-    if (g.nsplit > 1) return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, true, true, NH>(g, units, st);
+    if constexpr (SINGLE) { if (g.nsplit > 1) return CQ_ERR_UNSUPPORTED; }
+    else if (g.nsplit > 1) return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, true, true, NH>(g, units, st);
     if (g.mask || g.r_dev) return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, false, true, NH>(g, units, st);
     return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, false, false, NH>(g, units, st);
 }
@@ -41,8 +45,11 @@ static int launch_matrix_bits(const DecodeGeom& g, int hpb, int nh, int nt, unsi
     if (nt == 512) {
         if (hpb == 4 && nh == 3) return launch_matrix_unit<BITS, 4, DT, 512, kRegPair, 3>(g, units, st);
         if (hpb == 4) return launch_matrix_unit<BITS, 4, DT, 512, kRegPair>(g, units, st);
-        return most ? launch_matrix_unit<BITS, 2, DT, 512, kRegMost>(g, units, st)
-                    : launch_matrix_unit<BITS, 2, DT, 512, kRegPair>(g, units, st);
+        if constexpr (BITS == 1) {   // (two bits: two heads per unit only where there are few units)
+            if (hpb == 2) return most ? launch_matrix_unit<BITS, 2, DT, 512, kRegMost, 2, false, true>(g, units, st)
+                                      : launch_matrix_unit<BITS, 2, DT, 512, kRegPair, 2, false, true>(g, units, st);
+        }
+        return CQ_ERR_UNSUPPORTED;
     }
     if (hpb == 4 && nh == 3) return launch_matrix_unit<BITS, 4, DT, 1024, kRegLong, 3>(g, units, st);
     if (hpb == 4) return launch_matrix_unit<BITS, 4, DT, 1024, kRegLong>(g, units, st);
@@ -55,7 +62,6 @@ static int launch_matrix_bits(const DecodeGeom& g, int hpb, int nh, int nt, unsi
 // nt threads per workgroup, g.chunk tokens at most: the plan's (cq_decode.hip: make_plan)
 template <typename DT>
 int launch_matrix(const DecodeGeom& g, int bits, int hpb, int nh, int nt, unsigned units, hipStream_t st) {
-    if (nt == 512 && hpb == 1) return CQ_ERR_UNSUPPORTED;
     return bits == 1 ? launch_matrix_bits<1, DT>(g, hpb, nh, nt, units, st) : launch_matrix_bits<2, DT>(g, hpb, nh, nt, units, st);
 }
 
@@ -63,10 +69,12 @@ int launch_matrix(const DecodeGeom& g, int bits, int hpb, int nh, int nt, unsign
 // 4 096 tokens (the sixteen registers more of eight rounds do not fit beside the statistics of the values), eight above.
 template <int BITS, int HPB, typename DT>
 static int launch_token_unit(const DecodeGeom& g, unsigned units, hipStream_t st) {
-    static_assert(Lay<BITS, HPB, true, 1024, 0>::max_chunk() <= kRegPair * 1024, "the plan's chunks fit eight rounds");
+    constexpr int most = Lay<BITS, HPB, true, 1024, 0>::max_chunk();   // tokens of a plan's chunks
+    static_assert(most <= kRegPair * 1024, "the plan's chunks fit eight rounds");
     if (launch_rounds(true, HPB, 1024, g.chunk) == kRegTwoBit)
         return launch_matrix_unit<BITS, HPB, DT, 1024, kRegTwoBit, HPB, true>(g, units, st);
-    return launch_matrix_unit<BITS, HPB, DT, 1024, kRegPair, HPB, true>(g, units, st);
+    if constexpr (most > kRegTwoBit * 1024) return launch_matrix_unit<BITS, HPB, DT, 1024, kRegPair, HPB, true>(g, units, st);
+    return CQ_ERR_UNSUPPORTED;
 }
 
 template <typename DT>

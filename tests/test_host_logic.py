@@ -92,7 +92,7 @@ def test_decode_launch_plan_invariants_over_random_shapes():
         a = _lib.DecodeArgs()
         a.dtype, a.D, a.Hkv, a.Hq = int(rng.integers(0, 2)), 128, Hkv, Hkv * G
         a.B = int(rng.choice([1, 2, 3, 8, 16, 31, 32, 33, 64, 100, 256, 1000]))
-        a.T = int(rng.choice([0, 1, 63, 64, 65, 1000, 3328, 3392, 4096, 4097, 4288, 5000, 9984, 10240, 10241, 32768, 100000]))
+        a.T = int(rng.choice([0, 1, 63, 64, 65, 1000, 3328, 3392, 4096, 4097, 4160, 4288, 5000, 9984, 10240, 10241, 32768, 100000]))
         a.R = int(rng.choice([0, 1, 64, 128, 129, 1000])) if a.T else int(rng.choice([1, 64, 500]))
         a.bits = int(rng.integers(1, 3))
         a.v_mode = int(rng.integers(0, 2))
@@ -120,6 +120,11 @@ def test_decode_launch_plan_invariants_over_random_shapes():
             assert lib.cq_decode_attn_workspace(ctypes.byref(a)) == want, shape
         if a.v_mode == 1:
             assert p.threads == 1024 and p.register_logits in (4, 8), shape
+        # forms without an instantiation: 512 threads for one head, for two at 2 bits or in chunks; eight rounds of
+        # per-token values for four heads
+        if p.threads == 512:
+            assert p.heads_per_unit >= 3 or (p.heads_per_unit == 2 and a.bits == 1 and p.chunks == 1), shape
+        assert a.v_mode == 0 or p.heads_per_unit < 4 or p.register_logits == 4, shape
 
 
 def test_c_abi_rejects_bad_arguments_without_touching_the_gpu():
