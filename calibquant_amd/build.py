@@ -28,11 +28,6 @@ FLAGS = [
     "-Wall", "-Wno-unused-command-line-argument",
     "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
 ]
-# per-source additions (the profiling build's decode kernel is part of cq_decode.hip; the shipped ones, in
-# cq_decode_matrix*.hip, are scheduled by default)
-EXTRA_FLAGS = {
-    "cq_decode.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
-}
 
 
 def build(verbose: bool = True, jobs: int = 8) -> str:
@@ -41,7 +36,7 @@ def build(verbose: bool = True, jobs: int = 8) -> str:
     for src in SOURCES:
         obj = os.path.join(LIBDIR, src.replace(".hip", ".o"))
         objs.append(obj)
-        cmd = [HIPCC, *FLAGS, *EXTRA_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj]
+        cmd = [HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
         procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
@@ -111,7 +106,7 @@ def build_phase_stops(verbose: bool = True) -> str:
             continue
         obj = os.path.join(LIBDIR, src.replace(".hip", ".phases.o" if src == "cq_decode.hip" else ".o"))
         if src == "cq_decode.hip" or not os.path.exists(obj):
-            extra = EXTRA_FLAGS.get(src, []) + (["-DCQ_PHASE_STOPS"] if src == "cq_decode.hip" else [])
+            extra = ["-DCQ_PHASE_STOPS"] if src == "cq_decode.hip" else []
             cmd = [HIPCC, *FLAGS, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
             if verbose:
                 print(" ".join(cmd), flush=True)
