@@ -23,7 +23,8 @@
 // When the chunk does not cover all T tokens (long context or small batch)
 // a first launch computes every chunk's logits and publishes the per-chunk min / max;
 // the main launch recomputes its chunk's logits, exponentiates against the global min / max and writes an (m, l, acc)
-// partial; the last workgroup of a unit to get there combines the unit's partials.
+// partial; the last workgroup of a unit to get there combines the unit's partials.  Where all the chunks' workgroups
+// fit the device at once, one launch does both: the chunks exchange their min / max inside it.
 #pragma once
 #include "cq_common.h"
 
@@ -46,7 +47,7 @@ constexpr int kMatrixK = 4, kMatrixV = 4, kMatrixE = 2;
 constexpr int kLdsMax = 160 * 1024;
 constexpr int kDefaultUnits = 256; // compute units of a whole MI355X, assumed when no device can be asked
 constexpr int kRegPair = 8;        // rounds of logits a thread of a 512-thread workgroup keeps in registers (4 096 tokens)
-constexpr int kRegTwoBit = 4;      // ... of the 2-bit kernel with four heads per unit (4 096 tokens)
+constexpr int kRegTwoBit = 4;      // ... of a 1024-thread workgroup with per-token values and a short chunk (4 096 tokens); plans at 2 bits are cut with it too
 constexpr int kRegLong = 10;       // ... of a 1024-thread workgroup that holds a long chunk in one launch (10 240 tokens)
 constexpr int kRegMost = 16;       // ... of the longest chunks a plan for fewer than four heads per unit can have (16 384 tokens)
 constexpr float kLog2e = 1.4426950408889634f;
@@ -284,22 +285,24 @@ __device__ __forceinline__ void clear_handover(const DecodeGeom& g, int64_t unit
 // exact integers, put together in fp32.  Packed codes are masked in place, the upper half of a byte after one shift of
 // the word - one AND per 4 codes; a code then counts 2^s, s = 0 .. 3, which the fixed-point operand (logits) or the
 // closing fold (sums) takes back.
-// Measured, us per step, look-up form before and this one: batch 64 x 3 328 + 128, 1 bit 26.4 -> 19.4, 2 bits 47.8 -> 28.2;
-// batch 256 x 3 328 88 -> 55 (49 % of the rate of a large copy); 16 x 9 984, six heads 38.3 -> 23.5; 8 x 32 768 in
-// chunks 35.8 -> 29.0; batch 1 x 1 024 7.7 -> 6.4.  A 64-token tile of four heads takes about 140 vector instructions
-// (1 500 before) and 16 MFMAs; what bounds a launch now is the latency of its phases, then the memory.
-// Error against 64 bits: a weight is off by 2^-31 at most, a channel's q.s_k by 2^-27 of the head's largest (s = 3 costs
-// three of the grid's bits; masked in place all through, the top bit of a byte would cost seven), then the fp32 roundings.
+// Measured, us per step in turn on one box, look-up form before and this one: batch 64 x 3 328 + 128, 1 bit 28.5 -> 20.2,
+// 2 bits 48.9 -> 28.4; batch 256 x 3 328 99.7 -> 58.3 (3.9 TB/s); 16 x 9 984, six heads 38.4 -> 21.7; 8 x 32 768 in chunks
+// 36.8 -> 26.8; batch 1 x 1 024 7.7 -> 6.7.  A wave with 6.5 tiles of 64 tokens and four heads issues 1 810 vector
+// instructions (3 097 before), the set-up and the window's 350 among them: 84 a tile for the logits, 125 for weights and
+// values, 16 of these MFMAs.  What bounds a launch now is the latency of its phases, then the memory.
+// Error against 64 bits: a weight is off by 2^-31 at most; a channel's q.s_k by 2^(s - 30) of the head's
+// largest (s = 3: 2^-27, three of the grid's bits; masked in place all through, the top bit of a byte would cost seven),
+// then the fp32 roundings.
 // The look-up form added fp32 partial sums on the K side and held the weights as fp16 on the V side.  Root-mean-square
 // logit error over its own (a model of both on the CPU, keys with outlier channels of 1, 10, 100 and 1 000 times the
 // others): 0.59, 0.57, 0.56, 0.55 at 1 bit - 0.93, 1.4, 2.2, 2.8 masked in place -, 0.55, 0.52, 0.56, 0.53 at 2 bits.
 // (The shift costs batch 64 x 3 328 0.25 us at 1 bit and nothing at 2 bits.)
-// fp16 outputs lie 2.0e-4 from 64 bits, which is their own rounding, 7e-4 to 1.3e-3 there.
+// fp16 outputs lie 2.0e-4 to 2.2e-4 from 64 bits, which is their own rounding, 8e-4 to 1.6e-3 there (nine shapes).
 typedef int I4 __attribute__((ext_vector_type(4)));
 typedef int I2 __attribute__((ext_vector_type(2)));
 typedef uint32_t U2 __attribute__((ext_vector_type(2)));
 
-// four signed byte digits of x, |x| < 2^31 - 2^23 (digit 0 in the lowest byte)
+// four signed byte digits of x, -2^31 <= x <= 2^31 - 1 - 0x808080 (digit 0 in the lowest byte; above that the top digit wraps)
 __device__ __forceinline__ uint32_t byte_digits(int x) {
     return (static_cast<uint32_t>(x) + 0x00808080u) ^ 0x00808080u;
 }
@@ -439,9 +442,10 @@ template <int BITS> __device__ __forceinline__ void matrix_fold(const I4* acc, f
 // byte shifted by four, the one half a byte higher: 16 columns of the result are 16 channels, two MFMAs are a group.
 // The grid is a head's own largest e * scale of the group among the wave's tokens - the weighted scale, because a token
 // without weight (masked, or out of this head's sight) may have a scale of any size; sums of e * minimum stay in fp32.
-// Measured at batch 64 x 3 328 + 128, 1 bit, us per step: look-up form 58.1, this one 36.7 (1 024 threads, one workgroup per
-// compute unit: the four groups' operands, converted and read back one after the other, are what bounds it).  Grids of the
-// scales alone, as wide as the least weighted token makes them, were 36.9 there and 2.5 % faster in the middle of 60 shapes.
+// Measured at batch 64 x 3 328 + 128, 1 bit, us per step in turn on one box: look-up form 58.6, this one 38.9 (1 024 threads,
+// one workgroup per compute unit: the four groups' operands, converted and read back one after the other, are what bounds
+// it).  Grids of the scales alone, as wide as the least weighted token makes them, were within 1 % there and 2.5 % faster in
+// the middle of 60 shapes.
 // Weights and scales have 32 bits here, the look-up tables held their products and short sums as fp16.
 // st: the lane's own token's scales and minima (layout of `stats` below); pw: the head's grid, 2^(30 - e) per group.
 template <int BITS, typename DT>
@@ -563,15 +567,14 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     const int lane = tid & 63;
     const int wv = tid >> 6;
     const int G = g.G;
-    // Wave priorities of the paired launch (two 512-thread workgroups per compute unit, all of them
-    // resident from the first cycle).  Left to the hardware's own arbitration the workgroup that was
-    // dispatched first gets most of the issue slots: it ends after about 56 K cycles and the other one
-    // after 77 K, the last 20 K alone on the unit with too few waves to hide its own latencies.  With the
-    // short, latency-bound phases (set-up, table build, reductions, staging, exp) above the throughput
-    // phases, the first workgroup ahead in the K look-ups and the second ahead in the packed-V loop,
-    // both end together (measured at the benchmark shape: 36.0 -> 33.8 us, same results).  Launches with
-    // more workgroups than fit at once start their later workgroups as earlier ones end, which staggers
-    // them by itself; there the priorities are left alone (with them: 66 -> 84 us at batch 128).
+    // Wave priorities of the paired launch (two 512-thread workgroups per compute unit, all of them resident from
+    // the first cycle).  Left to the hardware's own arbitration the workgroup that was dispatched first gets most of
+    // the issue slots, and the other one ends alone on the unit with too few waves to hide its latencies.  So the
+    // short, latency-bound phases (set-up, reductions) go above the throughput phases, the first workgroup ahead in
+    // the logits and the second in the packed-V loop.  Measured with and without, us per step at 3 328 + 128 tokens:
+    // batch 33, 2 bits 21.1 -> 19.8; batch 40 19.3 -> 18.6; batch 64, 2 bits 27.4 -> 26.6, 1 bit 21.3 -> 21.2; two heads
+    // per unit 17.8 -> 18.1.  Launches with more workgroups than fit at once start their later workgroups as earlier
+    // ones end, which staggers them by itself; there the priorities are left alone.
     // `second`: the workgroup that shares its unit with an older one (workgroups are handed out unit by
     // unit, g.ncu at a time).
     const bool prio_on = NT == 512 && g.ncu > 0;
@@ -681,7 +684,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     };
 
     CQ_PHASE(1);   // prologue, requests of q and the statistics
-    // ---- phase 0: q, per-bit weights ---------------------------------------------------
+    // ---- phase 0: q onto its grid ---------------------------------------------------
     if (tid < HPB * kD) {
         const int h = tid / kD, d = tid % kD;
         const float qraw = Cvt<DT>::to_float(q_raw);
@@ -706,11 +709,8 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         fx[L::F_VSZ + kD + d] = Cvt<DT>::to_float(z_raw);
     }
     if (tid < 3 * HPB) reinterpret_cast<int*>(red)[tid] = static_cast<int>(0x80000000u);   // block_max's meeting words
-    // The packed K rows are requested only now: a wave that has to queue 64 KB of requests
-    // first gets to phase 0 thousands of cycles later, and the table build below covers
-    // their latency anyway.
-    // (requested any later - after the table build, or all but the first round - the launch is slower;
-    // requested at kernel entry, ahead of q, as well)
+    // The packed K rows are requested only now, behind what phase 0 waits for: a wave that has to queue these
+    // requests first gets to phase 0 later.
     uint4 kc[L::KR][BITS];
 #pragma unroll
     for (int r = 0; r < L::KR; ++r) {
@@ -753,7 +753,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         for (int r = 0; r < kVEarly; ++r) request_v(r);
     }
 
-    CQ_PHASE(2);   // q, per-bit weights, first packed K rows requested
+    CQ_PHASE(2);   // q on its grid, first packed K rows requested
     // the wave's first token, and the head whose results this lane holds (lanes beyond the unit's heads repeat
     // the last one)
     const int wt0 = __builtin_amdgcn_readfirstlane(tid);
@@ -822,7 +822,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
 
         if constexpr (CHUNKED) {
             // One launch: this chunk's min / max go out now (write-through stores, waited for, then the arrival
-            // count); the other chunks' are collected further down, after the staging of the first V block.
+            // count); the other chunks' are collected further down.
             if (g.fused && has_img && tid == 0) {
                 unsigned long long* o = g.rec + ((unit * HPB) * g.nsplit + split) * 2;
                 const unsigned long long tag = static_cast<unsigned long long>(g.epoch) << 32;
