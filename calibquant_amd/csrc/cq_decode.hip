@@ -49,17 +49,15 @@ static int pair_units() {
 static inline int ngroups(int G, int hpb) { return (G + hpb - 1) / hpb; }
 
 struct Plan {
-    int hpb, nh, nt, nsplit, chunk, nx, cap;   // hpb: heads an entry is wide; nh: heads a unit serves
+    int hpb, nh, nt, nsplit, chunk, nx;   // hpb: heads an entry is wide; nh: heads a unit serves
     bool fused;   // chunked step in one launch: every chunk's workgroup fits the device at once
     size_t ws_mm, ws_part, ws_cnt;   // chunked launch: min / max, partials, counters
 };
 
-template <int BITS, int HPB, bool VTOK, int NT = 1024, int REGL = 0>
-static void plan_for(const cq_decode_args* a, Plan* p, int nh = HPB) {
-    using L = Lay<BITS, HPB, VTOK, NT, REGL>;
+// units of nh heads (entries hpb wide) in workgroups of nt threads, chunks of at most maxc tokens
+static void plan_for(const cq_decode_args* a, Plan* p, int hpb, int nh, int nt, int maxc) {
     const int G = a->Hq / a->Hkv;
     const int64_t units = static_cast<int64_t>(a->B) * a->Hkv * ngroups(G, nh);
-    const int maxc = L::max_chunk();
     int nsplit = 1;
     if (a->T > 0) {
         const int need = (a->T + maxc - 1) / maxc;
@@ -79,19 +77,18 @@ static void plan_for(const cq_decode_args* a, Plan* p, int nh = HPB) {
     int chunk = a->T > 0 ? ((a->T + nsplit - 1) / nsplit + 63) / 64 * 64 : 64;
     if (chunk > maxc) chunk = maxc;
     nsplit = a->T > 0 ? (a->T + chunk - 1) / chunk : 1;
-    p->hpb = HPB;
+    p->hpb = hpb;
     p->nh = nh;
-    p->nt = NT;
+    p->nt = nt;
     p->nsplit = nsplit;
     p->chunk = chunk;
     p->nx = nsplit + ((nsplit > 1 && a->R > 0) ? 1 : 0);
-    p->cap = a->T > 0 ? chunk : 64;
     const size_t rows = static_cast<size_t>(a->B) * a->Hq;
     p->ws_mm = nsplit > 1 ? ((rows * nsplit * 2 * sizeof(float) + 255) / 256 * 256) : 0;
     p->ws_part = nsplit > 1 ? (rows * p->nx * (kD + 2) * sizeof(float) + 255) / 256 * 256 : 0;
     // counters: [unit] partials written (4 or 8 bytes), then the min / max records of the single-launch step
     p->ws_cnt = nsplit > 1 ? (static_cast<size_t>(units) * sizeof(unsigned long long) + 255) / 256 * 256 +
-                                 static_cast<size_t>(units) * HPB * nsplit * 16 : 0;
+                                 static_cast<size_t>(units) * hpb * nsplit * 16 : 0;
     p->fused = false;
 }
 
@@ -110,68 +107,42 @@ static int make_plan(const cq_decode_args* a, Plan* p) {
     // heads a unit with four-wide entries serves: three when that divides the group exactly and four does not
     // (G = 3, 6, 9: exact units instead of a padded last one; per-channel values only)
     const int nh4 = (!vtok && G % 3 == 0 && G % 4 != 0) ? 3 : 4;
-    if (a->bits == 1) {
-        // G = 3, 5, 6, 7, ...: units of four heads with the last one partly padding (two units per kv head at
-        // G = 6) do less work than units of two heads or one (three or six of them, each walking all the packed rows)
-        const bool pad4 = G % 4 != 0 && G > 2;
-        if (G % 4 == 0 || pad4) vtok ? plan_for<1, 4, true>(a, p) : plan_for<1, 4, false>(a, p, nh4);
-        else if (G % 2 == 0) vtok ? plan_for<1, 2, true>(a, p) : plan_for<1, 2, false>(a, p);
-        else vtok ? plan_for<1, 1, true>(a, p) : plan_for<1, 1, false>(a, p);
-        // More units than compute units: 512-thread workgroups, two resident per compute unit, need fewer
-        // instructions per unit than one 1024-thread workgroup after the other (half as many waves pay
-        // the per-wave set-up, reductions and folds) - when a unit's whole layout fits half the LDS.
-        // Four heads per unit, enough units to fill the device, and T beyond the layout with fp32 logits in
-        // the token slots: with the logits in registers (half the bytes per token slot) the layout may still
-        // hold all T tokens in one launch, which saves the min/max launch's second pass over the packed K rows.
-        if (p->hpb == 4 && !vtok && a->force_splits == 0 && p->nsplit > 1 &&
-            static_cast<int64_t>(a->B) * a->Hkv * ngroups(G, nh4) >= kPairUnits * 3 / 4) {
-            Plan q;
-            plan_for<1, 4, false, 1024, kRegLong>(a, &q, nh4);
+    auto plan = [&](Plan* o, int hpb, int nh) { plan_for(a, o, hpb, nh, 1024, plan_chunk(a->bits, vtok, hpb)); };
+    // G = 3, 5, 6, 7, ...: units of four heads with the last one partly padding (two units per kv head at
+    // G = 6) do less work than units of two heads or one (three or six of them, each walking all the packed rows).
+    // Per-token values at 2 bits: two heads per unit, padded for odd G (there is no form with four).
+    if (vtok && a->bits == 2) plan(p, G >= 2 ? 2 : 1, G >= 2 ? 2 : 1);
+    else if (G > 2) plan(p, 4, nh4);
+    else plan(p, G, G);
+    if (!vtok && a->force_splits == 0 && p->hpb >= 2) {
+        // Four heads per unit at 1 bit, enough units to fill the device, and T beyond the chunk: the longer chunk may
+        // still hold all T tokens in one launch, which saves the min/max launch's second pass over the packed K rows.
+        const int64_t units = static_cast<int64_t>(a->B) * a->Hkv * ngroups(G, p->nh);
+        Plan q;
+        if (a->bits == 1 && p->hpb == 4 && p->nsplit > 1 && units >= kPairUnits * 3 / 4) {
+            plan_for(a, &q, 4, nh4, 1024, kPlanLong);
             if (q.nsplit == 1) *p = q;
         }
-        // Single launch: only if the 512-thread layout also holds all T tokens.  Chunked launch (four heads
-        // per unit): the chunks are units of their own.
-        const int64_t units = static_cast<int64_t>(a->B) * a->Hkv * ngroups(G, p->nh);
-        if (!vtok && a->force_splits == 0 && p->hpb >= 2) {
-            Plan q;
-            if (p->hpb == 4) plan_for<1, 4, false, 512, kRegPair>(a, &q, nh4); else plan_for<1, 2, false, 512, 0>(a, &q);
+        // More units than compute units: 512-thread workgroups, two resident per compute unit, need fewer
+        // instructions per unit than one 1024-thread workgroup after the other (half as many waves pay
+        // the per-wave set-up, reductions and folds).  Single launch: only if their chunk also holds all T tokens.
+        // Chunked launch (four heads per unit): the chunks are units of their own.
+        if (p->hpb == 4 || a->bits == 1) {
+            plan_for(a, &q, p->hpb, p->nh, 512, p->hpb == 4 ? kPlanPair4 : kPlanPair2);
             const bool single = p->nsplit == 1 && q.nsplit == 1 && units > kPairUnits;
             const bool chunked = p->hpb == 4 && p->nsplit > 1 && q.nsplit > 1 && units * q.nsplit > kPairUnits;
             if (single || chunked) *p = q;
         }
-    } else {
-        // four heads per unit need the two-pass K table; with per-token values their LDS layout
-        // would not hold a 3 328-token chunk, so that mode keeps two heads per unit
-        // (the first pass's partial logits wait in registers, four tokens per thread: -3 % against the token slots)
-        if ((G % 4 == 0 || G > 2) && !vtok) {
-            plan_for<2, 4, false, 1024, kRegTwoBit>(a, p, nh4);
-            // more units than compute units: two 512-thread workgroups per compute unit (K table in two passes)
-            const int64_t units = static_cast<int64_t>(a->B) * a->Hkv * ngroups(G, nh4);
-            if (a->force_splits == 0) {
-                Plan q;
-                plan_for<2, 4, false, 512, kRegPair>(a, &q, nh4);
-                const bool single = p->nsplit == 1 && q.nsplit == 1 && units > kPairUnits;
-                const bool chunked = p->nsplit > 1 && q.nsplit > 1 && units * q.nsplit > kPairUnits;
-                if (single || chunked) *p = q;
-            }
-        }
-        else if (G >= 2) vtok ? plan_for<2, 2, true>(a, p) : plan_for<2, 2, false>(a, p);   // (per-token values: two heads per unit, padded for odd G)
-        else vtok ? plan_for<2, 1, true>(a, p) : plan_for<2, 1, false>(a, p);
     }
     // A handful of units leave most compute units idle, and a launch then lasts as long as one unit: fewer
-    // heads per unit make the units cheaper (18.8 / 15.5 / 14.2 us for four / two / one head at 3 328 + 128 tokens)
-    // and there are compute units for two or four times as many of them.
+    // heads per unit make the units cheaper and there are compute units for two or four times as many of them.
+    // (Where the lines lie was measured with the look-up form: 18.8 / 15.5 / 14.2 us for four / two / one head at
+    // 3 328 + 128 tokens.)
     if (a->force_splits == 0 && p->nsplit == 1 && p->hpb == 4) {
         const int64_t u4 = static_cast<int64_t>(a->B) * a->Hkv * ngroups(G, p->nh);
         const int h = u4 <= 32 ? 1 : (u4 <= 64 && G % 2 == 0) ? 2 : 4;
         Plan q = *p;
-        if (a->bits == 1) {
-            if (h == 1) vtok ? plan_for<1, 1, true>(a, &q) : plan_for<1, 1, false>(a, &q);
-            if (h == 2) vtok ? plan_for<1, 2, true>(a, &q) : plan_for<1, 2, false>(a, &q);
-        } else {
-            if (h == 1) vtok ? plan_for<2, 1, true>(a, &q) : plan_for<2, 1, false>(a, &q);
-            if (h == 2) vtok ? plan_for<2, 2, true>(a, &q) : plan_for<2, 2, false>(a, &q);
-        }
+        if (h < 4) plan(&q, h, h);
         if (q.nsplit == 1) *p = q;
     }
     const int64_t blocks = static_cast<int64_t>(a->B) * a->Hkv * ngroups(G, p->nh) * p->nx;
@@ -337,7 +308,6 @@ static int decode_entry(const cq_decode_args* a, void* workspace, size_t workspa
     g.B = a->B; g.Hq = a->Hq; g.Hkv = a->Hkv; g.T = a->T; g.R = a->R; g.S = a->sprompt_len;
     g.nsplit = p.nsplit; g.chunk = p.chunk; g.nx = p.nx;
     g.calib = a->calibrate; g.off_max = a->calib_off_max; g.off_min = a->calib_off_min;
-    g.cap = p.cap;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool vtok = a->v_mode == CQ_V_PER_TOKEN;
     if (a->dtype == CQ_BF16) return dispatch<BF16>(g, p, a->bits, vtok, st);

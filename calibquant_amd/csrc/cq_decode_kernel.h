@@ -40,14 +40,13 @@
 namespace cq {
 
 constexpr int kD = 128;
-constexpr int kPF = 4;             // 16-byte loads kept in flight per thread and stream
-// matrix-core form: 16-byte pieces of packed K and V rows in flight per thread, and of the V rows how many are requested
+// 16-byte pieces of packed K and V rows in flight per thread, and of the V rows how many are requested
 // ahead of the logits
 constexpr int kMatrixK = 4, kMatrixV = 4, kMatrixE = 2;
 constexpr int kLdsMax = 160 * 1024;
 constexpr int kDefaultUnits = 256; // compute units of a whole MI355X, assumed when no device can be asked
 constexpr int kRegPair = 8;        // rounds of logits a thread of a 512-thread workgroup keeps in registers (4 096 tokens)
-constexpr int kRegTwoBit = 4;      // ... of a 1024-thread workgroup with per-token values and a short chunk (4 096 tokens); plans at 2 bits are cut with it too
+constexpr int kRegTwoBit = 4;      // ... of a 1024-thread workgroup with per-token values and a short chunk (4 096 tokens)
 constexpr int kRegLong = 10;       // ... of a 1024-thread workgroup that holds a long chunk in one launch (10 240 tokens)
 constexpr int kRegMost = 16;       // ... of the longest chunks a plan for fewer than four heads per unit can have (16 384 tokens)
 constexpr float kLog2e = 1.4426950408889634f;
@@ -102,7 +101,6 @@ struct DecodeGeom {
     int nsplit, chunk, nx;
     int calib;
     float off_max, off_min;
-    int cap;      // logits capacity of the LDS layout, tokens
     FastDiv d_ng, d_nx, d_hkv;   // divisors of the unit decomposition: head groups, chunks (+ residual unit), kv heads
     int G;        // query heads per kv head
     int ncu;      // paired launch whose workgroups are all resident from the start (at most two per compute unit):
@@ -110,16 +108,12 @@ struct DecodeGeom {
 };
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
-constexpr int cmin(int a, int b) { return a < b ? a : b; }
 
 // VTOK: values quantised per token and per group of 32 channels (scale * code + minimum, codes in little-endian
 // 32-bit words, first channel in the lowest bits) instead of per channel.
-// REGL: rounds of kNT tokens whose logits a thread keeps in registers.
-// MX: the layout the kernel runs with: region A holds one 64-token tile of weights and of packed V rows per wave,
-// later the folds' partials.  Without it the struct describes the table layout of the look-up form this kernel had before;
-// plans are still cut with it (max_chunk, and the LDS a plan reports), so that chunks and workspace sizes are the ones
-// callers have laid out: its fields are sizes only.
-template <int BITS, int HPB, bool VTOK = false, int NT_ = 1024, int REGL = 0, bool MX = false> struct Lay {
+// Region A of the LDS holds the query's digits while the logits are worked out, then one 64-token tile of weights and of
+// packed V rows per wave, later the folds' partials; the words a whole workgroup shares lie behind it.
+template <int BITS, int HPB, bool VTOK = false, int NT_ = 1024> struct Lay {
     static constexpr int kNT = NT_;                 // threads per workgroup
     static constexpr int kNW = kNT / kWave;         // waves per workgroup
     // residual window: tiles of 128 rows for either workgroup size - a 512-thread workgroup puts 4 lanes on a
@@ -129,74 +123,32 @@ template <int BITS, int HPB, bool VTOK = false, int NT_ = 1024, int REGL = 0, bo
     static constexpr int NKP = 16 / LPR;            // 16-byte pieces of a row per lane
     static constexpr int RPW = kResTile / kNW;      // rows of a tile whose values one wave multiplies
     static constexpr int NB = 16 * BITS;            // bytes per packed row
-    static constexpr int PC = NB * 8;               // bit lanes per row
-    static constexpr int GPW = kWave / NB;          // 4-token groups per wave pass
-    static constexpr int MPL = 8 / GPW;             // bit lanes of a byte column handled by one lane
-    static constexpr int TPW = 4 * GPW;             // tokens per wave pass
-    static constexpr int ESZ = HPB * 4;             // bytes per fp32 table entry / logits slot
-    static constexpr int HW = HPB >= 2 ? HPB / 2 : 1;   // 32-bit words per packed-fp16 entry
-    static constexpr int ESZH = HW * 4;             // bytes per packed-fp16 table entry
-    // The byte-indexed K table covers NBP byte positions at a time: all of them when that fits the
-    // table's share of the LDS (64 KB; 32 KB for a 512-thread workgroup), else half of them in each of
-    // two (or a quarter in each of four) passes over the chunk's rows, the earlier passes' partial logits
-    // waiting in the token slots or, with REGL, in registers.
-    // INA (512-thread workgroup with the logits in registers): nothing else lives in LDS while the K table is
-    // in use, so the table takes all 64 KB of region A and the token slots, written only after the last
-    // look-up, sit in that region as well, behind the staged V block - one table pass at 1 bit (two at 2 bits)
-    // with 256-byte rows, i.e. single-permute look-up addresses, inside the 80 KB a paired workgroup may use.
-    // The table is then built straight from the per-bit weights (no nibble tables to find room for).
-    static constexpr bool INA = (NT_ == 512 && REGL > 0 && !MX);
-    static constexpr int KTMAX = ((NT_ == 512 && !INA) ? 32 : 64) * 1024;
-    static constexpr int KPASS = (NB * 256 * ESZ > 2 * KTMAX) ? 4 : (NB * 256 * ESZ > KTMAX) ? 2 : 1;
-    static constexpr int NBP = NB / KPASS;          // byte positions per pass
-    static constexpr int WPP = NBP / 4;             // 32-bit words of a row per pass
-    static constexpr int PCS = (WPP + 3) / 4;       // 16-byte pieces of a row a pass looks at
-    static constexpr int KT = NBP * 256 * ESZ;      // K table bytes
-    static_assert(NB * 256 * ESZ <= 4 * KTMAX, "at most four table passes");
-    static_assert(!(REGL > 0 && VTOK && !MX), "look-ups with logits in registers: per-channel values only");
-    static constexpr int SLOT = MX ? 0 : VTOK ? 16 : (REGL > 0 ? ESZH : ESZ);   // bytes per token slot: logits, later e (+ 4 group scales)
-    static constexpr int NGRP = VTOK ? kD / 32 : 1; // channel groups with tables of their own
-    static constexpr int WTAB = kNW * NGRP * GPW * 16 * ESZH;
-    static constexpr int RW = cmax(3 * HPB, VTOK ? (NGRP + 1) * HPB : 0);   // per-wave partials: min/max + masked max, or the closing sums
-    static constexpr int VSUB = kNT * kPF / BITS;   // V tokens staged at a time
-    static constexpr int KR = (MX ? kMatrixK : kPF) / BITS;           // K token rounds in flight per thread
-    static constexpr int RED = kNW * PC * ESZ;
-    static constexpr int RED2 = kNW * kD * ESZ;
-    // fixed small region (floats)
-    static constexpr int F_WBIT = 0;                          // NB*8*HPB
-    static constexpr int F_QSZ = F_WBIT + NB * 8 * HPB;       // NB*HPB: zero-point sum per byte position and head
-    static constexpr int F_QRAW = F_QSZ + NB * HPB;           // HPB*kD raw 16-bit q
-    static constexpr int F_RED = F_QRAW + HPB * kD / 2;       // kNW*HPB
-    static constexpr int F_STAT = F_RED + kNW * RW;           // 8*HPB: per-head softmax state
-    static constexpr int F_VSZ = F_STAT + 8 * HPB;            // 2*kD: value scale, zero-point (VTOK: NGRP*HPB minimum terms)
-    static constexpr int F_NIB = F_VSZ + 2 * kD;              // NB*32*HPB: nibble tables
-    // (REGL: the nibble tables live in the token slots, which are first written after the last table pass;
-    // INA: there are none)
-    static constexpr int NIBF = NB * 32 * HPB;
-    static constexpr int F_SRES = F_NIB + (REGL > 0 ? 0 : NIBF);  // kResTile*HPB
-    static constexpr int F_PRES = F_SRES + kResTile * HPB;    // kResTile*HPB
-    static constexpr int F_END = F_PRES + kResTile * HPB;
-    static constexpr int FIXED = ((F_END * 4 + 255) / 256) * 256;
-    // byte offset of the token slots: behind the fixed region, or (INA) inside region A behind the staged V block
-    static constexpr int slots_in_a(int cap) { return WTAB + cmin(VSUB, cap) * NB; }
-    // MX: bytes of a wave's tile: weights, then packed V rows (VTOK: weights and rows of one channel group, statistics)
+    static constexpr int KR = kMatrixK / BITS;      // K token rounds in flight per thread
+    // bytes of a wave's tile: weights, then packed V rows (VTOK: weights and rows of one channel group, statistics)
     static constexpr int MXT = VTOK ? 2560 : (1 + BITS) * 1024;
-    static constexpr int region_a(int cap) {
-        if (MX) return cmax(kNW * MXT, RED2);
-        return (cmax(cmax(KT, slots_in_a(cap) + (INA ? cap * SLOT : 0)), cmax(RED, RED2)) + 255) / 256 * 256;
-    }
-    static constexpr int lds_bytes(int cap) {
-        return region_a(cap) + FIXED + ((INA || MX) ? 0 : cmax(cap * SLOT, REGL > 0 ? NIBF * 4 : 0));
-    }
-    // largest chunk whose layout fits: the whole LDS for a 1024-thread workgroup, half of it for a
-    // 512-thread workgroup (two are meant to be resident per compute unit)
-    static constexpr int max_chunk() {
-        int best = 64;
-        for (int c = 64; c <= 16384; c += 64)
-            if (lds_bytes(c) <= (kNT == 512 ? kLdsMax / 2 : kLdsMax) && (REGL == 0 || c <= REGL * kNT)) best = c;
-        return best;
-    }
+    static constexpr int kRegionA = cmax(kNW * MXT, kNW * kD * HPB * 4);
+    // shared words, in floats (what is read as vectors first: each of these starts on 16 bytes)
+    static constexpr int F_QRAW = 0;                          // HPB*kD raw 16-bit q
+    static constexpr int F_SRES = F_QRAW + HPB * kD / 2;      // kResTile*HPB: logits of a tile of the window
+    static constexpr int F_PRES = F_SRES + kResTile * HPB;    // kResTile*HPB: its weights; before, the waves' closing sums
+    static constexpr int F_VSZ = F_PRES + kResTile * HPB;     // 2*kD: value scale, zero-point
+    static constexpr int F_QSZ = F_VSZ + (VTOK ? 0 : 2 * kD); // [head]: value of one grid step, zero-point sum
+    static constexpr int F_RED = F_QSZ + 2 * HPB;             // minima, maxima, masked maxima; from 4*HPB the chunks' fold and its flag
+    static constexpr int F_STAT = F_RED + 8 * HPB;            // 8*HPB: per-head softmax state
+    static constexpr int F_END = F_STAT + 8 * HPB;
+    static_assert(kNW * 5 * HPB <= kResTile * HPB, "the waves' closing sums fit the window's weights");
+    static constexpr int kLds = kRegionA + (F_END * 4 + 255) / 256 * 256;
 };
+
+// Tokens a chunk of a plan may have, for units of hpb heads in 1 024 threads.  These are what the LDS tables of an earlier
+// form of the kernel left room for (the limits of the forms below are of the same kind); the instantiations hold more, up to
+// launch_rounds() * threads.
+constexpr int plan_chunk(int bits, bool vtok, int hpb) {
+    if (vtok) return bits == 1 ? (hpb == 4 ? 3520 : hpb == 2 ? 4480 : 4736) : (hpb == 2 ? 4672 : 5120);
+    return bits == 1 ? (hpb == 4 ? 4480 : hpb == 2 ? 10560 : 16384) : (hpb == 4 ? 4096 : hpb == 2 ? 10176 : 16384);
+}
+constexpr int kPlanLong = 10048;                     // four heads at 1 bit, where that saves the chunks
+constexpr int kPlanPair4 = 4096, kPlanPair2 = 4736;  // 512 threads: four heads, two heads (1 bit)
 
 // What a launch of units of hpb heads in nt threads runs with: the rounds of logits its instantiation keeps in
 // registers for chunks of at most `chunk` tokens, and its dynamic LDS.  Launches pick by the first and check themselves
@@ -208,8 +160,7 @@ constexpr int launch_rounds(bool vtok, int hpb, int nt, int chunk) {
     return chunk <= few * nt ? few : kRegMost;
 }
 template <int BITS, bool VTOK, int NT> constexpr int launch_lds(int hpb) {
-    return hpb == 4 ? Lay<BITS, 4, VTOK, NT, kRegPair, true>::lds_bytes(0)
-         : hpb == 2 ? Lay<BITS, 2, VTOK, NT, kRegPair, true>::lds_bytes(0) : Lay<BITS, 1, VTOK, NT, kRegPair, true>::lds_bytes(0);
+    return hpb == 4 ? Lay<BITS, 4, VTOK, NT>::kLds : hpb == 2 ? Lay<BITS, 2, VTOK, NT>::kLds : Lay<BITS, 1, VTOK, NT>::kLds;
 }
 inline int launch_lds(int bits, bool vtok, int hpb, int nt) {
     if (vtok) return bits == 1 ? launch_lds<1, true, 1024>(hpb) : launch_lds<2, true, 1024>(hpb);
@@ -552,14 +503,13 @@ template <int BITS, int HPB, typename DT, bool MINMAX_ONLY, bool VTOK = false, i
 // (four waves per SIMD - at most 128 VGPRs - for either workgroup size: two 512-thread workgroups per compute
 // unit are only resident together within that)
 __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
-    using L = Lay<BITS, HPB, VTOK, NT, REGL, true>;
+    using L = Lay<BITS, HPB, VTOK, NT>;
     using V = Vec<HPB>;
     constexpr int NB = L::NB;
     constexpr int kNT = L::kNT, kNW = L::kNW, kResTile = L::kResTile;
     extern __shared__ __attribute__((aligned(256))) unsigned char smem[];
-    const int reg_a = L::region_a(g.cap);
     unsigned char* regA = smem;
-    float* fx = reinterpret_cast<float*>(smem + reg_a);
+    float* fx = reinterpret_cast<float*>(smem + L::kRegionA);
     float* qsz = fx + L::F_QSZ;
     float* red = fx + L::F_RED;
 
@@ -1276,11 +1226,10 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
 }
 
 // The min/max launch of a two-launch chunked step: no residual unit.
-static inline DecodeGeom minmax_geometry(const DecodeGeom& g, int cap) {
+static inline DecodeGeom minmax_geometry(const DecodeGeom& g) {
     DecodeGeom g1 = g;
     g1.nx = g.nsplit;
     g1.d_nx.set(static_cast<uint32_t>(g.nsplit));
-    g1.cap = cap;
     return g1;
 }
 

@@ -1,4 +1,4 @@
-// Launches of the matrix-core form of the decode step (kernel: cq_decode_kernel.h, template flag MX).
+// Launches of the matrix-core form of the decode step (kernel: cq_decode_kernel.h).
 #pragma once
 #include "cq_decode_kernel.h"
 
@@ -8,14 +8,14 @@ namespace cq {
 
 template <int BITS, int HPB, typename DT, bool VTOK, int NT, int REGL, bool CHUNKED, bool EXTRAS, int NH>
 static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st) {
-    constexpr int lds = Lay<BITS, HPB, VTOK, NT, REGL, true>::lds_bytes(0);
+    constexpr int lds = Lay<BITS, HPB, VTOK, NT>::kLds;
     static_assert(lds <= 64 * 1024, "no raised dynamic-LDS limit needed; two 512-thread workgroups share a compute unit");
     static_assert(lds == launch_lds<BITS, VTOK, NT>(HPB), "the LDS that plans report");
     if (launch_rounds(VTOK, HPB, NT, g.chunk) != REGL || g.chunk > REGL * NT) return CQ_ERR_UNSUPPORTED;   // (a token too many would be left out of the sum)
     if constexpr (CHUNKED) {
         if (!g.fused) {
-            const DecodeGeom g1 = minmax_geometry(g, 0);   // (this launch never looks at values)
-            constexpr int lds1 = Lay<BITS, HPB, false, NT, REGL, true>::lds_bytes(0);
+            const DecodeGeom g1 = minmax_geometry(g);   // (this launch never looks at values)
+            constexpr int lds1 = Lay<BITS, HPB, false, NT>::kLds;
             hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, true, false, NT, REGL, true, false, NH>),
                                dim3(units * g.nsplit), dim3(NT), lds1, st, g1);
             CQ_LAUNCH_CHECK();
@@ -69,7 +69,7 @@ int launch_matrix(const DecodeGeom& g, int bits, int hpb, int nh, int nt, unsign
 // 4 096 tokens (the sixteen registers more of eight rounds do not fit beside the statistics of the values), eight above.
 template <int BITS, int HPB, typename DT>
 static int launch_token_unit(const DecodeGeom& g, unsigned units, hipStream_t st) {
-    constexpr int most = Lay<BITS, HPB, true, 1024, 0>::max_chunk();   // tokens of a plan's chunks
+    constexpr int most = plan_chunk(BITS, true, HPB);
     static_assert(most <= kRegPair * 1024, "the plan's chunks fit eight rounds");
     if (launch_rounds(true, HPB, 1024, g.chunk) == kRegTwoBit)
         return launch_matrix_unit<BITS, HPB, DT, 1024, kRegTwoBit, HPB, true>(g, units, st);
