@@ -215,7 +215,7 @@ MID_BATCH = [
     # reps, Hq, Hkv, T, R, S, bits, dtype, mask, token values — 65..256 units of four heads: one 1024-thread workgroup
     # per unit, logits waiting in the token slots (smaller batches get fewer heads per unit)
     (6, 32, 8, 3328, 128, 0, 1, "bf16", False, False),
-    (6, 32, 8, 777, 60, 41, 2, "fp16", True, False),     # 2 bits: K table in two passes, partial logits in the slots
+    (6, 32, 8, 777, 60, 41, 2, "fp16", True, False),     # 2 bits
     (6, 32, 8, 1500, 33, 0, 1, "bf16", False, True),     # per-token values
     (5, 48, 8, 1000, 70, 3, 2, "bf16", False, False),    # six q heads per kv head: exact units of three heads
     (6, 32, 8, 0, 150, 5, 1, "fp16", False, False),      # window only
@@ -255,7 +255,7 @@ def test_decode_attn_mid_batch_four_heads_per_unit(ops, case):
 
 PAIRED = [
     # reps, Hq, Hkv, T, R, S, dtype, mask, calibrate — more than 256 units of work, a unit's layout within half the LDS:
-    # the launch uses 512-thread workgroups, two per compute unit (four heads per unit: logits kept in registers, K table in two passes)
+    # the launch uses 512-thread workgroups, two per compute unit (four heads per unit: eight rounds of logits in registers)
     (20, 32, 8, 777, 60, 41, "bf16", False, True),
     (20, 32, 8, 3328, 128, 0, "fp16", False, True),
     (20, 32, 8, 2100, 70, 5, "bf16", True, True),       # two blocks of staged value rows, mask
@@ -272,7 +272,7 @@ PAIRED = [
 
 
 PAIRED_2BIT = [
-    # reps, Hq, Hkv, T, R, S, dtype, mask — 2 bits, more than 256 four-head units: 512-thread workgroups, K table in four passes
+    # reps, Hq, Hkv, T, R, S, dtype, mask — 2 bits, more than 256 four-head units: 512-thread workgroups
     (20, 32, 8, 3328, 128, 0, "bf16", False),
     (20, 32, 8, 777, 60, 41, "fp16", True),
     (17, 48, 8, 2100, 33, 0, "bf16", False),     # padded four-head units, two blocks of staged value rows

@@ -160,7 +160,7 @@ def test_mask_of_the_lowest_value_over_every_packed_token(ops, T):
 
 
 def test_token_values_scales_far_apart(ops):
-    """Every wave takes its grid from the largest scale of a group among its tokens; a group of zero scales has none."""
+    """Every wave takes a head's grid from its largest weight times scale of a group; a group of zero scales has none."""
     c = _token_case(1, 32, 8, 300, 0, 1, "fp16", seed=3)
     c["sv"][:, :, 64:128] *= np.float32(2.0 ** -8)
     c["sv"][:, :, :, 1] = 0.0

@@ -89,9 +89,8 @@ def test_large_logits(ops, name, mult, qscale):
 @pytest.mark.parametrize("reps, T", [(20, 3328), (1, 3328), (1, 1000)])
 def test_value_sums_next_to_one(ops, reps, T):
     """One token in every 32 carries weight 1 and the other 31 a weight just under half a unit in the last
-    place of an fp16 1.0: the value loop adds the subset sums of 32 tokens as packed fp16 before it goes to
-    fp32, so these sums sit where that format rounds hardest.  The logits take exactly two values (one key
-    channel with a non-zero query weight), chosen so that the calibrated gap is ln(1 / 2.3e-4)."""
+    place of an fp16 1.0: sums of weights kept in that format would round hardest here.  The logits take exactly
+    two values (one key channel with a non-zero query weight), chosen so that the calibrated gap is ln(1 / 2.3e-4)."""
     B, Hq, Hkv, D, R = 2, 32, 8, 128, 0
     rng = np.random.default_rng(T)
     code = np.zeros((B, Hkv, T, D), np.uint8)
