@@ -1,8 +1,9 @@
 // Prefill quantise-and-pack for gfx950, and the unfused quant()/encode()
 // operators of the reference surface.
 //
-// Per-channel statistics need a column reduction over the token axis, so the
-// work is three launches on one stream:
+// Per-channel statistics need a column reduction over the token axis.  Rows of 128 channels go through the one-pass
+// kernel below, which keeps them in registers between the reduction and the codes.  What that does not take (other
+// widths, the unpacked codes of quant(), token axes beyond its part counts) is three launches on one stream:
 //   1. partial min/max per (batch, head, token chunk, channel)  - reads x once
 //   2. statistics: combine the chunks, run the storage-dtype op chain
 //      and, per channel, the input thresholds at which the code steps up
@@ -21,8 +22,7 @@
 
 #include <atomic>
 
-#include <mutex>
-#include <vector>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -38,13 +38,13 @@ struct QuantGeom {
     FastDiv dT, dH;       // divisors T and H of a flat (b, h, t) row index (per-token quantiser)
     FastDiv dTB;          // per-token quantiser: blocks of 16 tokens per (batch, head)
     int shared_stats;     // non-zero: one row of statistics / thresholds serves every (batch, head) (whole-tensor mode)
-    // One-pass kernel on a token axis that is longer than a workgroup's registers hold (SPLIT): 2^parts_log2
-    // workgroups share a slice, `part_rows` rows each, and exchange their channel minima / maxima through `rec`
-    // inside the launch: [virtual slice][channel][2] 64-bit records, the float's bits below the call's epoch, so a
-    // record is valid by itself and nothing has to be cleared.  The wait for the other parts is bounded
-    // (spin_limit polls); a lane that gives up sets *status (pinned host memory).
-    int parts_log2, part_rows;
-    int wide_map;         // one-pass kernel: which (batch, head) pairs share a die, see slice_of()
+    // One-pass kernel: `parts` workgroups share a (batch, head) pair, `part_rows` token rows each, and, if there are
+    // several, exchange their channel minima / maxima through `rec` inside the launch: [pair * parts + part][channel]
+    // 64-bit records, the two extremes as 16-bit keys below the call's epoch, so a record is valid by itself and nothing
+    // has to be cleared.  The wait for the other parts is bounded (spin_limit polls); a lane that gives up sets *status
+    // (pinned host memory).
+    int parts, part_rows;
+    FastDiv dP;           // divisor `parts`
     unsigned long long* rec;
     uint32_t epoch;
     int spin_limit;
@@ -412,31 +412,38 @@ __global__ __launch_bounds__(kQThreads) void emit_kernel(const uint16_t* __restr
 }
 
 // ---- one-pass quantise and pack ------------------------------------------------------------
-// A 1024-thread workgroup owns (batch, head, quarter of the channels): 32 channels = 64 bytes of
-// every token row, T <= 3328 tokens, which is 16 bytes x up to 13 rows per thread - the slice
-// stays in registers between the min/max and the emit, so x is read from HBM once.
-// thread = (row r = tid / 4 of a 256-row pass, 16-byte piece q = tid % 4).
-constexpr int kFThreads = 1024;
-constexpr int kFRows = 13;                  // rows per thread at most (13 x 256 = 12 tiles + thumbnail of 256 tokens)
-constexpr int kFMaxT = kFRows * (kFThreads / 4);
-constexpr int kFGridDefault = 256;          // workgroups of the persistent launch when no device can be asked: a whole MI355X
-// rows per thread of the next slice that are staged in LDS (16 KB each for the workgroup)
-// (not with the rotary embedding fused in: that instantiation has no registers to spare for the addresses).
-// The staged loads are assembly that the compiler does not see (m0, their own wait count): building with
-// -DCQ_NO_LDS_STAGE refills every row from memory through registers instead, for a toolchain that breaks them.
-#ifdef CQ_NO_LDS_STAGE
-constexpr int fused_stage_rows(int, bool) { return 0; }
-#else
-constexpr int fused_stage_rows(int nr, bool rope) { return (nr > 8 && !rope) ? 8 : 0; }
-#endif
+// A 256-thread workgroup owns a run of token rows of one (batch, head) pair: whole rows of 128 channels (256 bytes, LPR = 16
+// lanes a row), or, where there is little to do, a quarter of the channels (64 bytes, LPR = 4), 16 bytes x up to 52 rows per
+// thread, which stay in registers between the min / max and the emit, so x is read from HBM once.  A longer token axis is
+// shared by several workgroups (SPLIT), which exchange their channels' extremes inside the launch.
+// thread = (row r = tid / LPR of a pass of 256 / LPR rows, 16-byte piece tid % LPR).
+// Two workgroups are resident per compute unit (one wave per SIMD and 256 registers each), the next part's rows are
+// requested while this one's are packed.
+//
+// What bounds it: memory.  Batch 64 x 3 328 tokens x 8 heads, 1 bit, 464 MB, us: the strided key block of a fused projection 106
+// -> 92, a contiguous tensor 129 -> 93, 2 bits 130 -> 106; the loads alone 75, the code stores 10 - 12 more whatever their
+// form (a streaming kernel without any structure: 64 and 75).  Against a 1 024-thread workgroup per compute unit that
+// owned 64-byte quarters of 3 328 rows:
+//  - whole rows instead of 64-byte pieces: a contiguous tensor 129 -> 103 (its pieces lay 2 KB apart, on few channels);
+//  - non-temporal loads and stores (every line is used once, by one workgroup): 105 -> 94; only with 40 or more rows per
+//    thread, i.e. for tensors that the memory-side cache would not have held for the reader before;
+//  - codes from packed 16-bit comparisons (EmitPlan), about 15 vector instructions per 8 elements instead of 24;
+//  - the threshold search by inverting the op chain (threshold_key) instead of four rounds of 16-ary search.
+// More and smaller workgroups (3 x 24 rows, 4 x 16 or 20, 2 x 28) measured 99 to 127: the folds, the exchange and the
+// thresholds are paid per part.  Delaying every second workgroup's start so that the two of a unit run out of step: no change.
+// Small and long shapes: 1 x 64 tokens x 8 heads 6.0 -> 3.5, 1 x 3 328 12 -> 6.2, 8 x 1 024 7.6 -> 6.5, 64 x 256 37 -> 8.5,
+// 1 x 32 768 36 -> 22.5, 16 x 9 984 strided 105 -> 75, contiguous 109 -> 73.
+constexpr int kFThreads = 256;
+constexpr int kFRows = 52;                  // rows per thread at most
+constexpr int kFMaxT = 3328;                // token axis at most with the rotary embedding fused in
+constexpr int kFResident = 2;               // workgroups per compute unit of the persistent launch
+constexpr int kFGridDefault = 256;          // compute units when no device can be asked: a whole MI355X
 
 // Rotary embedding fused into the pass (ROPE): x is the un-rotated key block; every row is rotated as it
 // arrives - rnd(rnd(x * cos) + rotate_half(x) * sin), the arithmetic of the ops the reference runs on the
 // whole key tensor before it quantises the image slice (patch_internvl.py:125-134, 258-260, 295-297) - the
 // rotated row is written out once (the prefill attention and the caller's cache need it) and quantised from
-// the registers.  A channel d pairs with d + 64, so the 32 channels of a slice are then 16 of the lower half
-// and the matching 16 of the upper half (pieces 0, 1 / 2, 3 of a row's four lanes): the partner's raw values
-// are two lanes away, no second read of x.
+// the registers.  A channel d pairs with d + 64: the partner's raw values are eight lanes away.
 struct RopeArgs {
     const uint16_t* cos;      // (table_rows, 128) in the storage dtype
     const uint16_t* sin;
@@ -449,441 +456,481 @@ struct RopeArgs {
     int64_t gs = 0, og = 0;
 };
 
-// SPLIT: the token axis is longer than NR * 256 rows: 2^g.parts_log2 workgroups share a slice, each with g.part_rows
-// of its rows (<= NR * 256) in registers, and exchange their channels' min / max before the statistics - x is still
-// read once.  The parts of a slice are consecutive ids, i.e. they are worked on by different workgroups of the
-// persistent launch in the same step of their walks (the grid is a multiple of the part count), all of them
-// resident: whoever waits, waits for workgroups that are running.
-template <typename DT, int BITS, int NR, bool ROPE = false, bool SPLIT = false>   // NR: rows per thread (T <= NR * 256)
-__global__ __launch_bounds__(kFThreads) void fused_pack_kernel(const uint16_t* __restrict__ x, QuantGeom g, float clip,
+typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+typedef short S2 __attribute__((ext_vector_type(2)));
+typedef unsigned short US2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pk_max_s(uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(S2, a), __builtin_bit_cast(S2, b))); }
+__device__ __forceinline__ uint32_t pk_max_u(uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(US2, a), __builtin_bit_cast(US2, b))); }
+__device__ __forceinline__ uint32_t pk_min_s(uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(S2, a), __builtin_bit_cast(S2, b))); }
+// (maximum, minimum) pairs of monotone keys in the upper and lower half
+__device__ __forceinline__ uint32_t ext_fold(uint32_t a, uint32_t b) { return (pk_max_s(a, b) & 0xffff0000u) | (pk_min_s(a, b) & 0xffffu); }
+__device__ __forceinline__ uint32_t pk_min_u(uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(US2, a), __builtin_bit_cast(US2, b))); }
+__device__ __forceinline__ uint32_t pk_sub_sat(uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(S2, a), __builtin_bit_cast(S2, b))); }
+__device__ __forceinline__ uint32_t pk_sign(uint32_t a) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(S2, a) >> 15); }   // 0xffff where negative
+__device__ __forceinline__ uint32_t quad_xor(uint32_t v, std::integral_constant<int, 1>) { return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xB1, 0xf, 0xf, true)); }
+__device__ __forceinline__ uint32_t quad_xor(uint32_t v, std::integral_constant<int, 2>) { return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x4E, 0xf, 0xf, true)); }
+
+// The codes of a lane's eight channels of one row, four elements an instruction or two, from the raw 16-bit words.
+// Both storage types are sign-magnitude, so "x >= threshold" is an integer comparison of the words: the sign of a
+// saturating packed subtraction, which v_perm_b32 spreads over a byte per element (its selectors 8 .. 11) and a
+// four-byte dot product with the fields' weights (2^7 .. 2^0 for one bit) turns into the packed byte, modulo 256.
+// NaN inputs are kept out by the caller (sanitize()).
+// One bit: for a positive threshold the signed words compare as the values do (c = 0: the code is 1 where the
+// difference is not negative); for one <= 0 the unsigned words do, in reverse (c = 0x8000: 1 where it is).  Two bits: x is
+// made monotone once, y = x < 0 ? x ^ 0x7fff : x, and compared three times.
+template <int BITS> struct EmitPlan;
+template <> struct EmitPlan<1> {
+    uint32_t t[4], c[4], w[2];
+    int init;
+    __device__ __forceinline__ void load(const uint16_t (*thr)[128], const uint16_t* flip, int c0) {
+        const U4 tv = *reinterpret_cast<const U4*>(&thr[0][c0]), cv = *reinterpret_cast<const U4*>(flip + c0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { t[i] = tv[i]; c[i] = cv[i]; }
+        const uint32_t n0 = __builtin_amdgcn_perm(c[1], c[0], 0x0b0a0908u), n1 = __builtin_amdgcn_perm(c[3], c[2], 0x0b0a0908u);
+        w[0] = (n0 & 0xf0e0c080u) | (~n0 & 0x10204080u);
+        w[1] = (n1 & 0xfffefcf8u) | (~n1 & 0x01020408u);
+        init = __builtin_amdgcn_sdot4(static_cast<int>(~n1), static_cast<int>(0xfffefcf8u),
+                                      __builtin_amdgcn_sdot4(static_cast<int>(~n0), static_cast<int>(0xf0e0c080u), 0, false), false);
+    }
+    __device__ __forceinline__ uint32_t byte(const U4& x) const {   // bits 0 .. 7 are the packed byte
+        uint32_t d[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = pk_sub_sat(x[i] ^ c[i], t[i]);
+        const uint32_t p0 = __builtin_amdgcn_perm(d[1], d[0], 0x0b0a0908u), p1 = __builtin_amdgcn_perm(d[3], d[2], 0x0b0a0908u);
+        return static_cast<uint32_t>(__builtin_amdgcn_sdot4(static_cast<int>(p1), static_cast<int>(w[1]),
+                                                            __builtin_amdgcn_sdot4(static_cast<int>(p0), static_cast<int>(w[0]), init, false), false));
+    }
+};
+template <> struct EmitPlan<2> {
+    uint32_t t[3][4];
+    __device__ __forceinline__ void load(const uint16_t (*thr)[128], const uint16_t*, int c0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const U4 tv = *reinterpret_cast<const U4*>(&thr[k][c0]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t[k][i] = tv[i];
+        }
+    }
+    __device__ __forceinline__ void bytes(const U4& x, uint32_t& b0, uint32_t& b1) const {   // bits 0 .. 7 of either
+        uint32_t y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = x[i] ^ (pk_sign(x[i]) & 0x7fff7fffu);
+        int a0 = 255, a1 = 255;   // 3 * (64 + 16 + 4 + 1): every level reached, less what is not
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            uint32_t d[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[i] = pk_sub_sat(y[i], t[k][i]);
+            a0 = __builtin_amdgcn_sdot4(static_cast<int>(__builtin_amdgcn_perm(d[1], d[0], 0x0b0a0908u)), 0x01041040, a0, false);
+            a1 = __builtin_amdgcn_sdot4(static_cast<int>(__builtin_amdgcn_perm(d[3], d[2], 0x0b0a0908u)), 0x01041040, a1, false);
+        }
+        b0 = static_cast<uint32_t>(a0);
+        b1 = static_cast<uint32_t>(a1);
+    }
+};
+
+// NaN elements of a piece become -infinity, which every threshold leaves below it: code 0, as a comparison of floats gives
+template <typename DT> __device__ __forceinline__ void sanitize(U4& x) {
+    constexpr uint32_t kInf2 = static_cast<uint32_t>(Keys<DT>::hi) * 0x10001u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        // negative halves where the magnitude is beyond infinity's, spread over the half; in place (the assembly keeps
+        // the compiler from giving the result of this rarely taken branch registers of its own)
+        uint32_t m = pk_sub_sat(kInf2, x[i] & 0x7fff7fffu), w = x[i];
+        asm("v_pk_ashrrev_i16 %1, 15, %1 op_sel_hi:[0,1]\n\tv_bfi_b32 %0, %1, %2, %0" : "+v"(w), "+v"(m) : "v"(0x80008000u | kInf2));
+        x[i] = w;
+    }
+}
+
+// The smallest key (Keys<DT>) whose code is at least k, kNoKey if no value reaches it, for a lane pair that shares a
+// channel (odd: its second lane).  The op chain is inverted in fp32 - the value of y that rounds up to code k,
+// the quotient that rounds to it after the zero-point, the input that divides to that - which lands within a step or
+// two; the exact chain at four keys around the guess then decides, and a bisection over all keys does where they do not
+// bracket the step (degenerate statistics, values near zero).  The code is a non-decreasing function of x for every (scale,
+// zero-point) the chain can produce - also for scale 0 (x / 0 is -inf, NaN, +inf in that order and NaN maps to code 0)
+// and for NaN statistics (every code 0).
+constexpr int kNoKey = 0x7fff;
+template <typename DT> __device__ __forceinline__ int value_key(float f) {   // nearest storage value
+    const int p = static_cast<int>(Cvt<DT>::from_float(f) & 0xffffu);
+    return (p & 0x8000) ? -(p & 0x7fff) : p;
+}
+template <typename DT> __device__ __forceinline__ int key_from(float f, bool strict) {   // the smallest one not below f, or above it
+    const int k = value_key<DT>(f);
+    const float v = key_value<DT>(k);
+    return v < f || (strict && v == f) ? k + 1 : k;
+}
+template <typename DT>
+__device__ __forceinline__ int threshold_key(float s, float zp, float levels, int k, bool odd) {
+    const int half = value_key<DT>(static_cast<float>(k) - 0.5f);          // y at a tie: it rounds to the even code
+    const int ck = (k & 1) ? half + 1 : half;
+    const float m = 0.5f * (key_value<DT>(ck - 1) + key_value<DT>(ck));    // what rounds to ck or above
+    const int yk = key_from<DT>(m - zp, (k & 1) != 0);                     // (the tie between ck - 1 and ck goes to the even word)
+    const float q = 0.5f * (key_value<DT>(yk - 1) + key_value<DT>(yk));
+    const int guess = key_from<DT>(q * s, false);
+    const int first = min(max(guess - 2, Keys<DT>::lo), Keys<DT>::hi - 3);
+    auto reaches = [&](int key) { return quant_value<DT>(key_value<DT>(key), s, zp, levels) >= static_cast<float>(k); };
+    const int k0 = first + (odd ? 2 : 0);
+    int seen = (reaches(k0) ? 1 : 0) + (reaches(k0 + 1) ? 1 : 0);          // of this lane's two keys
+    seen += dpp_move_i<0xB1>(seen, 0);
+    int key = first + 4 - seen;
+    if (__ballot(seen == 0 || seen == 4)) {
+        int lo = Keys<DT>::lo - 1, hi = Keys<DT>::hi;   // code(lo) < k (lo may be the virtual floor), answer in (lo, hi]
+        const bool reach = reaches(hi);
+        while (hi - lo > 1) {   // (as many rounds in every lane)
+            const int mid = (lo + hi) >> 1;
+            if (reaches(mid)) hi = mid; else lo = mid;
+        }
+        if (seen == 0 || seen == 4) key = reach ? hi : kNoKey;
+    }
+    return key;
+}
+
+// The parts of a pair (or quarter) are consecutive ids; a workgroup walks ids blockIdx.x, blockIdx.x + gridDim.x, ... in increasing
+// order and all workgroups are resident: whoever waits for another part waits for a workgroup whose earlier ids belong to
+// the same or earlier pairs, so no two wait for each other.
+template <typename DT, int BITS, int NR, int LPR = 16, bool ROPE = false, bool SPLIT = false>   // NR: rows per thread
+__global__ __launch_bounds__(kFThreads, kFResident) void fused_pack_kernel(const uint16_t* __restrict__ x, QuantGeom g, float clip,
                                                               uint16_t* __restrict__ scale,
                                                               uint16_t* __restrict__ zero,
                                                               uint8_t* __restrict__ codes, RopeArgs ra) {
+    static_assert(NR % 4 == 0, "rows are packed and stored four at a time");
     constexpr int L = (1 << BITS) - 1;
     constexpr float levels = static_cast<float>(L);
-    __shared__ __attribute__((aligned(16))) float part_mn[32][kFThreads / 16];   // [channel][wave * 4 + row of 16 lanes]
-    __shared__ __attribute__((aligned(16))) float part_mx[32][kFThreads / 16];
-    __shared__ float s_s[32], s_z[32], s_thr[3][32];
-    // NP rows per thread of the NEXT slice travel through LDS: they are requested as soon as this slice's min / max
-    // fold has read the registers - global-to-LDS loads that need no register to land in - so HBM stays busy
-    // through the statistics and threshold phases, in which nothing else is in flight; the emit then refills those
-    // rows' registers from LDS and only the other NR - NP rows from memory.
-    constexpr int NP = fused_stage_rows(NR, ROPE);
-    extern __shared__ __attribute__((aligned(16))) unsigned char stage[];   // [NP][thread][16 bytes]
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int q4 = tid & 3, row = tid >> 2;
-    // A workgroup walks slices blockIdx.x, blockIdx.x + gridDim.x, ... (gridDim.x is a multiple
-    // of 32).  The four quarters of one (batch, head) sit on one XCD (slice ids 8 apart), so the
-    // four 4-byte pieces of a packed row meet in one L2.  While a slice's rows are emitted, every
-    // row's registers are refilled with the same row of the next slice: its loads are in flight
-    // during the emit and its min / max pass starts without a wait.
-    const int plog = SPLIT ? g.parts_log2 : 0;
-    const int64_t nbh = static_cast<int64_t>(g.B) * g.H;
-    // Slice vb -> (quarter, (batch, head) pair).  Workgroup l of the launch runs on die l % 8 and its ids are a
-    // multiple of 8 apart, so the low three bits of an id are the die: of an unsplit slice the low three bits of vb,
-    // of a slice split four ways the part and the lowest bit of vb.  The four quarters of a pair always share a
-    // die (their 4-byte pieces of a packed row meet in one L2, and two quarters share every 128-byte line of x).
-    // Narrow map: the low bits of vb are the low bits of the pair index - with eight heads, of the head.  Wide
-    // map: they select among eight runs of eight consecutive pairs - with eight heads, among batch rows - and the
-    // place in the run comes from bits 5-7.  For split slices of a contiguous (B, T, H, D) tensor the wide map
-    // puts all heads of a token row (one contiguous 2 KB) on one die, where the narrow one spreads them over two
-    // or more; the host picks it there (measured, see wide_map_for()).
-    const int wide = g.wide_map;
-    const int nslice = (wide ? static_cast<int>((nbh + 63) / 64) * 256 : static_cast<int>((nbh + 7) / 8) * 32) << plog;   // ids: slice * parts + part
-    auto slice_of = [&](int vb, int& quarter) -> int64_t {
-        if (wide) {
-            quarter = (vb >> 3) & 3;
-            return (static_cast<int64_t>(vb >> 8) * 8 + (vb & 7)) * 8 + ((vb >> 5) & 7);
-        }
-        quarter = (vb >> 3) & 3;
-        return static_cast<int64_t>(vb >> 5) * 8 + (vb & 7);
-    };
-    auto part_first = [&](int id) { return SPLIT ? (id & ((1 << plog) - 1)) * g.part_rows : 0; };        // first row of the id's part
-    auto part_len = [&](int id) { return SPLIT ? min(g.T - part_first(id), g.part_rows) : g.T; };       // rows of it
-    // The slice's base is the same for the whole workgroup and a row's piece sits at a 32-bit byte
-    // offset from it (the host checks T * row stride < 2^24 bytes): a load takes its address as
-    // scalar base + vector offset, one 24-bit multiply-add per row.
-    auto slice_base = [&](int id) -> const unsigned char* {   // slices past the last (batch, head) alias the last one
-        const int vb = id >> plog;
-        int quarter;
-        const uint32_t bh = static_cast<uint32_t>(min(slice_of(vb, quarter), nbh - 1));
-        const uint32_t b = g.dH.quot(bh), h = bh - b * g.dH.div;   // B * H < 2^31 on this path
+    static_assert(LPR == 16 || (LPR == 4 && !ROPE), "whole rows or quarters");
+    constexpr int kFPass = kFThreads / LPR;            // rows that one load of all threads covers
+    constexpr int kChan = 8 * LPR;                     // channels of the workgroup
+    constexpr int kLG = kFThreads / (kChan / 2);       // lanes that fold a pair of channels
+    constexpr int kLC = kLG / 2;                       // lanes per channel after that
+    constexpr bool kStream = LPR == 16 && NR >= 40;
+    // the threads' extremes as monotone 16-bit keys, two channels a word (the row pitch spreads what a wave reads together
+    // over the banks)
+    constexpr int kPitch = LPR == 16 ? 80 : 20;
+    __shared__ __attribute__((aligned(16))) uint32_t part_mn[kFPass][kPitch];
+    __shared__ __attribute__((aligned(16))) uint32_t part_mx[kFPass][kPitch];
+    __shared__ __attribute__((aligned(16))) uint16_t s_thr[L][128];   // thresholds as EmitPlan compares them
+    __shared__ __attribute__((aligned(16))) uint16_t s_flip[128];
+    const int tid = threadIdx.x, q4 = tid & 3;
+    const int piece = tid % LPR, row = tid / LPR;
+    const int npairs = g.B * g.H;
+    const int nids = npairs * (16 / LPR) * g.parts;   // (the host keeps this below 2^31)
+    // id = slice * parts + part; slice = quarter * pairs + pair: with eight heads the quarters of a pair, which share its
+    // lines of x and of the codes, come to lie on one die (ids a multiple of 8 apart)
+    auto slice_of = [&](int id) { return SPLIT ? static_cast<int>(g.dP.quot(static_cast<uint32_t>(id))) : id; };
+    auto quarter_of = [&](int slice) { return LPR == 16 ? 0 : (slice >= npairs) + (slice >= 2 * npairs) + (slice >= 3 * npairs); };
+    auto first_of = [&](int id) { return SPLIT ? (id - slice_of(id) * g.parts) * g.part_rows : 0; };  // first row of the id's part
+    auto rows_of = [&](int id) { return SPLIT ? min(g.T - first_of(id), g.part_rows) : g.T; };        // rows of it
+    auto base_of = [&](int id) -> const unsigned char* {
+        const int slice = slice_of(id), quarter = quarter_of(slice);
+        const uint32_t bh = static_cast<uint32_t>(slice - quarter * npairs);
+        const uint32_t b = g.dH.quot(bh), h = bh - b * g.dH.div;
         return reinterpret_cast<const unsigned char*>(x + static_cast<int64_t>(b) * g.sb + static_cast<int64_t>(h) * g.sh +
-                                                      static_cast<int64_t>(part_first(id)) * g.st + quarter * (ROPE ? 16 : 32));
+                                                      static_cast<int64_t>(first_of(id)) * g.st + quarter * 32);
     };
-    // first channel of the thread's piece, less the slice's own offset (quarter * 32, or quarter * 16 with ROPE)
-    const int chan_t = ROPE ? (q4 >> 1) * 64 + (q4 & 1) * 8 : q4 * 8;
-    const uint32_t st_bytes = static_cast<uint32_t>(g.st) * 2u, q_bytes = static_cast<uint32_t>(chan_t) * 2u;
-    auto row_offset = [&](int t, int len) -> uint32_t {   // byte offset of the thread's piece of row min(t, len - 1) of a slice (part)
-        return static_cast<uint32_t>(__umul24(static_cast<uint32_t>(min(t, len - 1)), st_bytes)) + q_bytes;
+    // A load takes its address as a scalar base (part, pass of rows) + a vector offset that is the same for every
+    // full pass; the last pass has an offset of its own, whose rows past the end repeat the last one (min / max unchanged,
+    // never written), and the passes behind it repeat the last pass.
+    const uint32_t st_bytes = static_cast<uint32_t>(g.st) * 2u;   // (the host checks that it is below 2^24)
+    const uint32_t pass_bytes = st_bytes * kFPass;
+    const uint32_t off_full = static_cast<uint32_t>(__umul24(static_cast<uint32_t>(row), st_bytes)) + piece * 16;
+    auto tail_offset = [&](int len) -> uint32_t {
+        return static_cast<uint32_t>(__umul24(static_cast<uint32_t>(min(row, (len - 1) & (kFPass - 1))), st_bytes)) + piece * 16;
     };
-    typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+    auto load_row = [&](const unsigned char* base, uint32_t pass_bytes, int i, int last_pass, uint32_t off_full, uint32_t off_last) -> U4 {
+        const unsigned char* p = base + static_cast<uint64_t>(static_cast<uint32_t>(min(i, last_pass))) * pass_bytes;
+        const U4* q = reinterpret_cast<const U4*>(p + (i < last_pass ? off_full : off_last));
+        if constexpr (kStream) return __builtin_nontemporal_load(q);
+        else return *q;
+    };
+    int id = blockIdx.x;
+    if (id >= nids) return;   // (the whole workgroup)
     U4 v[NR];
     {
-        const unsigned char* base = slice_base(blockIdx.x);
-        const int len0 = part_len(blockIdx.x);
+        const unsigned char* base = base_of(id);
+        const int len0 = rows_of(id);
+        const uint32_t off_last = tail_offset(len0);
 #pragma unroll
-        for (int i = 0; i < NR; ++i)   // rows past T re-read row T-1: min / max unchanged, never written
-            v[i] = *reinterpret_cast<const U4*>(base + row_offset(i * (kFThreads / 4) + row, len0));
+        for (int i = 0; i < NR; ++i) v[i] = load_row(base, pass_bytes, i, (len0 - 1) / kFPass, off_full, off_last);
     }
-    for (int id = blockIdx.x; id < nslice; id += gridDim.x) {
-    const int vb = id >> plog;
-    int quarter;
-    const int64_t bh = slice_of(vb, quarter);
-    const bool live = bh < nbh;                         // a padding slice computes and writes nothing
-    const bool has_next = id + static_cast<int>(gridDim.x) < nslice;
-    const int next_id = has_next ? id + gridDim.x : id;
-    const unsigned char* next_base = slice_base(next_id);
-    const int t_first = part_first(id), t_len = part_len(id), next_len = part_len(next_id);
-    int row_i = row;   // opaque per iteration: the row offsets below are recomputed, not kept in registers across the loop
-    asm volatile("" : "+v"(row_i));
+    // While a part's rows are emitted, every row's registers are refilled with the same row of the workgroup's next
+    // part: its loads are in flight during the emit and its min / max pass starts without a wait.
+    for (;;) {
+    const int slice = slice_of(id), quarter = quarter_of(slice);
+    const int bh = slice - quarter * npairs;
+    const int next_id = id + static_cast<int>(gridDim.x);
+    const bool has_next = next_id < nids;
+    const int t_first = first_of(id), t_len = rows_of(id);
     if constexpr (ROPE) {
-        const uint32_t bhc = static_cast<uint32_t>(min(bh, nbh - 1));
-        const uint32_t bb = g.dH.quot(bhc), hh = bhc - bb * g.dH.div;
-        const int chan0 = quarter * 16 + chan_t;
-        uint16_t* orow = ra.out + static_cast<int64_t>(bb) * ra.ob + static_cast<int64_t>(hh) * ra.oh + chan0;
-        const bool upper = (q4 >> 1) != 0;
+        const uint32_t bb = g.dH.quot(static_cast<uint32_t>(bh)), hh = static_cast<uint32_t>(bh) - bb * g.dH.div;
+        int row_i = row;   // opaque: the rows' addresses are worked out anew for each part, not kept across the loop
+        asm volatile("" : "+v"(row_i));
+        const int rope_last = (t_len - 1) / kFPass, row_l = min(row_i, (t_len - 1) & (kFPass - 1));
+        auto row_of = [&](int i) { return t_first + min(i, rope_last) * kFPass + (i < rope_last ? row_i : row_l); };   // the row that v[i] holds
+        uint16_t* orow = ra.out + static_cast<int64_t>(bb) * ra.ob + static_cast<int64_t>(hh) * ra.oh + piece * 8;
         const int64_t* pos_p = ra.pos ? ra.pos + static_cast<int64_t>(bb) * ra.pos_sb : reinterpret_cast<const int64_t*>(ra.cos);
         const int64_t pos_st = ra.pos ? ra.pos_st : 0;
         const int64_t trow_max = ra.table_rows - 1;
-        const uint32_t ysign = upper ? 0u : 0x80008000u;   // rotate_half(x) = (-x2, x1): the lower half takes minus its partner
+        const uint32_t ysign = piece >= 8 ? 0u : 0x80008000u;   // rotate_half(x) = (-x2, x1): the lower half takes minus its partner
         // the table rows of GR rows at a time are requested before the first of them is used: every request
-        // is a round trip to the L2, and one row after the other would make a slice wait for NR of them in turn
+        // is a round trip to the L2, and one row after the other would make a part wait for NR of them in turn
         constexpr int GR = 2;
 #pragma unroll
         for (int i0 = 0; i0 < NR; i0 += GR) {
             U4 cw[GR], sw[GR];
 #pragma unroll
             for (int k = 0; k < GR; ++k) {
-                if (i0 + k < NR) {
-                    const int t = min((i0 + k) * (kFThreads / 4) + row_i, g.T - 1);
-                    // no control flow around the loads (the compiler then requests a group's rows side by side):
-                    // without a position tensor the load reads a valid dummy and the select takes pos0 + t
-                    const int64_t pv = pos_p[static_cast<int64_t>(t) * pos_st];
-                    const int64_t pl = ra.pos ? pv : ra.pos0 + t;
-                    // clamped to the table in 32 bits (the host checks table_rows < 2^24)
-                    const uint32_t ps = static_cast<uint32_t>(pl < 0 ? 0 : (pl > trow_max ? trow_max : pl));
-                    cw[k] = *reinterpret_cast<const U4*>(ra.cos + __umul24(ps, 128u) + chan0);
-                    sw[k] = *reinterpret_cast<const U4*>(ra.sin + __umul24(ps, 128u) + chan0);
-                }
+                const int t = row_of(i0 + k);
+                // no control flow around the loads (the compiler then requests a group's rows side by side):
+                // without a position tensor the load reads a valid dummy and the select takes pos0 + t
+                const int64_t pv = pos_p[static_cast<int64_t>(t) * pos_st];
+                const int64_t pl = ra.pos ? pv : ra.pos0 + t;
+                // clamped to the table in 32 bits (the host checks table_rows < 2^24)
+                const uint32_t ps = static_cast<uint32_t>(pl < 0 ? 0 : (pl > trow_max ? trow_max : pl));
+                cw[k] = *reinterpret_cast<const U4*>(ra.cos + __umul24(ps, 128u) + piece * 8);
+                sw[k] = *reinterpret_cast<const U4*>(ra.sin + __umul24(ps, 128u) + piece * 8);
             }
 #pragma unroll
             for (int k = 0; k < GR; ++k) {
-                if (i0 + k < NR) {
-                    const int i = i0 + k;
-                    const int t = min(i * (kFThreads / 4) + row_i, g.T - 1);
-                    U4 pw;   // the partner's raw piece: the lane two away holds channel d +- 64 of the same row
+                const int i = i0 + k;
+                const int t = row_of(i);
+                U4 pw;   // the partner's raw piece: the lane eight away holds channel d +- 64 of the same row
 #pragma unroll
-                    for (int w = 0; w < 4; ++w)
-                        pw[w] = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v[i][w]), 0x4E, 0xf, 0xf, true)) ^ ysign;
-                    U4 r4;
+                for (int w = 0; w < 4; ++w) pw[w] = static_cast<uint32_t>(dpp_move_i<0x128>(static_cast<int>(v[i][w]), 0)) ^ ysign;   // row_ror:8
+                U4 r4;
 #pragma unroll
-                    for (int w = 0; w < 4; ++w) {   // a word (two elements) at a time: few values live at once
-                        const float x0 = Cvt<DT>::lo(v[i][w]), x1 = Cvt<DT>::hi(v[i][w]);
-                        const float y0 = Cvt<DT>::lo(pw[w]), y1 = Cvt<DT>::hi(pw[w]);
-                        const float c0 = Cvt<DT>::lo(cw[k][w]), c1 = Cvt<DT>::hi(cw[k][w]);
-                        const float s0 = Cvt<DT>::lo(sw[k][w]), s1 = Cvt<DT>::hi(sw[k][w]);
-                        const uint32_t o0 = Cvt<DT>::from_float(rnd<DT>(x0 * c0) + y0 * s0);   // y carries the sign of rotate_half
-                        const uint32_t o1 = Cvt<DT>::from_float(rnd<DT>(x1 * c1) + y1 * s1);
-                        r4[w] = o0 | (o1 << 16);
-                    }
-                    v[i] = r4;
-                    // unconditional store: a row past T repeats row T - 1 and a padding slice repeats the last
-                    // (batch, head), so whatever is written twice is written with the same bits
-                    *reinterpret_cast<U4*>(orow + static_cast<int64_t>(t) * ra.ot) = r4;
+                for (int w = 0; w < 4; ++w) {   // a word (two elements) at a time: few values live at once
+                    const float x0 = Cvt<DT>::lo(v[i][w]), x1 = Cvt<DT>::hi(v[i][w]);
+                    const float y0 = Cvt<DT>::lo(pw[w]), y1 = Cvt<DT>::hi(pw[w]);
+                    const float c0 = Cvt<DT>::lo(cw[k][w]), c1 = Cvt<DT>::hi(cw[k][w]);
+                    const float s0 = Cvt<DT>::lo(sw[k][w]), s1 = Cvt<DT>::hi(sw[k][w]);
+                    const uint32_t o0 = Cvt<DT>::from_float(rnd<DT>(x0 * c0) + y0 * s0);   // y carries the sign of rotate_half
+                    const uint32_t o1 = Cvt<DT>::from_float(rnd<DT>(x1 * c1) + y1 * s1);
+                    r4[w] = o0 | (o1 << 16);
                 }
+                v[i] = r4;
+                // unconditional store: a row past the end repeats an earlier one, so what is written twice is written with the same bits
+                *reinterpret_cast<U4*>(orow + static_cast<int64_t>(t) * ra.ot) = r4;
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    // Both storage types are sign-magnitude, so the extremes of a column follow from three packed
-    // 16-bit integer folds of the raw words, two elements per instruction and no unpacking: as
-    // signed integers the non-negative values are in value order (the signed maximum is the
-    // largest of them, if there is one); as unsigned integers the negative values lie above every
-    // non-negative one, in order of magnitude (the unsigned maximum is the most negative value,
-    // if there is one; the unsigned minimum is the smallest non-negative value, or with negatives
-    // only the one nearest to zero).  -0 counts as negative and orders below +0.
-    typedef short S2 __attribute__((ext_vector_type(2)));
-    typedef unsigned short US2 __attribute__((ext_vector_type(2)));
+    // Both storage types are sign-magnitude, so the extremes of a column follow from packed 16-bit integer folds of the
+    // raw words, two elements per instruction and no unpacking: as signed integers the non-negative values are in
+    // value order (the signed maximum is the largest of them, if there is one); as unsigned integers the negative
+    // values lie above every non-negative one, in order of magnitude (the unsigned maximum is the most negative value,
+    // if there is one).  A column of one sign among the thread's rows needs a third fold (the unsigned minimum: the
+    // smallest non-negative value, or with negatives only the one nearest to zero), which a wave
+    // without such a column leaves out.  -0 counts as negative and orders below +0.
     uint32_t k_smax[4], k_umin[4], k_umax[4];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) { k_smax[w] = 0x80008000u; k_umin[w] = 0xffffffffu; k_umax[w] = 0u; }
+    for (int w = 0; w < 4; ++w) { k_smax[w] = v[0][w]; k_umax[w] = v[0][w]; }
 #pragma unroll
-    for (int i = 0; i < NR; ++i) {
+    for (int i = 1; i < NR; ++i) {
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-            const uint32_t r = v[i][w];
-            k_smax[w] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(S2, k_smax[w]), __builtin_bit_cast(S2, r)));
-            k_umin[w] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(US2, k_umin[w]), __builtin_bit_cast(US2, r)));
-            k_umax[w] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(US2, k_umax[w]), __builtin_bit_cast(US2, r)));
+            k_smax[w] = pk_max_s(k_smax[w], v[i][w]);
+            k_umax[w] = pk_max_u(k_umax[w], v[i][w]);
         }
     }
-    if constexpr (NP > 0) {
-        if (has_next) {
-            // lane l of a wave lands at the wave's base + 16 l: thread tid's piece of row i at stage[i][tid].
-            // Written as assembly: the compiler waits for a global-to-LDS load it knows of before the next LDS
-            // instruction of any kind, which would take the loads out of flight again at once.  The fold's
-            // results are operands of the first statement only to place the loads after the fold, i.e. after the
-            // compiler's own wait for the rows that came through registers; unknown to the compiler, the loads
-            // can only make its later vector-memory waits stricter, never weaker, and the wait before the
-            // staged pieces are read back is written out below.  (m0, the LDS base of such a load, has no other
-            // use in this kernel; the compiler reserves it and does not accept it as a clobber.)
-            const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(stage)) +
-                                  static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(wv)) * 1024u;
+    uint32_t one_sign = 0, top_s = k_smax[0], top_u = k_umax[0];
 #pragma unroll
-            for (int i = 0; i < NP; ++i) {
-                const uint32_t off = row_offset(i * (kFThreads / 4) + row_i, next_len);
-                const uint32_t ldsa = lds0 + static_cast<uint32_t>(i) * (kFThreads * 16);
-                if (i == 0)
-                    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2"
-                                 :
-                                 : "v"(off), "s"(ldsa), "s"(next_base), "v"(k_smax[0]), "v"(k_smax[1]), "v"(k_smax[2]),
-                                   "v"(k_smax[3]), "v"(k_umin[0]), "v"(k_umin[1]), "v"(k_umin[2]), "v"(k_umin[3]),
-                                   "v"(k_umax[0]), "v"(k_umax[1]), "v"(k_umax[2]), "v"(k_umax[3])
-                                 : "memory");
-                else
-                    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2"
-                                 :
-                                 : "v"(off), "s"(ldsa), "s"(next_base)
-                                 : "memory");
-            }
-        }
+    for (int w = 0; w < 4; ++w) {
+        one_sign |= k_smax[w] | ~k_umax[w];
+        top_s = pk_max_s(top_s, k_smax[w]);
+        top_u = pk_max_u(top_u, k_umax[w]);
+        k_umin[w] = 0xffffffffu;
     }
-    float mn[8], mx[8];
+    if (__ballot((one_sign & 0x80008000u) != 0)) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int sh = 16 * (j & 1);
-        const uint32_t smax = (k_smax[j >> 1] >> sh) & 0xffffu, umin = (k_umin[j >> 1] >> sh) & 0xffffu,
-                       umax = (k_umax[j >> 1] >> sh) & 0xffffu;
-        mn[j] = Cvt<DT>::to_float((umax & 0x8000u) ? umax : umin);
-        mx[j] = Cvt<DT>::to_float((smax & 0x8000u) ? umin : smax);
-    }
-    // lanes l, l+4, l+8, l+12 of a row of 16 lanes hold the same channels: two rotations fold them
+        for (int i = 0; i < NR; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        mn[j] = fminf(mn[j], dpp_move<0x124>(mn[j], INFINITY));   // row_ror:4
-        mn[j] = fminf(mn[j], dpp_move<0x128>(mn[j], INFINITY));   // row_ror:8
-        mx[j] = fmaxf(mx[j], dpp_move<0x124>(mx[j], -INFINITY));
-        mx[j] = fmaxf(mx[j], dpp_move<0x128>(mx[j], -INFINITY));
+            for (int w = 0; w < 4; ++w) k_umin[w] = pk_min_u(k_umin[w], v[i][w]);
     }
-    if ((lane & 15) < 4) {
-        const int p = wv * 4 + (lane >> 4);
+    // a NaN of either sign is beyond the infinity of that sign
+    constexpr int kInf = Keys<DT>::hi;
+    const bool nan_here = static_cast<short>(top_s) > kInf || static_cast<short>(top_s >> 16) > kInf ||
+                          (top_u & 0xffffu) > (0x8000u | kInf) || (top_u >> 16) > (0x8000u | kInf);
+    if (__ballot(nan_here)) {   // (not a supported input; the codes of such elements are 0 all the same)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) { part_mn[q4 * 8 + j][p] = mn[j]; part_mx[q4 * 8 + j][p] = mx[j]; }
+        for (int i = 0; i < NR; ++i) sanitize<DT>(v[i]);
     }
-    __syncthreads();
-    // channel c of the quarter: 16 lanes fold its 64 partials (four each, then across the row),
-    // the first of them runs the statistics chain
-    if (tid < 32 * 16) {
-        const int c = tid >> 4, p16 = tid & 15;
-        const float4 a4 = *reinterpret_cast<const float4*>(&part_mn[c][4 * p16]);
-        const float4 z4 = *reinterpret_cast<const float4*>(&part_mx[c][4 * p16]);
-        float a = fminf(fminf(a4.x, a4.y), fminf(a4.z, a4.w));
-        float z = fmaxf(fmaxf(z4.x, z4.y), fmaxf(z4.z, z4.w));
-        a = row_reduce(a, OpMin(), INFINITY);
-        z = row_reduce(z, OpMax(), -INFINITY);
-        if constexpr (SPLIT) {
-            if (p16 == 0 && live) {
-                // This part's extremes of channel c go out as two self-validating records; then the records of all
-                // parts of the slice are polled (device-scope loads, a bounded number of times) and folded.  The
-                // other parts are being worked on right now by other workgroups of this launch.
-                const unsigned long long tag = static_cast<unsigned long long>(g.epoch) << 32;
-                unsigned long long* mine = g.rec + (static_cast<int64_t>(id) * 32 + c) * 2;
-                __hip_atomic_store(mine, tag | __float_as_uint(a), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(mine + 1, tag | __float_as_uint(z), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const int nparts = 1 << plog;
-                const unsigned long long* first = g.rec + (static_cast<int64_t>(id & ~(nparts - 1)) * 32 + c) * 2;
-                bool ok = false;
-                float fa = a, fz = z;
-                for (int it = 0; it < g.spin_limit && !ok; ++it) {
-                    ok = true;
-                    fa = a; fz = z;
-                    for (int pp = 0; pp < nparts; ++pp) {
-                        const unsigned long long lo = __hip_atomic_load(first + pp * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        const unsigned long long hi = __hip_atomic_load(first + pp * 64 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        ok = ok && static_cast<uint32_t>(lo >> 32) == g.epoch && static_cast<uint32_t>(hi >> 32) == g.epoch;
-                        // (a NaN extreme of any part stays one, as it does inside a part)
-                        const float pa = __uint_as_float(static_cast<uint32_t>(lo)), pz = __uint_as_float(static_cast<uint32_t>(hi));
-                        fa = (fa != fa || pa != pa) ? NAN : fminf(fa, pa);
-                        fz = (fz != fz || pz != pz) ? NAN : fmaxf(fz, pz);
-                    }
-                    if (!ok) __builtin_amdgcn_s_sleep(2);
-                }
-                if (ok) { a = fa; z = fz; }
-                else if (g.status) __hip_atomic_store(g.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);   // this call's result is not valid
-            }
-        }
-        if (p16 == 0 && live) {
-            const float x_min = rnd<DT>(a * clip);
-            const float x_max = rnd<DT>(z * clip);
-            const float diff = rnd<DT>(x_max - x_min);
-            const float sc = rnd<DT>(diff * __fdiv_rn(1.0f, levels));
-            const float zp = rnd<DT>(__fdiv_rn(-x_min, sc));
-            const int64_t o = bh * g.D + (ROPE ? (c >> 4) * 64 + quarter * 16 + (c & 15) : quarter * 32 + c);
-            if (!SPLIT || t_first == 0) {   // (one of the parts writes them)
-                scale[o] = static_cast<uint16_t>(Cvt<DT>::from_float(sc));
-                zero[o] = static_cast<uint16_t>(Cvt<DT>::from_float(zp));
-            }
-            s_s[c] = sc;
-            s_z[c] = zp;
-        }
-    }
-    __syncthreads();
-    // thresholds (see the statistics kernel): one 16-ary search per (channel, level) and group of
-    // 16 lanes, four rounds narrow the 2^16 ordered storage values down to one; a wave runs four
-    // searches side by side.  The code is a non-decreasing function of x for every (scale,
-    // zero-point) the chain can produce - also for scale 0 (x / 0 is -inf, NaN, +inf in that order
-    // and NaN maps to code 0) and for NaN statistics (every code 0) - so the search runs for
-    // every channel.
+    // the thread's extremes as monotone keys: y = x < 0 ? x ^ 0x7fff : x
     {
-        const int grp = lane >> 4, l16 = lane & 15;
-        for (int sid0 = wv * 4; sid0 < 32 * L; sid0 += kFThreads / 16) {
-            const int sid = min(sid0 + grp, 32 * L - 1);   // a group past the end repeats the last search
-            const int c = sid / L, k = sid % L + 1;
-            const float sc = s_s[c], zp = s_z[c];
-            int lo = Keys<DT>::lo - 1, hi = Keys<DT>::hi;   // code(lo) < k (lo may be the virtual floor), answer in (lo, hi]
-            bool reach = true;
+        U4 mn, mx;
 #pragma unroll
-            for (int round = 0; round < 4; ++round) {
-                const int step = (hi - lo + 15) / 16;
-                const int key = min(lo + (l16 + 1) * step, hi);
-                const bool pred = quant_value<DT>(key_value<DT>(key), sc, zp, levels) >= static_cast<float>(k);
-                const unsigned long long m = __ballot(pred);
-                const uint32_t mg = static_cast<uint32_t>(m >> (16 * grp)) & 0xffffu;   // the group's lanes
-                reach = reach && mg != 0;
-                const int f = mg ? __builtin_ctz(mg) : 0;
-                hi = min(lo + (f + 1) * step, hi);
-                lo = lo + f * step;
+        for (int w = 0; w < 4; ++w) {
+            const uint32_t neg = pk_sign(k_umax[w]), pos = ~pk_sign(k_smax[w]);   // there is a negative / a non-negative value
+            const uint32_t lo = (neg & k_umax[w]) | (~neg & k_umin[w]), hi = (pos & k_smax[w]) | (~pos & k_umin[w]);
+            mn[w] = lo ^ (pk_sign(lo) & 0x7fff7fffu);
+            mx[w] = hi ^ (pk_sign(hi) & 0x7fff7fffu);
+        }
+        *reinterpret_cast<U4*>(&part_mn[row][piece * 4]) = mn;
+        *reinterpret_cast<U4*>(&part_mx[row][piece * 4]) = mx;
+    }
+    __syncthreads();
+    // kLG lanes fold the partials of two channels, four each; then kLC lanes have a channel, run the statistics chain (all: the
+    // same instructions) and search the thresholds.
+    {
+        const int pair2 = tid / kLG, lg = tid % kLG;   // channels 2 * pair2, 2 * pair2 + 1
+        uint32_t a2 = part_mn[lg][pair2], z2 = part_mx[lg][pair2];
+#pragma unroll
+        for (int j = 1; j < kFPass / kLG; ++j) {
+            a2 = pk_min_s(a2, part_mn[lg + kLG * j][pair2]);
+            z2 = pk_max_s(z2, part_mx[lg + kLG * j][pair2]);
+        }
+        auto across = [&](auto ctrl) {
+            a2 = pk_min_s(a2, static_cast<uint32_t>(dpp_move_i<decltype(ctrl)::value>(static_cast<int>(a2), 0)));
+            z2 = pk_max_s(z2, static_cast<uint32_t>(dpp_move_i<decltype(ctrl)::value>(static_cast<int>(z2), 0)));
+        };
+        across(std::integral_constant<int, 0xB1>{});       // lane ^ 1
+        across(std::integral_constant<int, 0x4E>{});       // lane ^ 2
+        if constexpr (kLG == 16) {
+            across(std::integral_constant<int, 0x141>{});  // mirrored in eight lanes
+            across(std::integral_constant<int, 0x140>{});  // ... in sixteen
+        }
+        const int c = 2 * pair2 + lg / kLC, lc = lg % kLC;
+        const bool odd = (lc & 1) != 0, lead = lc == 0;
+        uint32_t ext = lg / kLC ? (z2 & 0xffff0000u) | (a2 >> 16) : (z2 << 16) | (a2 & 0xffffu);   // the channel's maximum, minimum
+        if constexpr (SPLIT) {
+            // This part's extremes of channel c go out as one self-validating record; then the records of all parts
+            // are polled (device-scope loads, a bounded number of times; each of the channel's lanes takes every kLC-th
+            // part, four at a time) and folded.  The other parts are being worked on right now by other workgroups of this launch.
+            unsigned long long* first = g.rec + static_cast<int64_t>(slice) * g.parts * kChan;
+            if (lead) __hip_atomic_store(first + static_cast<uint32_t>((id - slice * g.parts) * kChan + c), static_cast<unsigned long long>(g.epoch) << 32 | ext,
+                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            uint32_t fold = ext;
+            int polls = 0;
+            for (int p0 = lc; p0 < g.parts; p0 += 4 * kLC) {
+                unsigned long long r[4];   // in flight together; past the end the last part again
+                bool all = false;
+                while (!all && polls < g.spin_limit) {
+                    if (polls) __builtin_amdgcn_s_sleep(1);
+                    ++polls;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        r[k] = __hip_atomic_load(first + static_cast<uint32_t>(min(p0 + k * kLC, g.parts - 1) * kChan + c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    all = true;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) all = all && static_cast<uint32_t>(r[k] >> 32) == g.epoch;
+                }
+                if (!all) { polls = -1; break; }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) fold = ext_fold(fold, static_cast<uint32_t>(r[k]));
             }
-            // stays NaN if no value reaches code k
-            if (l16 == 0 && sid0 + grp < 32 * L) s_thr[k - 1][c] = reach ? key_value<DT>(hi) : NAN;
+            const bool ok = polls >= 0;
+            fold = ext_fold(fold, static_cast<uint32_t>(dpp_move_i<0xB1>(static_cast<int>(fold), 0)));
+            if constexpr (kLC == 8) {
+                fold = ext_fold(fold, static_cast<uint32_t>(dpp_move_i<0x4E>(static_cast<int>(fold), 0)));
+                fold = ext_fold(fold, static_cast<uint32_t>(dpp_move_i<0x141>(static_cast<int>(fold), 0)));
+            }
+            ext = fold;
+            if (!ok && g.status) __hip_atomic_store(g.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);   // this call's result is not valid
+        }
+        auto bits_of = [](uint32_t key) { return (key & 0x8000u) ? key ^ 0x7fffu : key; };   // (16 bits) the monotone map is its own inverse
+        const float x_min = rnd<DT>(Cvt<DT>::to_float(bits_of(ext & 0xffffu)) * clip);
+        const float x_max = rnd<DT>(Cvt<DT>::to_float(bits_of(ext >> 16)) * clip);
+        const float diff = rnd<DT>(x_max - x_min);
+        const float sc = rnd<DT>(diff * __fdiv_rn(1.0f, levels));
+        const float zp = rnd<DT>(__fdiv_rn(-x_min, sc));
+        if (lead && (!SPLIT || t_first == 0)) {   // (one of the parts writes them)
+            const int64_t o = static_cast<int64_t>(bh) * 128 + quarter * 32 + c;
+            scale[o] = static_cast<uint16_t>(Cvt<DT>::from_float(sc));
+            zero[o] = static_cast<uint16_t>(Cvt<DT>::from_float(zp));
+        }
+#pragma unroll
+        for (int k = 1; k <= L; ++k) {
+            const int key = threshold_key<DT>(sc, zp, levels, k, odd);
+            if (lead) {
+                // as EmitPlan compares: two bits, monotone words (-0 is one below +0, and belongs to a threshold of 0);
+                // one bit, signed words above 0 and reversed magnitudes up to it
+                if constexpr (BITS == 2) s_thr[k - 1][c] = static_cast<uint16_t>(key > 0 ? key : key - 1);
+                else {
+                    s_thr[0][c] = static_cast<uint16_t>(key > 0 ? key : 1 - key);
+                    s_flip[c] = static_cast<uint16_t>(key <= 0 ? 0x8000 : 0);
+                }
+            }
         }
     }
     __syncthreads();
-    float th[L][8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int k = 0; k < L; ++k) th[k][j] = s_thr[k][q4 * 8 + j];
+    EmitPlan<BITS> ep;
+    ep.load(s_thr, s_flip, piece * 8);
+    const unsigned char* next_base = base_of(has_next ? next_id : id);
+    const int next_len = rows_of(has_next ? next_id : id);
+    // opaque: what the rows' addresses are made of; they are worked out anew for each part, not kept across the loop
+    int next_last = (next_len - 1) / kFPass;
+    uint32_t next_full = off_full, next_off = tail_offset(next_len), next_pass = pass_bytes;
+    int t_out = q4 * kFPass + row;
+    asm volatile("" : "+v"(next_full), "+v"(next_off), "+v"(t_out), "+s"(next_last), "+s"(next_pass));
     constexpr int nb = 128 * BITS / 8;   // bytes per packed row
+    // lane q of a quad ends with row 4 j + q's bytes of all four pieces of the quad
+    uint8_t* orow = codes + (static_cast<int64_t>(bh) * g.T + t_first) * nb + (quarter + (piece >> 2)) * (nb / 4);
+    const uint32_t sel1 = (q4 & 1) ? 0x03070105u : 0x06020400u, sel2 = (q4 & 2) ? 0x03020706u : 0x05040100u;
+    auto emit = [&](auto refill) {
 #pragma unroll
-    for (int e = 0; e < NR; ++e) {
-        // the rows refilled from memory go first (their loads then have the rest of the emit to land), the
-        // staged rows after them
-        const int i = (e + NP) % NR;
-        if constexpr (NP > 0) {
-            if (e == NR - NP) {
-                // Every staged piece has landed once at most NR - NP younger memory operations are outstanding
-                // (the refills just issued; stores issued since only make the wait stricter).  A thread reads
-                // back exactly the bytes its own lane requested, so no barrier is needed.
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NR - NP) : "memory");
-            }
-        }
-        const int t = i * (kFThreads / 4) + row_i;
-        // (the empty statement keeps the compiler from carrying the unpacked floats of the
-        // min/max pass over to here: that would double the registers the slice needs)
-        asm volatile("" : "+v"(v[i]));
-        float f[8];
-        unpack8<DT>(v[i], f);
-        uint32_t code[8];
-        if constexpr (BITS == 2) {
+        for (int i0 = 0; i0 < NR; i0 += 4) {
+            uint32_t b[4][BITS];
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                code[j] = ((f[j] >= th[0][j]) ? 1u : 0u) + ((f[j] >= th[1][j]) ? 1u : 0u) + ((f[j] >= th[2][j]) ? 1u : 0u);
-        }
-        // ROPE: the quad's bytes are two pairs, the lower-half pair at quarter * nb / 8 and the upper-half pair nb / 2 further
-        uint8_t* o = codes + (min(bh, nbh - 1) * g.T + t_first + min(t, t_len - 1)) * nb + (ROPE ? quarter * (nb / 8) : quarter * (nb / 4));
-        if constexpr (BITS == 1) {
-            // The byte is built by eight add-with-carry steps, w = w + w + (f[j] >= th[j]): each
-            // comparison leaves its lane mask in a scalar register pair of its own and the add
-            // takes it as the carry-in (two instructions per element; a compare, a select and an
-            // OR otherwise).  The compares come first, so every mask is read at least two
-            // instructions after it is written, as this chip requires of a vector instruction
-            // that reads a scalar register written by another.
-            uint32_t w = 0;
-            unsigned long long m0, m1, m2, m3, m4, m5, m6, m7;
-            asm volatile(
-                "v_cmp_le_f32_e64 %[m0], %[t0], %[f0]\n\t"
-                "v_cmp_le_f32_e64 %[m1], %[t1], %[f1]\n\t"
-                "v_cmp_le_f32_e64 %[m2], %[t2], %[f2]\n\t"
-                "v_cmp_le_f32_e64 %[m3], %[t3], %[f3]\n\t"
-                "v_cmp_le_f32_e64 %[m4], %[t4], %[f4]\n\t"
-                "v_cmp_le_f32_e64 %[m5], %[t5], %[f5]\n\t"
-                "v_cmp_le_f32_e64 %[m6], %[t6], %[f6]\n\t"
-                "v_cmp_le_f32_e64 %[m7], %[t7], %[f7]\n\t"
-                "v_addc_co_u32_e64 %[w], %[m0], %[w], %[w], %[m0]\n\t"
-                "v_addc_co_u32_e64 %[w], %[m1], %[w], %[w], %[m1]\n\t"
-                "v_addc_co_u32_e64 %[w], %[m2], %[w], %[w], %[m2]\n\t"
-                "v_addc_co_u32_e64 %[w], %[m3], %[w], %[w], %[m3]\n\t"
-                "v_addc_co_u32_e64 %[w], %[m4], %[w], %[w], %[m4]\n\t"
-                "v_addc_co_u32_e64 %[w], %[m5], %[w], %[w], %[m5]\n\t"
-                "v_addc_co_u32_e64 %[w], %[m6], %[w], %[w], %[m6]\n\t"
-                "v_addc_co_u32_e64 %[w], %[m7], %[w], %[w], %[m7]"
-                : [w] "+v"(w), [m0] "=&s"(m0), [m1] "=&s"(m1), [m2] "=&s"(m2), [m3] "=&s"(m3),
-                  [m4] "=&s"(m4), [m5] "=&s"(m5), [m6] "=&s"(m6), [m7] "=&s"(m7)
-                : [t0] "v"(th[0][0]), [t1] "v"(th[0][1]), [t2] "v"(th[0][2]), [t3] "v"(th[0][3]),
-                  [t4] "v"(th[0][4]), [t5] "v"(th[0][5]), [t6] "v"(th[0][6]), [t7] "v"(th[0][7]),
-                  [f0] "v"(f[0]), [f1] "v"(f[1]), [f2] "v"(f[2]), [f3] "v"(f[3]),
-                  [f4] "v"(f[4]), [f5] "v"(f[5]), [f6] "v"(f[6]), [f7] "v"(f[7]));
-            w <<= 8 * q4;
-            w |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w), 0xB1, 0xf, 0xf, true));
-            w |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w), 0x4E, 0xf, 0xf, true));
-            if constexpr (ROPE) {
-                if ((q4 & 1) == 0 && t < t_len && live)
-                    *reinterpret_cast<uint16_t*>(o + (q4 >> 1) * (nb / 2)) = static_cast<uint16_t>(w >> (8 * q4));
-            } else {
-                if (q4 == 0 && t < t_len && live) *reinterpret_cast<uint32_t*>(o) = w;
+            for (int k = 0; k < 4; ++k) {
+                if constexpr (BITS == 1) b[k][0] = ep.byte(v[i0 + k]);
+                else ep.bytes(v[i0 + k], b[k][0], b[k][1]);
+                // the row is packed: its registers take the same row of the next part
+                if constexpr (decltype(refill)::value) v[i0 + k] = load_row(next_base, next_pass, i0 + k, next_last, next_full, next_off);
             }
-        } else {
-            const uint32_t b0 = (code[0] << 6) | (code[1] << 4) | (code[2] << 2) | code[3];
-            const uint32_t b1 = (code[4] << 6) | (code[5] << 4) | (code[6] << 2) | code[7];
-            const uint32_t half = b0 | (b1 << 8);
-            const uint32_t other = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(half), 0xB1, 0xf, 0xf, true));
-            if constexpr (ROPE) {
-                if ((q4 & 1) == 0 && t < t_len && live) *reinterpret_cast<uint32_t*>(o + (q4 >> 1) * (nb / 2)) = half | (other << 16);
+            if constexpr (BITS == 1) {
+                uint32_t w = __builtin_amdgcn_perm(b[1][0], b[0][0], 0x0c0c0400u) | __builtin_amdgcn_perm(b[3][0], b[2][0], 0x04000c0cu);
+                w = __builtin_amdgcn_perm(quad_xor(w, std::integral_constant<int, 1>{}), w, sel1);   // rows 0, 2 / 1, 3 of a lane pair
+                w = __builtin_amdgcn_perm(quad_xor(w, std::integral_constant<int, 2>{}), w, sel2);   // row q4 of the quad
+                if (t_out < t_len - i0 * kFPass)
+                    __builtin_nontemporal_store(w, reinterpret_cast<uint32_t*>(orow + i0 * kFPass * nb + static_cast<uint32_t>(t_out) * nb));
             } else {
-                if ((q4 & 1) == 0 && t < t_len && live) reinterpret_cast<uint32_t*>(o)[q4 >> 1] = half | (other << 16);
+                // two bytes a row and lane: rows 0, 1 and 2, 3 in a word each
+                uint32_t w01 = __builtin_amdgcn_perm(b[0][1], b[0][0], 0x0c0c0400u) | __builtin_amdgcn_perm(b[1][1], b[1][0], 0x04000c0cu);
+                uint32_t w23 = __builtin_amdgcn_perm(b[2][1], b[2][0], 0x0c0c0400u) | __builtin_amdgcn_perm(b[3][1], b[3][0], 0x04000c0cu);
+                const uint32_t selh = (q4 & 1) ? 0x03020706u : 0x05040100u;   // of a lane pair: row 0 (2) for the even lane, 1 (3) for the odd
+                w01 = __builtin_amdgcn_perm(quad_xor(w01, std::integral_constant<int, 1>{}), w01, selh);
+                w23 = __builtin_amdgcn_perm(quad_xor(w23, std::integral_constant<int, 1>{}), w23, selh);
+                const bool up = (q4 & 2) != 0;
+                const uint32_t keep = up ? w23 : w01, got = quad_xor(up ? w01 : w23, std::integral_constant<int, 2>{});
+                if (t_out < t_len - i0 * kFPass) {
+                    uint32_t* o = reinterpret_cast<uint32_t*>(orow + i0 * kFPass * nb + static_cast<uint32_t>(t_out) * nb);
+                    __builtin_nontemporal_store(up ? got : keep, o);   // (the codes are 4-byte aligned at least)
+                    __builtin_nontemporal_store(up ? keep : got, o + 1);
+                }
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        // the row is packed: its registers take the same row of the next slice
-        if (has_next) {
-            if (i < NP) v[i] = *reinterpret_cast<const U4*>(stage + (i * kFThreads + tid) * 16);
-            else v[i] = *reinterpret_cast<const U4*>(next_base + row_offset(t, next_len));
-        }
+    };
+    if (!has_next) {
+        emit(std::false_type{});
+        return;
     }
+    emit(std::true_type{});
+    id = next_id;
     }
 }
 
-// Raises a kernel's dynamic-LDS limit (the default stops at 64 KB); asked of the runtime once per kernel and device.
-static int allow_dynamic_lds(const void* kernel, int bytes) {
-    struct Done { const void* k; uint64_t devices; };
-    static std::mutex mu;
-    static std::vector<Done> done;
-    int dev = 0;
-    CQ_HIP_CHECK(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lock(mu);
-    for (auto& d : done)
-        if (d.k == kernel) {
-            if (d.devices >> (dev & 63) & 1) return CQ_OK;
-            CQ_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-            d.devices |= 1ull << (dev & 63);
-            return CQ_OK;
-        }
-    CQ_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-    done.push_back({kernel, 1ull << (dev & 63)});
-    return CQ_OK;
+// rows per thread of the instantiation for `need` passes: whole rows, quarters, with the rotary embedding
+static constexpr int fused_rows(int need, int lpr, bool rope) {
+    if (rope) return need <= 8 ? 8 : need <= 16 ? 16 : need <= 32 ? 32 : kFRows;
+    if (lpr == 4) return need <= 4 ? 4 : need <= 8 ? 8 : need <= 16 ? 16 : need <= 32 ? 32 : kFRows;
+    return need <= 4 ? 4 : need <= 8 ? 8 : need <= 16 ? 16 : need <= 24 ? 24 : need <= 32 ? 32 : need <= 40 ? 40 : kFRows;
 }
-
-template <typename DT, int BITS, int NR, bool ROPE, bool SPLIT = false>
-static int launch_fused(dim3 grid, hipStream_t st, const uint16_t* xp, const QuantGeom& g, float clip, uint16_t* sp,
-                        uint16_t* zp, uint8_t* codes, const RopeArgs& ra) {
-    constexpr int lds = fused_stage_rows(NR, ROPE) * kFThreads * 16;
-    auto kf = fused_pack_kernel<DT, BITS, NR, ROPE, SPLIT>;
-    if (lds) {
-        const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kf), lds);
-        if (rc != CQ_OK) return rc;
+template <typename DT, int BITS, int LPR, bool ROPE, bool SPLIT>
+static void launch_fused_rows(int nr, dim3 grid, hipStream_t st, const uint16_t* xp, const QuantGeom& g, float clip,
+                              uint16_t* sp, uint16_t* zp, uint8_t* codes, const RopeArgs& ra) {
+    auto go = [&](auto n) {
+        constexpr int NR = decltype(n)::value;
+        if constexpr (fused_rows(NR, LPR, ROPE) == NR)   // (no instantiation that the choice above does not name)
+            hipLaunchKernelGGL((fused_pack_kernel<DT, BITS, NR, LPR, ROPE, SPLIT>), grid, dim3(kFThreads), 0, st, xp, g, clip, sp, zp, codes, ra);
+    };
+    switch (nr) {
+        case 4: go(std::integral_constant<int, 4>{}); break;
+        case 8: go(std::integral_constant<int, 8>{}); break;
+        case 16: go(std::integral_constant<int, 16>{}); break;
+        case 24: go(std::integral_constant<int, 24>{}); break;
+        case 32: go(std::integral_constant<int, 32>{}); break;
+        case 40: go(std::integral_constant<int, 40>{}); break;
+        default: go(std::integral_constant<int, kFRows>{}); break;
     }
-    hipLaunchKernelGGL(kf, grid, dim3(kFThreads), lds, st, xp, g, clip, sp, zp, codes, ra);
-    return CQ_OK;
 }
 
 // true if the shape goes through the one-pass kernel (x read once, slice by slice in registers)
@@ -902,40 +949,46 @@ static int persistent_units() {
     return cu;
 }
 
-// ---- a token axis longer than one workgroup's registers: several workgroups per slice (SPLIT) ----------------
-// Parts per slice (a power of two up to 32, so that it divides the persistent grid), rows per part and per thread:
-// the choice that loads the fewest rows (a thread's rows past its part's end repeat the part's last row).  Only with
-// more than eight rows per thread, the instantiations that stage the next slice's rows through LDS: measured against
-// the three launches (partial min / max, statistics, emit - whose second read of x comes from the memory-side cache)
-// on one device, 1 bit, (batch, tokens, 8 heads): strided view of a fused projection (16, 9 984) 105 against 126 us,
-// (64, 5 000) 224 against 263 us, contiguous (16, 9 984) 123 against 123 us; with eight rows per thread and no
-// staging (8, 32 768) 265 against 205 us.
-struct SplitPlan { int plog, part_rows, nr; };
-static bool split_plan(int T, SplitPlan* sp) {
-    static const int kRowOptions[2] = {10, 13};
+// ---- how the work is cut ------------------------------------------------------------------------------------
+// Lanes per row, parts of the token axis, rows per part, rows per thread, workgroups of the launch.  Among the rows
+// per thread that give a part count that fits (at most 128; quarters only where all of them are resident at once) the one
+// that is expected to take the least, in hundredths of a microsecond: for each turn of a compute unit 0.08 us per row of
+// a thread and 0.4 us of folds and thresholds; with several parts 1 us for the exchange and what polling the other parts
+// costs.  Fitted to 20 shapes timed with every part count that fits: the choice is within 5 % of the best for 16 of them, 30 %
+// off for the worst (3 x 5 000 x 4 heads).
+// Why quarters at all, us of whole rows (best part count) / quarters: 4 x 320 x 8 heads 4.7 / 3.8, 1 x 1 024 4.9 / 4.2,
+// 8 x 1 024 7.2 / 6.4, 1 x 32 768 x 2 heads 11.8 / 8.3 (fewer channels to exchange per part).
+struct SplitPlan { int lpr, parts, part_rows, nr, grid; };
+constexpr int kFMostParts = 128;
+static bool split_plan(int64_t pairs, int T, bool rope, SplitPlan* sp) {
+    const int cu = persistent_units();
+    const int64_t room = static_cast<int64_t>(cu) * kFResident;
     int64_t best = -1;
-    for (int plog = 1; plog <= 5; ++plog) {
-        const int parts = 1 << plog;
-        const int rows = (T + parts - 1) / parts;
-        if (rows > kFMaxT || static_cast<int64_t>(parts - 1) * rows >= T) continue;
-        const int need = (rows + kFThreads / 4 - 1) / (kFThreads / 4);
-        int nr = 0;
-        for (int o : kRowOptions) if (!nr && o >= need) nr = o;
-        if (need <= 8) continue;   // (would be the unstaged instantiation)
-        const int64_t cost = static_cast<int64_t>(nr) * parts;
-        if (best < 0 || cost < best) { best = cost; sp->plog = plog; sp->part_rows = rows; sp->nr = nr; }
+    for (int lpr = 16; lpr >= (rope ? 16 : 4); lpr -= 12) {
+        const int pass = kFThreads / lpr;
+        const int64_t slices = pairs * (16 / lpr);
+        for (int n = 4; n <= kFRows; n = n < 8 ? 8 : n < 40 ? n + 8 : n + 12) {
+            if (fused_rows(n, lpr, rope) != n) continue;
+            // the fewest parts that n rows per thread hold (more of them only cost more); none of them empty
+            const int least = (T - 1) / (n * pass) + 1, rows = (T - 1) / least + 1, p = (T - 1) / rows + 1;
+            if (p > kFMostParts || p > room || (lpr == 4 && slices * p > room)) continue;   // (a pair's parts are resident together)
+            const int64_t turns = (slices * p + cu - 1) / cu;                                  // per compute unit
+            const int64_t cost = turns * (8 * n + 40) + (p > 1 ? 100 + (lpr == 16 ? 15 : 5) * p : 0);
+            if (best < 0 || cost < best) {
+                best = cost;
+                *sp = SplitPlan{lpr, p, rows, n, static_cast<int>(slices * p < room ? slices * p : room)};
+            }
+        }
     }
     return best >= 0;
 }
-static size_t split_records_bytes(int B, int H, int plog) {   // (for the map with more ids)
-    return ((static_cast<size_t>(B) * H + 63) / 64 * 256 << plog) * 32 * 2 * sizeof(unsigned long long);
-}
-// Which slices share a die (see slice_of() in the kernel).  Measured, 1 bit, batch 16 x 9 984 tokens x 8 heads split
-// four ways: contiguous (B, T, H, D) 122 -> 110 us with the wide map, the strided view of a fused projection 104 ->
-// 106 us; unsplit slices (batch 64 x 3 328) are indifferent to it (129 / 130 us contiguous, 106 / 106 us strided).
-// (the wide map pads the (batch, head) pairs to a multiple of 64: only where there are at least that many)
-static int wide_map_for(const QuantGeom& g, bool split) {
-    return (split && g.sh == g.D && static_cast<int64_t>(g.B) * g.H >= 64) ? 1 : 0;
+// records that the parts exchange (a pair's channels are the same number in whole rows and in quarters)
+static size_t split_records_bytes(int64_t pairs, int parts) { return static_cast<size_t>(pairs) * parts * 128 * sizeof(unsigned long long); }
+
+template <typename DT> static void launch_rope_rows(const uint16_t* x, const QuantGeom& g, const RopeArgs& ra, hipStream_t st);
+
+__global__ __launch_bounds__(256) void clear_records_kernel(unsigned long long* rec, int64_t n) {
+    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += gridDim.x * 256ll) rec[i] = 0ull;
 }
 
 // The wait of a part for the others is bounded; a lane that gives up sets a word of pinned host memory (one per
@@ -972,9 +1025,9 @@ static int* split_status_word(hipStream_t st) {
 }
 
 static bool one_pass_shape(const QuantGeom& g, const uint8_t* codes) {
-    return g.D == 128 && g.T <= kFMaxT && (reinterpret_cast<uintptr_t>(codes) & 3u) == 0 &&
-           static_cast<int64_t>(g.B) * g.H < (static_cast<int64_t>(1) << 31) && g.st > 0 && g.st * 2 < (1 << 24) &&
-           static_cast<int64_t>(g.T) * g.st * 2 < (static_cast<int64_t>(1) << 31);   // 32-bit row offsets
+    return g.D == 128 && (reinterpret_cast<uintptr_t>(codes) & 3u) == 0 &&
+           static_cast<int64_t>(g.B) * g.H < (static_cast<int64_t>(1) << 25) &&   // 32-bit ids
+           g.st > 0 && g.st * 2 < (1 << 24);   // 32-bit row offsets inside a pass
 }
 
 template <typename DT>
@@ -984,78 +1037,67 @@ static int run_quant(const void* x, QuantGeom g, int bits, float clip, uint8_t* 
     const uint16_t* xp = static_cast<const uint16_t*>(x);
     uint16_t* sp = static_cast<uint16_t*>(scale);
     uint16_t* zp = static_cast<uint16_t*>(zero);
-    if (rope && (xq || !one_pass_shape(g, codes))) return CQ_ERR_UNSUPPORTED;
-    if (!xq && one_pass_shape(g, codes)) {
-        // x fits a workgroup's registers slice by slice: one pass
-        const int64_t bh8 = (static_cast<int64_t>(g.B) * g.H + 7) / 8;
-        // persistent: at most one workgroup per compute unit and a multiple of 32 of them
-        g.wide_map = wide_map_for(g, false);
-        const int64_t nsl = g.wide_map ? (static_cast<int64_t>(g.B) * g.H + 63) / 64 * 256 : bh8 * 32;
-        // (the compute-unit count of the current device - a partitioned device reports its own share -
-        // rounded down to the multiple of 32 the slice walk needs)
-        const int cu = persistent_units();
-        const int64_t fmax = cu >= 32 ? cu / 32 * 32 : 32;
-        const dim3 fgrid(static_cast<unsigned>(nsl < fmax ? nsl : fmax));
-        const int nr = (g.T + kFThreads / 4 - 1) / (kFThreads / 4);
-        const RopeArgs ra = rope ? *rope : RopeArgs{};
-#define CQ_FUSED(B_, N_)                                                                          \
-        do {                                                                                      \
-            const int rc = rope ? launch_fused<DT, B_, N_, true>(fgrid, st, xp, g, clip, sp, zp, codes, ra)   \
-                                : launch_fused<DT, B_, N_, false>(fgrid, st, xp, g, clip, sp, zp, codes, ra); \
-            if (rc != CQ_OK) return rc;                                                           \
-        } while (0)
-        if (bits == 1) {
-            if (nr <= 4) CQ_FUSED(1, 4); else if (nr <= 8) CQ_FUSED(1, 8); else CQ_FUSED(1, 13);
-        } else {
-            if (nr <= 4) CQ_FUSED(2, 4); else if (nr <= 8) CQ_FUSED(2, 8); else CQ_FUSED(2, 13);
-        }
-#undef CQ_FUSED
-        CQ_LAUNCH_CHECK();
-        return CQ_OK;
-    }
+    if (rope && (xq || g.T > kFMaxT || !one_pass_shape(g, codes))) return CQ_ERR_UNSUPPORTED;
     SplitPlan spl;
-    // (the slice walk pads the (batch, head) pairs to a multiple of 8 and a padding slice costs what a live one does:
-    // measured, a single pair of 40 000 tokens takes 33 us split and 25 us in three launches, six pairs of 13 000
-    // tokens 19.5 against 25.7 us)
-    if (!xq && !rope && g.D == 128 && g.T > kFMaxT && static_cast<int64_t>(g.B) * g.H >= 4 && split_plan(g.T, &spl) &&
-        !g_split_off.load(std::memory_order_relaxed) &&
-        (reinterpret_cast<uintptr_t>(codes) & 3u) == 0 && static_cast<int64_t>(g.B) * g.H < (static_cast<int64_t>(1) << 26) &&
-        g.st > 0 && g.st * 2 < (1 << 24) && static_cast<int64_t>(spl.part_rows) * g.st * 2 < (static_cast<int64_t>(1) << 31)) {
-        // Still one pass over x: the slices are split along the token axis between workgroups of one persistent
-        // launch, which exchange their channel min / max inside it.
-        int* status = split_status_word(st);
-        if (status) {
-            if (*static_cast<volatile int*>(status) != 0) {
+    if (!xq && one_pass_shape(g, codes) && split_plan(static_cast<int64_t>(g.B) * g.H, g.T, rope != nullptr, &spl)) {
+        // one pass over x; several parts per pair need the word that tells when one gave up waiting
+        int* status = nullptr;
+        if (spl.parts > 1) {
+            status = g_split_off.load(std::memory_order_relaxed) ? nullptr : split_status_word(st);
+            if (status && *static_cast<volatile int*>(status) != 0) {
                 *static_cast<volatile int*>(status) = 0;
                 g_split_off.store(true, std::memory_order_relaxed);
                 return CQ_ERR_LAUNCH;   // an earlier split pass did not complete: its output is not valid
             }
-            g.wide_map = wide_map_for(g, true);
-            const int64_t nids = (g.wide_map ? (static_cast<int64_t>(g.B) * g.H + 63) / 64 * 256
-                                             : (static_cast<int64_t>(g.B) * g.H + 7) / 8 * 32) << spl.plog;
-            const int cu = persistent_units();
-            const int64_t fmax = cu >= 32 ? cu / 32 * 32 : 32;
-            const dim3 fgrid(static_cast<unsigned>(nids < fmax ? nids : fmax));
-            g.parts_log2 = spl.plog;
+        }
+        if (spl.parts == 1 || status) {
+            g.parts = spl.parts;
             g.part_rows = spl.part_rows;
+            g.dP.set(static_cast<uint32_t>(spl.parts));
             g.rec = reinterpret_cast<unsigned long long*>(ws);
-            uint32_t ep = g_qepoch.fetch_add(1, std::memory_order_relaxed) + 1;
-            g.epoch = ep ? ep : g_qepoch.fetch_add(1, std::memory_order_relaxed) + 1;
+            if (spl.parts > 1) {
+                uint32_t ep = g_qepoch.fetch_add(1, std::memory_order_relaxed) + 1;
+                g.epoch = ep ? ep : g_qepoch.fetch_add(1, std::memory_order_relaxed) + 1;
+            }
             g.spin_limit = g_qspin.load(std::memory_order_relaxed);
             g.status = status;
-            const RopeArgs ra{};
-            int rc = CQ_OK;
-#define CQ_SPLIT(B_, N_) rc = launch_fused<DT, B_, N_, false, true>(fgrid, st, xp, g, clip, sp, zp, codes, ra)
-            if (bits == 1) {
-                if (spl.nr == 10) CQ_SPLIT(1, 10); else CQ_SPLIT(1, 13);
-            } else {
-                if (spl.nr == 10) CQ_SPLIT(2, 10); else CQ_SPLIT(2, 13);
+            if (spl.parts > 1) {
+                // A recorded launch comes back with the same epoch: its records are emptied first, in the recording too.
+                // (0 is never an epoch)
+                hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+                if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
+                else if (cs != hipStreamCaptureStatusNone) {
+                    const int64_t n = static_cast<int64_t>(g.B) * g.H * spl.parts * 128;
+                    const int64_t blocks = (n + 255) / 256;
+                    hipLaunchKernelGGL(clear_records_kernel, dim3(static_cast<unsigned>(blocks < 1024 ? blocks : 1024)), dim3(256), 0, st, g.rec, n);
+                    CQ_LAUNCH_CHECK();
+                }
             }
-#undef CQ_SPLIT
-            if (rc != CQ_OK) return rc;
+            const dim3 fgrid(static_cast<unsigned>(spl.grid));
+            const RopeArgs ra = rope ? *rope : RopeArgs{};
+            auto launch = [&](auto b, auto l, auto r) {
+                constexpr int B_ = decltype(b)::value, L_ = decltype(l)::value;
+                constexpr bool R_ = decltype(r)::value;
+                if (spl.parts > 1) launch_fused_rows<DT, B_, L_, R_, true>(spl.nr, fgrid, st, xp, g, clip, sp, zp, codes, ra);
+                else launch_fused_rows<DT, B_, L_, R_, false>(spl.nr, fgrid, st, xp, g, clip, sp, zp, codes, ra);
+            };
+            auto with_bits = [&](auto b) {
+                if (rope) launch(b, std::integral_constant<int, 16>{}, std::true_type{});
+                else if (spl.lpr == 16) launch(b, std::integral_constant<int, 16>{}, std::false_type{});
+                else launch(b, std::integral_constant<int, 4>{}, std::false_type{});
+            };
+            if (bits == 1) with_bits(std::integral_constant<int, 1>{});
+            else with_bits(std::integral_constant<int, 2>{});
             CQ_LAUNCH_CHECK();
             return CQ_OK;
         }
+    }
+    if (rope) {
+        // no exchange inside a launch: the rotated rows first, then the three launches on them
+        launch_rope_rows<DT>(xp, g, *rope, st);
+        CQ_LAUNCH_CHECK();
+        xp = rope->out;
+        g.sb = rope->ob; g.st = rope->ot; g.sh = rope->oh;
     }
     hipLaunchKernelGGL(minmax_partial_kernel<DT>, grid, dim3(kQThreads), 0, st, xp, g, ws);
     CQ_LAUNCH_CHECK();
@@ -1165,6 +1207,11 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(const uint16_t* __restri
     uint16_t* orow = ra.out + b * ra.ob + static_cast<int64_t>(t) * ra.ot + static_cast<int64_t>(h) * ra.oh + gq * ra.og + p8 * 8;
     *reinterpret_cast<U4*>(orow) = r1;
     *reinterpret_cast<U4*>(orow + 64) = r2;
+}
+
+template <typename DT> static void launch_rope_rows(const uint16_t* x, const QuantGeom& g, const RopeArgs& ra, hipStream_t st) {
+    const int64_t blocks = (static_cast<int64_t>(g.B) * g.T * g.H * ra.gn * 8 + 255) / 256;   // (the callers keep it below 2^31)
+    hipLaunchKernelGGL(rope_rows_kernel<DT>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, x, g, ra);
 }
 
 static int check_rope(const void* cos_table, const void* sin_table, int64_t table_rows, const int64_t* pos,
@@ -1333,8 +1380,9 @@ size_t cq_quantize_pack_workspace(int B, int T, int H, int D) {
     size_t need = (static_cast<size_t>(B) * H * (static_cast<size_t>(cq::pick_chunks(B, T, H)) * 2 + 3) + 4) * D * sizeof(float);
     // (the records that the parts of a split slice exchange, when the one-pass kernel takes a long token axis)
     cq::SplitPlan spl;
-    if (D == 128 && T > cq::kFMaxT && cq::split_plan(T, &spl)) {
-        const size_t rec = cq::split_records_bytes(B, H, spl.plog);
+    for (int rope = 0; rope < 2; ++rope) {
+        if (D != 128 || !cq::split_plan(static_cast<int64_t>(B) * H, T, rope != 0, &spl) || spl.parts == 1) continue;
+        const size_t rec = cq::split_records_bytes(static_cast<int64_t>(B) * H, spl.parts);
         if (rec > need) need = rec;
     }
     return need;
@@ -1407,8 +1455,8 @@ int cq_rope_rows_grouped(const void* x, int dtype, int B, int T, int H, int G, i
     if (blocks > 0x7fffffff) return CQ_ERR_SHAPE;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint16_t* xp = static_cast<const uint16_t*>(x);
-    if (dtype == CQ_BF16) hipLaunchKernelGGL(cq::rope_rows_kernel<cq::BF16>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, xp, g, ra);
-    else hipLaunchKernelGGL(cq::rope_rows_kernel<cq::FP16>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, xp, g, ra);
+    if (dtype == CQ_BF16) cq::launch_rope_rows<cq::BF16>(xp, g, ra, st);
+    else cq::launch_rope_rows<cq::FP16>(xp, g, ra, st);
     CQ_LAUNCH_CHECK();
     return CQ_OK;
 }

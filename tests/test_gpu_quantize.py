@@ -214,3 +214,58 @@ def test_quantize_pack_split_slices_give_up_and_the_host_reports_it(ops):
     finally:
         lib.cq_quantize_pack_wait_polls(before)
     check()
+
+
+# What the one-pass kernel makes of a shape: whole rows or quarters, one part or several, one id per workgroup or a walk.
+# Edges of passes (16 and 64 rows), of the rows a thread holds, of the parts; pair counts that are no multiple of eight.
+CUT_SHAPES = [(1, 1, 1), (1, 2, 8), (2, 63, 3), (3, 65, 5), (1, 255, 2), (2, 833, 3), (1, 3329, 4), (5, 832, 8), (70, 831, 2),
+              (67, 16, 8), (90, 333, 8), (1, 4097, 8), (2, 6657, 7), (21, 1700, 8)]
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("shape", CUT_SHAPES)
+def test_quantize_pack_one_pass_cuts_bit_exact(ops, shape, bits, dtype):
+    """Codes and statistics equal the oracle's bit for bit; channels of one sign, of equal values, with zeros of
+    both signs and with infinities among them."""
+    B, T, H = shape
+    print(f"case quantize_pack cut shape={shape} bits={bits} dtype={dtype}", flush=True)
+    rng = np.random.default_rng(T * 31 + B)
+    x = O.round_to(rng.standard_normal((B, T, H, 128), dtype=np.float32), dtype)
+    x[..., 3] = np.abs(x[..., 3])
+    x[..., 50] = -np.abs(x[..., 50])
+    x[:, T // 2:, :, 51] = np.abs(x[:, T // 2:, :, 51])      # one sign in some threads' rows only
+    x[..., 77] = 1.5
+    x[..., 78] = -0.0
+    x[:, ::2, :, 79] = 0.0
+    x[:, T // 3, :, 90] = np.inf
+    x[:, T - 1, :, 91] = -np.inf
+    x[..., 127] *= O.round_to(np.float32(2.0 ** -12), dtype)
+    x = O.round_to(x, dtype)
+    with np.errstate(all="ignore"):
+        oc, os_, oz = O.quantize_pack(x, bits, CLIPS[bits][0], dtype)
+    codes, s, z = ops.quantize_pack(to_gpu(x, dtype), bits, CLIPS[bits][0])
+    torch.cuda.synchronize()
+    # (zero-points of equal value: the sign of a zero minimum is the only one that min() over +0 and -0 leaves open)
+    assert same_bits(to_np(s), os_) and np.array_equal(to_np(z), oz, equal_nan=True)
+    assert np.array_equal(codes.cpu().numpy(), oc)
+
+
+@pytest.mark.parametrize("shape", [(2, 3328, 8), (1, 20000, 2), (4, 300, 8)])
+def test_quantize_pack_recorded_and_replayed(ops, shape):
+    """A recorded pass whose parts exchange their extremes comes back with the same epoch: what an earlier replay left in
+    the workspace must not be taken for this one's.  New inputs in place for each replay, eager work between them."""
+    B, T, H = shape
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.randn((B, T, H, 128), generator=g, device="cuda").to(torch.bfloat16)
+    ops.quantize_pack(x, 1, 0.5)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ops.quantize_pack(x, 1, 0.5)
+    for k in range(4):
+        x.copy_(torch.randn((B, T, H, 128), generator=g, device="cuda").to(torch.bfloat16) * (3.0 if k == 0 else 1.0 / (k + 1)))
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(got, ops.quantize_pack(x, 1, 0.5)):
+            assert torch.equal(a, b)
