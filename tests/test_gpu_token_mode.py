@@ -32,6 +32,36 @@ def test_quantize_pack_token_is_bit_exact(bits, dtype):
     assert same_bits(to_np(scale), s_ref) and same_bits(to_np(mins), m_ref)
 
 
+# Four lanes a group below 24 576 rows, one lane a group from there on: either side of the line, partial passes of 16 and 64
+# tokens, a single token.
+TOKEN_SHAPES = [(1, 1, 1), (1, 17, 5), (2, 3071, 4), (3, 3073, 8), (24577, 1, 1), (6, 4127, 1)]
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("shape", TOKEN_SHAPES)
+def test_quantize_pack_token_cuts_bit_exact(shape, bits, dtype):
+    """Codes by comparison instead of division: groups whose quotients hit the rounding ties, subnormal and large
+    ranges, constant groups and infinities."""
+    from calibquant_amd import ops
+    B, T, H = shape
+    print(f"case token quantiser shape={shape} bits={bits} dtype={dtype}", flush=True)
+    rng = np.random.default_rng(T + 7 * B)
+    x = rng.standard_normal((B, T, H, 128)).astype(np.float32)
+    t = np.arange(T)[None, :, None]
+    x[..., :32] = np.where((t % 3 == 0)[..., None], np.round(x[..., :32] * 4) / 8, x[..., :32])     # many exact ties
+    x[..., 32:64] *= np.where((t % 4 == 1)[..., None], np.float32(2.0 ** -22), np.float32(1))        # fp16: subnormal steps
+    x[..., 64:96] = np.where((t % 5 == 2)[..., None], x[..., 64:65], x[..., 64:96])                  # equal values
+    x[..., 96:128] = x[..., 96:128] * 512 + np.where((t % 2 == 0)[..., None], np.float32(3000), np.float32(0))
+    x[0, T - 1, H - 1, 100] = np.inf
+    x = O.round_to(x, dtype)
+    words, scale, mins = ops.quantize_pack_token(to_gpu(x, dtype), bits)
+    torch.cuda.synchronize()
+    w_ref, s_ref, m_ref = O.kivi_quantize_pack(np.transpose(x, (0, 2, 1, 3)), 32, bits, dtype)
+    assert np.array_equal(words.cpu().numpy(), w_ref)
+    assert same_bits(to_np(scale), s_ref) and np.array_equal(to_np(mins), m_ref)
+
+
 def _token_case(B, Hq, Hkv, T, R, bits, dtype, seed):
     c = make_case(B, Hq, Hkv, 128, T, R, bits, dtype, seed)
     words, scale, mins = O.kivi_quantize_pack(np.transpose(c["v"], (0, 2, 1, 3)), 32, bits, dtype)
