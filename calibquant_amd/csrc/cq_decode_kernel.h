@@ -236,12 +236,16 @@ __device__ __forceinline__ void clear_handover(const DecodeGeom& g, int64_t unit
 // exact integers, put together in fp32.  Packed codes are masked in place, the upper half of a byte after one shift of
 // the word - one AND per 4 codes; a code then counts 2^s, s = 0 .. 3, which the fixed-point operand (logits) or the
 // closing fold (sums) takes back.
-// Measured, us per step in turn on one box, look-up form before and this one: batch 64 x 3 328 + 128, 1 bit 28.5 -> 20.2,
-// 2 bits 48.9 -> 28.4; batch 256 x 3 328 99.7 -> 58.3 (3.9 TB/s); 16 x 9 984, six heads 38.4 -> 21.7; 8 x 32 768 in chunks
-// 36.8 -> 26.8; batch 1 x 1 024 7.7 -> 6.7.  A wave with 6.5 tiles of 64 tokens and four heads issues 1 810 vector
-// instructions (3 097 before), the set-up and the window's 350 among them: 84 a tile for the logits, 125 for weights and
-// values, 16 of these MFMAs.  What bounds a launch now is the latency of its phases, then the memory.
-// Error against 64 bits: a weight is off by 2^-31 at most; a channel's q.s_k by 2^(s - 30) of the head's
+// Measured, us per step in turn on one box, look-up form before and this one: batch 64 x 3 328 + 128, 1 bit 28.5 -> 19.7,
+// 2 bits 48.9 -> 27.5; batch 256 x 3 328 99.7 -> 57; 16 x 9 984, six heads 38.4 -> 20.3; 8 x 32 768 in chunks
+// 36.8 -> 26.5; batch 1 x 1 024 7.7 -> 6.7.  A wave issues 66 vector instructions per 64 tokens and four heads for the logits, 66
+// for weights and values, beside 16 of these MFMAs, and about 600 for the rest (330 of them the window); at batch 256 the
+// vector units are busy for three quarters of a launch.  The matrix form first had 84 and 125 per tile: the logits stay in grid
+// steps (their scale and zero-point go into the exponent's factor and the calibration), V fields are taken in place,
+// a weight's digits are one fused multiply-add and a conversion, every lane calibrates its own head only, and the
+// rows' addresses are a scalar base and one bounded offset - start of these steps -> now: batch 64 21.3 -> 20.0, 2 bits
+// 29.0 -> 27.6, 16 x 9 984 23.1 -> 20.5, batch 256 60.1 -> 57.3, per-token values 39.4 -> 36.9 (one box, in turn).
+// Error against 64 bits: a weight is off by 2^-31, or by 2^-24 of itself; a channel's q.s_k by 2^(s - 30) of the head's
 // largest (s = 3: 2^-27, three of the grid's bits; masked in place all through, the top bit of a byte would cost seven),
 // then the fp32 roundings.
 // The look-up form added fp32 partial sums on the K side and held the weights as fp16 on the V side.  Root-mean-square
@@ -256,6 +260,12 @@ typedef uint32_t U2 __attribute__((ext_vector_type(2)));
 // four signed byte digits of x, -2^31 <= x <= 2^31 - 1 - 0x808080 (digit 0 in the lowest byte; above that the top digit wraps)
 __device__ __forceinline__ uint32_t byte_digits(int x) {
     return (static_cast<uint32_t>(x) + 0x00808080u) ^ 0x00808080u;
+}
+
+// A weight e in [0, 1] on its grid of 2^-30 as four byte digits: e * 2^30 + 0x808080 is a whole number in fp32 (at least
+// 2^23; rounded to even where e * 2^30 is not), which is off by 2^-31 or by 2^-24 of e, the rounding of any fp32 product.
+__device__ __forceinline__ uint32_t weight_digits(float e, float grid) {
+    return static_cast<uint32_t>(static_cast<int>(__builtin_fmaf(e, grid, 8421504.f))) ^ 0x00808080u;
 }
 
 // what field f (lowest first) of a masked byte of codes counts, as a shift: the upper half-byte's fields are moved down
@@ -300,9 +310,11 @@ template <int BITS> __device__ __forceinline__ void code_fields(uint32_t w, int*
 }
 
 // Logits of 64 tokens, one row per lane: a 4 x 4 exchange of dwords between the four groups of 16 lanes gives lane
-// (x, k) dword k of the tokens x, 16 + x, 32 + x, 48 + x - the right operand of four 16-token tiles.
+// (x, k) dword k of the tokens x, 16 + x, 32 + x, 48 + x - the right operand of four 16-token tiles.  The results are in grid
+// steps, before the zero-point: logit = result * step - zero-point sum, which the minima and maxima take (the map is
+// monotone) and the exponent's factor carries.
 template <int BITS>
-__device__ __forceinline__ void matrix_logits(const uint4* c, I4 a0, I4 a1, float inv, float zs, float* out) {
+__device__ __forceinline__ void matrix_logits(const uint4* c, I4 a0, I4 a1, float* out) {
     uint32_t w[BITS][4];
 #pragma unroll
     for (int s = 0; s < BITS; ++s) {
@@ -322,13 +334,21 @@ __device__ __forceinline__ void matrix_logits(const uint4* c, I4 a0, I4 a1, floa
         acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, I4{f[4], f[5], f[6], f[7]}, acc, 0, 0, 0);
         // digit sums are at most 128 * 128 * 12 in size: two of them meet as an integer
         const float l = static_cast<float>(acc[0] + (acc[1] << 8)), u = static_cast<float>(acc[2] + (acc[3] << 8));
-        out[j] = __builtin_fmaf(__builtin_fmaf(u, 65536.f, l), inv, -zs);
+        out[j] = __builtin_fmaf(u, 65536.f, l);
     }
 }
 
 // Eight rows of one byte column per lane: of a [row][16 bytes] tile in LDS, lane x of 16 gets byte x of eight rows
 __device__ __forceinline__ I2 column8(const unsigned char* p) {
     return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) I2*)(p));
+}
+
+// The fields of a packed V byte in place, each sum counting 2^shift (the fold takes it back); the byte itself instead of
+// the topmost, as a signed number - at 1 bit -128 b7 + the others; at 2 bits, with the top bit flipped, the byte less 128, which
+// needs the sum of the weights as well (accumulator 8).  One AND or XOR per four codes less than a shift and four masks.
+template <int BITS> __device__ __forceinline__ constexpr int value_mask(int i) {
+    if (BITS == 1) return i < 7 ? 0x01010101 << i : 0;
+    return i < 3 ? 0x03030303 << (2 * i) : static_cast<int>(0x80808080u);
 }
 
 // Weighted code sums of 64 tokens.  The weights (lane: head lane / 16, tokens 16 j + x) go through the wave's LDS tile
@@ -340,11 +360,7 @@ __device__ __forceinline__ void matrix_values(unsigned char* tile, const float* 
 #pragma unroll
     for (int s = 0; s < BITS; ++s) *reinterpret_cast<U4*>(tile + (1 + s) * 1024 + lane * 16) = v[s];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        // (a weight is at most 1; the cap keeps the digits in range whatever comes)
-        const float xs = fminf(e[j] * 1073741824.f, 2130706432.f);
-        *reinterpret_cast<uint32_t*>(tile + (16 * j + x) * 16 + 4 * k) = byte_digits(__float2int_rn(xs));
-    }
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint32_t*>(tile + (16 * j + x) * 16 + 4 * k) = weight_digits(e[j], 1073741824.f);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -355,31 +371,43 @@ __device__ __forceinline__ void matrix_values(unsigned char* tile, const float* 
     for (int s = 0; s < BITS; ++s) {
         const I2 v0 = column8(col + (1 + s) * 1024), v1 = column8(col + (1 + s) * 1024 + 128);
         const int w[4] = {v0[0], v0[1], v1[0], v1[1]};
-        int f[4][8];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) code_fields<BITS>(static_cast<uint32_t>(w[r]), f[r]);
         constexpr int NF = 8 / BITS;
 #pragma unroll
-        for (int i = 0; i < NF; ++i)
-            acc[s * NF + i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, I4{f[0][i], f[1][i], f[2][i], f[3][i]}, acc[s * NF + i], 0, 0, 0);
+        for (int i = 0; i < NF; ++i) {
+            const int m = value_mask<BITS>(i);
+            I4 f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) f[r] = i < NF - 1 ? w[r] & m : w[r] ^ m;
+            acc[s * NF + i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, f, acc[s * NF + i], 0, 0, 0);
+        }
     }
+    if constexpr (BITS == 2) acc[8] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, I4{0x01010101, 0x01010101, 0x01010101, 0x01010101}, acc[8], 0, 0, 0);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
 
-// the lane's sums (one head, byte column x) as floats in channel order
+// the lane's sums (one head, byte column x) as floats in channel order (sums of digits are whole numbers below 2^28)
 template <int BITS> __device__ __forceinline__ void matrix_fold(const I4* acc, float* out, int x) {
     constexpr int NF = 8 / BITS;
 #pragma unroll
     for (int s = 0; s < BITS; ++s) {
+        I4 top = -acc[s * NF + NF - 1];
+        if constexpr (BITS == 1) {
+#pragma unroll
+            for (int i = 0; i < NF - 1; ++i) top += acc[i];                     // 128 x the topmost field's sums
+        } else {
+            top = 128 * acc[8] - top;                                           // the unsigned bytes' sums
+#pragma unroll
+            for (int i = 0; i < NF - 1; ++i) top -= acc[s * NF + i];            // 64 x
+        }
         Vec<4> o[NF / 4];
 #pragma unroll
         for (int i = 0; i < NF; ++i) {
-            const I4 a = acc[s * NF + i];
+            const I4 a = i < NF - 1 ? acc[s * NF + i] : top;
             float r = static_cast<float>(a[3]);
 #pragma unroll
             for (int p = 2; p >= 0; --p) r = __builtin_fmaf(r, 256.f, static_cast<float>(a[p]));
-            const float unit = 1.f / (1073741824.f * static_cast<float>(1 << field_shift<BITS>(i)));
+            const float unit = 1.f / (1073741824.f * static_cast<float>(1 << (BITS * i)));
             o[(NF - 1 - i) / 4].v[(NF - 1 - i) % 4] = r * unit;   // first channel of a byte in its top bits
         }
 #pragma unroll
@@ -432,7 +460,7 @@ __device__ __forceinline__ void matrix_values_token(unsigned char* tile, const f
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             // (at most 2^30: the grid comes from this very product)
-            *reinterpret_cast<uint32_t*>(tile + (16 * j + x) * 16 + 4 * k) = byte_digits(__float2int_rn(sc[j][gi % 2] * pw[gi]));
+            *reinterpret_cast<uint32_t*>(tile + (16 * j + x) * 16 + 4 * k) = weight_digits(sc[j][gi % 2], pw[gi]);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -600,8 +628,6 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     const int64_t code_off = has_img ? (bh * g.T + t0) * NB : 0;   // one offset for both code streams
     const uint4* ckp = reinterpret_cast<const uint4*>(has_img ? g.ck + code_off : static_cast<const uint8_t*>(g.q));
     const uint4* cvp = reinterpret_cast<const uint4*>((has_img ? g.cv : static_cast<const uint8_t*>(g.q)) + code_off);
-    const U4* cvp4 = reinterpret_cast<const U4*>(cvp);
-    const int last_u = has_img ? n * NB / 16 - 1 : 0;   // last valid 16-byte unit of either stream
     const int last_row = has_img ? n - 1 : 0;
     // residual tile: K slice (row = tid / LPR, 128 / LPR elements); V: a wave owns RPW rows of the tile and a
     // lane one channel pair of each of them, so the value products need no fold inside the wave
@@ -633,7 +659,27 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         }
     };
 
-    CQ_PHASE(1);   // prologue, requests of q and the statistics
+    // The first packed K rows are requested behind q and the statistics, before either is looked at: they arrive while q
+    // goes onto its grid.  (us, requested after that: 3 328 + 128 tokens, batch 64, 1 bit 20.4 -> 20.0, per-token values
+    // 36.7 -> 35.7; 16 x 9 984 20.8 -> 20.3; batch 1 and 6 within 1 %.)
+    __builtin_amdgcn_sched_barrier(0);
+    // Round r's row of a thread: a scalar base and the thread's offset in the round, both kept inside the chunk (rounds and
+    // rows past its end repeat the last row).
+    auto row_at = [&](const void* p, int r) {
+        const int r0 = min(r * kNT, last_row);
+        return reinterpret_cast<const unsigned char*>(p) + static_cast<int64_t>(r0) * NB + min(static_cast<uint32_t>(tid) * NB, static_cast<uint32_t>(last_row - r0) * NB);
+    };
+    uint4 kc[L::KR][BITS];
+    auto request_k = [&](int r) {
+        const uint4* p = reinterpret_cast<const uint4*>(row_at(ckp, r));
+#pragma unroll
+        for (int i = 0; i < BITS; ++i) kc[r % L::KR][i] = p[i];
+    };
+#pragma unroll
+    for (int r = 0; r < L::KR; ++r) request_k(r);
+    __builtin_amdgcn_sched_barrier(0);
+
+    CQ_PHASE(1);   // prologue, requests of q, the statistics and the first packed K rows
     // ---- phase 0: q onto its grid ---------------------------------------------------
     if (tid < HPB * kD) {
         const int h = tid / kD, d = tid % kD;
@@ -659,15 +705,6 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         fx[L::F_VSZ + kD + d] = Cvt<DT>::to_float(z_raw);
     }
     if (tid < 3 * HPB) reinterpret_cast<int*>(red)[tid] = static_cast<int>(0x80000000u);   // block_max's meeting words
-    // The packed K rows are requested only now, behind what phase 0 waits for: a wave that has to queue these
-    // requests first gets to phase 0 later.
-    uint4 kc[L::KR][BITS];
-#pragma unroll
-    for (int r = 0; r < L::KR; ++r) {
-#pragma unroll
-        for (int i = 0; i < BITS; ++i)
-            kc[r][i] = ckp[min(tid + r * kNT, last_row) * BITS + i];
-    }
     // Chunked launch: the chunks' logit min / max, lane s the pair of chunk s for every head (all in flight
     // together; they are folded across the wave where the calibration needs them).
     struct alignas(8) MinMax { float lo, hi; };
@@ -689,21 +726,21 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
 
     float* stat = fx + L::F_STAT;   // [alpha | m_res | l_res | m_img | l_img][HPB]
     float o_res = 0.f;
-    float mn[HPB], mx[HPB];
-#pragma unroll
-    for (int h = 0; h < HPB; ++h) { mn[h] = h < NH ? INFINITY : 0.f; mx[h] = h < NH ? -INFINITY : 0.f; }
+    float mn = INFINITY, mx = -INFINITY;   // of the lane's head (hl)
     // First block of packed V rows: half of it is requested here, behind the packed K rows, the
     // rest as the K registers free up, so it has arrived when the logits are done.
     constexpr int kVF = VTOK ? (REGL > 4 ? 1 : 2) * BITS : kMatrixV;   // 16-byte pieces of packed V rows in flight per thread
     U4 vc[kVF];
-    auto request_v = [&](int r) { vc[r] = cvp4[min((tid + (r / BITS) * kNT) * BITS + r % BITS, last_u)]; };
+    auto request_v = [&](int slot, int piece) {   // piece: round * BITS + 16-byte piece of the row
+        vc[slot] = reinterpret_cast<const U4*>(row_at(cvp, piece / BITS))[piece % BITS];
+    };
     constexpr int kVEarly = VTOK ? BITS : kMatrixE;
     if constexpr (!MINMAX_ONLY) {
 #pragma unroll
-        for (int r = 0; r < kVEarly; ++r) request_v(r);
+        for (int r = 0; r < kVEarly; ++r) request_v(r, r);
     }
 
-    CQ_PHASE(2);   // q on its grid, first packed K rows requested
+    CQ_PHASE(2);   // q on its grid
     // the wave's first token, and the head whose results this lane holds (lanes beyond the unit's heads repeat
     // the last one)
     const int wt0 = __builtin_amdgcn_readfirstlane(tid);
@@ -715,22 +752,18 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     if (has_img) {
         const I4* aq = reinterpret_cast<const I4*>(regA);
         const I4 a0 = aq[lane], a1 = aq[64 + lane];
-        const float inv = qsz[2 * hl], zs = qsz[2 * hl + 1];
         float lo = INFINITY, hi = -INFINITY;
         phase_priority(std::integral_constant<int, 1>{});
 #pragma unroll
         for (int rd = 0; rd < REGL; ++rd) {
             if (wt0 + rd * kNT < n) {
-                matrix_logits<BITS>(kc[rd % L::KR], a0, a1, inv, zs, lx[rd]);
-                if (rd + L::KR < REGL) {
-#pragma unroll
-                    for (int i = 0; i < BITS; ++i) kc[rd % L::KR][i] = ckp[min(tid + (rd + L::KR) * kNT, last_row) * BITS + i];
-                }
+                matrix_logits<BITS>(kc[rd % L::KR], a0, a1, lx[rd]);
+                if (rd + L::KR < REGL) request_k(rd + L::KR);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) { lo = fminf(lo, lx[rd][j]); hi = fmaxf(hi, lx[rd][j]); }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (!MINMAX_ONLY && rd < kVF - kVEarly) request_v(kVEarly + rd);   // the rest of the first packed V rows
+            if (!MINMAX_ONLY && rd < kVF - kVEarly) request_v(kVEarly + rd, kVEarly + rd);   // the rest of the first packed V rows
         }
         phase_priority(std::integral_constant<int, 2>{});
         if constexpr (VTOK && !MINMAX_ONLY) {   // they arrive during the min / max and the calibration
@@ -745,42 +778,33 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             __hip_atomic_fetch_max(redi + HPB + hl, khi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
         __syncthreads();
-#pragma unroll
-        for (int h = 0; h < HPB; ++h) {
-            mn[h] = -key_float(__builtin_amdgcn_readfirstlane(redi[h]));
-            mx[h] = key_float(__builtin_amdgcn_readfirstlane(redi[HPB + h]));
-        }
+        mn = -key_float(redi[hl]);
+        mx = key_float(redi[HPB + hl]);
     }
 
     CQ_PHASE(4);   // block min / max
+    const bool speaks = wv == 0 && (lane & 15) == 0 && (lane >> 4) < nh;   // one lane per real head, for what a workgroup writes per head
     if constexpr (MINMAX_ONLY) {
-#pragma unroll
-        for (int h = 0; h < HPB; ++h) {
-            if (n > 0 && tid == h && h < nh) {
-                float* o = g.mm + ((static_cast<int64_t>(b) * g.Hq + hq0 + h) * g.nsplit + split) * 2;
-                o[0] = mn[h];
-                o[1] = mx[h];
-            }
+        if (n > 0 && speaks) {
+            float* o = g.mm + ((static_cast<int64_t>(b) * g.Hq + hq0 + hl) * g.nsplit + split) * 2;
+            o[0] = mn;
+            o[1] = mx;
         }
         if (split == 0 && tid == 0) g.cnt[unit] = 0;   // the main launch counts the unit's partials from 0
         return;
     } else {
-        float m_img[HPB];
-#pragma unroll
-        for (int h = 0; h < HPB; ++h) m_img[h] = -INFINITY;
+        float m_img = -INFINITY;   // of the lane's head
         float o_img = 0.f;  // thread (h, d) = (tid / kD, tid % kD) for tid < HPB*kD
 
         if constexpr (CHUNKED) {
             // One launch: this chunk's min / max go out now (write-through stores, waited for, then the arrival
             // count); the other chunks' are collected further down.
-            if (g.fused && has_img && tid == 0) {
-                unsigned long long* o = g.rec + ((unit * HPB) * g.nsplit + split) * 2;
+            // (padding heads repeat the last real one: every head of the unit's layout has its records)
+            if (g.fused && has_img && wv == 0 && (lane & 15) == 0 && (lane >> 4) < HPB) {
+                unsigned long long* o = g.rec + ((unit * HPB + hl) * g.nsplit + split) * 2;
                 const unsigned long long tag = static_cast<unsigned long long>(g.epoch) << 32;
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) {
-                    __hip_atomic_store(o + h * g.nsplit * 2, tag | __float_as_uint(mn[h]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(o + h * g.nsplit * 2 + 1, tag | __float_as_uint(mx[h]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
+                __hip_atomic_store(o, tag | __float_as_uint(mn), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(o + 1, tag | __float_as_uint(mx), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
 
@@ -830,8 +854,8 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                         if (*last) clear_handover<HPB, kNT>(g, unit, tid);
                         return;
                     }
-#pragma unroll
-                    for (int h = 0; h < HPB; ++h) { mn[h] = -fold[h]; mx[h] = fold[HPB + h]; }
+                    mn = -fold[hl];
+                    mx = fold[HPB + hl];
                 } else {
                 // one fold for both: max of (-min, max) over the chunks
                 float mm2[2 * HPB];
@@ -848,34 +872,32 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     }
                 }
                 wave_reduce_n<2 * HPB>(mm2, OpMax(), -INFINITY);
+                mn = -mm2[0];
+                mx = mm2[HPB];
 #pragma unroll
-                for (int h = 0; h < HPB; ++h) { mn[h] = -mm2[h]; mx[h] = mm2[HPB + h]; }
+                for (int h = 1; h < HPB; ++h) { mn = hl == h ? -mm2[h] : mn; mx = hl == h ? mm2[HPB + h] : mx; }
                 }
             }
-            float slope[HPB], tmin[HPB];
-#pragma unroll
-            for (int h = 0; h < HPB; ++h) {
-                if (g.calib) {
-                    const float tgt_max = mx[h] + g.off_max;
-                    tmin[h] = mn[h] + g.off_min;
-                    // (the hardware reciprocal, one unit in the last place: far inside the tolerance of the map)
-                    slope[h] = (tgt_max - tmin[h]) * __builtin_amdgcn_rcpf(mx[h] - mn[h] + 1e-8f);
-                } else {
-                    tmin[h] = mn[h];
-                    slope[h] = 1.0f;
-                }
+            // Up to here minima and maxima are in grid steps before the zero-point, as the logits stay; the calibration takes
+            // the logits themselves (all chunks of a unit have the same step and zero-point sum: the same query and statistics).
+            // Every lane works out its own head's.
+            const float step = qsz[2 * hl], zs = qsz[2 * hl + 1];
+            const float real_mn = __builtin_fmaf(mn, step, -zs), real_mx = __builtin_fmaf(mx, step, -zs);
+            float slope = 1.0f, tmin = real_mn;
+            if (g.calib) {
+                const float tgt_max = real_mx + g.off_max;
+                tmin = real_mn + g.off_min;
+                // (the hardware reciprocal, one unit in the last place: far inside the tolerance of the map)
+                slope = (tgt_max - tmin) * __builtin_amdgcn_rcpf(real_mx - real_mn + 1e-8f);
             }
-            // a value of the lane's head
-            auto mine = [&](const float* v) {
-                auto uni = [](float f) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f))); };
-                float r = uni(v[0]);   // (wave-uniform: scalar operands, and no array that would be indexed by the lane)
-#pragma unroll
-                for (int h = 1; h < HPB; ++h) r = hl == h ? uni(v[h]) : r;
-                return r;
-            };
+            // e = exp(x - M) with x = (w - mn) * slope + tmin, as exp2((w - peak) * ea): `peak` is the logit whose x is M, so no
+            // weight is above 1 - which the fixed-point weights rely on - however large the logits are or far from 0 they lie
+            // (a constant that takes M back is off by M's own rounding), and a degenerate logit range, whose slope is
+            // ~1e8, meets the exact zero of (w - peak).
+            float eal, pkl;
             if (EXTRAS && g.mask) {
                 const float* mk = g.mask + b * g.mask_sb + g.S + t0;
-                const float mnl = mine(mn), sl = mine(slope), tl = mine(tmin);
+                const float sl = slope * step;
                 float top = -INFINITY;
 #pragma unroll
                 for (int rd = 0; rd < REGL; ++rd) {
@@ -883,7 +905,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             const float mv = mk[min(wt0 + rd * kNT + 16 * j + (lane & 15), n - 1)];
-                            lx[rd][j] = (lx[rd][j] - mnl) * sl + tl + mv;
+                            lx[rd][j] = (lx[rd][j] - mn) * sl + tmin + mv;
                             top = fmaxf(top, lx[rd][j]);
                         }
                     }
@@ -893,31 +915,20 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 if ((lane & 15) == 0 && (lane >> 4) < HPB)
                     __hip_atomic_fetch_max(redi + hl, kt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 __syncthreads();
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) {
-                    m_img[h] = key_float(__builtin_amdgcn_readfirstlane(redi[h]));
-                    slope[h] = 1.0f;
-                }
+                m_img = key_float(redi[hl]);
+                eal = kLog2e;
+                pkl = m_img;
+                if (m_img == -INFINITY) { eal = 1.f; pkl = INFINITY; }   // every position masked out
             } else {
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) m_img[h] = fmaxf(tmin[h], (mx[h] - mn[h]) * slope[h] + tmin[h]);
+                m_img = fmaxf(tmin, (real_mx - real_mn) * slope + tmin);
+                eal = slope * kLog2e * step;
+                pkl = slope < 0.f ? mn : mx;
+                if (m_img == -INFINITY) { eal = 1.f; pkl = INFINITY; }
             }
-            // e = exp(x - M) with x = (w - mn) * slope + tmin, as exp2((w - peak) * ea): `peak` is the logit whose x is M, so no
-            // weight is above 1 - which the fixed-point weights rely on - however large the logits are or far from 0 they lie
-            // (a constant that takes M back is off by M's own rounding), and a degenerate logit range, whose slope is
-            // ~1e8, meets the exact zero of (w - peak).
-            float ea[HPB], peak[HPB];
-#pragma unroll
-            for (int h = 0; h < HPB; ++h) {
-                const bool dead = (m_img[h] == -INFINITY);   // every position masked out
-                ea[h] = dead ? 1.f : slope[h] * kLog2e;
-                peak[h] = dead ? INFINITY : (EXTRAS && g.mask) ? m_img[h] : slope[h] < 0.f ? mn[h] : mx[h];
-            }
-            const float eal = mine(ea), pkl = mine(peak);
             float lsum = 0.f;
-            I4 acc[8];
+            I4 acc[BITS == 2 && !VTOK ? 9 : 8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) acc[i] = I4{0, 0, 0, 0};
+            for (int i = 0; i < (BITS == 2 && !VTOK ? 9 : 8); ++i) acc[i] = I4{0, 0, 0, 0};
             unsigned char* et = regA + wv * L::MXT;
             constexpr int KV = kVF / BITS;   // rounds of packed V rows in flight
             U2 ssc[VTOK ? KV : 1], smin[VTOK ? KV : 1];   // VTOK: the statistics of the lane's own tokens, as many rounds ahead
@@ -979,8 +990,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     __builtin_amdgcn_sched_barrier(0);   // one round at a time: interleaved, they do not fit the registers
                     if (rd + KV < REGL) {
 #pragma unroll
-                        for (int i = 0; i < BITS; ++i)
-                            vc[(rd % KV) * BITS + i] = cvp4[min((tid + (rd + KV) * kNT) * BITS + i, last_u)];
+                        for (int i = 0; i < BITS; ++i) request_v((rd % KV) * BITS + i, (rd + KV) * BITS + i);
                         if constexpr (VTOK) {
                             ssc[rd % KV] = vsp[min(tid + (rd + KV) * kNT, n - 1)];
                             smin[rd % KV] = vmp[min(tid + (rd + KV) * kNT, n - 1)];
@@ -1141,12 +1151,9 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             }
         }
 
-#pragma unroll
-        for (int h = 0; h < HPB; ++h) {
-            if (tid == h) {
-                stat[3 * HPB + h] = m_img[h];
-                if (n == 0) stat[4 * HPB + h] = 0.f;
-            }
+        if (speaks) {
+            stat[3 * HPB + hl] = m_img;
+            if (n == 0) stat[4 * HPB + hl] = 0.f;
         }
         CQ_PHASE(9);   // residual window
         // ---- phase 7: merge / write ---------------------------------------------------------
