@@ -86,7 +86,7 @@ static void plan_for(const cq_decode_args* a, Plan* p, int hpb, int nh, int nt, 
     const size_t rows = static_cast<size_t>(a->B) * a->Hq;
     p->ws_mm = nsplit > 1 ? ((rows * nsplit * 2 * sizeof(float) + 255) / 256 * 256) : 0;
     p->ws_part = nsplit > 1 ? (rows * p->nx * (kD + 2) * sizeof(float) + 255) / 256 * 256 : 0;
-    // counters: [unit] partials written (4 or 8 bytes), then the min / max records of the single-launch step
+    // counters: [unit] partials written, then the min / max records of the single-launch step
     p->ws_cnt = nsplit > 1 ? (static_cast<size_t>(units) * sizeof(unsigned long long) + 255) / 256 * 256 +
                                  static_cast<size_t>(units) * hpb * nsplit * 16 : 0;
     p->fused = false;
@@ -291,7 +291,8 @@ static int decode_entry(const cq_decode_args* a, void* workspace, size_t workspa
         const int G = a->Hq / a->Hkv;
         const size_t units = static_cast<size_t>(a->B) * a->Hkv * ngroups(G, p.nh);
         char* c0 = reinterpret_cast<char*>(g.cnt);
-        g.done64 = reinterpret_cast<unsigned long long*>(c0);
+        g.done = reinterpret_cast<unsigned long long*>(workspace);
+        g.done_res = reinterpret_cast<unsigned long long*>(c0);
         g.rec = reinterpret_cast<unsigned long long*>(c0 + (units * sizeof(unsigned long long) + 255) / 256 * 256);
     }
 #ifdef CQ_PHASE_STOPS

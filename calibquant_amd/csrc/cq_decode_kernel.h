@@ -79,17 +79,20 @@ struct DecodeGeom {
     const int32_t* r_dev;   // optional: residual row count read at run time (R is then the capacity)
     float* mm;    // [B][Hq][nsplit][2] chunk logit min / max
     float* part;  // [B][Hq][nx][kD + 2] partials (m, l, acc)
-    int* cnt;     // chunked launch: [unit] count of the unit's chunks (+ residual unit) that have written their
-                  // partial; the one that finds all the others done merges them
+    int* cnt;     // chunked step in two launches: [unit] count of the unit's chunks (+ residual unit) that have written
+                  // their partial; the one that finds all the others done merges them
     // Chunked step in ONE launch (every chunk's workgroup resident at once): the chunks of a unit exchange their
     // logit min / max inside the launch.  rec: [unit][head][chunk][2] 64-bit records, a float (min, then max)
     // in the lower half and the call's epoch in the upper half - a record is valid by itself, so a chunk
     // publishes with plain write-through stores and waits for nothing, and the others poll the records
-    // (whatever an earlier call or an uninitialised workspace left there has another epoch).  done64: [unit]
-    // partials written, tagged with the epoch the same way.  status: host-visible word that a workgroup sets
+    // (whatever an earlier call or an uninitialised workspace left there has another epoch).  done: [unit][chunk] words of
+    // the same kind (in the place of the two-launch form's min / max), and done_res [unit] for the window's workgroup (in
+    // that of its counters), set to the epoch's tag when the workgroup's partial is written: the unit's first workgroup
+    // waits for them and merges.  status: host-visible word that a workgroup sets
     // when it gives up waiting (spin_limit polls); NULL: nowhere to report.
     unsigned long long* rec;
-    unsigned long long* done64;
+    unsigned long long* done;
+    unsigned long long* done_res;
     int* status;
     uint32_t epoch;
     int fused;
@@ -194,38 +197,38 @@ __device__ __forceinline__ void publish(float* p, float v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// One more arrival at an epoch-tagged counter; returns the arrivals of this epoch including this one.
-// Measured on this device: an atomic read-modify-write is executed at the memory side whatever scope it names
-// (about 2 us a round trip, those on one address one after the other), so such counters are for counting once
-// per workgroup, never for polling.
-// peek64: the current value of a 64-bit word as the memory side holds it, a compare-and-swap of 0 for 0.  (Not a
-// read-modify-write that changes nothing, such as OR 0: the compiler turns those into plain loads, which a
-// compute unit's own cache may answer with what it read earlier.)
-template <int SCOPE>
-__device__ __forceinline__ unsigned long long peek64(unsigned long long* c) {
-    unsigned long long v = 0ull;
-    __hip_atomic_compare_exchange_strong(c, &v, 0ull, __ATOMIC_RELAXED, __ATOMIC_RELAXED, SCOPE);
-    return v;
+// The partials of a unit are announced with plain write-through stores, not counted: an atomic read-modify-write is executed
+// at the memory side whatever scope it names (about 2 us a round trip, those on one address one after the other; with
+// a compare-and-swap counter that a unit's workgroups retried on, us, counter -> words: 8 chunks a unit (8 x 32 768) 27.5 ->
+// 25.0, 16 (4 x 16 384 + 200, 2 bits) 40.4 -> 25.2, 32 (1 x 32 768 + 100) 68.6 -> 20.7).  The first wave of the
+// unit's first workgroup polls the others' words, a bounded number of times of its own (every other workgroup ends
+// without waiting for this one, so the bound only matters where they are not all resident together).
+constexpr int kDonePolls = 1 << 18;
+__device__ __forceinline__ unsigned long long* done_word(const DecodeGeom& g, int64_t unit, int split) {
+    return split < g.nsplit ? g.done + unit * g.nsplit + split : g.done_res + unit;
 }
-
-template <int SCOPE>
-__device__ __forceinline__ uint32_t arrive(unsigned long long* c, uint32_t epoch) {
-    unsigned long long old = peek64<SCOPE>(c);
-    for (;;) {   // every failed exchange is another workgroup's success: at most as many rounds as workgroups
-        const unsigned long long want = (static_cast<uint32_t>(old >> 32) == epoch)
-                                            ? old + 1 : ((static_cast<unsigned long long>(epoch) << 32) | 1u);
-        if (__hip_atomic_compare_exchange_strong(c, &old, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED, SCOPE))
-            return static_cast<uint32_t>(want);
+__device__ __forceinline__ void announce(const DecodeGeom& g, int64_t unit, int split) {
+    __hip_atomic_store(done_word(g, unit, split), static_cast<unsigned long long>(g.epoch) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool others_done(const DecodeGeom& g, int64_t unit, int lane) {
+    bool ok = false;
+    for (int it = 0; it < kDonePolls && !ok; ++it) {
+        bool all = true;
+        for (int s = 1 + lane; s < g.nx; s += 64)
+            all = all && static_cast<uint32_t>(__hip_atomic_load(done_word(g, unit, s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32) == g.epoch;
+        ok = __builtin_amdgcn_ballot_w64(!all) == 0;
+        if (!ok) __builtin_amdgcn_s_sleep(1);
     }
+    return ok;
 }
 
-// The single-launch chunked step's records and arrival counter of one unit back to empty: by the unit's last
-// workgroup, once every other one is past both.
+// The single-launch chunked step's hand-over words of one unit back to empty: by the unit's first workgroup, once every
+// other one is past them (a recorded launch comes back with the same epoch).
 template <int HPB, int NT>
 __device__ __forceinline__ void clear_handover(const DecodeGeom& g, int64_t unit, int tid) {
     for (int i = tid; i < HPB * g.nsplit * 2; i += NT)
         __hip_atomic_store(g.rec + unit * HPB * g.nsplit * 2 + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (tid == 0) __hip_atomic_store(g.done64 + unit, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = tid; i <= g.nsplit; i += NT) __hip_atomic_store(done_word(g, unit, i), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---- the step on the matrix cores --------------------------------------------------------------
@@ -845,11 +848,18 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     }
                     __syncthreads();
                     if (!*flag) {
-                        // Given up: no result from this workgroup, but it is still counted, so that the unit's
-                        // last workgroup - this one or another - leaves the records and the counter empty and a
-                        // replay of this very launch (same epoch) does not take this launch's records for its own.
+                        // Given up: no result from this workgroup, but it still announces itself, so that the unit's
+                        // first workgroup leaves the hand-over words empty and a replay of this very launch (same epoch)
+                        // does not take this launch's records for its own.
+                        if (split != 0) {
+                            if (tid == 0) announce(g, unit, split);
+                            return;
+                        }
                         int* last = reinterpret_cast<int*>(red);
-                        if (tid == 0) *last = arrive<__HIP_MEMORY_SCOPE_AGENT>(g.done64 + unit, g.epoch) == static_cast<uint32_t>(g.nx);
+                        if (wv == 0) {
+                            const bool ok = others_done(g, unit, lane);
+                            if (lane == 0) *last = ok ? 1 : 0;
+                        }
                         __syncthreads();
                         if (*last) clear_handover<HPB, kNT>(g, unit, tid);
                         return;
@@ -1178,18 +1188,30 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             }
         }
         if constexpr (CHUNKED) {
-            // The unit's chunks (and its residual unit) each leave an (m, l, acc) partial; the workgroup that
-            // finds all the others' already counted combines them.  The partials are device-scope atomic stores
+            // The unit's chunks (and its residual unit) each leave an (m, l, acc) partial.  Two launches: the workgroup that
+            // finds all the others' already counted combines them; one launch: the first chunk's, when the others have
+            // announced theirs.  The partials are device-scope atomic stores
             // (written through to the level all compute units share, so no cache has to be written back as a
             // whole): every thread waits for its own stores to complete, the barrier collects the workgroup,
-            // then one thread counts.
+            // then one thread counts or announces.
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
             int* last = reinterpret_cast<int*>(red);
-            if (tid == 0) {
-                if (g.fused) *last = arrive<__HIP_MEMORY_SCOPE_AGENT>(g.done64 + unit, g.epoch) == static_cast<uint32_t>(g.nx);
-                else *last = __hip_atomic_fetch_add(g.cnt + unit, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.nx - 1;
+            if (g.fused) {
+                if (split != 0) {
+                    if (tid == 0) announce(g, unit, split);
+                    return;
+                }
+                if (wv == 0) {
+                    const bool ok = others_done(g, unit, lane);
+                    if (lane == 0) {
+                        *last = ok ? 1 : 0;
+                        if (!ok && g.status) __hip_atomic_store(g.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    }
+                }
+            } else if (tid == 0) {
+                *last = __hip_atomic_fetch_add(g.cnt + unit, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.nx - 1;
             }
             __syncthreads();
             if (*last) {
@@ -1224,8 +1246,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     }
                     store_elem<DT>(g.out, row * kD + d, num / den);
                 }
-                // every other workgroup of the unit is past both counters: leave them empty for a replay of this
-                // very launch (a recorded step comes back with the same epoch)
+                // every other workgroup of the unit is past the hand-over words
                 if (g.fused) clear_handover<HPB, kNT>(g, unit, tid);
             }
         }
