@@ -173,7 +173,8 @@ static DecodeGeom unit_geometry(const DecodeGeom& g, int nh, int nt) {
 
 template <typename DT>
 static int dispatch(const DecodeGeom& g, const Plan& p, int bits, bool vtok, hipStream_t st) {
-    const DecodeGeom gm = unit_geometry(g, p.nh, p.nt);
+    DecodeGeom gm = unit_geometry(g, p.nh, p.nt);
+    gm.stream = launch_streams(bits, vtok, p.hpb, p.nt, ngroups(gm.G, p.nh), g.nsplit, static_cast<int64_t>(g.B) * g.Hkv * g.T);
     const unsigned units = static_cast<unsigned>(g.B) * g.Hkv * ngroups(gm.G, p.nh);
 #ifdef CQ_PHASE_STOPS
     if (vtok || !std::is_same<DT, BF16>::value || bits != 1 || p.hpb != 4 || p.nh != 4 || p.nt != 512 || g.nsplit > 1)

@@ -96,6 +96,7 @@ struct DecodeGeom {
     int* status;
     uint32_t epoch;
     int fused;
+    int stream;   // launch_streams()
     int spin_limit;
 #ifdef CQ_PHASE_STOPS
     int stop;     // phase boundary at which the launch ends (-1: runs to the end)
@@ -152,6 +153,17 @@ constexpr int plan_chunk(int bits, bool vtok, int hpb) {
 }
 constexpr int kPlanLong = 10048;                     // four heads at 1 bit, where that saves the chunks
 constexpr int kPlanPair4 = 4096, kPlanPair2 = 4736;  // 512 threads: four heads, two heads (1 bit)
+
+// Launches whose packed rows (and per-token statistics) are more than half of the 256 MB memory-side cache, each read by one
+// unit: nothing of them would be found there again, and non-temporal loads stream faster.  us, ordinary / non-temporal:
+// batch 256 x 3 328 (218 MB) 57.3 / 53.6, batch 64 x 3 328 at 2 bits (109 MB) 27.6 / 27.7, with per-token values (109 MB)
+// 36.9 / 35.3; below, or where two units share the rows: 8 x 32 768 (67 MB) 26.7 / 28.0, 16 x 9 984 with two units per
+// kv head 20.5 / 21.9.  Instantiated for the forms that such launches take (four heads per unit in 512 threads; per-token
+// values with the most heads a unit has).
+constexpr bool stream_form(int bits, bool vtok, int hpb, int nt) { return vtok ? hpb == (bits == 1 ? 4 : 2) : hpb == 4 && nt == 512; }
+inline bool launch_streams(int bits, bool vtok, int hpb, int nt, int groups, int nsplit, int64_t tokens) {   // tokens: over all (batch, kv head) pairs
+    return stream_form(bits, vtok, hpb, nt) && groups == 1 && nsplit == 1 && tokens * (32 * bits + (vtok ? 16 : 0)) >= (static_cast<int64_t>(100) << 20);
+}
 
 // What a launch of units of hpb heads in nt threads runs with: the rounds of logits its instantiation keeps in
 // registers for chunks of at most `chunk` tokens, and its dynamic LDS.  Launches pick by the first and check themselves
@@ -526,11 +538,12 @@ template <int BITS> __device__ __forceinline__ void matrix_fold_token(const I4* 
 // none of their code.  EXTRAS: an additive mask or a residual row count read from device memory may be present; a
 // call with neither runs an instantiation without their code (the kernel sits at the register limit of its occupancy,
 // and code that never runs still costs registers).
+// STREAM: the packed rows are read with non-temporal loads (see launch_streams()).
 // NH: query heads a unit serves, at most HPB.  Operands and partials are laid out HPB heads wide either way; with
 // NH = 3 the fourth head's rows are padding - six query heads per kv-head (InternLM2-20B) make two exact units of
 // three instead of two units of four that carry two padding heads between them.
 template <int BITS, int HPB, typename DT, bool MINMAX_ONLY, bool VTOK = false, int NT = 1024, int REGL = 0,
-          bool CHUNKED = MINMAX_ONLY, bool EXTRAS = !MINMAX_ONLY, int NH = HPB>
+          bool CHUNKED = MINMAX_ONLY, bool EXTRAS = !MINMAX_ONLY, int NH = HPB, bool STREAM = false>
 // (four waves per SIMD - at most 128 VGPRs - for either workgroup size: two 512-thread workgroups per compute
 // unit are only resident together within that)
 __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
@@ -674,9 +687,9 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     };
     uint4 kc[L::KR][BITS];
     auto request_k = [&](int r) {
-        const uint4* p = reinterpret_cast<const uint4*>(row_at(ckp, r));
+        const U4* p = reinterpret_cast<const U4*>(row_at(ckp, r));
 #pragma unroll
-        for (int i = 0; i < BITS; ++i) kc[r % L::KR][i] = p[i];
+        for (int i = 0; i < BITS; ++i) kc[r % L::KR][i] = __builtin_bit_cast(uint4, STREAM ? __builtin_nontemporal_load(p + i) : p[i]);
     };
 #pragma unroll
     for (int r = 0; r < L::KR; ++r) request_k(r);
@@ -735,7 +748,8 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     constexpr int kVF = VTOK ? (REGL > 4 ? 1 : 2) * BITS : kMatrixV;   // 16-byte pieces of packed V rows in flight per thread
     U4 vc[kVF];
     auto request_v = [&](int slot, int piece) {   // piece: round * BITS + 16-byte piece of the row
-        vc[slot] = reinterpret_cast<const U4*>(row_at(cvp, piece / BITS))[piece % BITS];
+        const U4* p = reinterpret_cast<const U4*>(row_at(cvp, piece / BITS)) + piece % BITS;
+        vc[slot] = STREAM ? __builtin_nontemporal_load(p) : *p;
     };
     constexpr int kVEarly = VTOK ? BITS : kMatrixE;
     if constexpr (!MINMAX_ONLY) {

@@ -21,6 +21,14 @@ static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st
             CQ_LAUNCH_CHECK();
         }
     }
+    if constexpr (!CHUNKED && stream_form(BITS, VTOK, HPB, NT)) {
+        if (g.stream) {
+            hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, false, VTOK, NT, REGL, CHUNKED, EXTRAS, NH, true>), dim3(units * g.nx),
+                               dim3(NT), lds, st, g);
+            CQ_LAUNCH_CHECK();
+            return CQ_OK;
+        }
+    }
     hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, false, VTOK, NT, REGL, CHUNKED, EXTRAS, NH>), dim3(units * g.nx),
                        dim3(NT), lds, st, g);
     CQ_LAUNCH_CHECK();

@@ -2,6 +2,7 @@
 workgroup, and the fixed-point operands' range."""
 import numpy as np
 import pytest
+import torch
 
 from oracle import cq_oracle as O
 from tests.test_gpu_decode import _oracle, _run
@@ -203,3 +204,36 @@ def test_token_values_large_scale_of_a_token_without_weight(ops, dtype, far, bit
     for b in range(2):
         for h in range(32):
             _close(got[b, h], want[b, h], 2.0 ** -11 if dtype == "fp16" else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("bits, vals, G, option", [(1, "channel", 4, "none"), (1, "channel", 3, "device-rows"), (2, "channel", 4, "mask"),
+                                                   (1, "token", 4, "none"), (2, "token", 2, "device-rows")])
+def test_decode_attn_streamed_rows_equal_a_small_batch(ops, bits, vals, G, option):
+    """Launches that read more than half of the memory-side cache take their packed rows with non-temporal loads: the
+    same arithmetic, so the first rows of such a batch equal a batch of their own in units of the same form, bit for
+    bit."""
+    per = 32 * bits + (16 if vals == "token" else 0)
+    H, T, R, S = 8, 1800, 20, 3
+    B = (100 << 20) // (per * H * T) + 2
+    g = torch.Generator(device="cuda").manual_seed(B)
+    k = torch.randn((B, T, H, 128), generator=g, device="cuda").to(torch.bfloat16)
+    v = torch.randn((B, T, H, 128), generator=g, device="cuda").to(torch.bfloat16)
+    ck, sk, zk = ops.quantize_pack(k, bits, 0.5)
+    cv, sv, zv = ops.quantize_pack_token(v, bits) if vals == "token" else ops.quantize_pack(v, bits, 0.5)
+    del k, v
+    q = torch.randn((B, H * G, 128), generator=g, device="cuda").to(torch.bfloat16)
+    kr, vr = (torch.randn((B, H, R, 128), generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    mask = torch.where(torch.rand((B, T + R), generator=g, device="cuda") < 0.1, -1e4, 0.0) if option == "mask" else None
+
+    def run(n):
+        r_dev = torch.full((1,), R - 1, dtype=torch.int32, device="cuda") if option == "device-rows" else None
+        call = ops.DecodeCall(q[:n].contiguous(), ck[:n], cv[:n], sk[:n], zk[:n], sv[:n], zv[:n], kr[:n], vr[:n], sprompt_len=S, bits=bits,
+                              mask=None if mask is None else mask[:n].contiguous(), r_dev=r_dev, v_mode=vals)
+        out = call.run().clone()
+        torch.cuda.synchronize()
+        p = call.plan()
+        return out, (p["threads"], p["heads_per_unit"], p["chunks"])
+    big, form = run(B)
+    small, form2 = run(40)
+    assert form == form2 and form[2] == 1
+    assert torch.equal(big[:40], small)
