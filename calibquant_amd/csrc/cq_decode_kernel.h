@@ -1038,10 +1038,11 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     for (int gi = 0; gi < 4; ++gi) lpart[(wv * kParts + 1 + gi) * HPB + hl] = cm[gi];
                 }
             }
-            __syncthreads();
-            float* redv = reinterpret_cast<float*>(regA);   // [wave][head][channel]
+            // a wave's sums, [head][channel], take the place of its own tile: nobody else reads or writes there
+            static_assert(HPB * kD * 4 <= L::MXT, "a wave's sums fit its tile");
+            const float* redv = reinterpret_cast<const float*>(regA);
             if ((lane >> 4) < HPB) {
-                float* o = redv + (wv * HPB + hl) * kD;
+                float* o = reinterpret_cast<float*>(et) + hl * kD;
                 if constexpr (VTOK) matrix_fold_token<BITS>(acc, vpw, o, lane & 15);
                 else matrix_fold<BITS>(acc, o, lane & 15);
             }
@@ -1050,7 +1051,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 const int h = tid / kD, d = tid % kD;
                 float a = 0.f, lh = 0.f;
 #pragma unroll
-                for (int w = 0; w < kNW; ++w) { a += redv[(w * HPB + h) * kD + d]; lh += lpart[w * kParts * HPB + h]; }
+                for (int w = 0; w < kNW; ++w) { a += redv[w * (L::MXT / 4) + h * kD + d]; lh += lpart[w * kParts * HPB + h]; }
                 if constexpr (VTOK) {
                     float cmin = 0.f;
 #pragma unroll
@@ -1061,7 +1062,8 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 }
                 if (d == 0) stat[4 * HPB + h] = lh;
             }
-            __syncthreads();
+            // (no barrier: what was read here - the sums, the waves' sums of e - is next written behind barriers of the
+            // window, and `stat` is read behind the one of the merge)
         }
 
         if (n == 0) load_res_k(0, rk);
