@@ -1161,7 +1161,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     }
                 }
             }
-            __syncthreads();
+            // (regA was last read by the packed part's sum, behind which lie the tiles' barriers)
             float* red2 = reinterpret_cast<float*>(regA);  // [wave][head][kD]: the fold reads consecutive words
 #pragma unroll
             for (int h = 0; h < HPB; ++h) {
