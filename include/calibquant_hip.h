@@ -67,16 +67,18 @@ int cq_quantize_pack(const void* x, int dtype, int B, int T, int H, int D,
                      uint8_t* codes, void* scale, void* zero,
                      void* workspace, size_t workspace_bytes, cq_stream_t stream);
 
-/* With D = 128 and more than 3 328 tokens (what one workgroup's registers hold of a slice of 32 channels),
- * cq_quantize_pack still reads x once: two to thirty-two workgroups of its persistent launch share a slice along
- * the token axis and exchange the channels' minima and maxima through the workspace inside the launch.  The wait
+/* With D = 128, cq_quantize_pack reads x once: a workgroup keeps up to 832 token rows of a (batch, head) pair in registers
+ * (up to 3 328 rows of a quarter of the channels where there is little to do), and a longer token axis is shared by up to
+ * 128 workgroups of the launch, which exchange the channels' minima and maxima through the workspace inside it.  The wait
  * for the other parts is bounded: after `polls` polls (about a microsecond each; default 262 144) a workgroup goes
  * on with what it has and sets a word of pinned host memory (64 bytes per device, allocated at the first such
  * call outside a stream capture and kept until the process ends).  The next such call on that device then returns
  * CQ_ERR_LAUNCH once (the previous call's output is not valid) and the process goes on with three launches per
- * tensor (partial min / max, statistics, emit; x read twice).  This call sets the bound (polls >= 0; it also
- * re-enables the single launch after a give-up) and returns the previous one; polls < 0 only queries.  No
- * counterpart in the reference, whose quant() is a chain of whole-tensor torch ops (calibquant.py:24-42). */
+ * tensor (partial min / max, statistics, emit; x read twice).  Three launches are also what is recorded while a stream
+ * is captured before that word exists.  A recorded exchange empties its records first, so it may be replayed.  This call
+ * sets the bound (polls >= 0; it also re-enables the single launch after a give-up) and returns the previous one;
+ * polls < 0 only queries.  No counterpart in the reference, whose quant() is a chain of whole-tensor torch ops
+ * (calibquant.py:24-42). */
 int cq_quantize_pack_wait_polls(int polls);
 
 /* ------------------------------------------------------------------------
@@ -95,7 +97,8 @@ int cq_quantize_pack_wait_polls(int polls);
  * t*pos_stride_t] (clamped to the table), or NULL for positions pos0 + t.
  * x_rot: (B, T, H, 128) through element strides (multiples of 8).
  * codes / scale / zero / workspace as for cq_quantize_pack; the results are
- * bit-identical to cq_quantize_pack on the rotated tensor.
+ * bit-identical to cq_quantize_pack on the rotated tensor.  (Where the one launch is not available - see
+ * cq_quantize_pack_wait_polls - the rows are rotated first and quantised by three launches.)
  * Shapes outside the one-pass path (T > 3 328, D != 128) return
  * CQ_ERR_UNSUPPORTED: rotate with cq_rope_rows, then cq_quantize_pack. */
 int cq_rope_quantize_pack(const void* x, int dtype, int B, int T, int H, int D,
