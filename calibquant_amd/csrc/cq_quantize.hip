@@ -1625,9 +1625,10 @@ int cq_quantize_pack_token(const void* x, int dtype, int B, int T, int H, int D,
     g.nchunk = 1; g.chunk = T;
     g.dT.set(static_cast<uint32_t>(T));
     g.dH.set(static_cast<uint32_t>(H));
-    // A lane per group from 24 K rows on: us, four lanes a group / one, 1 x 1 024 tokens x 8 heads 2.4 / 3.1, 2 x 1 600 3.5 / 3.6,
-    // 4 x 3 328 7.7 / 7.1, 64 x 256 9.5 / 8.3, 64 x 3 328 strided 109 / 92.
-    const bool grouped = static_cast<int64_t>(B) * T * H >= 24 * 1024;
+    // A lane per group from 56 K rows on, where it has enough workgroups to fill the chip: us, four lanes a group / one (bf16, 1 bit),
+    // 24 x 150 tokens x 8 heads 3.8 / 4.3, 3 x 1 700 4.3 / 4.6, 2 x 3 328 5.0 / 4.9 (2 bits 5.9 / 6.0, fp16 5.0 / 5.3), 4 x 2 000 5.8 / 5.3 (2 bits
+    // 6.8 / 6.2, fp16 5.9 / 5.6), 4 x 3 328 8.9 / 7.2, 1 x 32 768 17.8 / 14.6, 64 x 3 328 strided 109 / 92.
+    const bool grouped = static_cast<int64_t>(B) * T * H >= 56 * 1024;
     const int64_t ntb = (static_cast<int64_t>(T) + cq::token_rows(grouped) - 1) / cq::token_rows(grouped);
     g.dTB.set(static_cast<uint32_t>(ntb));
     const int64_t nblk = static_cast<int64_t>(B) * H * ntb;

@@ -32,9 +32,9 @@ def test_quantize_pack_token_is_bit_exact(bits, dtype):
     assert same_bits(to_np(scale), s_ref) and same_bits(to_np(mins), m_ref)
 
 
-# Four lanes a group below 24 576 rows, one lane a group from there on: either side of the line, partial passes of 16 and 64
+# Four lanes a group below 57 344 rows, one lane a group from there on: either side of the line, partial passes of 16 and 64
 # tokens, a single token.
-TOKEN_SHAPES = [(1, 1, 1), (1, 17, 5), (2, 3071, 4), (3, 3073, 8), (24577, 1, 1), (6, 4127, 1)]
+TOKEN_SHAPES = [(1, 1, 1), (1, 17, 5), (2, 3071, 4), (3, 3073, 8), (24577, 1, 1), (6, 4127, 1), (2, 7167, 4), (57345, 1, 1), (14, 4127, 1)]
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
