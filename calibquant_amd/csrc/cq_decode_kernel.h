@@ -27,6 +27,7 @@
 // fit the device at once, one launch does both: the chunks exchange their min / max inside it.
 #pragma once
 #include "cq_common.h"
+#include "cq_digits.h"
 
 // The kernels below lean on behaviour of this architecture family that the HIP memory model does not
 // promise (see the in-launch merge of the chunked step) and on its LDS size, DPP controls and
@@ -253,14 +254,15 @@ __device__ __forceinline__ void clear_handover(const DecodeGeom& g, int64_t unit
 // closing fold (sums) takes back.
 // Measured, us per step in turn on one box, look-up form before and this one: batch 64 x 3 328 + 128, 1 bit 28.5 -> 19.7,
 // 2 bits 48.9 -> 27.5; batch 256 x 3 328 99.7 -> 57; 16 x 9 984, six heads 38.4 -> 20.3; 8 x 32 768 in chunks
-// 36.8 -> 26.5; batch 1 x 1 024 7.7 -> 6.7.  A wave issues 66 vector instructions per 64 tokens and four heads for the logits, 66
+// 36.8 -> 26.5; batch 1 x 1 024 7.7 -> 6.7.  A wave issues 66 vector instructions per 64 tokens and four heads for the logits, 74
 // for weights and values, beside 16 of these MFMAs, and about 600 for the rest (330 of them the window); at batch 256 the
 // vector units are busy for three quarters of a launch.  The matrix form first had 84 and 125 per tile: the logits stay in grid
 // steps (their scale and zero-point go into the exponent's factor and the calibration), V fields are taken in place,
-// a weight's digits are one fused multiply-add and a conversion, every lane calibrates its own head only, and the
+// every lane calibrates its own head only, and the
 // rows' addresses are a scalar base and one bounded offset - start of these steps -> now: batch 64 21.3 -> 20.0, 2 bits
 // 29.0 -> 27.6, 16 x 9 984 23.1 -> 20.5, batch 256 60.1 -> 57.3, per-token values 39.4 -> 36.9 (one box, in turn).
-// Error against 64 bits: a weight is off by 2^-31, or by 2^-24 of itself; a channel's q.s_k by 2^(s - 30) of the head's
+// Error against 64 bits: a weight is off by 2^-31 at most and exact from 2^-7 on (weight_digits(); with the digits' offset added
+// before the conversion instead, which rounds once more, 1.5 % less time: batch 64 18.41 -> 18.17, batch 256 52.7 -> 51.9); a channel's q.s_k by 2^(s - 30) of the head's
 // largest (s = 3: 2^-27, three of the grid's bits; masked in place all through, the top bit of a byte would cost seven),
 // then the fp32 roundings.
 // The look-up form added fp32 partial sums on the K side and held the weights as fp16 on the V side.  Root-mean-square
@@ -271,17 +273,6 @@ __device__ __forceinline__ void clear_handover(const DecodeGeom& g, int64_t unit
 typedef int I4 __attribute__((ext_vector_type(4)));
 typedef int I2 __attribute__((ext_vector_type(2)));
 typedef uint32_t U2 __attribute__((ext_vector_type(2)));
-
-// four signed byte digits of x, -2^31 <= x <= 2^31 - 1 - 0x808080 (digit 0 in the lowest byte; above that the top digit wraps)
-__device__ __forceinline__ uint32_t byte_digits(int x) {
-    return (static_cast<uint32_t>(x) + 0x00808080u) ^ 0x00808080u;
-}
-
-// A weight e in [0, 1] on its grid of 2^-30 as four byte digits: e * 2^30 + 0x808080 is a whole number in fp32 (at least
-// 2^23; rounded to even where e * 2^30 is not), which is off by 2^-31 or by 2^-24 of e, the rounding of any fp32 product.
-__device__ __forceinline__ uint32_t weight_digits(float e, float grid) {
-    return static_cast<uint32_t>(static_cast<int>(__builtin_fmaf(e, grid, 8421504.f))) ^ 0x00808080u;
-}
 
 // what field f (lowest first) of a masked byte of codes counts, as a shift: the upper half-byte's fields are moved down
 template <int BITS> __device__ __forceinline__ constexpr int field_shift(int f) { return (BITS * f) & 3; }
