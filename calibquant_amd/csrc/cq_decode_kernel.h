@@ -897,13 +897,14 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             // the logits themselves (all chunks of a unit have the same step and zero-point sum: the same query and statistics).
             // Every lane works out its own head's.
             const float step = qsz[2 * hl], zs = qsz[2 * hl + 1];
-            const float real_mn = __builtin_fmaf(mn, step, -zs), real_mx = __builtin_fmaf(mx, step, -zs);
-            float slope = 1.0f, tmin = real_mn;
+            // The range is that of the grid steps: the difference of the two logits carries their roundings, and a slope from it does
+            // not fit the steps where the logits differ by little beside their size.
+            const float range = (mx - mn) * step;
+            float slope = 1.0f, tmin = __builtin_fmaf(mn, step, -zs);
             if (g.calib) {
-                const float tgt_max = real_mx + g.off_max;
-                tmin = real_mn + g.off_min;
+                tmin += g.off_min;
                 // (the hardware reciprocal, one unit in the last place: far inside the tolerance of the map)
-                slope = (tgt_max - tmin) * __builtin_amdgcn_rcpf(real_mx - real_mn + 1e-8f);
+                slope = (range + (g.off_max - g.off_min)) * __builtin_amdgcn_rcpf(range + 1e-8f);
             }
             // e = exp(x - M) with x = (w - mn) * slope + tmin, as exp2((w - peak) * ea): `peak` is the logit whose x is M, so no
             // weight is above 1 - which the fixed-point weights rely on - however large the logits are or far from 0 they lie
@@ -935,7 +936,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 pkl = m_img;
                 if (m_img == -INFINITY) { eal = 1.f; pkl = INFINITY; }   // every position masked out
             } else {
-                m_img = fmaxf(tmin, (real_mx - real_mn) * slope + tmin);
+                m_img = fmaxf(tmin, range * slope + tmin);
                 eal = slope * kLog2e * step;
                 pkl = slope < 0.f ? mn : mx;
                 if (m_img == -INFINITY) { eal = 1.f; pkl = INFINITY; }

@@ -237,3 +237,26 @@ def test_decode_attn_streamed_rows_equal_a_small_batch(ops, bits, vals, G, optio
     small, form2 = run(40)
     assert form == form2 and form[2] == 1
     assert torch.equal(big[:40], small)
+
+
+@pytest.mark.parametrize("form", ["single", "mask", "chunked"])
+@pytest.mark.parametrize("log_scale", [-13, -11, -9, -6])
+def test_logit_range_below_the_resolution_of_the_logits(ops, form, log_scale):
+    """Keys that differ by little beside what they share: logits of about 560 (one last place of fp32: 6e-5) that range over
+    1e-5 to 1.4e-3.  The calibration stretches that range, so it is taken from the differences, not from the rounded
+    logits."""
+    T = 40000 if form == "chunked" else 300
+    B, Hq, Hkv = 1, 4, 1
+    rng = np.random.default_rng(6)
+    c = make_case(B, Hq, Hkv, 128, T, 0, 1, "fp16", seed=6)
+    bit = np.zeros((B, Hkv, T, 128), np.uint8)
+    bit[..., 0] = rng.integers(0, 2, size=(B, Hkv, T))
+    c["ck"] = O.encode(bit, 1)
+    c["q"] = np.ones_like(c["q"])
+    c["sk"] = np.ones_like(c["sk"])
+    c["sk"][..., 0] = 2.0 ** log_scale
+    c["zk"] = np.full_like(c["zk"], 50.0)
+    mask = np.zeros((B, T), np.float32) if form == "mask" else None
+    got = _run(ops, c, "fp16", 0, 1, mask=mask)
+    want = O.decode_attention(c["q"], c["ck"], c["cv"], c["sk"], c["zk"], c["sv"], c["zv"], None, None, 0, 1, mask=mask, ftype=np.float64)
+    _close(got, want)
