@@ -86,9 +86,9 @@ struct DecodeGeom {
     // logit min / max inside the launch.  rec: [unit][head][chunk][2] 64-bit records, a float (min, then max)
     // in the lower half and the call's epoch in the upper half - a record is valid by itself, so a chunk
     // publishes with plain write-through stores and waits for nothing, and the others poll the records
-    // (whatever an earlier call or an uninitialised workspace left there has another epoch).  done: [unit][chunk] words of
-    // the same kind (in the place of the two-launch form's min / max), and done_res [unit] for the window's workgroup (in
-    // that of its counters), set to the epoch's tag when the workgroup's partial is written: the unit's first workgroup
+    // (whatever an earlier call or an uninitialised workspace left there has another epoch).  done: [unit][chunk] words
+    // (in the place of the two-launch form's min / max), and done_res [unit] for the window's workgroup (in
+    // that of its counters), set to done_tag() of the epoch when the workgroup's partial is written: the unit's first workgroup
     // waits for them and merges.  status: host-visible word that a workgroup sets
     // when it gives up waiting (spin_limit polls); NULL: nowhere to report.
     unsigned long long* rec;
@@ -210,38 +210,60 @@ __device__ __forceinline__ void publish(float* p, float v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The partials of a unit are announced with plain write-through stores, not counted: an atomic read-modify-write is executed
-// at the memory side whatever scope it names (about 2 us a round trip, those on one address one after the other; with
+// The partials of a unit are announced in a word each, not counted: read-modify-writes are executed at the memory side
+// whatever scope they name (about 2 us a round trip, those on one address one after the other; with
 // a compare-and-swap counter that a unit's workgroups retried on, us, counter -> words: 8 chunks a unit (8 x 32 768) 27.5 ->
 // 25.0, 16 (4 x 16 384 + 200, 2 bits) 40.4 -> 25.2, 32 (1 x 32 768 + 100) 68.6 -> 20.7).  The first wave of the
-// unit's first workgroup polls the others' words, a bounded number of times of its own (every other workgroup ends
+// unit's first workgroup polls the others' words, as many times as the caller's bound says (every other workgroup ends
 // without waiting for this one, so the bound only matters where they are not all resident together).
-constexpr int kDonePolls = 1 << 18;
+// Whoever is last leaves the unit's words empty, because a recorded launch comes back with the same epoch.  That is the
+// first workgroup if its wait succeeds.  If not, it takes the words over with another mark and leaves the number of
+// workgroups still to come in its own word; one that finds the mark as it announces itself counts down, and the last clears.
+// (Announcing by exchange, whose result nothing waits for but the workgroup's own end, instead of by a store: no difference.)
+// A word is the epoch and its complement, so nothing else that a workspace may hold passes for one.
 __device__ __forceinline__ unsigned long long* done_word(const DecodeGeom& g, int64_t unit, int split) {
     return split < g.nsplit ? g.done + unit * g.nsplit + split : g.done_res + unit;
 }
-__device__ __forceinline__ void announce(const DecodeGeom& g, int64_t unit, int split) {
-    __hip_atomic_store(done_word(g, unit, split), static_cast<unsigned long long>(g.epoch) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ unsigned long long done_tag(uint32_t epoch) { return static_cast<unsigned long long>(epoch) << 32 | static_cast<uint32_t>(~epoch); }
+__device__ __forceinline__ unsigned long long left_tag(uint32_t epoch) { return static_cast<unsigned long long>(epoch) << 32 | epoch; }
+
+// The single-launch chunked step's hand-over words of one unit back to empty, by `nt` threads, once every other workgroup is past them.
+template <int HPB>
+__device__ __forceinline__ void clear_handover(const DecodeGeom& g, int64_t unit, int tid, int nt) {
+    for (int i = tid; i < HPB * g.nsplit * 2; i += nt)
+        __hip_atomic_store(g.rec + unit * HPB * g.nsplit * 2 + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = tid; i <= g.nsplit; i += nt) __hip_atomic_store(done_word(g, unit, i), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// One thread of a workgroup other than the unit's first, when its partial (if it has one) is written.
+template <int HPB>
+__device__ __forceinline__ void announce(const DecodeGeom& g, int64_t unit, int split) {
+    if (__hip_atomic_exchange(done_word(g, unit, split), done_tag(g.epoch), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != left_tag(g.epoch)) return;
+    if (__hip_atomic_fetch_add(g.done + unit * g.nsplit, ~0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1ull) clear_handover<HPB>(g, unit, 0, 1);
+}
+// One wave of the unit's first workgroup: true when every other one has announced itself; false when the bound is used
+// up, and the unit's words are no longer this workgroup's business.
 __device__ __forceinline__ bool others_done(const DecodeGeom& g, int64_t unit, int lane) {
-    bool ok = false;
-    for (int it = 0; it < kDonePolls && !ok; ++it) {
+    for (int it = 0; it < g.spin_limit; ++it) {
         bool all = true;
         for (int s = 1 + lane; s < g.nx; s += 64)
-            all = all && static_cast<uint32_t>(__hip_atomic_load(done_word(g, unit, s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32) == g.epoch;
-        ok = __builtin_amdgcn_ballot_w64(!all) == 0;
-        if (!ok) __builtin_amdgcn_s_sleep(1);
+            all = all && __hip_atomic_load(done_word(g, unit, s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == done_tag(g.epoch);
+        if (__builtin_amdgcn_ballot_w64(!all) == 0) return true;
+        __builtin_amdgcn_s_sleep(1);
     }
-    return ok;
-}
-
-// The single-launch chunked step's hand-over words of one unit back to empty: by the unit's first workgroup, once every
-// other one is past them (a recorded launch comes back with the same epoch).
-template <int HPB, int NT>
-__device__ __forceinline__ void clear_handover(const DecodeGeom& g, int64_t unit, int tid) {
-    for (int i = tid; i < HPB * g.nsplit * 2; i += NT)
-        __hip_atomic_store(g.rec + unit * HPB * g.nsplit * 2 + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int i = tid; i <= g.nsplit; i += NT) __hip_atomic_store(done_word(g, unit, i), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // The count is in place (its exchange has returned) before the first mark is.
+    unsigned long long* count = g.done + unit * g.nsplit;
+    if (lane == 0) __hip_atomic_exchange(count, static_cast<unsigned long long>(g.nx), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    int here = 1;   // this workgroup and those that came before the mark
+    for (int s0 = 1; s0 < g.nx; s0 += 64) {
+        const int s = s0 + lane;
+        const bool came = s < g.nx && __hip_atomic_exchange(done_word(g, unit, s), left_tag(g.epoch), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == done_tag(g.epoch);
+        here += __builtin_popcountll(__builtin_amdgcn_ballot_w64(came));
+    }
+    bool last = false;
+    if (lane == 0) last = __hip_atomic_fetch_add(count, ~0ull * static_cast<unsigned>(here), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == static_cast<unsigned long long>(here);
+    return __builtin_amdgcn_ballot_w64(last) != 0;   // (all of them are past their words after all)
 }
 
 // ---- the step on the matrix cores --------------------------------------------------------------
@@ -854,10 +876,10 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     __syncthreads();
                     if (!*flag) {
                         // Given up: no result from this workgroup, but it still announces itself, so that the unit's
-                        // first workgroup leaves the hand-over words empty and a replay of this very launch (same epoch)
+                        // hand-over words are left empty and a replay of this very launch (same epoch)
                         // does not take this launch's records for its own.
                         if (split != 0) {
-                            if (tid == 0) announce(g, unit, split);
+                            if (tid == 0) announce<HPB>(g, unit, split);
                             return;
                         }
                         int* last = reinterpret_cast<int*>(red);
@@ -866,7 +888,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                             if (lane == 0) *last = ok ? 1 : 0;
                         }
                         __syncthreads();
-                        if (*last) clear_handover<HPB, kNT>(g, unit, tid);
+                        if (*last) clear_handover<HPB>(g, unit, tid, kNT);
                         return;
                     }
                     mn = -fold[hl];
@@ -1208,7 +1230,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             int* last = reinterpret_cast<int*>(red);
             if (g.fused) {
                 if (split != 0) {
-                    if (tid == 0) announce(g, unit, split);
+                    if (tid == 0) announce<HPB>(g, unit, split);
                     return;
                 }
                 if (wv == 0) {
@@ -1255,7 +1277,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     store_elem<DT>(g.out, row * kD + d, num / den);
                 }
                 // every other workgroup of the unit is past the hand-over words
-                if (g.fused) clear_handover<HPB, kNT>(g, unit, tid);
+                if (g.fused) clear_handover<HPB>(g, unit, tid, kNT);
             }
         }
     }

@@ -307,8 +307,9 @@ typedef struct cq_decode_plan {
 int cq_decode_attn_plan(const cq_decode_args* args, cq_decode_plan* plan);
 
 /* The single-launch chunked step (plan: chunks > 1, launches == 1) makes the workgroups of a unit wait for each
- * other's logit min / max inside the launch.  That is only sound while they are all resident together, which the
- * plan works out from the device's compute-unit count; the wait is therefore bounded: after `polls` polls (about a
+ * other's logit min / max inside the launch, and the first of them for the others' partial results.  That is only
+ * sound while they are all resident together, which the
+ * plan works out from the device's compute-unit count; either wait is therefore bounded: after `polls` polls (about a
  * microsecond each; default 262 144) a workgroup gives up, ends without a result and sets a word of pinned host
  * memory (64 bytes per device, allocated at the first such call outside a stream capture - the one allocation
  * this library makes - and kept until the process ends).  The next chunked cq_decode_attn on that device then

@@ -169,3 +169,51 @@ def test_single_launch_chunked_step_gives_up_and_the_host_reports_it(ops):
     again = call.run().clone()
     torch.cuda.synchronize()
     assert torch.equal(again, good)
+
+
+@pytest.mark.parametrize("B, T, R, bits", [(1, 32768, 100, 1), (4, 16384, 200, 2), (2, 20000, 0, 1)])
+def test_single_launch_chunked_step_leaves_nothing_behind_when_its_merge_gives_up(ops, B, T, R, bits):
+    """With no polls the first workgroup of a unit does not wait for the others' partial results either: some of them
+    announce themselves before it has left, some after.  Whoever is last empties the hand-over words, so that replays
+    of the same recorded launch and later launches on the workspace start clean."""
+    from calibquant_amd import _lib
+    lib = _lib.load()
+    print(f"case merge gives up B={B} T={T} R={R} bits={bits}", flush=True)
+    Hq, Hkv = 32, 8
+    g = torch.Generator(device="cuda").manual_seed(T)
+    n = lambda *s: torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)  # noqa: E731
+    codes = [torch.randint(0, 256, (B, Hkv, T, 16 * bits), generator=g, device="cuda", dtype=torch.uint8) for _ in range(2)]
+    stats = [n(B, Hkv, 128).abs() for _ in range(4)]
+    kr, vr = (n(B, Hkv, R, 128), n(B, Hkv, R, 128)) if R else (None, None)
+    call = ops.DecodeCall(n(B, Hq, 128), codes[0], codes[1], *stats, kr, vr, bits=bits)
+    p = call.plan()
+    assert p["chunks"] > 1 and p["launches"] == 1
+    good = call.run().clone()
+    torch.cuda.synchronize()
+    units, heads, chunks = B * Hkv * (Hq // Hkv // p["heads_per_unit"]), p["heads_per_unit"], p["chunks"]
+    rec = units * heads * chunks * 16
+    cnt = (units * 8 + 255) // 256 * 256 + rec
+
+    def empty():
+        # [unit][chunk] words at the start of the workspace; the window's words and the records at its end
+        ws = call.workspace[:call.workspace_bytes]
+        return not (ws[:units * chunks * 8].any() or ws[-cnt:][:units * 8].any() or ws[-rec:].any())
+    assert empty()
+    before = lib.cq_decode_attn_wait_polls(0)
+    try:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            call.run()
+        for _ in range(30):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert empty()
+        assert lib.cq_decode_attn_gave_up() == 1
+        with pytest.raises(_lib.CalibQuantError):
+            call.run()
+    finally:
+        lib.cq_decode_attn_wait_polls(before)
+    for _ in range(3):
+        call.run()
+        torch.cuda.synchronize()
+        assert empty() and torch.equal(call.out, good)
