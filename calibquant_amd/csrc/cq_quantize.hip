@@ -39,9 +39,10 @@ struct QuantGeom {
     FastDiv dTB;          // per-token quantiser: workgroup passes per (batch, head)
     int shared_stats;     // non-zero: one row of statistics / thresholds serves every (batch, head) (whole-tensor mode)
     // One-pass kernel: `parts` workgroups share a (batch, head) pair, `part_rows` token rows each, and, if there are
-    // several, exchange their channel minima / maxima through `rec` inside the launch: [pair * parts + part][channel]
-    // 64-bit records, the two extremes as 16-bit keys below the call's epoch, so a record is valid by itself and nothing
-    // has to be cleared.  The wait for the other parts is bounded (spin_limit polls); a lane that gives up sets *status
+    // several, exchange their channel minima / maxima through `rec` inside the launch: [pair * parts + part][two channels]
+    // records of two 64-bit words: the minima as 16-bit keys, below the call's epoch xor the maxima; the maxima, below its
+    // complement xor the minima.  A record is valid by itself - 64 bits of it must fit, and a word of it beside one that the
+    // workspace held before does not - and nothing has to be cleared.  The wait for the other parts is bounded (spin_limit polls); a lane that gives up sets *status
     // (pinned host memory).
     int parts, part_rows;
     FastDiv dP;           // divisor `parts`
@@ -462,8 +463,6 @@ typedef unsigned short US2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pk_max_s(uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(S2, a), __builtin_bit_cast(S2, b))); }
 __device__ __forceinline__ uint32_t pk_max_u(uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(US2, a), __builtin_bit_cast(US2, b))); }
 __device__ __forceinline__ uint32_t pk_min_s(uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(S2, a), __builtin_bit_cast(S2, b))); }
-// (maximum, minimum) pairs of monotone keys in the upper and lower half
-__device__ __forceinline__ uint32_t ext_fold(uint32_t a, uint32_t b) { return (pk_max_s(a, b) & 0xffff0000u) | (pk_min_s(a, b) & 0xffffu); }
 __device__ __forceinline__ uint32_t pk_min_u(uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(US2, a), __builtin_bit_cast(US2, b))); }
 __device__ __forceinline__ uint32_t pk_sub_sat(uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(S2, a), __builtin_bit_cast(S2, b))); }
 __device__ __forceinline__ uint32_t pk_sign(uint32_t a) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(S2, a) >> 15); }   // 0xffff where negative
@@ -781,50 +780,62 @@ __global__ __launch_bounds__(kFThreads, kFResident) void fused_pack_kernel(const
             a2 = pk_min_s(a2, static_cast<uint32_t>(dpp_move_i<decltype(ctrl)::value>(static_cast<int>(a2), 0)));
             z2 = pk_max_s(z2, static_cast<uint32_t>(dpp_move_i<decltype(ctrl)::value>(static_cast<int>(z2), 0)));
         };
-        across(std::integral_constant<int, 0xB1>{});       // lane ^ 1
-        across(std::integral_constant<int, 0x4E>{});       // lane ^ 2
-        if constexpr (kLG == 16) {
-            across(std::integral_constant<int, 0x141>{});  // mirrored in eight lanes
-            across(std::integral_constant<int, 0x140>{});  // ... in sixteen
-        }
-        const int c = 2 * pair2 + lg / kLC, lc = lg % kLC;
-        const bool odd = (lc & 1) != 0, lead = lc == 0;
-        uint32_t ext = lg / kLC ? (z2 & 0xffff0000u) | (a2 >> 16) : (z2 << 16) | (a2 & 0xffffu);   // the channel's maximum, minimum
+        auto fold_lanes = [&] {
+            across(std::integral_constant<int, 0xB1>{});       // lane ^ 1
+            across(std::integral_constant<int, 0x4E>{});       // lane ^ 2
+            if constexpr (kLG == 16) {
+                across(std::integral_constant<int, 0x141>{});  // mirrored in eight lanes
+                across(std::integral_constant<int, 0x140>{});  // ... in sixteen
+            }
+        };
+        fold_lanes();
         if constexpr (SPLIT) {
-            // This part's extremes of channel c go out as one self-validating record; then the records of all parts
-            // are polled (device-scope loads, a bounded number of times; each of the channel's lanes takes every kLC-th
-            // part, four at a time) and folded.  The other parts are being worked on right now by other workgroups of this launch.
-            unsigned long long* first = g.rec + static_cast<int64_t>(slice) * g.parts * kChan;
-            if (lead) __hip_atomic_store(first + static_cast<uint32_t>((id - slice * g.parts) * kChan + c), static_cast<unsigned long long>(g.epoch) << 32 | ext,
-                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            uint32_t fold = ext;
+            // This part's extremes of the two channels go out as one self-validating record; then the records of all parts
+            // are polled (device-scope loads, a bounded number of times; each of the channels' lanes takes every kLG-th
+            // part, two at a time) and folded.  The other parts are being worked on right now by other workgroups of this launch.
+            unsigned long long* first = g.rec + static_cast<int64_t>(slice) * g.parts * kChan;   // (two words for two channels)
+            if (lg == 0) {
+                unsigned long long* mine = first + static_cast<uint32_t>((id - slice * g.parts) * kChan + 2 * pair2);
+                __hip_atomic_store(mine, static_cast<unsigned long long>(g.epoch ^ z2) << 32 | a2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(mine + 1, static_cast<unsigned long long>(~g.epoch ^ a2) << 32 | z2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            auto whole = [&](unsigned long long lo, unsigned long long hi) {
+                return (static_cast<uint32_t>(lo >> 32) ^ static_cast<uint32_t>(hi)) == g.epoch && (static_cast<uint32_t>(hi >> 32) ^ static_cast<uint32_t>(lo)) == ~g.epoch;
+            };
             int polls = 0;
-            for (int p0 = lc; p0 < g.parts; p0 += 4 * kLC) {
-                unsigned long long r[4];   // in flight together; past the end the last part again
+            for (int base = 0; base < g.parts; base += 2 * kLG) {
+                const bool two = base + kLG < g.parts;
+                unsigned long long lo[2], hi[2];   // past the end the last part again
                 bool all = false;
                 while (!all && polls < g.spin_limit) {
                     if (polls) __builtin_amdgcn_s_sleep(1);
                     ++polls;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        r[k] = __hip_atomic_load(first + static_cast<uint32_t>(min(p0 + k * kLC, g.parts - 1) * kChan + c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     all = true;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) all = all && static_cast<uint32_t>(r[k] >> 32) == g.epoch;
+                    for (int k = 0; k < 2; ++k) {
+                        if (k && !two) continue;
+                        unsigned long long* theirs = first + static_cast<uint32_t>(min(base + k * kLG + lg, g.parts - 1) * kChan + 2 * pair2);
+                        lo[k] = __hip_atomic_load(theirs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        hi[k] = __hip_atomic_load(theirs + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+#pragma unroll
+                    for (int k = 0; k < 2; ++k)
+                        if (k == 0 || two) all = all && whole(lo[k], hi[k]);
                 }
                 if (!all) { polls = -1; break; }
 #pragma unroll
-                for (int k = 0; k < 4; ++k) fold = ext_fold(fold, static_cast<uint32_t>(r[k]));
+                for (int k = 0; k < 2; ++k) {
+                    if (k && !two) continue;
+                    a2 = pk_min_s(a2, static_cast<uint32_t>(lo[k]));
+                    z2 = pk_max_s(z2, static_cast<uint32_t>(hi[k]));
+                }
             }
-            const bool ok = polls >= 0;
-            fold = ext_fold(fold, static_cast<uint32_t>(dpp_move_i<0xB1>(static_cast<int>(fold), 0)));
-            if constexpr (kLC == 8) {
-                fold = ext_fold(fold, static_cast<uint32_t>(dpp_move_i<0x4E>(static_cast<int>(fold), 0)));
-                fold = ext_fold(fold, static_cast<uint32_t>(dpp_move_i<0x141>(static_cast<int>(fold), 0)));
-            }
-            ext = fold;
-            if (!ok && g.status) __hip_atomic_store(g.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);   // this call's result is not valid
+            if (polls < 0 && g.status) __hip_atomic_store(g.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);   // this call's result is not valid
+            fold_lanes();
         }
+        const int c = 2 * pair2 + lg / kLC, lc = lg % kLC;
+        const bool odd = (lc & 1) != 0, lead = lc == 0;
+        const uint32_t ext = lg / kLC ? (z2 & 0xffff0000u) | (a2 >> 16) : (z2 << 16) | (a2 & 0xffffu);   // the channel's maximum, minimum
         auto bits_of = [](uint32_t key) { return (key & 0x8000u) ? key ^ 0x7fffu : key; };   // (16 bits) the monotone map is its own inverse
         const float x_min = rnd<DT>(Cvt<DT>::to_float(bits_of(ext & 0xffffu)) * clip);
         const float x_max = rnd<DT>(Cvt<DT>::to_float(bits_of(ext >> 16)) * clip);

@@ -269,3 +269,36 @@ def test_quantize_pack_recorded_and_replayed(ops, shape):
         torch.cuda.synchronize()
         for a, b in zip(got, ops.quantize_pack(x, 1, 0.5)):
             assert torch.equal(a, b)
+
+
+def test_quantize_pack_takes_no_record_from_what_the_workspace_held(ops):
+    """The parts' exchange records are recognised by their contents, and the workspace is whatever memory was free.  Here its
+    words hold the coming call's epoch above extremes that no part has - half of them taken from the upper half of the
+    first record's first word (what the minima stand below), half from that and the maxima."""
+    from calibquant_amd import _lib
+    lib = _lib.load()
+    B, T, H, D = 4, 9984, 8, 128
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn((B, T, H, D), generator=g, device="cuda").to(torch.bfloat16)
+    ws = torch.zeros(lib.cq_quantize_pack_workspace(B, T, H, D), dtype=torch.uint8, device="cuda")
+
+    def call():
+        codes = torch.empty((B, H, T, D // 8), dtype=torch.uint8, device="cuda")
+        s, z = (torch.empty((B, H, D), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        _lib.check(lib.cq_quantize_pack(x.data_ptr(), 0, B, T, H, D, *x.stride()[:3], 1, 0.5, codes.data_ptr(), s.data_ptr(),
+                                        z.data_ptr(), ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream), "cq_quantize_pack")
+        torch.cuda.synchronize()
+        return codes, s, z
+    want = call()
+    words = ws[:ws.numel() // 32 * 32].view(torch.int64)
+
+    def first_record():
+        lo, hi = (int(w) & (1 << 64) - 1 for w in words[:2])
+        return lo >> 32, lo >> 32 ^ hi & 0xffffffff
+    upper, epoch = first_record()
+    assert epoch != 0, "several parts per pair leave their records in the workspace"
+    for i, e in enumerate((upper, epoch, epoch, upper)):
+        words[i::4] = torch.tensor(((e + 1) << 32 | 0x7f008080) - (1 << 64 if e >> 31 else 0), device="cuda")
+    for a, b in zip(call(), want):
+        assert torch.equal(a, b)
+    assert first_record()[1] == epoch + 1
