@@ -42,8 +42,10 @@ struct QuantGeom {
     // several, exchange their channel minima / maxima through `rec` inside the launch: [pair * parts + part][two channels]
     // records of two 64-bit words: the minima as 16-bit keys, below the call's epoch xor the maxima; the maxima, below its
     // complement xor the minima.  A record is valid by itself - 64 bits of it must fit, and a word of it beside one that the
-    // workspace held before does not - and nothing has to be cleared.  The wait for the other parts is bounded (spin_limit polls); a lane that gives up sets *status
-    // (pinned host memory).
+    // workspace held before does not - and nothing has to be cleared.  The wait
+    // for the other parts is bounded (spin_limit polls); what is not there by then is read from x again (rows_again()), so the
+    // result does not depend on the workgroups being resident together.  spin_limit 0: a part goes on with what it has and
+    // sets *status (pinned host memory).
     int parts, part_rows;
     FastDiv dP;           // divisor `parts`
     unsigned long long* rec;
@@ -584,9 +586,40 @@ __device__ __forceinline__ int threshold_key(float s, float zp, float levels, in
     return key;
 }
 
+// Two neighbouring channels of the token rows [t, end) of a pair, read (and rotated) again, folded onto the minima and maxima.
+template <typename DT, bool ROPE>
+__device__ __forceinline__ void rows_again(const uint16_t* x, const QuantGeom& g, const RopeArgs& ra, int bh, int channel, int t, int end,
+                                           uint32_t& a2, uint32_t& z2) {
+    const uint32_t b = g.dH.quot(static_cast<uint32_t>(bh)), h = static_cast<uint32_t>(bh) - b * g.dH.div;
+    const uint16_t* col = x + static_cast<int64_t>(b) * g.sb + static_cast<int64_t>(h) * g.sh;
+    auto word = [](const uint16_t* p) { return *reinterpret_cast<const uint32_t*>(p); };
+    auto take = [&](uint32_t v) {
+        v ^= pk_sign(v) & 0x7fff7fffu;
+        a2 = pk_min_s(a2, v);
+        z2 = pk_max_s(z2, v);
+    };
+    if constexpr (ROPE) {
+        const uint32_t sign = channel < 64 ? 0x80008000u : 0u;   // of rotate_half
+#pragma unroll 1
+        for (; t < end; ++t) {
+            const uint16_t* xp = col + static_cast<int64_t>(t) * g.st;
+            const int64_t pl = ra.pos ? ra.pos[static_cast<int64_t>(b) * ra.pos_sb + static_cast<int64_t>(t) * ra.pos_st] : ra.pos0 + t;
+            const int64_t ps = (pl < 0 ? 0 : pl >= ra.table_rows ? ra.table_rows - 1 : pl) * 128 + channel;
+            const uint32_t v = word(xp + channel), y = word(xp + (channel ^ 64)) ^ sign, cw = word(ra.cos + ps), sw = word(ra.sin + ps);
+            take(Cvt<DT>::from_float(rnd<DT>(Cvt<DT>::lo(v) * Cvt<DT>::lo(cw)) + Cvt<DT>::lo(y) * Cvt<DT>::lo(sw)) |
+                 Cvt<DT>::from_float(rnd<DT>(Cvt<DT>::hi(v) * Cvt<DT>::hi(cw)) + Cvt<DT>::hi(y) * Cvt<DT>::hi(sw)) << 16);
+        }
+    } else {
+const uint16_t* p = col + static_cast<int64_t>(t) * g.st + channel;
+#pragma unroll 1
+        for (int rows = end - t; rows > 0; --rows, p += g.st) take(word(p));
+    }
+}
+
 // The parts of a pair (or quarter) are consecutive ids; a workgroup walks ids blockIdx.x, blockIdx.x + gridDim.x, ... in increasing
-// order and all workgroups are resident: whoever waits for another part waits for a workgroup whose earlier ids belong to
-// the same or earlier pairs, so no two wait for each other.
+// order.  With all workgroups resident, whoever waits for another part waits for a workgroup whose earlier ids belong to
+// the same or earlier pairs, so no two wait for each other; where they are not (other streams' kernels, compute-unit masks), a wait
+// ends after its bound and the missing rows are read again.
 template <typename DT, int BITS, int NR, int LPR = 16, bool ROPE = false, bool SPLIT = false>   // NR: rows per thread
 __global__ __launch_bounds__(kFThreads, kFResident) void fused_pack_kernel(const uint16_t* __restrict__ x, QuantGeom g, float clip,
                                                               uint16_t* __restrict__ scale,
@@ -792,7 +825,8 @@ __global__ __launch_bounds__(kFThreads, kFResident) void fused_pack_kernel(const
         if constexpr (SPLIT) {
             // This part's extremes of the two channels go out as one self-validating record; then the records of all parts
             // are polled (device-scope loads, a bounded number of times; each of the channels' lanes takes every kLG-th
-            // part, two at a time) and folded.  The other parts are being worked on right now by other workgroups of this launch.
+            // part, two at a time) and folded.  The other parts are being worked on right now by other workgroups of this launch,
+            // unless something else holds the compute units they need.
             unsigned long long* first = g.rec + static_cast<int64_t>(slice) * g.parts * kChan;   // (two words for two channels)
             if (lg == 0) {
                 unsigned long long* mine = first + static_cast<uint32_t>((id - slice * g.parts) * kChan + 2 * pair2);
@@ -830,7 +864,25 @@ __global__ __launch_bounds__(kFThreads, kFResident) void fused_pack_kernel(const
                     z2 = pk_max_s(z2, static_cast<uint32_t>(hi[k]));
                 }
             }
-            if (polls < 0 && g.status) __hip_atomic_store(g.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);   // this call's result is not valid
+            if (polls < 0) {
+                if (g.spin_limit <= 0) {   // this call's result is not valid
+                    if (g.status) __hip_atomic_store(g.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                } else {
+                    // Not all of them within the bound: what is still not there of the lane's parts it reads itself.
+#pragma unroll 1
+                    for (int p = lg; p < g.parts; p += kLG) {
+                        unsigned long long* theirs = first + static_cast<uint32_t>(p * kChan + 2 * pair2);
+                        const unsigned long long lo = __hip_atomic_load(theirs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        const unsigned long long hi = __hip_atomic_load(theirs + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if (whole(lo, hi)) {
+                            a2 = pk_min_s(a2, static_cast<uint32_t>(lo));
+                            z2 = pk_max_s(z2, static_cast<uint32_t>(hi));
+                        } else {
+                            rows_again<DT, ROPE>(x, g, ra, bh, quarter * 32 + 2 * pair2, p * g.part_rows, min(g.T, (p + 1) * g.part_rows), a2, z2);
+                        }
+                    }
+                }
+            }
             fold_lanes();
         }
         const int c = 2 * pair2 + lg / kLC, lc = lg % kLC;
@@ -1002,14 +1054,15 @@ __global__ __launch_bounds__(256) void clear_records_kernel(unsigned long long* 
     for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += gridDim.x * 256ll) rec[i] = 0ull;
 }
 
-// The wait of a part for the others is bounded; a lane that gives up sets a word of pinned host memory (one per
-// device, allocated at the first such call outside a stream capture, never freed).  The next call on the device
-// finds it, reports CQ_ERR_LAUNCH once, and the process goes on with the three-launch path.
+// A part that waits in vain reads the others' rows itself.  Only with the bound set to 0 (cq_quantize_pack_wait_polls) do
+// parts go on alone and set a word of pinned host memory (one per device, allocated at the first such call outside a stream
+// capture, never freed): the next call on the device reports CQ_ERR_LAUNCH once, and the process goes on with three
+// launches.
 constexpr int kQMaxDevices = 64;
 static std::atomic<int*> g_qstatus[kQMaxDevices];
 static std::atomic<bool> g_split_off{false};
 static std::atomic<uint32_t> g_qepoch{0x51ab0000u};
-static std::atomic<int> g_qspin{1 << 18};
+static std::atomic<int> g_qspin{1 << 12};   // polls of about a microsecond each
 
 static int* split_status_word(hipStream_t st) {
     int dev = 0;
@@ -1041,6 +1094,21 @@ static bool one_pass_shape(const QuantGeom& g, const uint8_t* codes) {
            g.st > 0 && g.st * 2 < (1 << 24);   // 32-bit row offsets inside a pass
 }
 
+// Rotated rows that overwrite rows of x: parts that may read each other's rows of x again do not take that.
+static bool rope_overlaps(const uint16_t* x, const QuantGeom& g, const RopeArgs& ra) {
+    auto span = [&](const uint16_t* p, int64_t sb, int64_t st, int64_t sh, uintptr_t* lo, uintptr_t* hi) {
+        int64_t a = 0, z = 128;
+        const int64_t ends[3] = {(g.B - 1) * sb, (g.T - 1) * st, (g.H - 1) * sh};
+        for (int64_t e : ends) (e < 0 ? a : z) += e;
+        *lo = reinterpret_cast<uintptr_t>(p) + static_cast<uintptr_t>(a * 2);
+        *hi = reinterpret_cast<uintptr_t>(p) + static_cast<uintptr_t>(z * 2);
+    };
+    uintptr_t x0, x1, o0, o1;
+    span(x, g.sb, g.st, g.sh, &x0, &x1);
+    span(ra.out, ra.ob, ra.ot, ra.oh, &o0, &o1);
+    return x0 < o1 && o0 < x1;
+}
+
 template <typename DT>
 static int run_quant(const void* x, QuantGeom g, int bits, float clip, uint8_t* codes, void* xq, void* scale,
                      void* zero, float* ws, hipStream_t st, const RopeArgs* rope = nullptr) {
@@ -1050,10 +1118,11 @@ static int run_quant(const void* x, QuantGeom g, int bits, float clip, uint8_t* 
     uint16_t* zp = static_cast<uint16_t*>(zero);
     if (rope && (xq || g.T > kFMaxT || !one_pass_shape(g, codes))) return CQ_ERR_UNSUPPORTED;
     SplitPlan spl;
-    if (!xq && one_pass_shape(g, codes) && split_plan(static_cast<int64_t>(g.B) * g.H, g.T, rope != nullptr, &spl)) {
-        // one pass over x; several parts per pair need the word that tells when one gave up waiting
+    if (!xq && one_pass_shape(g, codes) && split_plan(static_cast<int64_t>(g.B) * g.H, g.T, rope != nullptr, &spl) &&
+        !(rope && spl.parts > 1 && rope_overlaps(xp, g, *rope))) {
+        const int spin = g_qspin.load(std::memory_order_relaxed);
         int* status = nullptr;
-        if (spl.parts > 1) {
+        if (spl.parts > 1 && spin == 0) {
             status = g_split_off.load(std::memory_order_relaxed) ? nullptr : split_status_word(st);
             if (status && *static_cast<volatile int*>(status) != 0) {
                 *static_cast<volatile int*>(status) = 0;
@@ -1061,7 +1130,7 @@ static int run_quant(const void* x, QuantGeom g, int bits, float clip, uint8_t* 
                 return CQ_ERR_LAUNCH;   // an earlier split pass did not complete: its output is not valid
             }
         }
-        if (spl.parts == 1 || status) {
+        if (spl.parts == 1 || spin > 0 || status) {
             g.parts = spl.parts;
             g.part_rows = spl.part_rows;
             g.dP.set(static_cast<uint32_t>(spl.parts));
@@ -1070,7 +1139,7 @@ static int run_quant(const void* x, QuantGeom g, int bits, float clip, uint8_t* 
                 uint32_t ep = g_qepoch.fetch_add(1, std::memory_order_relaxed) + 1;
                 g.epoch = ep ? ep : g_qepoch.fetch_add(1, std::memory_order_relaxed) + 1;
             }
-            g.spin_limit = g_qspin.load(std::memory_order_relaxed);
+            g.spin_limit = spin;
             g.status = status;
             if (spl.parts > 1) {
                 // A recorded launch comes back with the same epoch: its records are emptied first, in the recording too.

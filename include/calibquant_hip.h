@@ -70,14 +70,15 @@ int cq_quantize_pack(const void* x, int dtype, int B, int T, int H, int D,
 /* With D = 128, cq_quantize_pack reads x once: a workgroup keeps up to 832 token rows of a (batch, head) pair in registers
  * (up to 3 328 rows of a quarter of the channels where there is little to do), and a longer token axis is shared by up to
  * 128 workgroups of the launch, which exchange the channels' minima and maxima through the workspace inside it.  The wait
- * for the other parts is bounded: after `polls` polls (about a microsecond each; default 262 144) a workgroup goes
- * on with what it has and sets a word of pinned host memory (64 bytes per device, allocated at the first such
- * call outside a stream capture and kept until the process ends).  The next such call on that device then returns
- * CQ_ERR_LAUNCH once (the previous call's output is not valid) and the process goes on with three launches per
- * tensor (partial min / max, statistics, emit; x read twice).  Three launches are also what is recorded while a stream
- * is captured before that word exists.  A recorded exchange empties its records first, so it may be replayed.  This call
- * sets the bound (polls >= 0; it also re-enables the single launch after a give-up) and returns the previous one;
- * polls < 0 only queries.  No counterpart in the reference, whose quant() is a chain of whole-tensor torch ops
+ * for the other parts is bounded: after `polls` polls (about a microsecond each; default 4 096) a workgroup reads
+ * the rows of the parts it misses itself, so the result is the same whether or not the workgroups are resident together
+ * - several such passes on several streams, or beside other work, only take longer.  A recorded exchange empties its
+ * records first, so it may be replayed.  This call sets the bound (polls >= 0) and returns the previous one; polls < 0
+ * only queries.  polls = 0 takes the exchange out of service instead: a part goes on with what it has and sets a
+ * word of pinned host memory (64 bytes per device, allocated at the first such call outside a stream capture and kept
+ * until the process ends); the next such call on that device then returns CQ_ERR_LAUNCH once (the previous call's
+ * output is not valid) and calls take three launches per tensor (partial min / max, statistics, emit; x read twice)
+ * until the bound is set again.  No counterpart in the reference, whose quant() is a chain of whole-tensor torch ops
  * (calibquant.py:24-42). */
 int cq_quantize_pack_wait_polls(int polls);
 
@@ -98,7 +99,7 @@ int cq_quantize_pack_wait_polls(int polls);
  * x_rot: (B, T, H, 128) through element strides (multiples of 8).
  * codes / scale / zero / workspace as for cq_quantize_pack; the results are
  * bit-identical to cq_quantize_pack on the rotated tensor.  (Where the one launch is not available - see
- * cq_quantize_pack_wait_polls - the rows are rotated first and quantised by three launches.)
+ * cq_quantize_pack_wait_polls - or x_rot overlaps x, the rows are rotated first and quantised by three launches.)
  * Shapes outside the one-pass path (T > 3 328, D != 128) return
  * CQ_ERR_UNSUPPORTED: rotate with cq_rope_rows, then cq_quantize_pack. */
 int cq_rope_quantize_pack(const void* x, int dtype, int B, int T, int H, int D,
@@ -312,7 +313,7 @@ int cq_decode_attn_plan(const cq_decode_args* args, cq_decode_plan* plan);
  * plan works out from the device's compute-unit count; either wait is therefore bounded: after `polls` polls (about a
  * microsecond each; default 262 144) a workgroup gives up, ends without a result and sets a word of pinned host
  * memory (64 bytes per device, allocated at the first such call outside a stream capture - the one allocation
- * this library makes - and kept until the process ends).  The next chunked cq_decode_attn on that device then
+ * this library makes in ordinary use - and kept until the process ends).  The next chunked cq_decode_attn on that device then
  * returns CQ_ERR_LAUNCH once (the previous step's output is not valid) and the process goes on with two launches
  * per step.  cq_decode_attn_static always takes two launches.  This call sets the bound (polls >= 0; it also
  * re-enables the single launch after a give-up) and returns the previous one; polls < 0 only queries.

@@ -302,3 +302,61 @@ def test_quantize_pack_takes_no_record_from_what_the_workspace_held(ops):
     for a, b in zip(call(), want):
         assert torch.equal(a, b)
     assert first_record()[1] == epoch + 1
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("shape", [(4, 9984, 8), (1, 9984, 8), (3, 3329, 2), (1, 40000, 1), (64, 1700, 8)])
+def test_quantize_pack_parts_that_wait_in_vain_read_the_rows_themselves(ops, shape, bits, dtype):
+    """With a bound of one poll nearly every part misses others' extremes and reads those rows again: the same result,
+    nothing is reported, and the next call is an ordinary one."""
+    from calibquant_amd import _lib
+    lib = _lib.load()
+    B, T, H = shape
+    print(f"case quantize_pack in vain shape={shape} bits={bits} dtype={dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T + B)
+    x = torch.randn((B, T, H, 128), generator=g, device="cuda").to(torch.bfloat16 if dtype == "bf16" else torch.float16)
+    x[..., 3] = x[..., 3].abs()
+    x[:, T // 2:, :, 50] = -x[:, T // 2:, :, 50].abs()
+    x[:, T // 3, :, 90] = float("inf")
+    x[..., 91] = 0.0
+    x[:, ::2, :, 91] = -0.0
+    want = ops.quantize_pack(x, bits, 0.5)
+    torch.cuda.synchronize()
+    before = lib.cq_quantize_pack_wait_polls(1)
+    try:
+        for _ in range(2):
+            for a, b in zip(ops.quantize_pack(x, bits, 0.5), want):
+                assert same_bits(to_np(a), to_np(b)) if a.is_floating_point() else torch.equal(a, b)
+            torch.cuda.synchronize()
+    finally:
+        lib.cq_quantize_pack_wait_polls(before)
+    for a, b in zip(ops.quantize_pack(x, bits, 0.5), want):
+        assert same_bits(to_np(a), to_np(b)) if a.is_floating_point() else torch.equal(a, b)
+
+
+def test_quantize_pack_on_two_streams(ops):
+    """Two passes whose parts exchange their extremes share the device, with a chunked decode step of one launch on a
+    third stream: the results are those of each alone."""
+    B, T, H = 24, 2400, 8
+    g = torch.Generator(device="cuda").manual_seed(12)
+    xs = [torch.randn((B, T, H, 128), generator=g, device="cuda").to(torch.bfloat16) for _ in range(2)]
+    want = [ops.quantize_pack(x, 1, 0.5) for x in xs]
+    n = lambda *s: torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)  # noqa: E731
+    codes = [torch.randint(0, 256, (4, H, 32768, 16), generator=g, device="cuda", dtype=torch.uint8) for _ in range(2)]
+    decode = ops.DecodeCall(n(4, 32, 128), *codes, *[n(4, H, 128).abs() for _ in range(4)], None, None, bits=1)
+    assert decode.plan()["launches"] == 1 and decode.plan()["chunks"] > 1
+    good = decode.run().clone()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    for _ in range(6):
+        got = []
+        for x, s in zip(xs, streams):
+            with torch.cuda.stream(s):
+                got.append(ops.quantize_pack(x, 1, 0.5))
+        with torch.cuda.stream(streams[2]):
+            decode.run()
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert all(torch.equal(u, v) for u, v in zip(a, b))
+        assert torch.equal(decode.out, good)

@@ -155,3 +155,30 @@ def test_attention_prefill_same_state_through_every_rotary_path(dtype):
         if dtype == torch.bfloat16 or other == 1:   # (torch's fp16 addcmul rounds once: window rows may differ in the last bit)
             assert torch.equal(got[0][3], got[other][3]) and torch.equal(got[0][4], got[other][4])
     assert torch.equal(got[0][5], got[1][5])
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("B, T, Hkv", [(4, 300, 8), (2, 3328, 4), (3, 1111, 5)])
+def test_rope_quantize_pack_parts_that_wait_in_vain(ops, B, T, Hkv, bits, dtype):
+    """With a bound of one poll the parts of a pair rotate each other's rows again for the extremes they miss; the rows
+    may also be rotated in place."""
+    from calibquant_amd import _lib
+    lib = _lib.load()
+    print(f"case rope_quantize_pack in vain B={B} T={T} Hkv={Hkv} bits={bits} dtype={dtype}", flush=True)
+    torch.manual_seed(T)
+    x = torch.randn(B, T, Hkv, 128, device="cuda").to(TDT[dtype])
+    cos, sin = _tables(T + 60, 128, dtype)
+    pos = (torch.arange(T, device="cuda")[None] + torch.arange(B, device="cuda")[:, None] * 7).contiguous()
+    two = ops.rope_rows(x, cos, sin, pos)
+    want = ops.quantize_pack(two, bits, CLIPS[bits][0])
+    before = lib.cq_quantize_pack_wait_polls(1)
+    try:
+        for in_place in (False, True):
+            target = x.clone() if in_place else torch.empty_like(x)
+            got = ops.rope_quantize_pack(target if in_place else x, cos, sin, pos, target, bits, CLIPS[bits][0])
+            torch.cuda.synchronize()
+            assert torch.equal(target, two)
+            assert torch.equal(got[0], want[0]) and all(same_bits(to_np(a), to_np(b)) for a, b in zip(got[1:], want[1:]))
+    finally:
+        lib.cq_quantize_pack_wait_polls(before)
