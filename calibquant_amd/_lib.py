@@ -19,7 +19,7 @@ SYMBOLS = (
     "cq_quantize_pack_workspace", "cq_quantize_pack", "cq_rope_quantize_pack", "cq_rope_rows", "cq_rope_rows_grouped", "cq_quant", "cq_quant_tensor", "cq_encode",
     "cq_lut_vecmat_qk", "cq_lut_vecmat_pv",
     "cq_decode_attn_workspace", "cq_decode_attn", "cq_decode_attn_static", "cq_decode_attn_static_limit",
-    "cq_decode_attn_plan", "cq_decode_attn_wait_polls", "cq_decode_attn_gave_up", "cq_quantize_pack_wait_polls", "cq_decode_attn_single_launch", "cq_rope_append", "cq_quantize_pack_token",
+    "cq_decode_attn_plan", "cq_decode_attn_wait_polls", "cq_decode_attn_gave_up", "cq_quantize_pack_wait_polls", "cq_quantize_pack_plan", "cq_decode_attn_single_launch", "cq_rope_append", "cq_quantize_pack_token",
 )
 
 
@@ -27,6 +27,11 @@ class DecodePlan(C.Structure):
     """Mirror of `cq_decode_plan`."""
     _fields_ = [("threads", C.c_int), ("heads_per_unit", C.c_int), ("chunks", C.c_int), ("chunk_tokens", C.c_int),
                 ("launches", C.c_int), ("lds_bytes", C.c_int), ("register_logits", C.c_int)]
+
+
+class QuantizePlan(C.Structure):
+    """Mirror of `cq_quantize_plan`."""
+    _fields_ = [("channels", C.c_int), ("rows_per_thread", C.c_int), ("parts", C.c_int), ("part_rows", C.c_int), ("workgroups", C.c_int)]
 
 
 class DecodeArgs(C.Structure):
@@ -104,6 +109,8 @@ def load() -> C.CDLL:
     lib.cq_decode_attn.argtypes = [C.POINTER(DecodeArgs), vp]
     lib.cq_decode_attn_wait_polls.restype = i
     lib.cq_decode_attn_wait_polls.argtypes = [i]
+    lib.cq_quantize_pack_plan.restype = i
+    lib.cq_quantize_pack_plan.argtypes = [i, i, i, i, C.POINTER(QuantizePlan)]
     lib.cq_quantize_pack_wait_polls.restype = i
     lib.cq_quantize_pack_wait_polls.argtypes = [i]
     lib.cq_decode_attn_gave_up.restype = i

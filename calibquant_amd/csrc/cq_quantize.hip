@@ -20,6 +20,7 @@
 // only compares - the per-element IEEE division would otherwise bound the pass.
 #include "cq_common.h"
 
+#include <algorithm>
 #include <atomic>
 
 #include <type_traits>
@@ -996,7 +997,6 @@ static void launch_fused_rows(int nr, dim3 grid, hipStream_t st, const uint16_t*
     }
 }
 
-// true if the shape goes through the one-pass kernel (x read once, slice by slice in registers)
 // Compute units of the current device, asked once per process.
 static int persistent_units() {
     static std::atomic<int> cached{0};
@@ -1016,11 +1016,18 @@ static int persistent_units() {
 // Lanes per row, parts of the token axis, rows per part, rows per thread, workgroups of the launch.  Among the rows
 // per thread that give a part count that fits (at most 128; quarters only where all of them are resident at once) the one
 // that is expected to take the least, in hundredths of a microsecond: for each turn of a compute unit 0.08 us per row of
-// a thread and 0.4 us of folds and thresholds; with several parts 1 us for the exchange and what polling the other parts
-// costs.  Fitted to 20 shapes timed with every part count that fits: the choice is within 5 % of the best for 16 of them, 30 %
-// off for the worst (3 x 5 000 x 4 heads).
+// a thread and 0.4 us of folds and thresholds, a little more with the 52 rows that leave no register over; with several parts 1 us
+// for the exchange and what polling the other parts costs.  Fitted to 29 shapes, contiguous and strided, timed with every part
+// count that fits: 4 % from the best on average, 42 % for the worst (6 x 2 700 x 8 heads contiguous, from memory).
 // Why quarters at all, us of whole rows (best part count) / quarters: 4 x 320 x 8 heads 4.7 / 3.8, 1 x 1 024 4.9 / 4.2,
-// 8 x 1 024 7.2 / 6.4, 1 x 32 768 x 2 heads 11.8 / 8.3 (fewer channels to exchange per part).
+// 8 x 1 024 7.2 / 6.4, 1 x 32 768 x 2 heads 11.8 / 8.3 (fewer channels to exchange per part).  The quarters of a pair share
+// its 128-byte lines, and lie on one die only if the pairs are a multiple of eight; otherwise two dies fetch every line,
+// which a row then costs more the more of the chip asks for them (up to 0.2 us): 15 x 2 590 x 4 heads 12.2 / 17.5,
+// 30 x 3 300 x 2 heads 14.3 / 19.8, 19 x 1 994 x 2 heads 7.1 / 9.0; 1 x 12 171 x 4 heads, 64 workgroups, 10.3 / 8.2.
+// With the rotary embedding a row costs ten times as much, and of two workgroups on a compute unit the second takes little less
+// than the first, us, rows per thread 52 / 32 / 16 / 8: 6 x 3 328 x 8 heads 42 / 31 / 33 / 37, 64 x 1 300 x 2 heads 41 / 31 / 33 / 35,
+// 40 x 600 x 4 heads 31 / 28 / 19 / 23, 64 x 3 328 x 8 heads 263 / 292 / 298 / 374 (18 shapes: 1 % from the best on average,
+// 12 % for the worst).
 struct SplitPlan { int lpr, parts, part_rows, nr, grid; };
 constexpr int kFMostParts = 128;
 static bool split_plan(int64_t pairs, int T, bool rope, SplitPlan* sp) {
@@ -1036,7 +1043,10 @@ static bool split_plan(int64_t pairs, int T, bool rope, SplitPlan* sp) {
             const int least = (T - 1) / (n * pass) + 1, rows = (T - 1) / least + 1, p = (T - 1) / rows + 1;
             if (p > kFMostParts || p > room || (lpr == 4 && slices * p > room)) continue;   // (a pair's parts are resident together)
             const int64_t turns = (slices * p + cu - 1) / cu;                                  // per compute unit
-            const int64_t cost = turns * (8 * n + 40) + (p > 1 ? 100 + (lpr == 16 ? 15 : 5) * p : 0);
+            const int64_t row = lpr == 4 && pairs % 8 ? 8 + std::min<int64_t>(12, slices * p / 16) : 8;
+            const int64_t work = rope ? turns / 2 * (100 * n + 400) + turns % 2 * (65 * n + 300)
+                                      : turns * (row * n + (lpr == 16 && n == kFRows ? 65 : 40));
+            const int64_t cost = work + (p > 1 ? 100 + (rope ? 10 : 5) * p : 0);
             if (best < 0 || cost < best) {
                 best = cost;
                 *sp = SplitPlan{lpr, p, rows, n, static_cast<int>(slices * p < room ? slices * p : room)};
@@ -1613,6 +1623,19 @@ size_t cq_quantize_pack_workspace(int B, int T, int H, int D) {
         if (rec > need) need = rec;
     }
     return need;
+}
+
+int cq_quantize_pack_plan(int B, int T, int H, int rope, cq_quantize_plan* plan) {
+    if (!plan) return CQ_ERR_NULL;
+    if (B < 1 || T < 1 || H < 1) return CQ_ERR_SHAPE;
+    cq::SplitPlan spl;
+    if ((rope && T > cq::kFMaxT) || !cq::split_plan(static_cast<int64_t>(B) * H, T, rope != 0, &spl)) return CQ_ERR_UNSUPPORTED;
+    plan->channels = 8 * spl.lpr;
+    plan->rows_per_thread = spl.nr;
+    plan->parts = spl.parts;
+    plan->part_rows = spl.part_rows;
+    plan->workgroups = spl.grid;
+    return CQ_OK;
 }
 
 int cq_quantize_pack_wait_polls(int polls) {

@@ -81,6 +81,17 @@ int cq_quantize_pack(const void* x, int dtype, int B, int T, int H, int D,
  * until the bound is set again.  No counterpart in the reference, whose quant() is a chain of whole-tensor torch ops
  * (calibquant.py:24-42). */
 int cq_quantize_pack_wait_polls(int polls);
+/* How the one launch of cq_quantize_pack (rope = 0; cq_rope_quantize_pack: 1) cuts a (B, T, H, 128) tensor; nothing is
+ * launched, the only device call is a query of the compute-unit count, made once per process (256 without a device).
+ * CQ_ERR_UNSUPPORTED where there is no such launch (more rows than 128 parts hold).  No counterpart in the reference. */
+typedef struct cq_quantize_plan {
+    int channels;         /* channels of a workgroup: 128, or 32 (a quarter of the row) */
+    int rows_per_thread;  /* token rows that a thread keeps in registers at most */
+    int parts;            /* workgroups that share the token axis of a (batch, head) pair or of a quarter of it */
+    int part_rows;        /* token rows of a part (the last may have fewer) */
+    int workgroups;       /* of the launch; B * H * (128 / channels) * parts pieces of work go round them */
+} cq_quantize_plan;
+int cq_quantize_pack_plan(int B, int T, int H, int rope, cq_quantize_plan* plan);
 
 /* ------------------------------------------------------------------------
  * Prefill, keys: rotary embedding fused into the quantise-and-pack pass.

@@ -264,3 +264,28 @@ def test_host_shim_loads_and_matches_the_library():
     with pytest.raises(Exception):      # CPU tensors / wrong block size are refused before any launch
         shim.LayerStep(C.addressof(_lib.DecodeArgs()), 8, torch.zeros(1), torch.zeros(1), torch.zeros(1),
                        torch.zeros(1), 0, torch.zeros(1, dtype=torch.int64))
+
+
+def test_quantize_plan_of_shapes():
+    """How the one-pass quantiser cuts a tensor (256 compute units): quarters of the rows only for little work, and with many
+    rows each only where the quarters of a pair lie on one die (pairs a multiple of eight); with the rotary embedding
+    fused in, few rows per thread unless there are several turns for every compute unit."""
+    from calibquant_amd import _lib
+    lib = _lib.load()
+
+    def plan(B, T, H, rope=0):
+        p = _lib.QuantizePlan()
+        assert lib.cq_quantize_pack_plan(B, T, H, rope, ctypes.byref(p)) == 0
+        d = {n: getattr(p, n) for n, _ in p._fields_}
+        assert (d["parts"] - 1) * d["part_rows"] < T <= d["parts"] * d["part_rows"]
+        assert d["part_rows"] <= d["rows_per_thread"] * 256 * 8 // d["channels"] and d["workgroups"] <= 512
+        return d
+    for shape in ((15, 2590, 4), (30, 3300, 2), (60, 3328, 1), (19, 1994, 2)):
+        assert plan(*shape)["channels"] == 128, shape
+    assert plan(64, 3328, 8) == dict(channels=128, rows_per_thread=52, parts=4, part_rows=832, workgroups=512)
+    assert plan(1, 1024, 8)["channels"] == 32 and plan(1, 32768, 8)["channels"] == 32
+    assert plan(6, 3328, 8, 1)["rows_per_thread"] <= 32 and plan(64, 1300, 2, 1)["rows_per_thread"] <= 32
+    assert plan(40, 600, 4, 1)["rows_per_thread"] == 16 and plan(64, 3328, 8, 1)["rows_per_thread"] == 52
+    p = _lib.QuantizePlan()
+    assert lib.cq_quantize_pack_plan(1, 128 * 832, 1, 0, ctypes.byref(p)) == 0
+    assert lib.cq_quantize_pack_plan(1, 3329, 1, 1, ctypes.byref(p)) != 0 and lib.cq_quantize_pack_plan(1, 0, 1, 0, ctypes.byref(p)) != 0
