@@ -65,6 +65,12 @@ static inline int pick_chunks(int B, int T, int H) {
     return static_cast<int>(n);
 }
 
+// Extremes that keep a NaN, as torch's reductions and the one-pass kernel below do (one instruction each, as fminf / fmaxf).
+__device__ __forceinline__ float ext_min(float a, float b) { return __builtin_elementwise_minimum(a, b); }
+__device__ __forceinline__ float ext_max(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+struct OpExtMin { __device__ __forceinline__ float operator()(float a, float b) const { return ext_min(a, b); } };
+struct OpExtMax { __device__ __forceinline__ float operator()(float a, float b) const { return ext_max(a, b); } };
+
 // ---- 1. partial min / max -------------------------------------------------
 // grid (nchunk, H, B), 256 threads.  A row of D elements is covered by D/8
 // adjacent lanes with one 16-byte load each; 256/(D/8) rows per iteration.
@@ -94,7 +100,7 @@ __global__ __launch_bounds__(kQThreads) void minmax_partial_kernel(const uint16_
             float f[8];
             unpack8<DT>(v[u], f);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) { mn[i] = fminf(mn[i], f[i]); mx[i] = fmaxf(mx[i], f[i]); }
+            for (int i = 0; i < 8; ++i) { mn[i] = ext_min(mn[i], f[i]); mx[i] = ext_max(mx[i], f[i]); }
         }
     }
     __shared__ float smn[kQThreads * 8];
@@ -109,8 +115,8 @@ __global__ __launch_bounds__(kQThreads) void minmax_partial_kernel(const uint16_
     for (int d = threadIdx.x; d < g.D; d += kQThreads) {
         float a = INFINITY, z = -INFINITY;
         for (int r = 0; r < rows_per_iter; ++r) {
-            a = fminf(a, smn[r * g.D + d]);
-            z = fmaxf(z, smx[r * g.D + d]);
+            a = ext_min(a, smn[r * g.D + d]);
+            z = ext_max(z, smx[r * g.D + d]);
         }
         float* o = part + ((static_cast<int64_t>(b) * g.H + h) * g.nchunk + c) * 2 * g.D;
         o[d] = a;
@@ -160,15 +166,15 @@ __global__ void stats_kernel(const float* __restrict__ part, QuantGeom g, float 
     const float* p = part + static_cast<int64_t>(bh) * g.nchunk * 2 * g.D;
 #pragma unroll 4
     for (int c = pt; c < g.nchunk; c += nparts) {   // independent loads: four pairs in flight
-        a = fminf(a, p[c * 2 * g.D + d]);
-        z = fmaxf(z, p[c * 2 * g.D + g.D + d]);
+        a = ext_min(a, p[c * 2 * g.D + d]);
+        z = ext_max(z, p[c * 2 * g.D + g.D + d]);
     }
     sh[(pt * 2) * g.D + d] = a;
     sh[(pt * 2 + 1) * g.D + d] = z;
     __syncthreads();
     for (int q = 0; q < nparts; ++q) {
-        a = fminf(a, sh[(q * 2) * g.D + d]);
-        z = fmaxf(z, sh[(q * 2 + 1) * g.D + d]);
+        a = ext_min(a, sh[(q * 2) * g.D + d]);
+        z = ext_max(z, sh[(q * 2 + 1) * g.D + d]);
     }
     const float x_min = rnd<DT>(a * clip);
     const float x_max = rnd<DT>(z * clip);
@@ -229,14 +235,14 @@ __global__ __launch_bounds__(kStatThreads) void tensor_stats_kernel(const float*
     const int64_t n = npairs * 2 * D;
     for (int64_t e = tid; e < n; e += kStatThreads) {
         const float v = part[e];
-        if ((e / D) & 1) z = fmaxf(z, v); else a = fminf(a, v);   // [pair][min row | max row][D]
+        if ((e / D) & 1) z = ext_max(z, v); else a = ext_min(a, v);   // [pair][min row | max row][D]
     }
-    a = wave_min(a);
-    z = wave_max(z);
+    a = wave_reduce(a, OpExtMin(), INFINITY);
+    z = wave_reduce(z, OpExtMax(), -INFINITY);
     if ((tid & 63) == 0) { smn[tid >> 6] = a; smx[tid >> 6] = z; }
     __syncthreads();
     if (tid == 0) {
-        for (int w = 0; w < kStatThreads / kWave; ++w) { a = fminf(a, smn[w]); z = fmaxf(z, smx[w]); }
+        for (int w = 0; w < kStatThreads / kWave; ++w) { a = ext_min(a, smn[w]); z = ext_max(z, smx[w]); }
         const float x_min = rnd<DT>(a * clip);
         const float x_max = rnd<DT>(z * clip);
         const float diff = rnd<DT>(x_max - x_min);
@@ -782,7 +788,7 @@ __global__ __launch_bounds__(kFThreads, kFResident) void fused_pack_kernel(const
     constexpr int kInf = Keys<DT>::hi;
     const bool nan_here = static_cast<short>(top_s) > kInf || static_cast<short>(top_s >> 16) > kInf ||
                           (top_u & 0xffffu) > (0x8000u | kInf) || (top_u >> 16) > (0x8000u | kInf);
-    if (__ballot(nan_here)) {   // (not a supported input; the codes of such elements are 0 all the same)
+    if (__ballot(nan_here)) {   // (its channel's statistics are NaN and the codes 0, as the ops give; other channels are not touched)
 #pragma unroll
         for (int i = 0; i < NR; ++i) sanitize<DT>(v[i]);
     }

@@ -360,3 +360,36 @@ def test_quantize_pack_on_two_streams(ops):
         for a, b in zip(got, want):
             assert all(torch.equal(u, v) for u, v in zip(a, b))
         assert torch.equal(decode.out, good)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("shape", [(1, 70, 2, 128), (3, 333, 5, 128), (1, 4100, 2, 128), (20, 1700, 8, 128), (2, 300, 3, 64), (1, 500, 2, 256)])
+def test_quantize_pack_of_nan(ops, shape, bits, dtype):
+    """A NaN of either sign makes the statistics of its channel NaN and its codes 0, as the ops do, in the one-pass kernel (one
+    part, several, whole rows and quarters) and in the three launches alike; other channels are what they were."""
+    B, T, H, D = shape
+    print(f"case quantize_pack nan shape={shape} bits={bits} dtype={dtype}", flush=True)
+    x = O.round_to(np.random.default_rng(T).standard_normal(shape, dtype=np.float32), dtype)
+    clip = CLIPS[bits][0]
+    plain = ops.quantize_pack(to_gpu(x, dtype), bits, clip)
+    g = to_gpu(x, dtype)
+    raw = g.view(torch.int16)
+    raw[0, T // 2, 0, 5] = 0x7fff                    # the largest pattern of a positive NaN, the smallest of a negative one
+    raw[B - 1, T - 1, H - 1, 62] = -0x8000 | (0x7f81 if dtype == "bf16" else 0x7c01)
+    raw[B - 1, 0, H - 1, 63] = 0x7f81 if dtype == "bf16" else 0x7c01
+    hit = np.zeros((B, H, D), bool)
+    hit[0, 0, 5] = hit[B - 1, H - 1, 62] = hit[B - 1, H - 1, 63] = True
+    codes, s, z = ops.quantize_pack(g, bits, clip)
+    xq, s2, z2 = ops.quant_codes(g, bits, clip)
+    torch.cuda.synchronize()
+    with np.errstate(all="ignore"):
+        oc, os_, oz = O.quantize_pack(to_np(g), bits, clip, dtype)
+    assert np.isnan(os_[hit]).all() and not np.isnan(os_[~hit]).any()
+    assert np.array_equal(codes.cpu().numpy(), oc)
+    for a, b, p in ((s, os_, plain[1]), (z, oz, plain[2])):
+        assert np.array_equal(np.isnan(to_np(a)), hit) and same_bits(to_np(a)[~hit], b[~hit]) and same_bits(to_np(a)[~hit], to_np(p)[~hit])
+    # quant(): NaN statistics make every value of the channel NaN
+    assert np.array_equal(np.isnan(to_np(s2[:, 0])), hit) and np.array_equal(np.isnan(to_np(xq)), np.broadcast_to(hit[:, None], shape))
+    _, st, zt = ops.quant_codes_tensor(g, bits, clip)
+    assert bool(st.isnan()) and bool(zt.isnan())
