@@ -1134,7 +1134,8 @@ static int run_quant(const void* x, QuantGeom g, int bits, float clip, uint8_t* 
     uint16_t* zp = static_cast<uint16_t*>(zero);
     if (rope && (xq || g.T > kFMaxT || !one_pass_shape(g, codes))) return CQ_ERR_UNSUPPORTED;
     SplitPlan spl;
-    if (!xq && one_pass_shape(g, codes) && split_plan(static_cast<int64_t>(g.B) * g.H, g.T, rope != nullptr, &spl) &&
+    // (a negative clip factor swaps minimum and maximum: the code then falls with x, which the thresholds do not cover)
+    if (!xq && clip >= 0.0f && one_pass_shape(g, codes) && split_plan(static_cast<int64_t>(g.B) * g.H, g.T, rope != nullptr, &spl) &&
         !(rope && spl.parts > 1 && rope_overlaps(xp, g, *rope))) {
         const int spin = g_qspin.load(std::memory_order_relaxed);
         int* status = nullptr;

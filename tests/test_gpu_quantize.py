@@ -393,3 +393,14 @@ def test_quantize_pack_of_nan(ops, shape, bits, dtype):
     assert np.array_equal(np.isnan(to_np(s2[:, 0])), hit) and np.array_equal(np.isnan(to_np(xq)), np.broadcast_to(hit[:, None], shape))
     _, st, zt = ops.quant_codes_tensor(g, bits, clip)
     assert bool(st.isnan()) and bool(zt.isnan())
+
+
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("shape", [(2, 300, 3, 128), (2, 4100, 2, 128)])
+def test_quantize_pack_of_a_negative_clip_factor(ops, shape, bits):
+    """A negative factor gives a negative scale: the op chain still says what the codes are."""
+    x = O.round_to(np.random.default_rng(2).standard_normal(shape, dtype=np.float32), "bf16")
+    codes, s, z = ops.quantize_pack(to_gpu(x, "bf16"), bits, -0.5)
+    oc, os_, oz = O.quantize_pack(x, bits, -0.5, "bf16")
+    assert (os_ < 0).all() and same_bits(to_np(s), os_) and same_bits(to_np(z), oz)
+    assert np.array_equal(codes.cpu().numpy(), oc)
