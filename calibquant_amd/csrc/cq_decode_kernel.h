@@ -155,15 +155,19 @@ constexpr int plan_chunk(int bits, bool vtok, int hpb) {
 constexpr int kPlanLong = 10048;                     // four heads at 1 bit, where that saves the chunks
 constexpr int kPlanPair4 = 4096, kPlanPair2 = 4736;  // 512 threads: four heads, two heads (1 bit)
 
-// Launches whose packed rows (and per-token statistics) are more than half of the 256 MB memory-side cache, each read by one
-// unit: nothing of them would be found there again, and non-temporal loads stream faster.  us, ordinary / non-temporal:
-// batch 256 x 3 328 (218 MB) 57.3 / 53.6, batch 64 x 3 328 at 2 bits (109 MB) 27.6 / 27.7, with per-token values (109 MB)
-// 36.9 / 35.3; below, or where two units share the rows: 8 x 32 768 (67 MB) 26.7 / 28.0, 16 x 9 984 with two units per
-// kv head 20.5 / 21.9.  Instantiated for the forms that such launches take (four heads per unit in 512 threads; per-token
-// values with the most heads a unit has).
-constexpr bool stream_form(int bits, bool vtok, int hpb, int nt) { return vtok ? hpb == (bits == 1 ? 4 : 2) : hpb == 4 && nt == 512; }
+// Launches whose packed rows (and per-token statistics) are most of the 256 MB memory-side cache or more, each read by one
+// unit: hardly anything of them would be found there again, and non-temporal loads stream faster.  us at 3 328 + 128 tokens,
+// ordinary / non-temporal, with the rows from memory (a model's other layers in between) and, in brackets, the same call repeated:
+// 1 bit, 123 MB 45.2 / 43.4 (39.2 / 41.0), 150 MB 52.3 / 51.0 (46.5 / 48.3), 177 MB 61.0 / 58.5 (56.4 / 55.6), batch 256, 218 MB, 71.9 / 69.5
+// (72.8 / 65.5); with per-token values 82 MB 34.2 / 33.9 (31.3 / 32.7), 164 MB 66.6 / 64.7 (60.3 / 62.8), 204 MB 82.6 / 81.7 (80.6 / 80.0); 2 bits,
+// 109 MB 26.9 / 27.5 (23.3 / 27.0), 218 MB 52.2 / 52.5 (45.9 / 51.5), 245 MB 63.5 / 61.3 (60.9 / 61.2), 436 MB 101.0 / 101.5 (101.3 / 99.8), with
+// per-token values no difference at any size.  So the lines are 168 MiB and, at 2 bits, 228 MiB: from there on neither gets
+// slower.  Where two units share the rows: 16 x 9 984 with two units per kv head 20.5 / 21.9; in chunks: 8 x 32 768 (67 MB)
+// 26.7 / 28.0.  Instantiated for the forms that such launches take (four heads per unit).
+constexpr bool stream_form(int bits, bool vtok, int hpb, int nt) { return hpb == 4 && (vtok ? bits == 1 : nt == 512); }
 inline bool launch_streams(int bits, bool vtok, int hpb, int nt, int groups, int nsplit, int64_t tokens) {   // tokens: over all (batch, kv head) pairs
-    return stream_form(bits, vtok, hpb, nt) && groups == 1 && nsplit == 1 && tokens * (32 * bits + (vtok ? 16 : 0)) >= (static_cast<int64_t>(100) << 20);
+    return stream_form(bits, vtok, hpb, nt) && groups == 1 && nsplit == 1 &&
+           tokens * (32 * bits + (vtok ? 16 : 0)) >= (static_cast<int64_t>(bits == 1 ? 168 : 228) << 20);
 }
 
 // What a launch of units of hpb heads in nt threads runs with: the rounds of logits its instantiation keeps in

@@ -209,12 +209,12 @@ def test_token_values_large_scale_of_a_token_without_weight(ops, dtype, far, bit
 @pytest.mark.parametrize("bits, vals, G, option", [(1, "channel", 4, "none"), (1, "channel", 3, "device-rows"), (2, "channel", 4, "mask"),
                                                    (1, "token", 4, "none"), (2, "token", 2, "device-rows")])
 def test_decode_attn_streamed_rows_equal_a_small_batch(ops, bits, vals, G, option):
-    """Launches that read more than half of the memory-side cache take their packed rows with non-temporal loads: the
-    same arithmetic, so the first rows of such a batch equal a batch of their own in units of the same form, bit for
-    bit."""
+    """Launches that read most of the memory-side cache (168 MiB; at 2 bits 228 MiB) take their packed rows with
+    non-temporal loads: the same arithmetic, so the first rows of such a batch equal a batch of their own in units of
+    the same form, bit for bit.  (2 bits with per-token values: large, without such loads.)"""
     per = 32 * bits + (16 if vals == "token" else 0)
     H, T, R, S = 8, 1800, 20, 3
-    B = (100 << 20) // (per * H * T) + 2
+    B = ((168 if bits == 1 else 228) << 20) // (per * H * T) + 2
     g = torch.Generator(device="cuda").manual_seed(B)
     k = torch.randn((B, T, H, 128), generator=g, device="cuda").to(torch.bfloat16)
     v = torch.randn((B, T, H, 128), generator=g, device="cuda").to(torch.bfloat16)
