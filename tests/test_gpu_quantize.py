@@ -1,5 +1,7 @@
 """GPU parity of the prefill quantise-and-pack kernels against the oracle:
 bit-exact codes, scales and zero-points (through the C-ABI library)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -105,8 +107,8 @@ def test_quant_and_encode_operators(ops, bits, dtype):
 def test_quantize_pack_matches_torch_device_op_chain(ops, bits, B):
     """torch's own device kernels, run op by op on the 16-bit tensor, are the
     primitives the reference executes (calibquant.py:27-36).  At batch 64 (the benchmark's prefill
-    tensor) every workgroup of the one-pass kernel walks eight slices, the later ones with part of
-    their rows staged through LDS."""
+    tensor) every workgroup of the one-pass kernel walks four parts of pairs, whose rows it requests while it packs
+    the part before."""
     T, H, D = 3328, 8, 128
     g = torch.Generator(device="cuda").manual_seed(5)
     x = torch.randn((B, T, H, D), generator=g, device="cuda", dtype=torch.float32).to(torch.bfloat16)
@@ -146,16 +148,15 @@ def test_quantize_pack_full_size_properties(ops, bits):
     assert (un2 != un).float().mean().item() < 2e-3
 
 
-# Token axes beyond what one workgroup's registers hold of a slice (3 328 rows): the one-pass kernel splits a slice
-# between 2, 4, ... workgroups of its launch when a part then has more than 2 048 rows (parts x rows per part ->
-# rows per thread); the other shapes take three launches.
-LONG_SHAPES = [(2, 9984, 8, 128),    # 4 x 2496 -> 10: the 26B prompt's token count
-               (3, 3329, 2, 128),    # just beyond one workgroup: three launches
-               (4, 13000, 1, 128),   # 4 x 3250 -> 13
-               (2, 40000, 2, 128),   # 16 x 2500 -> 10
-               (1, 40000, 1, 128),   # a single (batch, head) pair: three launches
-               (9, 5000, 8, 128),    # 2 x 2500 -> 10; 288 slices x 2 parts: more ids than workgroups, 3 steps
-               (2, 7000, 8, 128)]    # three launches
+# Token axes beyond what one workgroup's registers hold (832 rows, 3 328 of a quarter of the channels): several parts of a
+# pair's rows, whose workgroups exchange their extremes.
+LONG_SHAPES = [(2, 9984, 8, 128),    # the 26B prompt's token count
+               (3, 3329, 2, 128),    # just beyond one workgroup
+               (4, 13000, 1, 128),
+               (2, 40000, 2, 128),
+               (1, 40000, 1, 128),   # a single (batch, head) pair
+               (9, 5000, 8, 128),    # more parts than workgroups
+               (2, 7000, 8, 128)]
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
@@ -187,10 +188,10 @@ def test_quantize_pack_long_token_axis_strided_view(ops):
 
 
 def test_quantize_pack_split_slices_give_up_and_the_host_reports_it(ops):
-    """The parts of a split slice wait for each other a bounded number of polls.  With the bound at zero every
-    part goes on alone (the kernel ends normally; its statistics are those of single parts, i.e. not valid): the
-    call returns success, the next call on the device reports the failure once, and from then on long token axes
-    take the three-launch path - bit-exact - until the bound is set again."""
+    """The parts of a pair wait for each other a bounded number of polls.  A bound of zero takes their exchange out of
+    service: every part goes on alone (the kernel ends normally; its statistics are those of single parts, i.e. not
+    valid), the call returns success, the next call on the device reports the failure once, and from then on shapes of
+    several parts take the three-launch path - bit-exact - until the bound is set again."""
     from calibquant_amd import _lib
     lib = _lib.load()
     B, T, H, D = 2, 9984, 2, 128
@@ -246,7 +247,7 @@ def test_quantize_pack_one_pass_cuts_bit_exact(ops, shape, bits, dtype):
         oc, os_, oz = O.quantize_pack(x, bits, CLIPS[bits][0], dtype)
     codes, s, z = ops.quantize_pack(to_gpu(x, dtype), bits, CLIPS[bits][0])
     torch.cuda.synchronize()
-    # (zero-points of equal value: the sign of a zero minimum is the only one that min() over +0 and -0 leaves open)
+    # (equal values: the sign of a zero minimum is the only one that min() over +0 and -0 leaves open)
     assert same_bits(to_np(s), os_) and np.array_equal(to_np(z), oz, equal_nan=True)
     assert np.array_equal(codes.cpu().numpy(), oc)
 
@@ -403,4 +404,31 @@ def test_quantize_pack_of_a_negative_clip_factor(ops, shape, bits):
     codes, s, z = ops.quantize_pack(to_gpu(x, "bf16"), bits, -0.5)
     oc, os_, oz = O.quantize_pack(x, bits, -0.5, "bf16")
     assert (os_ < 0).all() and same_bits(to_np(s), os_) and same_bits(to_np(z), oz)
+    assert np.array_equal(codes.cpu().numpy(), oc)
+
+
+# More parts than workgroups, so that a workgroup goes on to a second part whose rows it has requested while it packed the
+# first, with the parts of some pairs on either side of a turn (the grid is no multiple of the part count) and ragged last
+# parts.
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("bits", [1, 2])
+@pytest.mark.parametrize("shape", [(30, 2400, 8), (30, 2399, 8), (43, 3327, 3), (25, 3328, 8)])
+def test_quantize_pack_parts_across_turns_bit_exact(ops, shape, bits, dtype):
+    from calibquant_amd import _lib
+    B, T, H = shape
+    p = _lib.QuantizePlan()
+    _lib.check(_lib.load().cq_quantize_pack_plan(B, T, H, 0, ctypes.byref(p)), "plan")
+    assert p.channels == 128 and p.parts > 1 and B * H * p.parts > p.workgroups and p.workgroups % p.parts
+    print(f"case quantize_pack across turns shape={shape} bits={bits} dtype={dtype}", flush=True)
+    rng = np.random.default_rng(T)
+    x = O.round_to(rng.standard_normal((B, T, H, 128), dtype=np.float32), dtype)
+    # every part of a pair has the extremes of some channels
+    for part in range(p.parts):
+        x[:, part * p.part_rows, :, part] = 9.0
+        x[:, min(T, (part + 1) * p.part_rows) - 1, :, 64 + part] = -9.0
+    codes, s, z = ops.quantize_pack(to_gpu(x, dtype), bits, CLIPS[bits][0])
+    torch.cuda.synchronize()
+    oc, os_, oz = O.quantize_pack(x, bits, CLIPS[bits][0], dtype)
+    for a, b in ((s, os_), (z, oz)):     # (no zero minimum here: bit for bit)
+        assert np.array_equal(to_np(a).view(np.uint32), np.asarray(b, np.float32).view(np.uint32))
     assert np.array_equal(codes.cpu().numpy(), oc)

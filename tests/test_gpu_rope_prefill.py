@@ -2,6 +2,8 @@
 `rope_quantize_pack` (image block of the keys: rotation fused into the quantise-and-pack pass).
 Bit-exact against the oracle (`O.rope` then `O.quantize_pack`), against the same arithmetic
 written as separate torch ops on the device, and against the two-step HIP path."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -182,3 +184,23 @@ def test_rope_quantize_pack_parts_that_wait_in_vain(ops, B, T, Hkv, bits, dtype)
             assert torch.equal(got[0], want[0]) and all(same_bits(to_np(a), to_np(b)) for a, b in zip(got[1:], want[1:]))
     finally:
         lib.cq_quantize_pack_wait_polls(before)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("B, T, Hkv", [(30, 2399, 8), (40, 1700, 8)])
+def test_rope_quantize_pack_parts_across_turns(ops, B, T, Hkv, dtype):
+    """More parts than workgroups, and a grid that is no multiple of the part count: the bits of the two-step path."""
+    from calibquant_amd import _lib
+    p = _lib.QuantizePlan()
+    _lib.check(_lib.load().cq_quantize_pack_plan(B, T, Hkv, 1, ctypes.byref(p)), "plan")
+    assert p.parts > 1 and B * Hkv * p.parts > p.workgroups and p.workgroups % p.parts
+    print(f"case rope_quantize_pack across turns B={B} T={T} Hkv={Hkv} dtype={dtype}", flush=True)
+    torch.manual_seed(T)
+    x = torch.randn(B, T, Hkv, 128, device="cuda").to(TDT[dtype])
+    cos, sin = _tables(T + 60, 128, dtype)
+    out = torch.empty_like(x)
+    got = ops.rope_quantize_pack(x, cos, sin, 5, out, 1, 0.5)
+    two = ops.rope_rows(x, cos, sin, 5)
+    assert torch.equal(out, two)
+    for a, b in zip(got, ops.quantize_pack(two, 1, 0.5)):
+        assert torch.equal(a, b)
