@@ -86,7 +86,7 @@ static void plan_for(const cq_decode_args* a, Plan* p, int hpb, int nh, int nt, 
     const size_t rows = static_cast<size_t>(a->B) * a->Hq;
     p->ws_mm = nsplit > 1 ? ((rows * nsplit * 2 * sizeof(float) + 255) / 256 * 256) : 0;
     p->ws_part = nsplit > 1 ? (rows * p->nx * (kD + 2) * sizeof(float) + 255) / 256 * 256 : 0;
-    // counters: [unit] partials written, then the min / max records of the single-launch step
+    // counters: [unit] partials written (one launch: the window's announcement), then the min / max records of that form
     p->ws_cnt = nsplit > 1 ? (static_cast<size_t>(units) * sizeof(unsigned long long) + 255) / 256 * 256 +
                                  static_cast<size_t>(units) * hpb * nsplit * 16 : 0;
     p->fused = false;
@@ -306,7 +306,7 @@ static int decode_entry(const cq_decode_args* a, void* workspace, size_t workspa
     g.status = status;
     g.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
     uint32_t ep = g_epoch.fetch_add(1, std::memory_order_relaxed) + 1;
-    g.epoch = ep ? ep : g_epoch.fetch_add(1, std::memory_order_relaxed) + 1;   // 0 marks an empty counter
+    g.epoch = ep ? ep : g_epoch.fetch_add(1, std::memory_order_relaxed) + 1;   // (0 is never an epoch)
     g.B = a->B; g.Hq = a->Hq; g.Hkv = a->Hkv; g.T = a->T; g.R = a->R; g.S = a->sprompt_len;
     g.nsplit = p.nsplit; g.chunk = p.chunk; g.nx = p.nx;
     g.calib = a->calibrate; g.off_max = a->calib_off_max; g.off_min = a->calib_off_min;

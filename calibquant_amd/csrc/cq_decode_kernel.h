@@ -831,8 +831,8 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         float o_img = 0.f;  // thread (h, d) = (tid / kD, tid % kD) for tid < HPB*kD
 
         if constexpr (CHUNKED) {
-            // One launch: this chunk's min / max go out now (write-through stores, waited for, then the arrival
-            // count); the other chunks' are collected further down.
+            // One launch: this chunk's min / max go out now (write-through stores that nothing waits for); the other
+            // chunks' are collected further down.
             // (padding heads repeat the last real one: every head of the unit's layout has its records)
             if (g.fused && has_img && wv == 0 && (lane & 15) == 0 && (lane >> 4) < HPB) {
                 unsigned long long* o = g.rec + ((unit * HPB + hl) * g.nsplit + split) * 2;

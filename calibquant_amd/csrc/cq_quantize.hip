@@ -36,7 +36,7 @@ struct QuantGeom {
     int B, T, H, D;
     int64_t sb, st, sh;   // element strides of x
     int nchunk, chunk;    // token chunks
-    FastDiv dT, dH;       // divisors T and H of a flat (b, h, t) row index (per-token quantiser)
+    FastDiv dH;           // divisor H
     FastDiv dTB;          // per-token quantiser: workgroup passes per (batch, head)
     int shared_stats;     // non-zero: one row of statistics / thresholds serves every (batch, head) (whole-tensor mode)
     // One-pass kernel: `parts` workgroups share a (batch, head) pair, `part_rows` token rows each, and, if there are
@@ -431,12 +431,14 @@ __global__ __launch_bounds__(kQThreads) void emit_kernel(const uint16_t* __restr
 // requested while this one's are packed.
 //
 // What bounds it: memory.  Batch 64 x 3 328 tokens x 8 heads, 1 bit, 464 MB, us: the strided key block of a fused projection 106
-// -> 92, a contiguous tensor 129 -> 93, 2 bits 130 -> 106; the loads alone 75, the code stores 10 - 12 more whatever their
-// form (a streaming kernel without any structure: 64 and 75).  Against a 1 024-thread workgroup per compute unit that
+// -> 92, then 88 with the parts' records read once for two channels (no registers spilled); a contiguous tensor 129 -> 93, 2 bits
+// 130 -> 106; the loads alone 75, the code stores 10 - 12 more whatever their form (a streaming kernel without any structure: 64 and 75).  Against a 1 024-thread workgroup per compute unit that
 // owned 64-byte quarters of 3 328 rows:
 //  - whole rows instead of 64-byte pieces: a contiguous tensor 129 -> 103 (its pieces lay 2 KB apart, on few channels);
-//  - non-temporal loads and stores (every line is used once, by one workgroup): 105 -> 94; only with 40 or more rows per
-//    thread, i.e. for tensors that the memory-side cache would not have held for the reader before;
+//  - non-temporal loads (every line is used once, by one workgroup): 97 -> 89; with 40 or more rows per thread, which is what
+//    split_plan() gives large tensors and small ones of few channels.  us ordinary / non-temporal, from memory (and where the
+//    memory-side cache holds the tensor): 70 x 831 x 2 heads 9.3 / 9.5 (7.9 / 8.4), 25 x 600 x 8 10.2 / 9.6 (7.0 / 7.5), 21 x 1 700 x 8
+//    22.5 / 21.5 (20.7 / 19.5), 64 x 1 664 x 8 57 / 51 (49 / 50), 16 x 9 984 x 8 86 / 78;
 //  - codes from packed 16-bit comparisons (EmitPlan), about 15 vector instructions per 8 elements instead of 24;
 //  - the threshold search by inverting the op chain (threshold_key) instead of four rounds of 16-ary search.
 // More and smaller workgroups (3 x 24 rows, 4 x 16 or 20, 2 x 28) measured 99 to 127: the folds, the exchange and the
@@ -651,7 +653,7 @@ __global__ __launch_bounds__(kFThreads, kFResident) void fused_pack_kernel(const
     const int tid = threadIdx.x, q4 = tid & 3;
     const int piece = tid % LPR, row = tid / LPR;
     const int npairs = g.B * g.H;
-    const int nids = npairs * (16 / LPR) * g.parts;   // (the host keeps this below 2^31)
+    const int nids = npairs * (16 / LPR) * g.parts;   // (below 2^31 with the grid added: split_plan())
     // id = slice * parts + part; slice = quarter * pairs + pair: with eight heads the quarters of a pair, which share its
     // lines of x and of the codes, come to lie on one die (ids a multiple of 8 apart)
     auto slice_of = [&](int id) { return SPLIT ? static_cast<int>(g.dP.quot(static_cast<uint32_t>(id))) : id; };
@@ -1047,7 +1049,7 @@ static bool split_plan(int64_t pairs, int T, bool rope, SplitPlan* sp) {
             if (fused_rows(n, lpr, rope) != n) continue;
             // the fewest parts that n rows per thread hold (more of them only cost more); none of them empty
             const int least = (T - 1) / (n * pass) + 1, rows = (T - 1) / least + 1, p = (T - 1) / rows + 1;
-            if (p > kFMostParts || p > room || (lpr == 4 && slices * p > room)) continue;   // (a pair's parts are resident together)
+            if (p > kFMostParts || p > room || slices * p > 0x7fffffff - room || (lpr == 4 && slices * p > room)) continue;   // (a pair's parts are resident together)
             const int64_t turns = (slices * p + cu - 1) / cu;                                  // per compute unit
             const int64_t row = lpr == 4 && pairs % 8 ? 8 + std::min<int64_t>(12, slices * p / 16) : 8;
             const int64_t work = rope ? turns / 2 * (100 * n + 400) + turns % 2 * (65 * n + 300)
@@ -1262,7 +1264,6 @@ static int quant_entry(const void* x, int dtype, int B, int T, int H, int D, int
     g.sb = sb; g.st = st; g.sh = sh;
     g.nchunk = pick_chunks(B, T, H);
     g.chunk = (T + g.nchunk - 1) / g.nchunk;
-    g.dT.set(static_cast<uint32_t>(T));
     g.dH.set(static_cast<uint32_t>(H));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == CQ_BF16)
@@ -1733,7 +1734,6 @@ int cq_quantize_pack_token(const void* x, int dtype, int B, int T, int H, int D,
     g.B = B; g.T = T; g.H = H; g.D = D;
     g.sb = stride_b; g.st = stride_t; g.sh = stride_h;
     g.nchunk = 1; g.chunk = T;
-    g.dT.set(static_cast<uint32_t>(T));
     g.dH.set(static_cast<uint32_t>(H));
     // A lane per group from 56 K rows on, where it has enough workgroups to fill the chip: us, four lanes a group / one (bf16, 1 bit),
     // 24 x 150 tokens x 8 heads 3.8 / 4.3, 3 x 1 700 4.3 / 4.6, 2 x 3 328 5.0 / 4.9 (2 bits 5.9 / 6.0, fp16 5.0 / 5.3), 4 x 2 000 5.8 / 5.3 (2 bits
@@ -1793,7 +1793,6 @@ int cq_quant_tensor(const void* x, int dtype, int B, int T, int H, int D, int64_
     g.sb = stride_b; g.st = stride_t; g.sh = stride_h;
     g.nchunk = cq::pick_chunks(B, T, H);
     g.chunk = (T + g.nchunk - 1) / g.nchunk;
-    g.dT.set(static_cast<uint32_t>(T));
     g.dH.set(static_cast<uint32_t>(H));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == CQ_BF16)

@@ -189,9 +189,9 @@ def forward_internlm2_calibquant(self, hidden_states: torch.Tensor, attention_ma
     # The reference rotates the whole tensors with a chain of torch ops first (patch_internvl.py:258-260) and
     # quantises afterwards (:295-297).  With `cq_fused_rope` set on the module the image block of the keys is
     # rotated inside the quantise-and-pack pass instead (`cq_rope_quantize_pack`: un-rotated keys read once,
-    # rotated rows written once, quantised from the registers) - same bits, one launch fewer, but slower at the
-    # benchmark shape (348 against 309 us: a slice then reads two 32-byte pieces per row instead of one of 64,
-    # which HBM serves as 64-byte fetches), so it is not the default.
+    # rotated rows written once, quantised from the registers) - same bits, one launch fewer, but no faster at the
+    # benchmark shape (279 against 267 us per key tensor; the rotation, not the extra pass, is what takes the time), so it is
+    # not the default.
     hip_rope = (q_len > 1 and qkv.is_cuda and qkv.dtype in (torch.bfloat16, torch.float16) and D == 128
                 and position_ids is not None and position_ids.is_cuda and position_ids.dtype == torch.int64
                 and tuple(position_ids.shape) == (bsz, q_len))
