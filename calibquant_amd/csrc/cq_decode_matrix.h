@@ -36,8 +36,8 @@ static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st
 }
 
 // A chunked launch has one instantiation, with the mask and the row count.  Of the kernels that chunked plans ask for,
-// those of 512 threads and of per-token values keep within the 128 registers; those of ten rounds spill up to 22 (48 B of
-// scratch per lane), those of sixteen 78 to 126 (152 to 224 B; 7 to 28 in single launches without mask and row count).
+// those of 512 threads and of per-token values keep within the 128 registers; those of ten rounds spill up to 16 (36 B of
+// scratch per lane), those of sixteen 76 to 108 (2 to 13 in single launches without mask and row count).
 // SINGLE: no plan chunks such units.
 template <int BITS, int HPB, typename DT, int NT, int REGL, int NH = HPB, bool VTOK = false, bool SINGLE = false>
 static int launch_matrix_unit(const DecodeGeom& g, unsigned units, hipStream_t st) {

@@ -431,7 +431,7 @@ __global__ __launch_bounds__(kQThreads) void emit_kernel(const uint16_t* __restr
 // requested while this one's are packed.
 //
 // What bounds it: memory.  Batch 64 x 3 328 tokens x 8 heads, 1 bit, 464 MB, us: the strided key block of a fused projection 106
-// -> 92, then 88 with the parts' records read once for two channels (no registers spilled); a contiguous tensor 129 -> 93, 2 bits
+// -> 92, then 88 with the parts' records read once for two channels (4 registers spilled instead of 13); a contiguous tensor 129 -> 93, 2 bits
 // 130 -> 106; the loads alone 75, the code stores 10 - 12 more whatever their form (a streaming kernel without any structure: 64 and 75).  Against a 1 024-thread workgroup per compute unit that
 // owned 64-byte quarters of 3 328 rows:
 //  - whole rows instead of 64-byte pieces: a contiguous tensor 129 -> 103 (its pieces lay 2 KB apart, on few channels);

@@ -42,7 +42,7 @@ def empty_token_rows(B: int, T: int, H: int, D: int, dtype, device) -> torch.Ten
     """An uninitialised (B, T, H, D) tensor for keys or values that the quantiser will read: token rows of
     H * D elements, plus 128 bytes of padding per row where rows would otherwise lie a multiple of 2 KB apart,
     which spreads a head's rows over more memory channels.  (It took the quantiser from 129 to 105 us at batch 64 x 3 328
-    tokens x 8 heads while that read rows in 64-byte pieces; now that it reads them whole, a contiguous tensor takes 93.)
+    tokens x 8 heads while that read rows in 64-byte pieces; now that it reads them whole, a contiguous tensor takes no longer.)
     The result is a view; D stays contiguous."""
     row = H * D
     pad = 64 if (row * torch.empty((), dtype=dtype).element_size()) % 2048 == 0 else 0
