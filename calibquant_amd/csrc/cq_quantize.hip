@@ -619,7 +619,7 @@ __device__ __forceinline__ void rows_again(const uint16_t* x, const QuantGeom& g
                  Cvt<DT>::from_float(rnd<DT>(Cvt<DT>::hi(v) * Cvt<DT>::hi(cw)) + Cvt<DT>::hi(y) * Cvt<DT>::hi(sw)) << 16);
         }
     } else {
-const uint16_t* p = col + static_cast<int64_t>(t) * g.st + channel;
+        const uint16_t* p = col + static_cast<int64_t>(t) * g.st + channel;
 #pragma unroll 1
         for (int rows = end - t; rows > 0; --rows, p += g.st) take(word(p));
     }
