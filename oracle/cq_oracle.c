@@ -1,7 +1,7 @@
 /* C restatement of the CalibQuant decode-attention step and of the prefill
  * quantise-and-pack (fp32, OpenMP over independent (batch, head) units).
  *
- * TEST INFRASTRUCTURE ONLY: the checker for the HIP kernels and the timed
+ * TEST INFRASTRUCTURE ONLY: what the HIP kernels are held against and the timed
  * "CPU port" of the benchmark.  The shipped library never links it.
  * tests/test_oracle_c.py pins it against the numpy oracle (cq_oracle.py),
  * which in turn is pinned against library routines and closed forms.

@@ -1,6 +1,6 @@
 """CPU oracle for CalibQuant's quantized-KV decode path (numpy).
 
-TEST INFRASTRUCTURE ONLY.  This module is the checker the HIP kernels are
+TEST INFRASTRUCTURE ONLY.  This module is what the HIP kernels are
 compared against.  Only the test-suite, the smoke entry and the CPU-baseline
 leg of the benchmark may import it; the shipped package never does.
 
