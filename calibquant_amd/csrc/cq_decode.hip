@@ -152,7 +152,7 @@ static int make_plan(const cq_decode_args* a, Plan* p) {
     // the packed K rows, no logits buffer.  (The residual units wait for nobody and make room as they end.)
     if (p->nsplit > 1) {
         const int64_t waiting = static_cast<int64_t>(a->B) * a->Hkv * ngroups(G, p->nh) * p->nsplit;
-        const int64_t room = static_cast<int64_t>(kPairUnits) * (p->nt == 512 && launch_lds(a->bits, vtok, p->hpb, p->nt) <= kLdsMax / 2 ? 2 : 1);
+        const int64_t room = static_cast<int64_t>(kPairUnits) * (p->nt == 512 && launch_lds(a->bits, vtok, p->hpb, p->nt) + parked_lds(vtok, p->nt, launch_rounds(vtok, p->hpb, p->nt, p->chunk)) <= kLdsMax / 2 ? 2 : 1);
         // (one lane per chunk polls)
         if (waiting <= room && p->nsplit <= 64 && g_fused_wanted.load(std::memory_order_relaxed)) p->fused = true;
     }

@@ -7,18 +7,19 @@
 //
 //   loads    the packed K rows are requested at kernel entry, the first block of
 //            packed V rows behind them (half before the logits, half as the K
-//            registers free up), the first tile of residual K/V rows when the
-//            packed-V phase ends: each stream is in flight while the phase before
+//            registers free up), the window's first K rows ahead of the packed V rows and
+//            its V rows behind them: each stream is in flight while the phase before
 //            its consumer runs, and no phase starts behind a queue of requests
-//            it does not need.
-//   K side   the codes are small integers: q.s_k goes onto a fixed-point grid, four signed byte digits a value, and a
-//            tile's logits are 8-bit integer MFMAs (see "the step on the matrix cores" below); the fp16/bf16 K tensor
-//            is never materialised.  A thread keeps its logits in registers.
+//            it does not need.  (The window's rows at entry, or ahead of the logits: the packed K rows
+//            wait behind them.  us, batch 64 x 3 328 + 128 19.3 -> 20.8, 16 x 9 984 + 105 17.8 -> 19.1.)
+//   K side   the codes are small integers: q.s_k goes onto a fixed-point grid, eight 4-bit digits and a sign a value, and a
+//            tile's logits are exact products of 6-bit and 4-bit floats (see "the step on the matrix cores" below); the
+//            fp16/bf16 K tensor is never materialised.  A thread keeps its logits in registers, the last rounds' in LDS.
 //   stats    min / max of the image logits (calibration), then e = exp(w' - M).
 //   V side   e (times the token's group scale, for per-token values) as four byte digits against the packed V rows,
-//            on the same MFMAs.  Per-channel scale / zero-point are applied once at the end.
+//            on 8-bit integer products.  Per-channel scale / zero-point are applied once at the end.
 //   residual the full-precision rows run last as an online-softmax flash-decode in
-//            the same workgroup (packed dot2 for q.K) and are merged at the end.
+//            the same workgroup, on 16-bit products with the weights in three parts, and are merged at the end.
 //
 // When the chunk does not cover all T tokens (long context or small batch)
 // a first launch computes every chunk's logits and publishes the per-chunk min / max;
@@ -66,6 +67,22 @@ constexpr float kLog2e = 1.4426950408889634f;
 template <int N> struct alignas(N * 4) Vec { float v[N]; };
 // native 16-byte vector: copies are single vector moves (HIP's uint4 struct copies lower to memcpy)
 typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+typedef uint32_t U2 __attribute__((ext_vector_type(2)));
+typedef uint32_t Pair16 __attribute__((aligned(2)));   // two 16-bit values wherever they lie: q and the statistics need no alignment
+typedef float F4 __attribute__((ext_vector_type(4)));
+
+// Of a launch's rounds of logits, how many (the last ones) a thread keeps in LDS of its own instead of registers: all of them in registers
+// leave too few for the products' operands and the rows in flight, and a spilled row waits for its load (batch 64 18.4 -> 22.0 us with 16
+// registers spilled).  16 bytes a lane, written and read once each: no bank conflicts, no vector instruction.  The same LDS holds a tile of the window's rows later.
+constexpr int cmax(int a, int b) { return a > b ? a : b; }
+constexpr int parked_rounds(bool vtok, int nt, int rounds) {
+    if (vtok || rounds <= 4) return 0;
+    if (rounds > 10) return nt == 512 ? 7 : 6;
+    return nt == 512 ? 4 : 5;
+}
+
+// ... and the bytes of it (static LDS, beside the dynamic): at least a tile of 128 window rows
+constexpr int parked_lds(bool vtok, int nt, int rounds) { return cmax(parked_rounds(vtok, nt, rounds) * nt * 16, 128 * 256); }
 
 struct DecodeGeom {
     const void* q;
@@ -112,7 +129,6 @@ struct DecodeGeom {
                   // the number of compute units (the two workgroups of a unit are told apart by it); else 0
 };
 
-constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
 // VTOK: values quantised per token and per group of 32 channels (scale * code + minimum, codes in little-endian
 // 32-bit words, first channel in the lowest bits) instead of per channel.
@@ -135,7 +151,7 @@ template <int BITS, int HPB, bool VTOK = false, int NT_ = 1024> struct Lay {
     // shared words, in floats (what is read as vectors first: each of these starts on 16 bytes)
     static constexpr int F_QRAW = 0;                          // HPB*kD raw 16-bit q
     static constexpr int F_SRES = F_QRAW + HPB * kD / 2;      // kResTile*HPB: logits of a tile of the window
-    static constexpr int F_PRES = F_SRES + kResTile * HPB;    // kResTile*HPB: its weights; before, the waves' closing sums
+    static constexpr int F_PRES = F_SRES + kResTile * HPB;    // kResTile*HPB: the waves' closing sums
     static constexpr int F_VSZ = F_PRES + kResTile * HPB;     // 2*kD: value scale, zero-point
     static constexpr int F_QSZ = F_VSZ + (VTOK ? 0 : 2 * kD); // [head]: value of one grid step, zero-point sum
     static constexpr int F_RED = F_QSZ + 2 * HPB;             // minima, maxima, masked maxima; from 4*HPB the chunks' fold and its flag
@@ -198,15 +214,33 @@ __device__ __forceinline__ int virtual_block_id() {
     return l;
 }
 
-// Two-element dot product with fp32 accumulation on raw 16-bit pairs.
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-template <typename DT> __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c);
-template <> __device__ __forceinline__ float dot2<BF16>(uint32_t a, uint32_t b, float c) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
+// The window's products, 16 x 16 x 32 on raw 16-bit values; a lane's left (right) operand is row (column) lane % 16, k = 8 (lane / 16) + 0 .. 7
+typedef __bf16 B8 __attribute__((ext_vector_type(8)));
+typedef _Float16 H8 __attribute__((ext_vector_type(8)));
+typedef short S4 __attribute__((ext_vector_type(4)));
+template <typename DT> __device__ __forceinline__ F4 mfma16(U4 a, U4 b, F4 c);
+template <> __device__ __forceinline__ F4 mfma16<BF16>(U4 a, U4 b, F4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(B8, a), __builtin_bit_cast(B8, b), c, 0, 0, 0);
 }
-template <> __device__ __forceinline__ float dot2<FP16>(uint32_t a, uint32_t b, float c) {
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, a), __builtin_bit_cast(f16x2_t, b), c, false);
+template <> __device__ __forceinline__ F4 mfma16<FP16>(U4 a, U4 b, F4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(H8, a), __builtin_bit_cast(H8, b), c, 0, 0, 0);
+}
+
+// A weight 0 <= p <= 1 in three 16-bit parts, p = part 0 + kPartScale * part 1 + kPartScale^2 * part 2: bf16 holds 8 bits in each, all 24;
+// fp16 11, the lower parts scaled up so that none is lost to its small exponents.
+template <typename DT> constexpr float kPartScale = std::is_same<DT, FP16>::value ? 1.f / 4096.f : 1.f;
+template <typename DT> __device__ __forceinline__ void split_weight(float p, uint32_t* o) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        if constexpr (std::is_same<DT, BF16>::value) {
+            const uint32_t b = __float_as_uint(p) & 0xffff0000u;
+            o[i] = b >> 16;
+            p -= __uint_as_float(b);
+        } else {
+            o[i] = Cvt<DT>::from_float(p);
+            p = (p - Cvt<DT>::to_float(o[i])) * 4096.f;
+        }
+    }
 }
 
 // A float handed from one workgroup to another inside a launch: device-scope atomic store.
@@ -271,82 +305,114 @@ __device__ __forceinline__ bool others_done(const DecodeGeom& g, int64_t unit, i
 }
 
 // ---- the step on the matrix cores --------------------------------------------------------------
-// The codes are small integers, so both contractions run exactly on 8-bit integer MFMAs (16 x 16 x 64): what is not
+// The codes are small integers, so both contractions run exactly on the matrix cores: what is not
 // an integer - q.s_k, and the softmax weights - is put on a 32-bit fixed-point grid of its own maximum and split into
-// four signed byte digits.  16 rows of a tile are then four heads times four digits, the columns are tokens (logits)
-// or byte columns of the packed V rows (sums), and a lane of the result holds the four digits' sums of one head:
-// exact integers, put together in fp32.  Packed codes are masked in place, the upper half of a byte after one shift of
-// the word - one AND per 4 codes; a code then counts 2^s, s = 0 .. 3, which the fixed-point operand (logits) or the
-// closing fold (sums) takes back.
-// Measured, us per step in turn on one box, look-up form before and this one: batch 64 x 3 328 + 128, 1 bit 28.5 -> 19.7,
-// 2 bits 48.9 -> 27.5; batch 256 x 3 328 99.7 -> 57; 16 x 9 984, six heads 38.4 -> 20.3; 8 x 32 768 in chunks
-// 36.8 -> 26.5; batch 1 x 1 024 7.7 -> 6.7.  A wave issues 66 vector instructions per 64 tokens and four heads for the logits, 74
-// for weights and values, beside 16 of these MFMAs, and about 600 for the rest (330 of them the window); at batch 256 the
-// vector units are busy for three quarters of a launch.  The matrix form first had 84 and 125 per tile: the logits stay in grid
-// steps (their scale and zero-point go into the exponent's factor and the calibration), V fields are taken in place,
-// every lane calibrates its own head only, and the
-// rows' addresses are a scalar base and one bounded offset - start of these steps -> now: batch 64 21.3 -> 20.0, 2 bits
-// 29.0 -> 27.6, 16 x 9 984 23.1 -> 20.5, batch 256 60.1 -> 57.3, per-token values 39.4 -> 36.9 (one box, in turn).
-// Error against 64 bits: a weight is off by 2^-31 at most and exact from 2^-7 on (weight_digits(); with the digits' offset added
-// before the conversion instead, which rounds once more, 1.5 % less time: batch 64 18.41 -> 18.17, batch 256 52.7 -> 51.9); a channel's q.s_k by 2^(s - 30) of the head's
-// largest (s = 3: 2^-27, three of the grid's bits; masked in place all through, the top bit of a byte would cost seven),
-// then the fp32 roundings.
-// The look-up form added fp32 partial sums on the K side and held the weights as fp16 on the V side.  Root-mean-square
-// logit error over its own (a model of both on the CPU, keys with outlier channels of 1, 10, 100 and 1 000 times the
-// others): 0.59, 0.57, 0.56, 0.55 at 1 bit - 0.93, 1.4, 2.2, 2.8 masked in place -, 0.55, 0.52, 0.56, 0.53 at 2 bits.
-// (The shift costs batch 64 x 3 328 0.25 us at 1 bit and nothing at 2 bits.)
-// fp16 outputs lie 2.0e-4 to 2.2e-4 from 64 bits, which is their own rounding, 8e-4 to 1.6e-3 there (nine shapes).
+// digits.  The 16 rows of a tile are four heads times four digits (pairs of digits), the columns are tokens (logits)
+// or byte columns of the packed V rows (sums), and a lane of the result holds the sums of one head:
+// exact integers, put together in fp32.
+// Values: 8-bit integer products (16 x 16 x 64), weights as four signed byte digits, packed V bytes masked in place - a code then counts 2^s,
+// which the closing fold takes back.  Logits: 6-bit by 4-bit float products (16 x 16 x 128) take a token's 128 channels at twice the rate and
+// expand packed codes to half bytes, 5 instructions per 32 codes where byte fields take 9 (two bits: 3 per 16, 5).  The digits
+// then have 4 bits, so as many products are issued either way (2 x 4 per 64 tokens), but their sums come as floats that three
+// multiply-adds put together, without integer shifts and conversions: 53 vector instructions per 64 tokens and four heads for 66.
+// (8-bit floats on the left, which need no packing of digits, halve the rate.  The codes' rows loaded as the products read them,
+// 4 bytes of four rows to a lane, save the exchange between lanes, but a quarter of a load's lanes then covers 16 rows: batch 64 18.2 -> 20.0.)
+// What bounds it: a wave issues 53 vector instructions per 64 tokens and four heads for the logits, 70 for weights and values, and 16
+// products, which vector instructions of other waves do not overlap with here (8 integer products and 64 ANDs of four waves a
+// SIMD take the sum of their times).  At batch 256 that keeps the SIMDs busy for nine tenths of a launch.
+// Measured, us per step in turn on one box, against 8-bit integer products for the logits, the window on dot products, logits all in
+// registers and rounds that are skipped one by one: batch 64 x 3 328 + 128 18.6 -> 17.7, 2 bits 27.5 -> 27.0; batch 256 x 3 328 52.7 -> 51.6,
+// x 300 + 40 32.7 -> 27.3; 16 x 9 984 + 105, six heads 19.5 -> 18.8; 8 x 32 768 in chunks 24.2 -> 22.6; batch 1 and 6 no difference.
+// Error against 64 bits: a weight is off by 2^-31 at most and exact from 2^-7 on (weight_digits()); a channel's q.s_k by 2^(s - 32) of the head's
+// largest (s = 0 .. 2), then the fp32 roundings.  fp16 outputs lie 1.9e-4 to 2.3e-4 from 64 bits, bf16 1.5e-3 to 1.8e-3, which is their own
+// rounding (sixteen shapes, the same to four digits as with integer products).
 typedef int I4 __attribute__((ext_vector_type(4)));
 typedef int I2 __attribute__((ext_vector_type(2)));
-typedef uint32_t U2 __attribute__((ext_vector_type(2)));
 
-// what field f (lowest first) of a masked byte of codes counts, as a shift: the upper half-byte's fields are moved down
-template <int BITS> __device__ __forceinline__ constexpr int field_shift(int f) { return (BITS * f) & 3; }
+// The logits' operands.  Right: packed codes as 4-bit floats (E2M1), eight to a dword, masked in place: the fields of a half byte
+// read 0.5, 1 and 2 - the topmost would be the sign and is moved to the lowest place; a 2-bit code in the lower half of one reads
+// half its value, the upper is moved down.  Left: a channel's q.s_k on a 32-bit grid of the head's largest, divided by what its field counts,
+// as a sign and eight 4-bit digits in 6-bit floats (E2M3, where 0 .. 15 eighths are the codes 0 .. 15): rows (head, pair of
+// digits), the lower and the upper digit of a pair one product each, 16 apart by the product's own scale.  All sums are whole
+// numbers of sixteenths below 2^24, exact in fp32.
+// k order: lane (x, kg) has dword kg of a packed row (two bits: dwords kg and 4 + kg).
+// A wave prepares a head, a lane two neighbouring channels (query_pair() * 2 and the next): their fields are neighbours as well.  Lanes that
+// differ in bits 0, 1, 3 hold the eight nibbles of the same two dwords.
+template <int BITS> __device__ __forceinline__ int query_pair(int lane) {
+    const int j = ((lane & 3) | ((lane >> 1) & 4)) ^ 1, b2 = (lane >> 2) & 1;   // (nibble n of a dword is the higher of a byte's halves for odd n, the earlier channels)
+    return (lane & 0x30) | (BITS == 1 ? (j << 1) | b2 : (b2 << 3) | j);
+}
 
-// One channel of one head of q.s_k into the K contraction's left operand: row (head, digit), in the byte that meets
-// the channel's code.  A wave holds one half of a head, the other half's values come along for the common scale and
-// the zero-point sum.  scale: [head][2] = (value of one grid step, zero-point sum).
+// 4 nibbles (of the lower 16 bits) -> 24 bits, two empty bits above each
+__device__ __forceinline__ uint32_t spread6(uint32_t x) {
+    const uint32_t t = (x & 0xffu) | ((x << 4) & ~0xffu);
+    return ((t & 0x00f00fu) | ((t << 2) & ~0x00f00fu)) & 0x3cf3cfu;
+}
+
+// Eight lanes' numbers to 48 bits of codes: lane n ends with digit n of all of them, in nibble order.  (The butterfly of an 8 x 8 transposition of
+// nibbles; `neg`: the signs of the wave's lanes.)
+struct Codes { uint32_t lo, hi; };   // 24 bits each
+__device__ __forceinline__ Codes digit_codes(int x, int lane) {
+    uint32_t w = static_cast<uint32_t>(x < 0 ? -x : x);
+    const uint64_t neg = __builtin_amdgcn_ballot_w64(x < 0);
+    uint32_t t = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w), 0xB1, 0xf, 0xf, true));    // lane ^ 1
+    t = __builtin_amdgcn_alignbit(t, t, (lane & 1) ? 4 : 28);
+    const uint32_t own = (lane & 1) ? 0xf0f0f0f0u : 0x0f0f0f0fu;
+    w = (w & own) | (t & ~own);
+    t = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w), 0x4E, 0xf, 0xf, true));             // lane ^ 2
+    w = __builtin_amdgcn_perm(t, w, (lane & 2) ? 0x03070105u : 0x06020400u);
+    t = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w), 0x128, 0xf, 0xf, true));            // lane ^ 8
+    w = __builtin_amdgcn_perm(t, w, (lane & 8) ? 0x03020706u : 0x05040100u);
+    // (bit i of four times 0x108420 stands at i + 5 k + 5, once each: those at 6 i + 5 are kept)
+    const uint32_t sg = static_cast<uint32_t>(neg >> (lane & 0x34));
+    return {spread6(w) | (((sg & 15u) * 0x108420u) & 0x820820u), spread6(w >> 16) | ((((sg >> 8) & 15u) * 0x108420u) & 0x820820u)};
+}
+
+// One head of q.s_k into the left operand, by one wave.  qs: a lane's two channels.  In LDS: [lower, upper digits][lane] 24 bytes.
+// scale: (value of one step of the result, zero-point sum).
+constexpr int kQueryHalf = 64 * 24;
 template <int BITS>
-__device__ __forceinline__ void matrix_query(float qs, float qsz, float qv2, float s2, float z2, int h, int d,
-                                             unsigned char* regA, float* scale) {
-    const float qs2 = qv2 * s2;
-    const int top = wave_max_key(max(__builtin_bit_cast(int, qs) & 0x7fffffff, __builtin_bit_cast(int, qs2) & 0x7fffffff));
-    const float zs = wave_sum(qsz + qs2 * z2);
-    // the largest value lies in [2^(e-1), 2^e); a head that is all but zero keeps a grid of 2^-90
+__device__ __forceinline__ void matrix_query(const float* qs, float qz, int h, int lane, unsigned char* operand, float* scale) {
+    const int top = wave_max_key(max(__builtin_bit_cast(int, qs[0]) & 0x7fffffff, __builtin_bit_cast(int, qs[1]) & 0x7fffffff));
+    const float zs = wave_sum(qz);
+    // the largest value lies in [2^(e-1), 2^e); a head that is all but zero keeps a grid of 2^-91
     const int e = max((top >> 23) - 126, -60);
-    const int byte = BITS == 1 ? d >> 3 : d >> 2;                  // byte of the packed row
-    const int f = BITS == 1 ? 7 - (d & 7) : 3 - (d & 3);           // field of the byte, lowest first
-    const float x = qs * __builtin_bit_cast(float, (30 - e + 127) << 23) * __builtin_bit_cast(float, (127 - field_shift<BITS>(f)) << 23);
-    const uint32_t dg = byte_digits(__float2int_rn(x));
-    const int kg = (byte >> 2) & 3, b = byte & 3, i = BITS == 1 ? f : (byte >> 4) * 4 + f;   // operand dword i = 0 .. 7
-    unsigned char* o = regA + ((i >> 2) * 64 + kg * 16 + 4 * h) * 16 + (i & 3) * 4 + b;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) o[16 * p] = static_cast<unsigned char>(dg >> (8 * p));
-    if ((d & 127) == 0) {
+    const float grid = __builtin_bit_cast(float, (31 - e + 127) << 23);
+    // fields of the pair: at 1 bit 3 and 2, or 1 and 0; they count 2^shift, shift = 0, 2, 1, 0
+    const bool low = lane & 4;
+    const float c0 = BITS == 1 && low ? grid * 0.5f : grid, c1 = BITS == 1 && !low ? grid * 0.25f : grid;
+    const Codes odd = digit_codes(__float2int_rn(qs[0] * c0), lane), even = digit_codes(__float2int_rn(qs[1] * c1), lane);
+    const int digit = (lane & 3) | ((lane >> 1) & 4);
+    const int kg = BITS == 1 ? lane >> 4 : ((lane >> 4) & 1) * 2 + (low ? 1 : 0), part = BITS == 1 ? (low ? 0 : 1) : lane >> 5;   // k block, and which half of its 24 bytes
+    uint32_t* o = reinterpret_cast<uint32_t*>(operand + (digit & 1) * kQueryHalf + (kg * 16 + 4 * h + (digit >> 1)) * 24 + part * 12);
+    o[0] = even.lo | (even.hi << 24);
+    o[1] = (even.hi >> 8) | (odd.lo << 16);
+    o[2] = (odd.lo >> 16) | (odd.hi << 8);
+    if (lane == 0) {
         // an infinity or a NaN anywhere in the head makes all its logits NaN, as a floating-point sum would
-        scale[2 * h] = top >= 0x7f800000 ? __builtin_nanf("") : __builtin_bit_cast(float, (e - 30 + 127) << 23);
+        // (results count 16 grid steps: a digit is held as eighths, the lowest field as a half)
+        scale[2 * h] = top >= 0x7f800000 ? __builtin_nanf("") : __builtin_bit_cast(float, (e - 31 + 4 + 127) << 23);
         scale[2 * h + 1] = zs;
     }
 }
 
-// the right operand's dwords of one word of packed codes
-template <int BITS> __device__ __forceinline__ void code_fields(uint32_t w, int* o) {
-    constexpr uint32_t kCode = BITS == 1 ? 0x01010101u : 0x03030303u;
-    constexpr int kHalf = 4 / BITS;   // codes of half a byte
-    const uint32_t up = w >> 4;
-#pragma unroll
-    for (int i = 0; i < kHalf; ++i) {
-        o[i] = static_cast<int>(w & (kCode << (BITS * i)));
-        o[kHalf + i] = static_cast<int>(up & (kCode << (BITS * i)));
-    }
+typedef int I8 __attribute__((ext_vector_type(8)));
+struct QueryOperand { I8 lower, upper; };   // (6-bit floats: six dwords of each)
+__device__ __forceinline__ QueryOperand load_query(const unsigned char* regA, int lane) {
+    QueryOperand o;
+    const U2* p = reinterpret_cast<const U2*>(regA) + 3 * lane;
+    const U2 l0 = p[0], l1 = p[1], l2 = p[2], u0 = p[192], u1 = p[193], u2 = p[194];
+    o.lower = I8{static_cast<int>(l0.x), static_cast<int>(l0.y), static_cast<int>(l1.x), static_cast<int>(l1.y), static_cast<int>(l2.x), static_cast<int>(l2.y), 0, 0};
+    o.upper = I8{static_cast<int>(u0.x), static_cast<int>(u0.y), static_cast<int>(u1.x), static_cast<int>(u1.y), static_cast<int>(u2.x), static_cast<int>(u2.y), 0, 0};
+    return o;
 }
 
 // Logits of 64 tokens, one row per lane: a 4 x 4 exchange of dwords between the four groups of 16 lanes gives lane
-// (x, k) dword k of the tokens x, 16 + x, 32 + x, 48 + x - the right operand of four 16-token tiles.  The results are in grid
-// steps, before the zero-point: logit = result * step - zero-point sum, which the minima and maxima take (the map is
+// (x, kg) dword kg of the tokens x, 16 + x, 32 + x, 48 + x - the right operand of four 16-token tiles.  The results are in steps of
+// the query's grid, before the zero-point: logit = result * step - zero-point sum, which the minima and maxima take (the map is
 // monotone) and the exponent's factor carries.
 template <int BITS>
-__device__ __forceinline__ void matrix_logits(const uint4* c, I4 a0, I4 a1, float* out) {
+__device__ __forceinline__ void matrix_logits(const uint4* c, const QueryOperand& a, float* out) {
     uint32_t w[BITS][4];
 #pragma unroll
     for (int s = 0; s < BITS; ++s) {
@@ -358,15 +424,16 @@ __device__ __forceinline__ void matrix_logits(const uint4* c, I4 a0, I4 a1, floa
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        int f[8];
-        code_fields<BITS>(w[0][j], f);
-        if constexpr (BITS == 2) code_fields<BITS>(w[1][j], f + 4);
-        I4 acc = {0, 0, 0, 0};
-        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, I4{f[0], f[1], f[2], f[3]}, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, I4{f[4], f[5], f[6], f[7]}, acc, 0, 0, 0);
-        // digit sums are at most 128 * 128 * 12 in size: two of them meet as an integer
-        const float l = static_cast<float>(acc[0] + (acc[1] << 8)), u = static_cast<float>(acc[2] + (acc[3] << 8));
-        out[j] = __builtin_fmaf(u, 65536.f, l);
+        const uint32_t u = w[0][j], v = w[BITS - 1][j];
+        I8 f;
+        if constexpr (BITS == 1)
+            f = I8{static_cast<int>(u & 0x11111111u), static_cast<int>(u & 0x22222222u), static_cast<int>(u & 0x44444444u), static_cast<int>((u >> 3) & 0x11111111u), 0, 0, 0, 0};
+        else
+            f = I8{static_cast<int>(u & 0x33333333u), static_cast<int>((u >> 2) & 0x33333333u), static_cast<int>(v & 0x33333333u), static_cast<int>((v >> 2) & 0x33333333u), 0, 0, 0, 0};
+        F4 acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a.lower, f, F4{0.f, 0.f, 0.f, 0.f}, 2, 4, 0, 0x7f, 0, 0x7f);
+        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a.upper, f, acc, 2, 4, 0, 0x83, 0, 0x7f);   // x 2^4
+        const float lo = __builtin_fmaf(acc[1], 256.f, acc[0]), hi = __builtin_fmaf(acc[3], 256.f, acc[2]);
+        out[j] = __builtin_fmaf(hi, 65536.f, lo);
     }
 }
 
@@ -385,9 +452,9 @@ template <int BITS> __device__ __forceinline__ constexpr int value_mask(int i) {
 
 // Weighted code sums of 64 tokens.  The weights (lane: head lane / 16, tokens 16 j + x) go through the wave's LDS tile
 // as [token][head] words, i.e. rows of 16 digit bytes, the packed V rows as they are, [token][16 bytes]; both come
-// back by columns, 16 tokens of one column per lane.
+// back by columns, 16 tokens of one column per lane.  first: there are no sums yet.
 template <int BITS>
-__device__ __forceinline__ void matrix_values(unsigned char* tile, const float* e, const U4* v, I4* acc) {
+__device__ __forceinline__ void matrix_values(unsigned char* tile, const float* e, const U4* v, I4* acc, bool first) {
     const int lane = threadIdx.x & 63, x = lane & 15, k = lane >> 4;
 #pragma unroll
     for (int s = 0; s < BITS; ++s) *reinterpret_cast<U4*>(tile + (1 + s) * 1024 + lane * 16) = v[s];
@@ -410,16 +477,16 @@ __device__ __forceinline__ void matrix_values(unsigned char* tile, const float* 
             I4 f;
 #pragma unroll
             for (int r = 0; r < 4; ++r) f[r] = i < NF - 1 ? w[r] & m : w[r] ^ m;
-            acc[s * NF + i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, f, acc[s * NF + i], 0, 0, 0);
+            acc[s * NF + i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, f, first ? I4{0, 0, 0, 0} : acc[s * NF + i], 0, 0, 0);
         }
     }
-    if constexpr (BITS == 2) acc[8] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, I4{0x01010101, 0x01010101, 0x01010101, 0x01010101}, acc[8], 0, 0, 0);
+    if constexpr (BITS == 2) acc[8] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, I4{0x01010101, 0x01010101, 0x01010101, 0x01010101}, first ? I4{0, 0, 0, 0} : acc[8], 0, 0, 0);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
 
 // the lane's sums (one head, byte column x) as floats in channel order (sums of digits are whole numbers below 2^28)
-template <int BITS> __device__ __forceinline__ void matrix_fold(const I4* acc, float* out, int x) {
+template <int BITS> __device__ __forceinline__ void matrix_fold(const I4* acc, float* out, int x, int swz) {
     constexpr int NF = 8 / BITS;
 #pragma unroll
     for (int s = 0; s < BITS; ++s) {
@@ -443,7 +510,7 @@ template <int BITS> __device__ __forceinline__ void matrix_fold(const I4* acc, f
             o[(NF - 1 - i) / 4].v[(NF - 1 - i) % 4] = r * unit;   // first channel of a byte in its top bits
         }
 #pragma unroll
-        for (int q = 0; q < NF / 4; ++q) *reinterpret_cast<Vec<4>*>(out + (16 * s + x) * NF + 4 * q) = o[q];
+        for (int q = 0; q < NF / 4; ++q) *reinterpret_cast<Vec<4>*>(out + (((16 * s + x) * NF + 4 * q) ^ swz)) = o[q];
     }
 }
 
@@ -533,7 +600,7 @@ template <typename DT> __device__ __forceinline__ void token_tops(const float* e
 }
 
 // its sums as floats in channel order; pw: the grids
-template <int BITS> __device__ __forceinline__ void matrix_fold_token(const I4* acc, const float* pw, float* out, int x) {
+template <int BITS> __device__ __forceinline__ void matrix_fold_token(const I4* acc, const float* pw, float* out, int x, int swz) {
     const int byte = BITS == 1 ? x & 3 : x & 7, f = BITS == 1 ? x >> 2 : x >> 3;
     const float field = __builtin_bit_cast(float, (127 - BITS * f) << 23);   // the field counts 2^(BITS f)
 #pragma unroll
@@ -546,7 +613,7 @@ template <int BITS> __device__ __forceinline__ void matrix_fold_token(const I4* 
             float r = static_cast<float>(a[3]);
 #pragma unroll
             for (int p = 2; p >= 0; --p) r = __builtin_fmaf(r, 256.f, static_cast<float>(a[p]));
-            out[32 * gi + byte * (8 / BITS) + f + q * (4 / BITS)] = r * field * unit;
+            out[(32 * gi + byte * (8 / BITS) + f + q * (4 / BITS)) ^ swz] = r * field * unit;
         }
     }
 }
@@ -565,10 +632,11 @@ template <int BITS, int HPB, typename DT, bool MINMAX_ONLY, bool VTOK = false, i
 // unit are only resident together within that)
 __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     using L = Lay<BITS, HPB, VTOK, NT>;
-    using V = Vec<HPB>;
     constexpr int NB = L::NB;
     constexpr int kNT = L::kNT, kNW = L::kNW, kResTile = L::kResTile;
     extern __shared__ __attribute__((aligned(256))) unsigned char smem[];
+    constexpr int PARK = MINMAX_ONLY ? 0 : parked_rounds(VTOK, NT, REGL), RR = REGL - PARK;
+    __shared__ F4 parked[MINMAX_ONLY ? 1 : parked_lds(VTOK, NT, REGL) / 16];
     unsigned char* regA = smem;
     float* fx = reinterpret_cast<float*>(smem + L::kRegionA);
     float* qsz = fx + L::F_QSZ;
@@ -635,38 +703,29 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     // at q (always mapped, at least 256 bytes) and never looks at what comes back.
     const bool has_img = n > 0;
     const int64_t unit = bh * static_cast<int64_t>(g.d_ng.div) + hg;
+    // wave h < HPB: head h of q and the keys' statistics; the last wave: the values'
+    const int wvu = __builtin_amdgcn_readfirstlane(wv);
+    const int pair = query_pair<BITS>(lane);   // the two channels this lane sets up
     uint32_t q_raw, s_raw, z_raw;
-    constexpr bool kVSep = (HPB * kD > kNT - kD);
-    uint32_t vs_raw = 0, vz_raw = 0;
-    uint32_t q_raw2, s_raw2, z_raw2;   // the head's other half, for a wave that needs the whole head
     {
-        const int h = min(min(tid / kD, HPB - 1), nh - 1), d = tid % kD;   // a padding head repeats the last real one
-        const uint16_t* qp = static_cast<const uint16_t*>(g.q) + (static_cast<int64_t>(b) * g.Hq + hq0) * kD;
-        q_raw = qp[h * kD + d];
-        // the last kD threads fetch the value statistics, unless they are q threads as well
-        // (then the first kD threads fetch them with two loads of their own, below)
-        const bool vstat = tid >= kNT - kD && !kVSep;
-        const uint16_t* sp = has_img ? static_cast<const uint16_t*>((vstat && !VTOK) ? g.vs : g.ks) + bh * kD : qp;
-        const uint16_t* zp = has_img ? static_cast<const uint16_t*>((vstat && !VTOK) ? g.vz : g.kz) + bh * kD : qp;
-        s_raw = sp[d];
-        z_raw = zp[d];
-        q_raw2 = qp[h * kD + (d ^ 64)];
-        s_raw2 = sp[d ^ 64];
-        z_raw2 = zp[d ^ 64];
-        if constexpr (kVSep && !VTOK) {
-            vs_raw = (has_img ? static_cast<const uint16_t*>(g.vs) + bh * kD : qp)[d];
-            vz_raw = (has_img ? static_cast<const uint16_t*>(g.vz) + bh * kD : qp)[d];
-        }
+        const int h = min(min(wvu, HPB - 1), nh - 1);   // a padding head repeats the last real one
+        const Pair16* qp = reinterpret_cast<const Pair16*>(static_cast<const uint16_t*>(g.q) + (static_cast<int64_t>(b) * g.Hq + hq0 + h) * kD);
+        const bool vstat = !VTOK && wvu == kNW - 1;
+        const Pair16* sp = has_img ? reinterpret_cast<const Pair16*>(static_cast<const uint16_t*>(vstat ? g.vs : g.ks) + bh * kD) : qp;
+        const Pair16* zp = has_img ? reinterpret_cast<const Pair16*>(static_cast<const uint16_t*>(vstat ? g.vz : g.kz) + bh * kD) : qp;
+        q_raw = qp[pair];
+        s_raw = sp[pair];
+        z_raw = zp[pair];
     }
+    static_assert(HPB < kNW, "a wave is left for the values' statistics");
     const int64_t code_off = has_img ? (bh * g.T + t0) * NB : 0;   // one offset for both code streams
     const uint4* ckp = reinterpret_cast<const uint4*>(has_img ? g.ck + code_off : static_cast<const uint8_t*>(g.q));
     const uint4* cvp = reinterpret_cast<const uint4*>((has_img ? g.cv : static_cast<const uint8_t*>(g.q)) + code_off);
     const int last_row = has_img ? n - 1 : 0;
-    // residual tile: K slice (row = tid / LPR, 128 / LPR elements); V: a wave owns RPW rows of the tile and a
-    // lane one channel pair of each of them, so the value products need no fold inside the wave
+    // residual tile: a thread loads a slice of a K and of a V row (row = tid / LPR, 128 / LPR elements); a wave's rows go through its own
+    // part of the LDS
     constexpr int LPR = L::LPR, NKP = L::NKP, RPW = L::RPW;
     const int lq = tid % LPR, krow = tid / LPR;
-    const int wvr = __builtin_amdgcn_readfirstlane(wv);   // wave-uniform: scalar row arithmetic
     // (the strides are read where the other kernel arguments are, not behind the branch that needs them: one
     // round trip to the argument block instead of one more)
     // (a single launch: every workgroup has a window; of a chunked launch only the residual units do)
@@ -677,19 +736,11 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     const uint16_t* vbp = static_cast<const uint16_t*>(do_res ? g.vres : g.q) + res_off;
     const int last_r = do_res ? R - 1 : 0;
     const int64_t rs_r = do_res ? arg_rs_r : 0;
-    uint4 rk[NKP];
-    uint32_t rv[RPW];
-    auto load_res_k = [&](int r0, uint4* k2) {   // rows past R re-read row R-1 (their logit is masked)
-        const uint16_t* kp = kb + min(r0 + krow, last_r) * rs_r + lq * 8;
+    U4 rk[NKP], rv[NKP];
+    auto load_res = [&](const uint16_t* base, int r0, U4* o) {   // rows past R re-read row R-1 (their weight is 0)
+        const uint16_t* p = base + min(r0 + krow, last_r) * rs_r + lq * 8;
 #pragma unroll
-        for (int i = 0; i < NKP; ++i) k2[i] = *reinterpret_cast<const uint4*>(kp + i * (LPR * 8));   // piece i * LPR + lq
-    };
-    auto load_res_v = [&](int r0, uint32_t* v8) {   // rows past R re-read row R-1 (their weight is 0)
-#pragma unroll
-        for (int i = 0; i < RPW; ++i) {
-            const int r2 = min(r0 + wvr * RPW + i, last_r);
-            v8[i] = *reinterpret_cast<const uint32_t*>(vbp + r2 * rs_r + 2 * lane);
-        }
+        for (int i = 0; i < NKP; ++i) o[i] = *reinterpret_cast<const U4*>(p + i * (LPR * 8));   // piece i * LPR + lq
     };
 
     // The first packed K rows are requested behind q and the statistics, before either is looked at: they arrive while q
@@ -714,28 +765,16 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
 
     CQ_PHASE(1);   // prologue, requests of q, the statistics and the first packed K rows
     // ---- phase 0: q onto its grid ---------------------------------------------------
-    if (tid < HPB * kD) {
-        const int h = tid / kD, d = tid % kD;
-        const float qraw = Cvt<DT>::to_float(q_raw);
-        reinterpret_cast<uint16_t*>(fx + L::F_QRAW)[h * kD + d] = static_cast<uint16_t>(q_raw);
-        const float qv = qraw * inv_sqrt_d;
+    if (wvu < HPB) {
+        reinterpret_cast<uint32_t*>(fx + L::F_QRAW)[wvu * (kD / 2) + pair] = q_raw;
         if (n > 0) {
-            const float s = Cvt<DT>::to_float(s_raw);
-            const float z = Cvt<DT>::to_float(z_raw);
-            const float qs = qv * s;
-            matrix_query<BITS>(qs, qs * z, Cvt<DT>::to_float(q_raw2) * inv_sqrt_d, Cvt<DT>::to_float(s_raw2),
-                               Cvt<DT>::to_float(z_raw2), h, d, regA, qsz);
+            const float qs[2] = {Cvt<DT>::lo(q_raw) * inv_sqrt_d * Cvt<DT>::lo(s_raw), Cvt<DT>::hi(q_raw) * inv_sqrt_d * Cvt<DT>::hi(s_raw)};
+            matrix_query<BITS>(qs, qs[0] * Cvt<DT>::lo(z_raw) + qs[1] * Cvt<DT>::hi(z_raw), wvu, lane, regA, qsz);
         }
     }
-    if constexpr (kVSep) {
-        if (!VTOK && n > 0 && tid < kD) {
-            fx[L::F_VSZ + tid] = Cvt<DT>::to_float(vs_raw);
-            fx[L::F_VSZ + kD + tid] = Cvt<DT>::to_float(vz_raw);
-        }
-    } else if (!VTOK && n > 0 && tid >= kNT - kD) {
-        const int d = tid - (kNT - kD);
-        fx[L::F_VSZ + d] = Cvt<DT>::to_float(s_raw);
-        fx[L::F_VSZ + kD + d] = Cvt<DT>::to_float(z_raw);
+    if (!VTOK && n > 0 && wvu == kNW - 1) {
+        *reinterpret_cast<Vec<2>*>(fx + L::F_VSZ + 2 * pair) = Vec<2>{{Cvt<DT>::lo(s_raw), Cvt<DT>::hi(s_raw)}};
+        *reinterpret_cast<Vec<2>*>(fx + L::F_VSZ + kD + 2 * pair) = Vec<2>{{Cvt<DT>::lo(z_raw), Cvt<DT>::hi(z_raw)}};
     }
     if (tid < 3 * HPB) reinterpret_cast<int*>(red)[tid] = static_cast<int>(0x80000000u);   // block_max's meeting words
     // Chunked launch: the chunks' logit min / max, lane s the pair of chunk s for every head (all in flight
@@ -744,7 +783,25 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     MinMax mraw[HPB];
     // Logits: round rd's 64 tokens of a wave start at 64 * wv + rd * kNT; lane (x, h) = (lane & 15, lane >> 4) has the
     // logits of head h for the tokens 16 j + x of them
-    float lx[REGL][4];
+    float lx[RR][4];
+    auto get_logits = [&](int rd, float* o) {
+        if (rd < RR) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = lx[rd < RR ? rd : 0][j];
+        } else {
+            const F4 v = parked[(rd - RR) * NT + tid];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = v[j];
+        }
+    };
+    auto put_logits = [&](int rd, const float* o) {
+        if (rd < RR) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) lx[rd < RR ? rd : 0][j] = o[j];
+        } else {
+            parked[(rd - RR) * NT + tid] = F4{o[0], o[1], o[2], o[3]};
+        }
+    };
     if constexpr (!MINMAX_ONLY) {
         if (CHUNKED && has_img && !g.fused) {
 #pragma unroll
@@ -773,6 +830,21 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
 #pragma unroll
         for (int r = 0; r < kVEarly; ++r) request_v(r, r);
     }
+    // The mask's values of the first rounds and of the window's first tile, ahead of the phases that add them.  (No mask: q, always mapped.)
+    constexpr int kMaskAhead = EXTRAS ? (REGL < 2 ? REGL : 2) : 0;
+    const bool masked = EXTRAS && g.mask;
+    const float* mask_img = masked && n > 0 ? g.mask + b * g.mask_sb + g.S + t0 : reinterpret_cast<const float*>(g.q);
+    const float* mask_win = masked ? g.mask + b * g.mask_sb : reinterpret_cast<const float*>(g.q);
+    float mask_v[kMaskAhead ? kMaskAhead : 1][4], mask_w = 0.f;
+    if constexpr (kMaskAhead > 0) {
+        const int top = masked && n > 0 ? n - 1 : 0;
+#pragma unroll
+        for (int r = 0; r < kMaskAhead; ++r)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) mask_v[r][j] = mask_img[min((tid & ~63) + r * kNT + 16 * j + (lane & 15), top)];
+        const int r = min(wv * RPW + (lane & 15) % RPW, last_r);
+        mask_w = mask_win[masked && do_res ? (r < g.S ? r : g.T + r) : 0];
+    }
 
     CQ_PHASE(2);   // q on its grid
     // the wave's first token, and the head whose results this lane holds (lanes beyond the unit's heads repeat
@@ -784,19 +856,20 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     const U2* vmp = reinterpret_cast<const U2*>(has_img ? static_cast<const uint16_t*>(g.vz) + (bh * g.T + t0) * 4 : static_cast<const uint16_t*>(g.q));
     U2 ts[VTOK && !MINMAX_ONLY ? REGL : 1];   // the scales of the lane's own tokens
     if (has_img) {
-        const I4* aq = reinterpret_cast<const I4*>(regA);
-        const I4 a0 = aq[lane], a1 = aq[64 + lane];
+        const QueryOperand aq = load_query(regA, lane);
         float lo = INFINITY, hi = -INFINITY;
         phase_priority(std::integral_constant<int, 1>{});
 #pragma unroll
         for (int rd = 0; rd < REGL; ++rd) {
-            if (wt0 + rd * kNT < n) {
-                matrix_logits<BITS>(kc[rd % L::KR], a0, a1, lx[rd]);
-                if (rd + L::KR < REGL) request_k(rd + L::KR);
+            // (left at the wave's end, not skipped round by round: a wait then counts every load issued since its own)
+            if (wt0 + rd * kNT >= n) break;
+            float l[4];
+            matrix_logits<BITS>(kc[rd % L::KR], aq, l);
+            if (rd + L::KR < REGL) request_k(rd + L::KR);
+            if (!MINMAX_ONLY) put_logits(rd, l);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) { lo = fminf(lo, lx[rd][j]); hi = fmaxf(hi, lx[rd][j]); }
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            for (int j = 0; j < 4; ++j) { lo = fminf(lo, l[j]); hi = fmaxf(hi, l[j]); }
+            __builtin_amdgcn_sched_barrier(0);
             if (!MINMAX_ONLY && rd < kVF - kVEarly) request_v(kVEarly + rd, kVEarly + rd);   // the rest of the first packed V rows
         }
         phase_priority(std::integral_constant<int, 2>{});
@@ -828,7 +901,10 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         return;
     } else {
         float m_img = -INFINITY;   // of the lane's head
-        float o_img = 0.f;  // thread (h, d) = (tid / kD, tid % kD) for tid < HPB*kD
+        // From here a lane of the first eight waves owns channel `od` of head `hl`: as the window's products leave them
+        const int od = 16 * wv + (lane & 15);
+        const bool owns = wv < 8 && (lane >> 4) < HPB;
+        float o_img = 0.f;
 
         if constexpr (CHUNKED) {
             // One launch: this chunk's min / max go out now (write-through stores that nothing waits for); the other
@@ -937,19 +1013,21 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             // (a constant that takes M back is off by M's own rounding), and a degenerate logit range, whose slope is
             // ~1e8, meets the exact zero of (w - peak).
             float eal, pkl;
-            if (EXTRAS && g.mask) {
-                const float* mk = g.mask + b * g.mask_sb + g.S + t0;
+            if (masked) {
                 const float sl = slope * step;
                 float top = -INFINITY;
 #pragma unroll
                 for (int rd = 0; rd < REGL; ++rd) {
                     if (wt0 + rd * kNT < n) {
+                        float l[4];
+                        get_logits(rd, l);
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
-                            const float mv = mk[min(wt0 + rd * kNT + 16 * j + (lane & 15), n - 1)];
-                            lx[rd][j] = (lx[rd][j] - mn) * sl + tmin + mv;
-                            top = fmaxf(top, lx[rd][j]);
+                            const float mv = rd < kMaskAhead ? mask_v[rd < kMaskAhead ? rd : 0][j] : mask_img[min(wt0 + rd * kNT + 16 * j + (lane & 15), n - 1)];
+                            l[j] = (l[j] - mn) * sl + tmin + mv;
+                            top = fmaxf(top, l[j]);
                         }
+                        put_logits(rd, l);
                     }
                 }
                 const int kt = row_max_key(float_key(top));
@@ -969,8 +1047,10 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             }
             float lsum = 0.f;
             I4 acc[BITS == 2 && !VTOK ? 9 : 8];
+            if (VTOK || wt0 >= n) {   // (else the first round starts them)
 #pragma unroll
-            for (int i = 0; i < (BITS == 2 && !VTOK ? 9 : 8); ++i) acc[i] = I4{0, 0, 0, 0};
+                for (int i = 0; i < (BITS == 2 && !VTOK ? 9 : 8); ++i) acc[i] = I4{0, 0, 0, 0};
+            }
             unsigned char* et = regA + wv * L::MXT;
             constexpr int KV = kVF / BITS;   // rounds of packed V rows in flight
             U2 ssc[VTOK ? KV : 1], smin[VTOK ? KV : 1];   // VTOK: the statistics of the lane's own tokens, as many rounds ahead
@@ -982,11 +1062,13 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     smin[r] = vmp[min(tid + r * kNT, n - 1)];
                 }
             }
+            load_res(kb, 0, rk);   // the first tile of the window: its K rows arrive during the packed V rows
             phase_priority(std::integral_constant<int, 3>{});
             auto weights = [&](int rd, float* e) {   // of round rd's tile
                 const int tw = wt0 + rd * kNT;
+                get_logits(rd, e);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f((lx[rd][j] - pkl) * eal);
+                for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f((e[j] - pkl) * eal);
                 if (tw + kWave > n) {   // the chunk's last tile: what is past the end weighs nothing
 #pragma unroll
                     for (int j = 0; j < 4; ++j) e[j] = tw + 16 * j + (lane & 15) < n ? e[j] : 0.f;
@@ -1012,36 +1094,34 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             }
 #pragma unroll
             for (int rd = 0; rd < REGL; ++rd) {
-                const int tw = wt0 + rd * kNT;
-                if (tw < n) {
-                    float e[4];
+                if (wt0 + rd * kNT >= n) break;
+                float e[4];
+                if constexpr (VTOK) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) e[j] = lx[rd][j];
+                } else {
+                    weights(rd, e);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) lsum += e[j];
+                if constexpr (VTOK) {
+                    const U2 a = ssc[rd % KV], m = smin[rd % KV];
+                    matrix_values_token<BITS, DT>(et, e, vc + (rd % KV) * BITS, U4{a.x, m.x, a.y, m.y}, vpw, cm, acc);
+                } else {
+                    matrix_values<BITS>(et, e, vc + (rd % KV) * BITS, acc, rd == 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);   // one round at a time: interleaved, they do not fit the registers
+                if (rd + KV < REGL) {
+#pragma unroll
+                    for (int i = 0; i < BITS; ++i) request_v((rd % KV) * BITS + i, (rd + KV) * BITS + i);
                     if constexpr (VTOK) {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) e[j] = lx[rd][j];
-                    } else {
-                        weights(rd, e);
-                    }
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) lsum += e[j];
-                    if constexpr (VTOK) {
-                        const U2 a = ssc[rd % KV], m = smin[rd % KV];
-                        matrix_values_token<BITS, DT>(et, e, vc + (rd % KV) * BITS, U4{a.x, m.x, a.y, m.y}, vpw, cm, acc);
-                    } else {
-                        matrix_values<BITS>(et, e, vc + (rd % KV) * BITS, acc);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);   // one round at a time: interleaved, they do not fit the registers
-                    if (rd + KV < REGL) {
-#pragma unroll
-                        for (int i = 0; i < BITS; ++i) request_v((rd % KV) * BITS + i, (rd + KV) * BITS + i);
-                        if constexpr (VTOK) {
-                            ssc[rd % KV] = vsp[min(tid + (rd + KV) * kNT, n - 1)];
-                            smin[rd % KV] = vmp[min(tid + (rd + KV) * kNT, n - 1)];
-                        }
+                        ssc[rd % KV] = vsp[min(tid + (rd + KV) * kNT, n - 1)];
+                        smin[rd % KV] = vmp[min(tid + (rd + KV) * kNT, n - 1)];
                     }
                 }
             }
             phase_priority(std::integral_constant<int, 4>{});
-            load_res_k(0, rk);   // first residual tile's K rows: in flight during the fold below
+            load_res(vbp, 0, rv);   // ... its V rows: in flight during the fold and the window's logits
             float* lpart = fx + L::F_PRES;   // the waves' sums of e (not in `red`, which a slower wave may still read)
             lsum = row_reduce(lsum, OpSum(), 0.f);
             constexpr int kParts = VTOK ? 5 : 1;     // VTOK: and of e * minimum per channel group
@@ -1060,16 +1140,16 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             static_assert(HPB * kD * 4 <= L::MXT, "a wave's sums fit its tile");
             const float* redv = reinterpret_cast<const float*>(regA);
             if ((lane >> 4) < HPB) {
-                float* o = reinterpret_cast<float*>(et) + hl * kD;
-                if constexpr (VTOK) matrix_fold_token<BITS>(acc, vpw, o, lane & 15);
-                else matrix_fold<BITS>(acc, o, lane & 15);
+                float* o = reinterpret_cast<float*>(et) + hl * kD;   // (channels in the order channel ^ 16 * head: the fold reads them without bank conflicts)
+                if constexpr (VTOK) matrix_fold_token<BITS>(acc, vpw, o, lane & 15, hl << 4);
+                else matrix_fold<BITS>(acc, o, lane & 15, hl << 4);
             }
             __syncthreads();
-            if (tid < HPB * kD) {
-                const int h = tid / kD, d = tid % kD;
+            if (owns) {
+                const int h = hl, d = od;
                 float a = 0.f, lh = 0.f;
 #pragma unroll
-                for (int w = 0; w < kNW; ++w) { a += redv[w * (L::MXT / 4) + h * kD + d]; lh += lpart[w * kParts * HPB + h]; }
+                for (int w = 0; w < kNW; ++w) { a += redv[w * (L::MXT / 4) + h * kD + (d ^ (h << 4))]; lh += lpart[w * kParts * HPB + h]; }
                 if constexpr (VTOK) {
                     float cmin = 0.f;
 #pragma unroll
@@ -1084,7 +1164,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             // window, and `stat` is read behind the one of the merge)
         }
 
-        if (n == 0) load_res_k(0, rk);
+        if (n == 0) { load_res(kb, 0, rk); load_res(vbp, 0, rv); }
         CQ_PHASE(8);   // fold of the packed part
         // ---- phase 6: full-precision residual rows, online softmax.  Runs last: its first
         // tile is requested when the packed-V phase ends and arrives during that phase's fold.
@@ -1098,101 +1178,81 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         if (do_res) {
             float m_run = -INFINITY, l_run = 0.f;
             float* sres = fx + L::F_SRES;
-            float* pres = fx + L::F_PRES;
-            // raw 16-bit q, [head][kD], read per head as two 16-byte LDS loads
-            const uint4* q128 = reinterpret_cast<const uint4*>(fx + L::F_QRAW);
-            float accv[2][HPB];   // the lane's channel pair
+            unsigned char* wrows = reinterpret_cast<unsigned char*>(parked) + wv * 1024;   // a wave's rows: four to 1 KB, NT * 16 apart
+            auto row_piece = [&](int row, int piece) { return (row >> 2) * (NT * 16) + (row & 3) * 256 + ((piece ^ row) << 4); };
+            auto park_rows = [&](const U4* v) {
 #pragma unroll
-            for (int k = 0; k < 2; ++k)
-#pragma unroll
-                for (int h = 0; h < HPB; ++h) accv[k][h] = 0.f;
-            const float* mk = (EXTRAS && g.mask) ? g.mask + b * g.mask_sb : nullptr;
+                for (int i = 0; i < NKP; ++i) *reinterpret_cast<U4*>(wrows + row_piece(lane / LPR, i * LPR + lq)) = v[i];
+            };
+            const int x = lane & 15, kg = lane >> 4;
+            const unsigned char* q16 = smem + L::kRegionA + L::F_QRAW * 4 + min(x >> 2, HPB - 1) * (kD * 2) + kg * 16;   // left operand: rows 4 h .. 4 h + 3 are head h
+            constexpr int kPB = 272;   // bytes of a row of weight parts: 128 window rows and 16 bytes against bank conflicts
+            unsigned char* parts = regA;    // [4 * head + part][window row], read by the fold above before the tile's first barrier
+            static_assert(16 * kPB <= L::kRegionA, "the weights' parts fit region A");
+            F4 racc = {0.f, 0.f, 0.f, 0.f};
 
             for (int r0 = 0; r0 < R; r0 += kResTile) {
                 const bool more = r0 + kResTile < R;
-                const int r = r0 + krow;
-                load_res_v(r0, rv);   // the tile's value words: in flight while its logits and weights are worked out
-                float dot[HPB];
+                if (r0 > 0) __syncthreads();   // (the values of the tile before are read)
+                park_rows(rk);
+                if (more) load_res(kb, r0 + kResTile, rk);
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                F4 dot = {0.f, 0.f, 0.f, 0.f};
+                const int xr = x % RPW;   // (waves of eight rows: columns 8 .. 15 repeat them)
 #pragma unroll
-                for (int h = NH; h < HPB; ++h) dot[h] = 0.f;
-#pragma unroll
-                for (int h = 0; h < NH; ++h) {
-                    float a = 0.f;
-#pragma unroll
-                    for (int i = 0; i < NKP; ++i) {
-                        const uint4 qa = q128[h * (kD / 8) + i * LPR + lq];
-                        a = dot2<DT>(qa.x, rk[i].x, a); a = dot2<DT>(qa.y, rk[i].y, a);
-                        a = dot2<DT>(qa.z, rk[i].z, a); a = dot2<DT>(qa.w, rk[i].w, a);
-                    }
-                    dot[h] = (LPR == 4 ? quad_reduce(a, OpSum(), 0.f) : oct_reduce(a, OpSum(), 0.f)) * inv_sqrt_d;
-                    // one head's q pieces at a time: all of them side by side would not fit the registers
-                    if constexpr (NKP > 2) __builtin_amdgcn_sched_barrier(0);
+                for (int s = 0; s < 4; ++s)
+                    dot = mfma16<DT>(*reinterpret_cast<const U4*>(q16 + 64 * s), *reinterpret_cast<const U4*>(wrows + row_piece(xr, 4 * s + kg)), dot);
+                if (x < RPW && kg < HPB) {
+                    const int r = r0 + wv * RPW + x;
+                    float w = dot[0] * inv_sqrt_d;
+                    if (masked && r < R) w += r0 == 0 ? mask_w : mask_win[r < g.S ? r : g.T + r];
+                    sres[(wv * RPW + x) * HPB + kg] = r < R ? w : -INFINITY;
                 }
-                if (more) load_res_k(r0 + kResTile, rk);   // next tile's K slice, in place
-                if (lq == 0) {
-                    float mv = 0.f;
-                    if (mk && r < R) mv = mk[r < g.S ? r : g.T + r];
-#pragma unroll
-                    for (int h = 0; h < HPB; ++h) sres[krow * HPB + h] = (r < R) ? dot[h] + mv : -INFINITY;
-                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                park_rows(rv);
+                if (more) load_res(vbp, r0 + kResTile, rv);
                 __syncthreads();
-                if (wv < NH) {   // wave h keeps the running softmax state of head h
+                if (wv < NH) {   // wave h keeps the running softmax state of head h; a lane two neighbouring rows
                     const int h = wv;
-                    constexpr int kRL = kResTile / kWave;   // tile rows per lane
-                    float sv[kRL], smax = -INFINITY;
-#pragma unroll
-                    for (int i = 0; i < kRL; ++i) {
-                        sv[i] = sres[(lane + i * kWave) * HPB + h];
-                        smax = fmaxf(smax, sv[i]);
-                    }
-                    const float mnew = fmaxf(m_run, wave_max(smax));
+                    const float s0 = sres[2 * lane * HPB + h], s1 = sres[(2 * lane + 1) * HPB + h];
+                    const float mnew = fmaxf(m_run, wave_max(fmaxf(s0, s1)));
                     const bool dead = (mnew == -INFINITY);
-                    float psum = 0.f;
+                    const float p0 = dead ? 0.f : __expf(s0 - mnew), p1 = dead ? 0.f : __expf(s1 - mnew);
+                    uint32_t w0[3], w1[3];
+                    split_weight<DT>(p0, w0);
+                    split_weight<DT>(p1, w1);
 #pragma unroll
-                    for (int i = 0; i < kRL; ++i) {
-                        const float pi = dead ? 0.f : __expf(sv[i] - mnew);
-                        pres[(lane + i * kWave) * HPB + h] = pi;
-                        psum += pi;
-                    }
+                    for (int i = 0; i < 3; ++i) *reinterpret_cast<uint32_t*>(parts + (4 * h + i) * kPB + 4 * lane) = w0[i] | (w1[i] << 16);
                     const float al = dead ? 1.0f : __expf(m_run - mnew);
-                    l_run = l_run * al + wave_sum(psum);
+                    l_run = l_run * al + wave_sum(p0 + p1);
                     m_run = mnew;
                     if (lane == 0) { stat[h] = al; stat[HPB + h] = m_run; stat[2 * HPB + h] = l_run; }
                 }
                 __syncthreads();
-                if (r0 > 0) {
+                if (wv < 8) {   // 16 channels of all heads: a wave each
+                    if (r0 > 0) racc *= stat[hl];
 #pragma unroll
-                    for (int h = 0; h < NH; ++h) {
-                        const float al = stat[h];
-                        accv[0][h] *= al;
-                        accv[1][h] *= al;
+                    for (int s = 0; s < kResTile / 32; ++s) {
+                        const U4 w = *reinterpret_cast<const U4*>(parts + x * kPB + 64 * s + 16 * kg);
+                        U4 v;
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) {   // rows 32 s + 8 kg + 4 t + 0 .. 3: column x of four rows
+                            const int row = (8 * kg + 4 * t + (x >> 2)) % RPW;
+                            const unsigned char* o = reinterpret_cast<const unsigned char*>(parked) + ((32 * s + 8 * kg) / RPW) * 1024 +
+                                                     row_piece(row, 2 * wv + ((x >> 1) & 1)) + (x & 1) * 8;
+                            const U2 c = __builtin_bit_cast(U2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) S4*)(o)));
+                            v[2 * t] = c.x; v[2 * t + 1] = c.y;
+                        }
+                        racc = mfma16<DT>(w, v, racc);
                     }
                 }
-#pragma unroll
-                for (int i = 0; i < RPW; ++i) {
-                    const float f0 = Cvt<DT>::lo(rv[i]), f1 = Cvt<DT>::hi(rv[i]);
-                    const V p = reinterpret_cast<const V*>(pres)[wvr * RPW + i];   // the row's weights (0 past R), one address per wave
-#pragma unroll
-                    for (int h = 0; h < NH; ++h) {
-                        accv[0][h] = __builtin_fmaf(p.v[h], f0, accv[0][h]);
-                        accv[1][h] = __builtin_fmaf(p.v[h], f1, accv[1][h]);
-                    }
-                }
             }
-            // (regA was last read by the packed part's sum, behind which lie the tiles' barriers)
-            float* red2 = reinterpret_cast<float*>(regA);  // [wave][head][kD]: the fold reads consecutive words
-#pragma unroll
-            for (int h = 0; h < HPB; ++h) {
-                Vec<2> a2;
-                a2.v[0] = accv[0][h]; a2.v[1] = accv[1][h];
-                *reinterpret_cast<Vec<2>*>(red2 + (wv * HPB + h) * kD + 2 * lane) = a2;
-            }
-            __syncthreads();
-            if (tid < HPB * kD) {
-                const int h = tid / kD, d = tid % kD;
-#pragma unroll
-                for (int w = 0; w < kNW; ++w) o_res += red2[(w * HPB + h) * kD + d];
-            }
+            o_res = racc[0];
+            // (an infinite sum stays one: 0, a lower part's, times an infinite value would make it a NaN)
+            if (__builtin_fabsf(o_res) != INFINITY) o_res += kPartScale<DT> * (racc[1] + kPartScale<DT> * racc[2]);
         }
 
         if (speaks) {
@@ -1202,8 +1262,8 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         CQ_PHASE(9);   // residual window
         // ---- phase 7: merge / write ---------------------------------------------------------
         __syncthreads();
-        if (tid < nh * kD) {
-            const int h = tid / kD, d = tid % kD;
+        if (owns && hl < nh) {
+            const int h = hl, d = od;
             const float mr = stat[HPB + h], lr = stat[2 * HPB + h];
             const float mi = stat[3 * HPB + h], li = stat[4 * HPB + h];
             const int64_t row = static_cast<int64_t>(b) * g.Hq + hq0 + h;

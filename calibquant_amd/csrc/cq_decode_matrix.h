@@ -9,7 +9,8 @@ namespace cq {
 template <int BITS, int HPB, typename DT, bool VTOK, int NT, int REGL, bool CHUNKED, bool EXTRAS, int NH>
 static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st) {
     constexpr int lds = Lay<BITS, HPB, VTOK, NT>::kLds;
-    static_assert(lds <= 64 * 1024, "no raised dynamic-LDS limit needed; two 512-thread workgroups share a compute unit");
+    static_assert(lds <= 64 * 1024, "no raised dynamic-LDS limit needed");
+    static_assert(lds + parked_lds(VTOK, NT, REGL) <= kLdsMax / (NT == 512 ? 2 : 1), "two 512-thread workgroups share a compute unit");
     static_assert(lds == launch_lds<BITS, VTOK, NT>(HPB), "the LDS that plans report");
     if (launch_rounds(VTOK, HPB, NT, g.chunk) != REGL || g.chunk > REGL * NT) return CQ_ERR_UNSUPPORTED;   // (a token too many would be left out of the sum)
     if constexpr (CHUNKED) {
@@ -35,9 +36,8 @@ static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st
     return CQ_OK;
 }
 
-// A chunked launch has one instantiation, with the mask and the row count.  Of the kernels that chunked plans ask for,
-// those of 512 threads and of per-token values keep within the 128 registers; those of ten rounds spill up to 16 (36 B of
-// scratch per lane), those of sixteen 76 to 108 (2 to 13 in single launches without mask and row count).
+// A chunked launch has one instantiation, with the mask and the row count.  All kernels keep within the 128 registers, except those of
+// sixteen rounds with mask and row count (4 to 16 spilled).
 // SINGLE: no plan chunks such units.
 template <int BITS, int HPB, typename DT, int NT, int REGL, int NH = HPB, bool VTOK = false, bool SINGLE = false>
 static int launch_matrix_unit(const DecodeGeom& g, unsigned units, hipStream_t st) {

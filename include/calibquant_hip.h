@@ -313,7 +313,8 @@ typedef struct cq_decode_plan {
     int chunk_tokens;     /* packed tokens per chunk */
     int launches;         /* 1 or 2 (what the plan asks for; see cq_decode_attn_wait_polls for when one becomes two) */
     int lds_bytes;        /* dynamic LDS of the main launch */
-    int register_logits;  /* a thread keeps the fp32 logits of this many rounds of `threads` tokens in registers;
+    int register_logits;  /* a thread keeps the fp32 logits of this many rounds of `threads` tokens, in registers and,
+                           * the last of them, in LDS of its own (static, beside lds_bytes);
                            * chunk_tokens <= register_logits * threads */
 } cq_decode_plan;
 int cq_decode_attn_plan(const cq_decode_args* args, cq_decode_plan* plan);

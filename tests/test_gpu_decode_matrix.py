@@ -260,3 +260,57 @@ def test_logit_range_below_the_resolution_of_the_logits(ops, form, log_scale):
     got = _run(ops, c, "fp16", 0, 1, mask=mask)
     want = O.decode_attention(c["q"], c["ck"], c["cv"], c["sk"], c["zk"], c["sv"], c["zv"], None, None, 0, 1, mask=mask, ftype=np.float64)
     _close(got, want)
+
+
+def _window_case(B, Hq, Hkv, T, rows, dtype, seed):
+    c = make_case(B, Hq, Hkv, 128, max(T, 64), rows, 1, dtype, seed=seed)
+    if T == 0:
+        c["ck"], c["cv"] = c["ck"][:, :, :0], c["cv"][:, :, :0]
+    return c
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape", [(1, 4, 1), (3, 12, 4), (2, 16, 8), (40, 32, 8)])   # 1, 3 and 2 heads in 1 024 threads, 4 in 512
+def test_window_edges(ops, shape, dtype):
+    """Windows around a wave's 8 or 16 rows, a tile's 128 and the first row of the next, with and without packed tokens."""
+    B, Hq, Hkv = shape
+    for T, rows in ((0, 1), (0, 129), (70, 7), (70, 9), (70, 16), (70, 17), (70, 127), (70, 128), (70, 257)):
+        print(f"case window {shape} {dtype} T={T} rows={rows}", flush=True)
+        c = _window_case(B, Hq, Hkv, T, rows, dtype, rows)
+        _close(_run(ops, c, dtype, min(rows, 5), 1), _oracle(c, min(rows, 5), 1), 2.0 ** -11 if dtype == "fp16" else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+def test_window_weights_of_all_sizes(ops, dtype):
+    """One row weighs 1, the others 2^-12 to 2^-22 each but have values of 512 times its size, which adds up: the parts a weight is held in
+    keep small ones as exactly as large ones.  An infinite value makes its channel infinite and no other."""
+    B, Hq, Hkv, R = 1, 4, 1, 130
+    c = _window_case(B, Hq, Hkv, 0, R, dtype, 3)
+    c["q"][:] = 0
+    c["q"][..., 0] = 8.0
+    c["kr"][:] = 0
+    c["kr"][0, 0, :, 0] = -np.linspace(12, 21, R)
+    c["kr"][0, 0, 77, 0] = 0
+    c["vr"] = np.where(np.arange(R)[:, None] == 77, 0.25, 128.0 * (1 + np.arange(R)[:, None] % 7) / 7) * np.ones_like(c["vr"])
+    c["vr"] = O.round_to(c["vr"].astype(np.float32), dtype)
+    rounding = 2.0 ** -11 if dtype == "fp16" else 2.0 ** -8
+    _close(_run(ops, c, dtype, 0, 1), _oracle(c, 0, 1), rounding)
+    c["vr"][0, 0, 77, 3] = np.inf
+    got, want = _run(ops, c, dtype, 0, 1), _oracle(c, 0, 1)
+    assert (got[..., 3] == np.inf).all()   # (a weight of 1 on an infinite value, none on any other)
+    _close(np.delete(got, 3, -1), np.delete(want, 3, -1), rounding)
+
+
+def test_query_and_statistics_on_odd_addresses(ops):
+    """q and the statistics are read two values at a time and need no alignment beyond their own."""
+    def odd(t):
+        o = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+        return o.copy_(t)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda", dtype=torch.bfloat16)
+    ck, sk, zk = ops.quantize_pack(r(2, 150, 4, 128), 1, 0.5)
+    cv, sv, zv = ops.quantize_pack(r(2, 150, 4, 128), 1, 0.3)
+    q = r(2, 16, 128)
+    want = ops.decode_attn(q, ck, cv, sk, zk, sv, zv, None, None, sprompt_len=0, bits=1)
+    got = ops.decode_attn(odd(q), ck, cv, odd(sk), odd(zk), odd(sv), odd(zv), None, None, sprompt_len=0, bits=1)
+    assert torch.equal(got, want)
