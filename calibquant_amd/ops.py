@@ -6,6 +6,7 @@ and `decode_attn` replaces its decode branch (patch_internvl.py:344-436).  Both
 call the C-ABI library on torch's current stream; torch only owns the memory."""
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 from typing import Optional, Tuple
 
@@ -17,8 +18,17 @@ _DT = {torch.bfloat16: _lib.CQ_BF16, torch.float16: _lib.CQ_FP16, torch.float32:
        torch.int64: _lib.CQ_I64, torch.int32: _lib.CQ_I32, torch.uint8: _lib.CQ_U8}
 
 
+# The raw handle of torch's current stream (0.1 us; building the stream object around it takes 1.9 us), and the device switch only
+# where the thread's current device is another one: a small call is bound by the host (batch 1 x 1 024 tokens 6.9 -> 5.9 us).
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    return _SAME_DEVICE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 def _need_gpu(t: torch.Tensor, name: str) -> None:
@@ -60,7 +70,8 @@ def _decode_workspace(nbytes: int, device) -> Optional[torch.Tensor]:
     if nbytes == 0:
         return None
     dev = torch.device(device)
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(), torch.cuda.current_stream(dev).cuda_stream)
+    index = dev.index if dev.index is not None else torch.cuda.current_device()
+    key = (index, torch._C._cuda_getCurrentRawStream(index))
     ws = _decode_ws.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
@@ -83,7 +94,7 @@ def quantize_pack(x: torch.Tensor, bits: int, clip: float) -> Tuple[torch.Tensor
     scale = torch.empty((B, H, D), dtype=x.dtype, device=x.device)
     zero = torch.empty((B, H, D), dtype=x.dtype, device=x.device)
     ws = _workspace(lib.cq_quantize_pack_workspace(B, T, H, D), x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = lib.cq_quantize_pack(x.data_ptr(), dt, B, T, H, D, x.stride(0), x.stride(1), x.stride(2),
                                   bits, float(clip), codes.data_ptr(), scale.data_ptr(), zero.data_ptr(),
                                   ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0,
@@ -128,7 +139,7 @@ def rope_rows(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, pos, out: O
     if out is None:
         out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
     args, keep = _rope_args(x, cos, sin, pos, out)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = _lib.load().cq_rope_rows(*args, _stream(x))
     _lib.check(rc, "cq_rope_rows")
     return out
@@ -146,7 +157,7 @@ def rope_rows_grouped(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, pos
         raise _lib.CalibQuantError("rope: out must be shaped like x with a contiguous last axis")
     args, keep = _rope_args(x[:, :, :, 0], cos, sin, pos, out[:, :, :, 0])
     (xp, dt, B, T, H, D, sb, st_, sh, cp, sp, rows, pp, psb, pst, p0, op, ob, ot, oh) = args
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = _lib.load().cq_rope_rows_grouped(xp, dt, B, T, H, x.shape[3], D, sb, st_, sh, x.stride(3), cp, sp, rows,
                                               pp, psb, pst, p0, op, ob, ot, oh, out.stride(3), _stream(x))
     _lib.check(rc, "cq_rope_rows_grouped")
@@ -170,7 +181,7 @@ def rope_quantize_pack(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, po
     scale = torch.empty((B, H, D), dtype=x.dtype, device=x.device)
     zero = torch.empty((B, H, D), dtype=x.dtype, device=x.device)
     ws = _workspace(lib.cq_quantize_pack_workspace(B, T, H, D), x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = lib.cq_rope_quantize_pack(*args, int(bits), float(clip), codes.data_ptr(), scale.data_ptr(),
                                        zero.data_ptr(), ws.data_ptr(), ws.numel(), _stream(x))
     _lib.check(rc, "cq_rope_quantize_pack")
@@ -193,7 +204,7 @@ def quantize_pack_token(x: torch.Tensor, bits: int, group_size: int = 32):
     words = torch.empty((B, H, T, D * bits // 32), dtype=torch.int32, device=x.device)
     scale = torch.empty((B, H, T, D // group_size), dtype=x.dtype, device=x.device)
     mins = torch.empty_like(scale)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = lib.cq_quantize_pack_token(x.data_ptr(), dt, B, T, H, D, x.stride(0), x.stride(1), x.stride(2),
                                         int(bits), int(group_size), words.data_ptr(), scale.data_ptr(),
                                         mins.data_ptr(), _stream(x))
@@ -214,7 +225,7 @@ def quant_codes(x: torch.Tensor, bits: int, clip: float):
     scale = torch.empty((B, 1, H, D), dtype=x.dtype, device=x.device)
     zero = torch.empty((B, 1, H, D), dtype=x.dtype, device=x.device)
     ws = _workspace(lib.cq_quantize_pack_workspace(B, T, H, D), x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = lib.cq_quant(x.data_ptr(), dt, B, T, H, D, x.stride(0), x.stride(1), x.stride(2),
                           bits, float(clip), xq.data_ptr(), scale.data_ptr(), zero.data_ptr(),
                           ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _stream(x))
@@ -241,7 +252,7 @@ def quant_codes_tensor(x: torch.Tensor, bits: int, clip: float):
     xq = torch.empty((B, T, H, D), dtype=x.dtype, device=x.device)
     stats = torch.empty(16, dtype=x.dtype, device=x.device)        # scale at [0], zero-point at [8]
     ws = _workspace(lib.cq_quantize_pack_workspace(B, T, H, D), x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = lib.cq_quant_tensor(x4.data_ptr(), dt, B, T, H, D, x4.stride(0), x4.stride(1), x4.stride(2),
                                  bits, float(clip), xq.data_ptr(), stats[0:].data_ptr(), stats[8:].data_ptr(),
                                  ws.data_ptr(), ws.numel(), _stream(x))
@@ -258,7 +269,7 @@ def encode_indices(idx: torch.Tensor, bits: int) -> torch.Tensor:
     D = idx.shape[-1]
     rows = idx.numel() // D if D else 0
     out = torch.empty((*idx.shape[:-1], D * bits // 8), dtype=torch.uint8, device=idx.device)
-    with torch.cuda.device(idx.device):
+    with _on(idx.device):
         rc = _lib.load().cq_encode(idx.data_ptr(), _DT[idx.dtype], rows, D, bits, out.data_ptr(), _stream(idx))
     _lib.check(rc, "cq_encode")
     return out
@@ -277,7 +288,7 @@ def lut_vecmat(kind: str, lut: torch.Tensor, a: torch.Tensor, enc: torch.Tensor,
     D = nb * 8 // bits
     out = torch.empty((M, T if kind == "qk" else D), dtype=torch.float16, device=a.device)
     fn = _lib.load().cq_lut_vecmat_qk if kind == "qk" else _lib.load().cq_lut_vecmat_pv
-    with torch.cuda.device(a.device):
+    with _on(a.device):
         rc = fn(lut.data_ptr(), _DT[lut.dtype], lut.numel(), a.data_ptr(), _DT[a.dtype], enc.data_ptr(), M, T, D, bits,
                 out.data_ptr(), _stream(a))
     _lib.check(rc, f"cq_lut_vecmat_{kind}")
@@ -397,7 +408,7 @@ class DecodeCall:
         return self.run()
 
     def run(self) -> torch.Tensor:
-        rc = self._entry(self._ref, torch.cuda.current_stream(self.device).cuda_stream)
+        rc = self._entry(self._ref, torch._C._cuda_getCurrentRawStream(self.device.index))
         if rc:
             _lib.check(rc, "cq_decode_attn")
         return self.out
@@ -422,7 +433,7 @@ def decode_attn(q: torch.Tensor, codes_k: Optional[torch.Tensor], codes_v: Optio
     Returns (B, Hq, D)."""
     call = DecodeCall(q, codes_k, codes_v, k_scale, k_zero, v_scale, v_zero, k_res, v_res,
                       sprompt_len, bits, calibrate, calib_off_max, calib_off_min, mask, out, force_splits, r_dev, v_mode)
-    with torch.cuda.device(call.device):
+    with _on(call.device):
         return call.run()
 
 
@@ -471,6 +482,6 @@ class RopeAppendCall:
         self.run()
 
     def run(self) -> None:
-        rc = self._lib.cq_rope_append(*self._args, torch.cuda.current_stream(self.device).cuda_stream)
+        rc = self._lib.cq_rope_append(*self._args, torch._C._cuda_getCurrentRawStream(self.device.index))
         if rc:
             _lib.check(rc, "cq_rope_append")
