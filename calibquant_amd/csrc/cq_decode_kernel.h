@@ -81,8 +81,10 @@ constexpr int parked_rounds(bool vtok, int nt, int rounds) {
     return nt == 512 ? 4 : 5;
 }
 
-// ... and the bytes of it (static LDS, beside the dynamic): at least a tile of 128 window rows
-constexpr int parked_lds(bool vtok, int nt, int rounds) { return cmax(parked_rounds(vtok, nt, rounds) * nt * 16, 128 * 256); }
+// ... and the bytes of it (static LDS, beside the dynamic): at least a tile of 128 window rows; two for 1 024 threads, which have the
+// LDS to themselves and take the tiles in turn: no barrier between the values of one and the rows of the next
+constexpr int kWindowTile = 128 * 256;
+constexpr int parked_lds(bool vtok, int nt, int rounds) { return cmax(parked_rounds(vtok, nt, rounds) * nt * 16, nt == 1024 ? 2 * kWindowTile : kWindowTile); }
 
 struct DecodeGeom {
     const void* q;
@@ -212,6 +214,17 @@ __device__ __forceinline__ int virtual_block_id() {
     const int l = blockIdx.x;
     if ((n & 7) == 0) return (l & 7) * (n >> 3) + (l >> 3);
     return l;
+}
+
+// Two-element dot product with fp32 accumulation on raw 16-bit pairs.
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+template <typename DT> __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c);
+template <> __device__ __forceinline__ float dot2<BF16>(uint32_t a, uint32_t b, float c) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
+}
+template <> __device__ __forceinline__ float dot2<FP16>(uint32_t a, uint32_t b, float c) {
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, a), __builtin_bit_cast(f16x2_t, b), c, false);
 }
 
 // The window's products, 16 x 16 x 32 on raw 16-bit values; a lane's left (right) operand is row (column) lane % 16, k = 8 (lane / 16) + 0 .. 7
@@ -718,6 +731,9 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         z_raw = zp[pair];
     }
     static_assert(HPB < kNW, "a wave is left for the values' statistics");
+    // Two heads or one: few units (or few heads), where a launch lasts as long as its phases in a row; dot products straight from the loaded rows
+    // are the shorter chain (us, 2 x 800 + 250, 16 / 4 heads 8.0 for 8.3; 1 x 300 + 60 6.25 for 6.45).
+    constexpr bool kDotWindow = HPB <= 2;
     const int64_t code_off = has_img ? (bh * g.T + t0) * NB : 0;   // one offset for both code streams
     const uint4* ckp = reinterpret_cast<const uint4*>(has_img ? g.ck + code_off : static_cast<const uint8_t*>(g.q));
     const uint4* cvp = reinterpret_cast<const uint4*>((has_img ? g.cv : static_cast<const uint8_t*>(g.q)) + code_off);
@@ -1062,7 +1078,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                     smin[r] = vmp[min(tid + r * kNT, n - 1)];
                 }
             }
-            load_res(kb, 0, rk);   // the first tile of the window: its K rows arrive during the packed V rows
+            if constexpr (!kDotWindow) load_res(kb, 0, rk);   // the first tile of the window: its K rows arrive during the packed V rows
             phase_priority(std::integral_constant<int, 3>{});
             auto weights = [&](int rd, float* e) {   // of round rd's tile
                 const int tw = wt0 + rd * kNT;
@@ -1121,7 +1137,8 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 }
             }
             phase_priority(std::integral_constant<int, 4>{});
-            load_res(vbp, 0, rv);   // ... its V rows: in flight during the fold and the window's logits
+            if constexpr (kDotWindow) load_res(kb, 0, rk);
+            else load_res(vbp, 0, rv);   // ... its V rows: in flight during the fold and the window's logits
             float* lpart = fx + L::F_PRES;   // the waves' sums of e (not in `red`, which a slower wave may still read)
             lsum = row_reduce(lsum, OpSum(), 0.f);
             constexpr int kParts = VTOK ? 5 : 1;     // VTOK: and of e * minimum per channel group
@@ -1164,7 +1181,10 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             // window, and `stat` is read behind the one of the merge)
         }
 
-        if (n == 0) { load_res(kb, 0, rk); load_res(vbp, 0, rv); }
+        if (n == 0) {
+            load_res(kb, 0, rk);
+            if constexpr (!kDotWindow) load_res(vbp, 0, rv);
+        }
         CQ_PHASE(8);   // fold of the packed part
         // ---- phase 6: full-precision residual rows, online softmax.  Runs last: its first
         // tile is requested when the packed-V phase ends and arrives during that phase's fold.
@@ -1176,83 +1196,188 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
             }
         }
         if (do_res) {
-            float m_run = -INFINITY, l_run = 0.f;
-            float* sres = fx + L::F_SRES;
-            unsigned char* wrows = reinterpret_cast<unsigned char*>(parked) + wv * 1024;   // a wave's rows: four to 1 KB, NT * 16 apart
-            auto row_piece = [&](int row, int piece) { return (row >> 2) * (NT * 16) + (row & 3) * 256 + ((piece ^ row) << 4); };
-            auto park_rows = [&](const U4* v) {
+            if constexpr (kDotWindow) {
+                float m_run = -INFINITY, l_run = 0.f;
+                float* sres = fx + L::F_SRES;
+                float* pres = fx + L::F_PRES;
+                // raw 16-bit q, [head][kD], read per head as two 16-byte LDS loads
+                const uint4* q128 = reinterpret_cast<const uint4*>(fx + L::F_QRAW);
+                float accv[2][HPB];   // the lane's channel pair
 #pragma unroll
-                for (int i = 0; i < NKP; ++i) *reinterpret_cast<U4*>(wrows + row_piece(lane / LPR, i * LPR + lq)) = v[i];
-            };
-            const int x = lane & 15, kg = lane >> 4;
-            const unsigned char* q16 = smem + L::kRegionA + L::F_QRAW * 4 + min(x >> 2, HPB - 1) * (kD * 2) + kg * 16;   // left operand: rows 4 h .. 4 h + 3 are head h
-            constexpr int kPB = 272;   // bytes of a row of weight parts: 128 window rows and 16 bytes against bank conflicts
-            unsigned char* parts = regA;    // [4 * head + part][window row], read by the fold above before the tile's first barrier
-            static_assert(16 * kPB <= L::kRegionA, "the weights' parts fit region A");
-            F4 racc = {0.f, 0.f, 0.f, 0.f};
+                for (int k = 0; k < 2; ++k)
+#pragma unroll
+                    for (int h = 0; h < HPB; ++h) accv[k][h] = 0.f;
 
-            for (int r0 = 0; r0 < R; r0 += kResTile) {
-                const bool more = r0 + kResTile < R;
-                if (r0 > 0) __syncthreads();   // (the values of the tile before are read)
-                park_rows(rk);
-                if (more) load_res(kb, r0 + kResTile, rk);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                F4 dot = {0.f, 0.f, 0.f, 0.f};
-                const int xr = x % RPW;   // (waves of eight rows: columns 8 .. 15 repeat them)
+                for (int r0 = 0; r0 < R; r0 += kResTile) {
+                    const bool more = r0 + kResTile < R;
+                    const int r = r0 + krow;
+                    uint32_t vw[RPW];   // the tile's value words, a channel pair of the wave's rows: in flight while its logits and weights are worked out
 #pragma unroll
-                for (int s = 0; s < 4; ++s)
-                    dot = mfma16<DT>(*reinterpret_cast<const U4*>(q16 + 64 * s), *reinterpret_cast<const U4*>(wrows + row_piece(xr, 4 * s + kg)), dot);
-                if (x < RPW && kg < HPB) {
-                    const int r = r0 + wv * RPW + x;
-                    float w = dot[0] * inv_sqrt_d;
-                    if (masked && r < R) w += r0 == 0 ? mask_w : mask_win[r < g.S ? r : g.T + r];
-                    sres[(wv * RPW + x) * HPB + kg] = r < R ? w : -INFINITY;
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                park_rows(rv);
-                if (more) load_res(vbp, r0 + kResTile, rv);
-                __syncthreads();
-                if (wv < NH) {   // wave h keeps the running softmax state of head h; a lane two neighbouring rows
-                    const int h = wv;
-                    const float s0 = sres[2 * lane * HPB + h], s1 = sres[(2 * lane + 1) * HPB + h];
-                    const float mnew = fmaxf(m_run, wave_max(fmaxf(s0, s1)));
-                    const bool dead = (mnew == -INFINITY);
-                    const float p0 = dead ? 0.f : __expf(s0 - mnew), p1 = dead ? 0.f : __expf(s1 - mnew);
-                    uint32_t w0[3], w1[3];
-                    split_weight<DT>(p0, w0);
-                    split_weight<DT>(p1, w1);
+                    for (int i = 0; i < RPW; ++i) vw[i] = *reinterpret_cast<const uint32_t*>(vbp + min(r0 + wvu * RPW + i, last_r) * rs_r + 2 * lane);
+                    float dot[HPB];
 #pragma unroll
-                    for (int i = 0; i < 3; ++i) *reinterpret_cast<uint32_t*>(parts + (4 * h + i) * kPB + 4 * lane) = w0[i] | (w1[i] << 16);
-                    const float al = dead ? 1.0f : __expf(m_run - mnew);
-                    l_run = l_run * al + wave_sum(p0 + p1);
-                    m_run = mnew;
-                    if (lane == 0) { stat[h] = al; stat[HPB + h] = m_run; stat[2 * HPB + h] = l_run; }
-                }
-                __syncthreads();
-                if (wv < 8) {   // 16 channels of all heads: a wave each
-                    if (r0 > 0) racc *= stat[hl];
+                    for (int h = NH; h < HPB; ++h) dot[h] = 0.f;
 #pragma unroll
-                    for (int s = 0; s < kResTile / 32; ++s) {
-                        const U4 w = *reinterpret_cast<const U4*>(parts + x * kPB + 64 * s + 16 * kg);
-                        U4 v;
+                    for (int h = 0; h < NH; ++h) {
+                        float a = 0.f;
 #pragma unroll
-                        for (int t = 0; t < 2; ++t) {   // rows 32 s + 8 kg + 4 t + 0 .. 3: column x of four rows
-                            const int row = (8 * kg + 4 * t + (x >> 2)) % RPW;
-                            const unsigned char* o = reinterpret_cast<const unsigned char*>(parked) + ((32 * s + 8 * kg) / RPW) * 1024 +
-                                                     row_piece(row, 2 * wv + ((x >> 1) & 1)) + (x & 1) * 8;
-                            const U2 c = __builtin_bit_cast(U2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) S4*)(o)));
-                            v[2 * t] = c.x; v[2 * t + 1] = c.y;
+                        for (int i = 0; i < NKP; ++i) {
+                            const uint4 qa = q128[h * (kD / 8) + i * LPR + lq];
+                            a = dot2<DT>(qa.x, rk[i].x, a); a = dot2<DT>(qa.y, rk[i].y, a);
+                            a = dot2<DT>(qa.z, rk[i].z, a); a = dot2<DT>(qa.w, rk[i].w, a);
                         }
-                        racc = mfma16<DT>(w, v, racc);
+                        dot[h] = (LPR == 4 ? quad_reduce(a, OpSum(), 0.f) : oct_reduce(a, OpSum(), 0.f)) * inv_sqrt_d;
+                    }
+                    if (more) load_res(kb, r0 + kResTile, rk);   // next tile's K slice, in place
+                    if (lq == 0) {
+                        float mv = 0.f;
+                        if (masked && r < R) mv = mask_win[r < g.S ? r : g.T + r];
+#pragma unroll
+                        for (int h = 0; h < HPB; ++h) sres[krow * HPB + h] = (r < R) ? dot[h] + mv : -INFINITY;
+                    }
+                    __syncthreads();
+                    if (wv < NH) {   // wave h keeps the running softmax state of head h
+                        const int h = wv;
+                        constexpr int kRL = kResTile / kWave;   // tile rows per lane
+                        float sv[kRL], smax = -INFINITY;
+#pragma unroll
+                        for (int i = 0; i < kRL; ++i) {
+                            sv[i] = sres[(lane + i * kWave) * HPB + h];
+                            smax = fmaxf(smax, sv[i]);
+                        }
+                        const float mnew = fmaxf(m_run, wave_max(smax));
+                        const bool dead = (mnew == -INFINITY);
+                        float psum = 0.f;
+#pragma unroll
+                        for (int i = 0; i < kRL; ++i) {
+                            const float pi = dead ? 0.f : __expf(sv[i] - mnew);
+                            pres[(lane + i * kWave) * HPB + h] = pi;
+                            psum += pi;
+                        }
+                        const float al = dead ? 1.0f : __expf(m_run - mnew);
+                        l_run = l_run * al + wave_sum(psum);
+                        m_run = mnew;
+                        if (lane == 0) { stat[h] = al; stat[HPB + h] = m_run; stat[2 * HPB + h] = l_run; }
+                    }
+                    __syncthreads();
+                    if (r0 > 0) {
+#pragma unroll
+                        for (int h = 0; h < NH; ++h) {
+                            const float al = stat[h];
+                            accv[0][h] *= al;
+                            accv[1][h] *= al;
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < RPW; ++i) {
+                        const float f0 = Cvt<DT>::lo(vw[i]), f1 = Cvt<DT>::hi(vw[i]);
+                        const Vec<HPB> p = reinterpret_cast<const Vec<HPB>*>(pres)[wvu * RPW + i];   // the row's weights (0 past R), one address per wave
+#pragma unroll
+                        for (int h = 0; h < NH; ++h) {
+                            accv[0][h] = __builtin_fmaf(p.v[h], f0, accv[0][h]);
+                            accv[1][h] = __builtin_fmaf(p.v[h], f1, accv[1][h]);
+                        }
                     }
                 }
+                // (regA was last read by the packed part's sum, behind which lie the tiles' barriers)
+                float* red2 = reinterpret_cast<float*>(regA);  // [wave][head][kD]: the fold reads consecutive words
+#pragma unroll
+                for (int h = 0; h < HPB; ++h) {
+                    Vec<2> a2;
+                    a2.v[0] = accv[0][h]; a2.v[1] = accv[1][h];
+                    *reinterpret_cast<Vec<2>*>(red2 + (wv * HPB + h) * kD + 2 * lane) = a2;
+                }
+                __syncthreads();
+                if (owns) {
+#pragma unroll
+                    for (int w = 0; w < kNW; ++w) o_res += red2[(w * HPB + hl) * kD + od];
+                }
+            } else {
+                float m_run = -INFINITY, l_run = 0.f;
+                float* sres = fx + L::F_SRES;
+                unsigned char* tile_rows = reinterpret_cast<unsigned char*>(parked);
+                unsigned char* wrows = tile_rows + wv * 1024;   // a wave's rows: four to 1 KB, NT * 16 apart
+                auto row_piece = [&](int row, int piece) { return (row >> 2) * (NT * 16) + (row & 3) * 256 + ((piece ^ row) << 4); };
+                auto park_rows = [&](const U4* v) {
+#pragma unroll
+                    for (int i = 0; i < NKP; ++i) *reinterpret_cast<U4*>(wrows + row_piece(lane / LPR, i * LPR + lq)) = v[i];
+                };
+                const int x = lane & 15, kg = lane >> 4;
+                const unsigned char* q16 = smem + L::kRegionA + L::F_QRAW * 4 + min(x >> 2, HPB - 1) * (kD * 2) + kg * 16;   // left operand: rows 4 h .. 4 h + 3 are head h
+                constexpr int kPB = 272;   // bytes of a row of weight parts: 128 window rows and 16 bytes against bank conflicts
+                unsigned char* parts = regA;    // [4 * head + part][window row], read by the fold above before the tile's first barrier
+                static_assert(16 * kPB <= L::kRegionA, "the weights' parts fit region A");
+                F4 racc = {0.f, 0.f, 0.f, 0.f};
+
+                for (int r0 = 0; r0 < R; r0 += kResTile) {
+                    const bool more = r0 + kResTile < R;
+                    if (r0 > 0) {
+                        if constexpr (NT == 1024) {
+                            const int other = (r0 / kResTile) % 2 ? kWindowTile : -kWindowTile;
+                            tile_rows += other;
+                            wrows += other;
+                        } else {
+                            __syncthreads();   // (the values of the tile before are read)
+                        }
+                    }
+                    park_rows(rk);
+                    if (more) load_res(kb, r0 + kResTile, rk);
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    F4 dot = {0.f, 0.f, 0.f, 0.f};
+                    const int xr = x % RPW;   // (waves of eight rows: columns 8 .. 15 repeat them)
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        dot = mfma16<DT>(*reinterpret_cast<const U4*>(q16 + 64 * s), *reinterpret_cast<const U4*>(wrows + row_piece(xr, 4 * s + kg)), dot);
+                    if (x < RPW && kg < HPB) {
+                        const int r = r0 + wv * RPW + x;
+                        float w = dot[0] * inv_sqrt_d;
+                        if (masked && r < R) w += r0 == 0 ? mask_w : mask_win[r < g.S ? r : g.T + r];
+                        sres[(wv * RPW + x) * HPB + kg] = r < R ? w : -INFINITY;
+                    }
+                    __syncthreads();
+                    if (wv < NH) {   // wave h keeps the running softmax state of head h; a lane two neighbouring rows
+                        const int h = wv;
+                        const float s0 = sres[2 * lane * HPB + h], s1 = sres[(2 * lane + 1) * HPB + h];
+                        const float mnew = fmaxf(m_run, wave_max(fmaxf(s0, s1)));
+                        const bool dead = (mnew == -INFINITY);
+                        const float p0 = dead ? 0.f : __expf(s0 - mnew), p1 = dead ? 0.f : __expf(s1 - mnew);
+                        uint32_t w0[3], w1[3];
+                        split_weight<DT>(p0, w0);
+                        split_weight<DT>(p1, w1);
+#pragma unroll
+                        for (int i = 0; i < 3; ++i) *reinterpret_cast<uint32_t*>(parts + (4 * h + i) * kPB + 4 * lane) = w0[i] | (w1[i] << 16);
+                        const float al = dead ? 1.0f : __expf(m_run - mnew);
+                        l_run = l_run * al + wave_sum(p0 + p1);
+                        m_run = mnew;
+                        if (lane == 0) { stat[h] = al; stat[HPB + h] = m_run; stat[2 * HPB + h] = l_run; }
+                    }
+                    park_rows(rv);   // (over the wave's K rows; behind the weights, so that these do not wait for the values)
+                    if (more) load_res(vbp, r0 + kResTile, rv);
+                    __syncthreads();
+                    if (wv < 8) {   // 16 channels of all heads: a wave each
+                        if (r0 > 0) racc *= stat[hl];
+#pragma unroll
+                        for (int s = 0; s < kResTile / 32; ++s) {
+                            const U4 w = *reinterpret_cast<const U4*>(parts + x * kPB + 64 * s + 16 * kg);
+                            U4 v;
+#pragma unroll
+                            for (int t = 0; t < 2; ++t) {   // rows 32 s + 8 kg + 4 t + 0 .. 3: column x of four rows
+                                const int row = (8 * kg + 4 * t + (x >> 2)) % RPW;
+                                const unsigned char* o = tile_rows + ((32 * s + 8 * kg) / RPW) * 1024 +
+                                                         row_piece(row, 2 * wv + ((x >> 1) & 1)) + (x & 1) * 8;
+                                const U2 c = __builtin_bit_cast(U2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) S4*)(o)));
+                                v[2 * t] = c.x; v[2 * t + 1] = c.y;
+                            }
+                            racc = mfma16<DT>(w, v, racc);
+                        }
+                    }
+                }
+                o_res = racc[0];
+                // (an infinite sum stays one: 0, a lower part's, times an infinite value would make it a NaN)
+                if (__builtin_fabsf(o_res) != INFINITY) o_res += kPartScale<DT> * (racc[1] + kPartScale<DT> * racc[2]);
             }
-            o_res = racc[0];
-            // (an infinite sum stays one: 0, a lower part's, times an infinite value would make it a NaN)
-            if (__builtin_fabsf(o_res) != INFINITY) o_res += kPartScale<DT> * (racc[1] + kPartScale<DT> * racc[2]);
         }
 
         if (speaks) {

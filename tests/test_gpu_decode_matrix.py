@@ -270,7 +270,7 @@ def _window_case(B, Hq, Hkv, T, rows, dtype, seed):
 
 
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
-@pytest.mark.parametrize("shape", [(1, 4, 1), (3, 12, 4), (2, 16, 8), (40, 32, 8)])   # 1, 3 and 2 heads in 1 024 threads, 4 in 512
+@pytest.mark.parametrize("shape", [(1, 4, 1), (6, 32, 8), (30, 12, 4), (20, 16, 4), (40, 32, 8)])   # 1, 2, 3 and 4 heads in 1 024 threads, 4 in 512
 def test_window_edges(ops, shape, dtype):
     """Windows around a wave's 8 or 16 rows, a tile's 128 and the first row of the next, with and without packed tokens."""
     B, Hq, Hkv = shape
@@ -280,22 +280,23 @@ def test_window_edges(ops, shape, dtype):
         _close(_run(ops, c, dtype, min(rows, 5), 1), _oracle(c, min(rows, 5), 1), 2.0 ** -11 if dtype == "fp16" else 2.0 ** -8)
 
 
+@pytest.mark.parametrize("batch", [1, 70, 300])   # 1 head in 1 024 threads, 4 in 1 024, 4 in 512
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
-def test_window_weights_of_all_sizes(ops, dtype):
+def test_window_weights_of_all_sizes(ops, dtype, batch):
     """One row weighs 1, the others 2^-12 to 2^-22 each but have values of 512 times its size, which adds up: the parts a weight is held in
     keep small ones as exactly as large ones.  An infinite value makes its channel infinite and no other."""
-    B, Hq, Hkv, R = 1, 4, 1, 130
+    B, Hq, Hkv, R = batch, 4, 1, 130
     c = _window_case(B, Hq, Hkv, 0, R, dtype, 3)
     c["q"][:] = 0
     c["q"][..., 0] = 8.0
     c["kr"][:] = 0
-    c["kr"][0, 0, :, 0] = -np.linspace(12, 21, R)
-    c["kr"][0, 0, 77, 0] = 0
+    c["kr"][:, 0, :, 0] = -np.linspace(12, 21, R)
+    c["kr"][:, 0, 77, 0] = 0
     c["vr"] = np.where(np.arange(R)[:, None] == 77, 0.25, 128.0 * (1 + np.arange(R)[:, None] % 7) / 7) * np.ones_like(c["vr"])
     c["vr"] = O.round_to(c["vr"].astype(np.float32), dtype)
     rounding = 2.0 ** -11 if dtype == "fp16" else 2.0 ** -8
     _close(_run(ops, c, dtype, 0, 1), _oracle(c, 0, 1), rounding)
-    c["vr"][0, 0, 77, 3] = np.inf
+    c["vr"][:, 0, 77, 3] = np.inf
     got, want = _run(ops, c, dtype, 0, 1), _oracle(c, 0, 1)
     assert (got[..., 3] == np.inf).all()   # (a weight of 1 on an infinite value, none on any other)
     _close(np.delete(got, 3, -1), np.delete(want, 3, -1), rounding)
