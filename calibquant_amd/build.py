@@ -17,7 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIBPATH = os.path.join(LIBDIR, "libcalibquant_hip.so")
 SOURCES = ["cq_core.hip", "cq_quantize.hip", "cq_lutvecmat.hip", "cq_decode.hip", "cq_decode_matrix_bf16.hip",
-           "cq_decode_matrix_fp16.hip", "cq_decode_matrix_token_bf16.hip", "cq_decode_matrix_token_fp16.hip", "cq_rope.hip"]
+           "cq_decode_matrix_fp16.hip", "cq_decode_matrix_token_bf16.hip", "cq_decode_matrix_token_fp16.hip", "cq_rope.hip", "cq_linear.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

@@ -90,6 +90,17 @@ __device__ __forceinline__ void store_elem(void* p, int64_t i, float f) {
     static_cast<uint16_t*>(p)[i] = static_cast<uint16_t>(Cvt<DT>::from_float(f));
 }
 
+// Two-element dot product with fp32 accumulation on raw 16-bit pairs.
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+template <typename DT> __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c);
+template <> __device__ __forceinline__ float dot2<BF16>(uint32_t a, uint32_t b, float c) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
+}
+template <> __device__ __forceinline__ float dot2<FP16>(uint32_t a, uint32_t b, float c) {
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, a), __builtin_bit_cast(f16x2_t, b), c, false);
+}
+
 // Division of indices (< 2^31) by a small run-time constant without the integer-division
 // expansion: q = (mulhi(n, mul) + n) >> shift, with mul and shift worked out on the host.
 struct FastDiv {

@@ -216,17 +216,6 @@ __device__ __forceinline__ int virtual_block_id() {
     return l;
 }
 
-// Two-element dot product with fp32 accumulation on raw 16-bit pairs.
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-template <typename DT> __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c);
-template <> __device__ __forceinline__ float dot2<BF16>(uint32_t a, uint32_t b, float c) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
-}
-template <> __device__ __forceinline__ float dot2<FP16>(uint32_t a, uint32_t b, float c) {
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, a), __builtin_bit_cast(f16x2_t, b), c, false);
-}
-
 // The window's products, 16 x 16 x 32 on raw 16-bit values; a lane's left (right) operand is row (column) lane % 16, k = 8 (lane / 16) + 0 .. 7
 typedef __bf16 B8 __attribute__((ext_vector_type(8)));
 typedef _Float16 H8 __attribute__((ext_vector_type(8)));

@@ -67,14 +67,9 @@ class LayerStep {
     py::object step(const at::Tensor& qkv, const at::Tensor& pos, const at::Tensor& past_k) {
         const int64_t B = a_.B, Hq = a_.Hq, Hkv = a_.Hkv, D = a_.D;
         const int64_t R = len_ + 1;
-        if (pos.dim() < 1 || !qkv.is_cuda() || qkv.scalar_type() != dtype_ || !qkv.is_contiguous() ||
-            qkv.numel() != B * (Hq + 2 * Hkv) * D || qkv.device() != k_.device())
+        if (!qkv.is_cuda() || qkv.scalar_type() != dtype_ || !qkv.is_contiguous() ||
+            qkv.numel() != B * (Hq + 2 * Hkv) * D || qkv.device() != k_.device() || !next_token(pos, past_k))
             return py::none();
-        if (!pos.is_cuda() || pos.scalar_type() != at::kLong || pos.device() != k_.device() || pos.size(0) != B ||
-            !(pos.dim() == 1 || (pos.dim() == 2 && pos.size(1) == 1)))
-            return py::none();
-        if (past_k.data_ptr() != k_.data_ptr() || past_k.dim() != 4 || past_k.size(2) != len_) return py::none();
-        if (R + a_.T > cos_.size(0) || R > ramp_.numel()) return py::none();
         c10::hip::HIPGuardMasqueradingAsCUDA guard(k_.device());
         if (R > k_.size(2)) grow(R);
         auto opts = qkv.options();
@@ -100,11 +95,49 @@ class LayerStep {
         return py::make_tuple(out, k_.narrow(2, 0, R), v_.narrow(2, 0, R));
     }
 
+    // The same with both projections: hidden (B, 1, K), the weights of wqkv ((Hq + 2 Hkv) D, K) and wo (N, Hq D), no bias.  The projections
+    // of a few rows run in the library (cq_linear_rows); None where those do not take the sizes or the step is not the steady-state
+    // one.  The first of the results is wo's output.  (A library product of such rows costs 20 us of host time to launch.)
+    py::object step_rows(const at::Tensor& hidden, const at::Tensor& wqkv, const at::Tensor& wo, const at::Tensor& pos, const at::Tensor& past_k) {
+        const int64_t B = a_.B, NQ = static_cast<int64_t>(a_.Hq + 2 * a_.Hkv) * a_.D, KO = static_cast<int64_t>(a_.Hq) * a_.D;
+        auto ours = [&](const at::Tensor& t) {
+            return t.is_cuda() && t.scalar_type() == dtype_ && t.device() == k_.device() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+        };
+        if (hidden.dim() != 3 || hidden.size(0) != B || hidden.size(1) != 1 || wqkv.dim() != 2 || wo.dim() != 2 || wqkv.size(0) != NQ ||
+            wqkv.size(1) != hidden.size(2) || wo.size(1) != KO || hidden.size(2) > INT32_MAX || wo.size(0) > INT32_MAX)
+            return py::none();
+        const int K = static_cast<int>(hidden.size(2)), N = static_cast<int>(wo.size(0));
+        if (!cq_linear_rows_takes(a_.B, K, static_cast<int>(NQ)) || !cq_linear_rows_takes(a_.B, static_cast<int>(KO), N) || !ours(hidden) ||
+            hidden.stride(2) != 1 || hidden.stride(0) % 8 != 0 || !ours(wqkv) || !wqkv.is_contiguous() || !ours(wo) || !wo.is_contiguous() ||
+            !next_token(pos, past_k))
+            return py::none();
+        c10::hip::HIPGuardMasqueradingAsCUDA guard(k_.device());
+        hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(k_.device().index()).stream();
+        at::Tensor qkv = at::empty({B, 1, NQ}, hidden.options());
+        check(cq_linear_rows(hidden.data_ptr(), hidden.stride(0), a_.dtype, a_.B, K, wqkv.data_ptr(), static_cast<int>(NQ), qkv.data_ptr(), stream), "cq_linear_rows");
+        py::object got = step(qkv, pos, past_k);
+        if (got.is_none()) return got;
+        const py::tuple t = got;
+        const at::Tensor att = t[0].cast<at::Tensor>();
+        at::Tensor out = at::empty({B, 1, N}, hidden.options());
+        check(cq_linear_rows(att.data_ptr(), KO, a_.dtype, a_.B, static_cast<int>(KO), wo.data_ptr(), N, out.data_ptr(), stream), "cq_linear_rows");
+        return py::make_tuple(out, t[1], t[2]);
+    }
+
     int64_t length() const { return len_; }
     int64_t steps() const { return steps_; }
     int64_t capacity() const { return k_.size(2); }
 
   private:
+    // the caller's position and window are those of the next token of the window this object handed out, within the tables
+    bool next_token(const at::Tensor& pos, const at::Tensor& past_k) const {
+        if (!pos.is_cuda() || pos.scalar_type() != at::kLong || pos.device() != k_.device() || pos.dim() < 1 || pos.size(0) != a_.B ||
+            !(pos.dim() == 1 || (pos.dim() == 2 && pos.size(1) == 1)))
+            return false;
+        if (past_k.data_ptr() != k_.data_ptr() || past_k.dim() != 4 || past_k.size(2) != len_) return false;
+        return len_ + 1 + a_.T <= cos_.size(0) && len_ + 1 <= ramp_.numel();
+    }
+
     // New buffers with head-room; the rows held so far are copied once (the reference copies the
     // whole window on every step, patch_internvl.py:264-266).
     void grow(int64_t need) {
@@ -133,6 +166,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     py::class_<LayerStep>(m, "LayerStep")
         .def(py::init<uintptr_t, size_t, at::Tensor, at::Tensor, at::Tensor, at::Tensor, int64_t, at::Tensor>())
         .def("step", &LayerStep::step)
+        .def("step_rows", &LayerStep::step_rows)
         .def_property_readonly("length", &LayerStep::length)
         .def_property_readonly("steps", &LayerStep::steps)
         .def_property_readonly("capacity", &LayerStep::capacity);

@@ -21,6 +21,7 @@ import warnings
 from typing import Optional, Tuple
 
 import torch
+from torch.nn.modules import module as _module
 
 from . import _lib, ops
 from ._lib import CalibQuantError
@@ -129,6 +130,21 @@ def _image_token_num(self) -> int:
     return int(n)
 
 
+def _plain_products(*modules) -> bool:
+    """Whether calling the modules would be nothing but a product with their weights: plain `nn.Linear`s without bias, hooks or a
+    replaced `forward`, outside of autograd, autocast, tracing, compilation, function transforms and tensor modes."""
+    if (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None
+            or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or _module._global_forward_hooks or _module._global_forward_pre_hooks):
+        return False
+    for m in modules:
+        if (type(m) is not torch.nn.Linear or m.bias is not None or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                or m._backward_pre_hooks or "forward" in m.__dict__ or type(m.weight) not in (torch.nn.Parameter, torch.Tensor)):
+            return False
+    return True
+
+
 def forward_internlm2_calibquant(self, hidden_states: torch.Tensor, attention_mask: Optional[torch.Tensor] = None,
                                  position_ids: Optional[torch.LongTensor] = None,
                                  past_key_value: Optional[Tuple[torch.Tensor]] = None,
@@ -147,6 +163,10 @@ def forward_internlm2_calibquant(self, hidden_states: torch.Tensor, attention_ma
     fast = self.__dict__.get("_cq_step")
     if (fast is not None and attention_mask is None and past_key_value is not None and position_ids is not None
             and not kwargs and hidden_states.shape[1] == 1):
+        if hidden_states.shape[0] <= 8 and _plain_products(self.wqkv, self.wo):
+            got = fast[0].step_rows(hidden_states, self.wqkv.weight, self.wo.weight, position_ids, past_key_value[0])
+            if got is not None:
+                return got[0], None, ((got[1], got[2]) if use_cache else None)
         got = fast[0].step(self.wqkv(hidden_states), position_ids, past_key_value[0])
         if got is not None:
             return self.wo(got[0]), None, ((got[1], got[2]) if use_cache else None)

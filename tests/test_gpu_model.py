@@ -400,3 +400,73 @@ def test_two_prefills_follow_the_environment_variable(monkeypatch):
             assert np.array_equal(att.encoded_features_v.cpu().numpy(), cv)
         with pytest.raises(CalibQuantError):
             pi.forward_internlm2_calibquant(att, x, torch.zeros(B, 1, N, N, device="cuda"), pos, None, False, True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 2048, 8), (2, 2560, 24), (3, 4096, 520), (4, 4096, 6144), (5, 6144, 1032), (8, 4096, 4096)])
+def test_linear_rows(shape, dtype):
+    """Rows beside the instantiated 1, 2, 4 and 8, slices beside the eight in flight, rows of x apart; against 64 bits, no further off than the
+    library's product beyond one unit of the sums' last places."""
+    import ctypes as C
+    from calibquant_amd import _lib
+    M, K, N = shape
+    print(f"case linear rows {shape} {dtype}", flush=True)
+    lib = _lib.load()
+    assert lib.cq_linear_rows_takes(M, K, N)
+    g = torch.Generator(device="cuda").manual_seed(K + M)
+    x = torch.randn((M, 2, K), generator=g, device="cuda", dtype=dtype)[:, 1]
+    w = torch.randn((N, K), generator=g, device="cuda", dtype=dtype) * K ** -0.5
+    out = torch.full((M + 1, N), 7.0, device="cuda", dtype=dtype)
+    rc = lib.cq_linear_rows(C.c_void_p(x.data_ptr()), x.stride(0), _lib.CQ_BF16 if dtype == torch.bfloat16 else _lib.CQ_FP16, M, K,
+                            C.c_void_p(w.data_ptr()), N, C.c_void_p(out.data_ptr()), C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert (out[M] == 7).all()
+    want = x.double() @ w.double().T
+    err = lambda t: ((t.double() - want).norm() / want.norm()).item()
+    ours, library = err(out[:M]), err(torch.nn.functional.linear(x, w))
+    print(f"rel. distance to 64 bits {ours:.4e}, library {library:.4e}")
+    # (both are the rounding of the result, 2^-9 or 2^-12 of it at most; fp32 sums of K products are within K * 2^-24 of their size)
+    assert ours <= library + K * 2.0 ** -24 * 1e-2
+    assert not lib.cq_linear_rows_takes(9, K, N) and not lib.cq_linear_rows_takes(M, K + 8, N) and not lib.cq_linear_rows_takes(M, K, N + 4)
+    assert not lib.cq_linear_rows_takes(8, 8192, N) and not lib.cq_linear_rows_takes(M, 1536, N)
+
+
+def test_small_batch_step_takes_its_projections_along():
+    """The steady-state step of a few rows runs both projections in the shim; a hook, autograd or autocast, which want the module called, keep the
+    module call, and the results agree to the rounding of the projections."""
+    from calibquant_amd import patch_internvl as pi
+    from calibquant_amd.internlm2 import InternLM2Attention, InternLM2Config
+    cfg = InternLM2Config.internvl2_5_8b()
+    B, S, T, TXT = 3, 4, 130, 9
+    N, dtype = S + T + TXT, torch.bfloat16
+    att = InternLM2Attention(cfg).cuda().to(dtype)
+    att.cq_sprompt_len, att.cq_image_token_num = S, T
+    x = torch.randn(B, N + 6, cfg.hidden_size, device="cuda", dtype=dtype)
+    pos = torch.arange(N + 6, device="cuda")[None].expand(B, N + 6)
+    seen = []
+
+    def steps(hook):
+        calls = seen.clear()
+        h = att.wqkv.register_forward_hook(lambda *a: seen.append(1)) if hook else None
+        outs = []
+        with torch.no_grad():
+            _, _, past = pi.forward_internlm2_calibquant(att, x[:, :N], None, pos[:, :N], None, False, True)
+            for i in range(N, N + 6):
+                o, _, past = pi.forward_internlm2_calibquant(att, x[:, i:i + 1], None, pos[:, i:i + 1], past, False, True)
+                outs.append(o)
+        if h:
+            h.remove()
+        assert att._cq_step[0].steps == 5
+        return torch.stack(outs).float(), past
+
+    with torch.no_grad():
+        assert pi._plain_products(att.wqkv, att.wo)
+        with torch.autocast("cuda", dtype=dtype):
+            assert not pi._plain_products(att.wqkv, att.wo)
+    assert not pi._plain_products(att.wqkv, att.wo)
+    a, pa = steps(False)
+    b, pb = steps(True)
+    assert len(seen) == 7                                     # prefill and six steps
+    assert (a - b).norm() / b.norm() < 8e-3                   # two roundings to bf16 (2^-9 each) and the attention between them
+    assert (pa[0].float() - pb[0].float()).norm() / pb[0].float().norm() < 4e-3
