@@ -21,6 +21,7 @@ import warnings
 from typing import Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad as _forward_ad
 from torch.nn.modules import module as _module
 
 from . import _lib, ops
@@ -130,17 +131,24 @@ def _image_token_num(self) -> int:
     return int(n)
 
 
+_LINEAR = (torch.nn.Linear.forward, torch.nn.functional.linear)
+
+
 def _plain_products(*modules) -> bool:
     """Whether calling the modules would be nothing but a product with their weights: plain `nn.Linear`s without bias, hooks or a
-    replaced `forward`, outside of autograd, autocast, tracing, compilation, function transforms and tensor modes."""
-    if (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None
+    replaced `forward`, outside of autograd in either direction, autocast, tracing, compilation, function transforms and tensor modes."""
+    if (torch.is_grad_enabled() or _forward_ad._current_level >= 0 or (torch.nn.Linear.forward, torch.nn.functional.linear) != _LINEAR
+            or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None
             or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
             or torch._C._functorch.peek_interpreter_stack() is not None
             or _module._global_forward_hooks or _module._global_forward_pre_hooks):
         return False
     for m in modules:
-        if (type(m) is not torch.nn.Linear or m.bias is not None or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                or m._backward_pre_hooks or "forward" in m.__dict__ or type(m.weight) not in (torch.nn.Parameter, torch.Tensor)):
+        if type(m) is not torch.nn.Linear:
+            return False
+        d = m.__dict__   # (an attribute that is a parameter takes the module's slow look-up)
+        if ("forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]
+                or d["_parameters"].get("bias") is not None or type(d["_parameters"].get("weight")) is not torch.nn.Parameter):
             return False
     return True
 

@@ -289,3 +289,42 @@ def test_quantize_plan_of_shapes():
     p = _lib.QuantizePlan()
     assert lib.cq_quantize_pack_plan(1, 128 * 832, 1, 0, ctypes.byref(p)) == 0
     assert lib.cq_quantize_pack_plan(1, 3329, 1, 1, ctypes.byref(p)) != 0 and lib.cq_quantize_pack_plan(1, 0, 1, 0, ctypes.byref(p)) != 0
+
+
+def test_plain_products_are_plain():
+    """The decode step takes the projections from the modules only where calling them would be a product with their weights and nothing else."""
+    from torch.autograd import forward_ad
+    from calibquant_amd.patch_internvl import _plain_products as plain
+    make = lambda bias=False: torch.nn.Linear(8, 8, bias=bias)
+
+    class Other(torch.nn.Linear):
+        pass
+
+    with torch.no_grad():
+        m = make()
+        assert plain(m, make())
+        assert not plain(m, make(True)) and not plain(Other(8, 8, bias=False))
+        with forward_ad.dual_level():
+            assert not plain(m)
+        for hook in (m.register_forward_hook(lambda *a: None), m.register_forward_pre_hook(lambda *a: None),
+                     torch.nn.modules.module.register_module_forward_hook(lambda *a: None)):
+            assert not plain(m)
+            hook.remove()
+        replaced = make()
+        replaced.forward = lambda x: x
+        assert not plain(replaced)
+        held = make()
+        weight = held.weight
+        del held.weight
+        held.weight = weight.detach()
+        assert not plain(held)
+        old = torch.nn.Linear.forward
+        torch.nn.Linear.forward = lambda self, x: x
+        try:
+            assert not plain(m)
+        finally:
+            torch.nn.Linear.forward = old
+        seen = []
+        torch.func.vmap(lambda x: (seen.append(plain(m)), x)[1])(torch.zeros(2, 8))
+        assert seen == [False] and plain(m)
+    assert not plain(m)
