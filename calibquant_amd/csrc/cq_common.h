@@ -90,6 +90,21 @@ __device__ __forceinline__ void store_elem(void* p, int64_t i, float f) {
     static_cast<uint16_t*>(p)[i] = static_cast<uint16_t>(Cvt<DT>::from_float(f));
 }
 
+// native 16-byte vector: copies are single vector moves (HIP's uint4 struct copies lower to memcpy)
+typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+typedef float F4 __attribute__((ext_vector_type(4)));
+
+// Matrix product 16 x 16 x 32 on raw 16-bit values; a lane's left (right) operand is row (column) lane % 16, k = 8 (lane / 16) + 0 .. 7
+typedef __bf16 B8 __attribute__((ext_vector_type(8)));
+typedef _Float16 H8 __attribute__((ext_vector_type(8)));
+template <typename DT> __device__ __forceinline__ F4 mfma16(U4 a, U4 b, F4 c);
+template <> __device__ __forceinline__ F4 mfma16<BF16>(U4 a, U4 b, F4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(B8, a), __builtin_bit_cast(B8, b), c, 0, 0, 0);
+}
+template <> __device__ __forceinline__ F4 mfma16<FP16>(U4 a, U4 b, F4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(H8, a), __builtin_bit_cast(H8, b), c, 0, 0, 0);
+}
+
 // Two-element dot product with fp32 accumulation on raw 16-bit pairs.
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));

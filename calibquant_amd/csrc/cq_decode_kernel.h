@@ -65,11 +65,8 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 
 template <int N> struct alignas(N * 4) Vec { float v[N]; };
-// native 16-byte vector: copies are single vector moves (HIP's uint4 struct copies lower to memcpy)
-typedef uint32_t U4 __attribute__((ext_vector_type(4)));
 typedef uint32_t U2 __attribute__((ext_vector_type(2)));
 typedef uint32_t Pair16 __attribute__((aligned(2)));   // two 16-bit values wherever they lie: q and the statistics need no alignment
-typedef float F4 __attribute__((ext_vector_type(4)));
 
 // Of a launch's rounds of logits, how many (the last ones) a thread keeps in LDS of its own instead of registers: all of them in registers
 // leave too few for the products' operands and the rows in flight, and a spilled row waits for its load (batch 64 18.4 -> 22.0 us with 16
@@ -216,18 +213,7 @@ __device__ __forceinline__ int virtual_block_id() {
     return l;
 }
 
-// The window's products, 16 x 16 x 32 on raw 16-bit values; a lane's left (right) operand is row (column) lane % 16, k = 8 (lane / 16) + 0 .. 7
-typedef __bf16 B8 __attribute__((ext_vector_type(8)));
-typedef _Float16 H8 __attribute__((ext_vector_type(8)));
 typedef short S4 __attribute__((ext_vector_type(4)));
-template <typename DT> __device__ __forceinline__ F4 mfma16(U4 a, U4 b, F4 c);
-template <> __device__ __forceinline__ F4 mfma16<BF16>(U4 a, U4 b, F4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(B8, a), __builtin_bit_cast(B8, b), c, 0, 0, 0);
-}
-template <> __device__ __forceinline__ F4 mfma16<FP16>(U4 a, U4 b, F4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(H8, a), __builtin_bit_cast(H8, b), c, 0, 0, 0);
-}
-
 // A weight 0 <= p <= 1 in three 16-bit parts, p = part 0 + kPartScale * part 1 + kPartScale^2 * part 2: bf16 holds 8 bits in each, all 24;
 // fp16 11, the lower parts scaled up so that none is lost to its small exponents.
 template <typename DT> constexpr float kPartScale = std::is_same<DT, FP16>::value ? 1.f / 4096.f : 1.f;

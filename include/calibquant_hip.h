@@ -370,8 +370,8 @@ int cq_rope_append(const void* qkv, int dtype, int B, int Hq, int Hkv, int D,
                    int64_t win_stride_r, int capacity, const int64_t* row_dev, cq_stream_t stream);
 
 /* Projection of a few rows: out (M, N) = x (M, K) times w (N, K) transposed, storage dtype, fp32 sums, one rounding; out and w
- * contiguous, rows of x ldx elements apart (a multiple of 8).  For the decode step of a small batch (M <= 8, K a multiple of 512 from 2 048 on, M * K * 2 <= 65 536 bytes, N a multiple of 8:
- * cq_linear_rows_takes() is non-zero; else CQ_ERR_UNSUPPORTED).  x and w on 16 bytes. */
+ * contiguous, rows of x ldx elements apart (a multiple of 8).  For the decode step of a small batch (M <= 8, K a multiple of 512 from 2 048 on,
+ * N a multiple of 8: cq_linear_rows_takes() is non-zero; else CQ_ERR_UNSUPPORTED).  x and w on 16 bytes. */
 int cq_linear_rows_takes(int M, int K, int N);
 int cq_linear_rows(const void* x, int64_t ldx, int dtype, int M, int K, const void* w, int N, void* out, cq_stream_t stream);
 

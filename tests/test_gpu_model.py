@@ -403,10 +403,11 @@ def test_two_prefills_follow_the_environment_variable(monkeypatch):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("shape", [(1, 2048, 8), (2, 2560, 24), (3, 4096, 520), (4, 4096, 6144), (5, 6144, 1032), (8, 4096, 4096)])
+@pytest.mark.parametrize("shape", [(1, 2048, 8), (2, 2560, 24), (3, 4096, 520), (4, 4096, 6144), (5, 6144, 1032), (8, 4096, 4096),
+                                   (1, 4096, 6144), (7, 2048, 6144), (8, 8192, 40), (2, 16896, 16)])
 def test_linear_rows(shape, dtype):
-    """Rows beside the instantiated 1, 2, 4 and 8, slices beside the eight in flight, rows of x apart; against 64 bits, no further off than the
-    library's product beyond one unit of the sums' last places."""
+    """Dot products (one row, two) and one to three tiles a workgroup, pieces and slices beside the eight in flight, rows of x apart; against 64 bits, no further off than
+    the library's product beyond one unit of the sums' last places."""
     import ctypes as C
     from calibquant_amd import _lib
     M, K, N = shape
@@ -429,7 +430,7 @@ def test_linear_rows(shape, dtype):
     # (both are the rounding of the result, 2^-9 or 2^-12 of it at most; fp32 sums of K products are within K * 2^-24 of their size)
     assert ours <= library + K * 2.0 ** -24 * 1e-2
     assert not lib.cq_linear_rows_takes(9, K, N) and not lib.cq_linear_rows_takes(M, K + 8, N) and not lib.cq_linear_rows_takes(M, K, N + 4)
-    assert not lib.cq_linear_rows_takes(8, 8192, N) and not lib.cq_linear_rows_takes(M, 1536, N)
+    assert not lib.cq_linear_rows_takes(M, 1536, N)
 
 
 def test_small_batch_step_takes_its_projections_along():
