@@ -100,3 +100,56 @@ extern "C" int cq_rope_append(const void* qkv, int dtype, int B, int Hq, int Hkv
     CQ_LAUNCH_CHECK();
     return CQ_OK;
 }
+
+namespace cq {
+
+struct WindowGeom {
+    const uint16_t* in[2];        // keys, values (B, N, Hkv, D) through strides
+    int64_t s_b[2], s_t[2], s_h[2];
+    uint16_t* win[2];             // (B, Hkv, capacity, D) through strides
+    int64_t ws_b, ws_h, ws_r;
+    int rows, S, T, Hkv;
+    int64_t total;                // B * rows * Hkv
+};
+
+// The window's first rows, after a prefill: the rows of keys and values around the image block, [0, S) and [S + T, N), one launch for both tensors.
+// grid (16 rows of 256 bytes, tensor), a lane moves 16 bytes; rows go in the order in which they are read (all heads of a token).
+// Bound by its launch: at 4 x 64 rows x 8 heads it takes 3.3 us and replaces two concatenations of 6.4 and two copies of 4 us, which passed over
+// the rows twice.
+__global__ __launch_bounds__(256) void window_rows_kernel(WindowGeom g) {
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * 16 + (threadIdx.x >> 4);
+    if (row >= g.total) return;
+    const uint32_t n = static_cast<uint32_t>(row), br = n / static_cast<uint32_t>(g.Hkv), h = n % static_cast<uint32_t>(g.Hkv);   // (total < 2^31)
+    const uint32_t b = br / static_cast<uint32_t>(g.rows), r = br % static_cast<uint32_t>(g.rows);
+    const int64_t t = static_cast<int64_t>(r) + (static_cast<int>(r) < g.S ? 0 : g.T);
+    const int i = blockIdx.y, d = (threadIdx.x & 15) * 8;
+    const U4* from = reinterpret_cast<const U4*>(g.in[i] + b * g.s_b[i] + t * g.s_t[i] + h * g.s_h[i] + d);
+    *reinterpret_cast<U4*>(g.win[i] + b * g.ws_b + h * g.ws_h + r * g.ws_r + d) = *from;
+}
+
+}  // namespace cq
+
+extern "C" int cq_window_rows(const void* k, int64_t k_stride_b, int64_t k_stride_t, int64_t k_stride_h, const void* v, int64_t v_stride_b,
+                              int64_t v_stride_t, int64_t v_stride_h, int dtype, int B, int N, int Hkv, int D, int S, int T, void* k_win, void* v_win,
+                              int64_t win_stride_b, int64_t win_stride_h, int64_t win_stride_r, cq_stream_t stream) {
+    if (!k || !v || !k_win || !v_win) return CQ_ERR_NULL;
+    if (dtype != CQ_BF16 && dtype != CQ_FP16) return CQ_ERR_DTYPE;
+    if (D != cq::kRD) return CQ_ERR_UNSUPPORTED;
+    if (B < 1 || N < 1 || Hkv < 1 || S < 0 || T < 0 || static_cast<int64_t>(S) + T > N) return CQ_ERR_SHAPE;
+    const int64_t total = static_cast<int64_t>(B) * (N - T);
+    if (total > 0x7fffffff / Hkv) return CQ_ERR_SHAPE;
+    if (((k_stride_b | k_stride_t | k_stride_h | v_stride_b | v_stride_t | v_stride_h | win_stride_b | win_stride_h | win_stride_r) & 7) != 0 ||
+        !cq::aligned16(k) || !cq::aligned16(v) || !cq::aligned16(k_win) || !cq::aligned16(v_win))
+        return CQ_ERR_ALIGN;
+    if (total == 0) return CQ_OK;
+    cq::WindowGeom g;
+    g.in[0] = static_cast<const uint16_t*>(k); g.in[1] = static_cast<const uint16_t*>(v);
+    g.s_b[0] = k_stride_b; g.s_t[0] = k_stride_t; g.s_h[0] = k_stride_h;
+    g.s_b[1] = v_stride_b; g.s_t[1] = v_stride_t; g.s_h[1] = v_stride_h;
+    g.win[0] = static_cast<uint16_t*>(k_win); g.win[1] = static_cast<uint16_t*>(v_win);
+    g.ws_b = win_stride_b; g.ws_h = win_stride_h; g.ws_r = win_stride_r;
+    g.rows = N - T; g.S = S; g.T = T; g.Hkv = Hkv; g.total = total * Hkv;
+    hipLaunchKernelGGL(cq::window_rows_kernel, dim3(static_cast<unsigned>((g.total + 15) / 16), 2), dim3(256), 0, static_cast<hipStream_t>(stream), g);
+    CQ_LAUNCH_CHECK();
+    return CQ_OK;
+}

@@ -437,6 +437,26 @@ def decode_attn(q: torch.Tensor, codes_k: Optional[torch.Tensor], codes_v: Optio
         return call.run()
 
 
+def window_rows(k: torch.Tensor, v: torch.Tensor, sprompt_len: int, image_tokens: int, k_win: torch.Tensor, v_win: torch.Tensor) -> bool:
+    """Rows [0, S) and [S + T, N) of keys and values (B, N, Hkv, D) into the first N - T rows of the window buffers (B, Hkv, capacity, D), one launch
+    (the reference concatenates the two parts, patch_internvl.py:461-476).  False, and nothing done, where the kernel does not take the layout."""
+    _need_gpu(k, "k")
+    dt = _storage_dtype(k, "k")
+    B, N, H, D = k.shape
+    R = N - image_tokens
+    if (v.shape != k.shape or k_win.shape != v_win.shape or k_win.stride() != v_win.stride() or k_win.shape[:2] != (B, H) or k_win.shape[2] < R
+            or k_win.shape[3] != D or any(t.dtype != k.dtype or t.device != k.device or t.stride(3) != 1 for t in (v, k_win, v_win)) or k.stride(3) != 1):
+        raise _lib.CalibQuantError("window_rows: keys, values and the window buffers do not match")
+    if (D != 128 or B * R * H >= 2 ** 31 or any(t.data_ptr() % 16 or any(s % 8 for s in t.stride()[:3]) for t in (k, v, k_win, v_win))):
+        return False
+    with _on(k.device):
+        rc = _lib.load().cq_window_rows(k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), dt,
+                                        B, N, H, D, int(sprompt_len), int(image_tokens), k_win.data_ptr(), v_win.data_ptr(), k_win.stride(0),
+                                        k_win.stride(1), k_win.stride(2), _stream(k))
+    _lib.check(rc, "cq_window_rows")
+    return True
+
+
 class RopeAppendCall:
     """A prepared `cq_rope_append` launch over fixed buffers: the token's fused projection output
     `qkv` (B, 1, (Hq + 2 Hkv) * D) or (B, Hkv, Hq/Hkv + 2, D), rotary tables (rows, D), device

@@ -285,10 +285,18 @@ def forward_internlm2_calibquant(self, hidden_states: torch.Tensor, attention_ma
             self.encoded_features_k = self.encoded_features_v = None
             self._cq_stats = None
         if use_cache:
-            k_st = torch.cat([key_states[:, :, :S], key_states[:, :, S + T:]], dim=2)
-            v_st = torch.cat([value_states[:, :, :S], value_states[:, :, S + T:]], dim=2)
             self._cq_window = GrowingKV()
-            past_key_value = self._cq_window.append(None, k_st, v_st)
+            past_key_value = None
+            if hip_rope and not torch.is_grad_enabled() and _forward_ad._current_level < 0:
+                # straight into the window's buffers, one launch; with a derivative to carry, torch's operations below
+                R = q_len - T
+                k_win, v_win = self._cq_window.reserve(None, R, key_states, (bsz, Hkv), D)
+                if ops.window_rows(k_rot, qkv[..., -1, :], S, T, k_win, v_win):
+                    past_key_value = self._cq_window.extended(R)
+            if past_key_value is None:
+                k_st = torch.cat([key_states[:, :, :S], key_states[:, :, S + T:]], dim=2)
+                v_st = torch.cat([value_states[:, :, :S], value_states[:, :, S + T:]], dim=2)
+                past_key_value = self._cq_window.append(None, k_st, v_st)
         else:
             past_key_value = None
         # full-precision causal attention over the whole prompt, in query chunks

@@ -369,6 +369,13 @@ int cq_rope_append(const void* qkv, int dtype, int B, int Hq, int Hkv, int D,
                    void* k_win, void* v_win, int64_t win_stride_b, int64_t win_stride_h,
                    int64_t win_stride_r, int capacity, const int64_t* row_dev, cq_stream_t stream);
 
+/* The first rows of the full-precision window after a prefill: rows [0, S) and [S + T, N) of keys and values (B, N, Hkv, D), any strides with a
+ * contiguous last axis, into rows [0, N - T) of the buffers (B, Hkv, capacity >= N - T, D).  D = 128; pointers on 16 bytes, strides multiples of 8;
+ * B * (N - T) * Hkv < 2^31. */
+int cq_window_rows(const void* k, int64_t k_stride_b, int64_t k_stride_t, int64_t k_stride_h, const void* v, int64_t v_stride_b,
+                   int64_t v_stride_t, int64_t v_stride_h, int dtype, int B, int N, int Hkv, int D, int S, int T, void* k_win, void* v_win,
+                   int64_t win_stride_b, int64_t win_stride_h, int64_t win_stride_r, cq_stream_t stream);
+
 /* Projection of a few rows: out (M, N) = x (M, K) times w (N, K) transposed, storage dtype, fp32 sums, one rounding; out and w
  * contiguous, rows of x ldx elements apart (a multiple of 8).  For the decode step of a small batch (M <= 8, K a multiple of 512 from 2 048 on,
  * N a multiple of 8: cq_linear_rows_takes() is non-zero; else CQ_ERR_UNSUPPORTED).  x and w on 16 bytes. */

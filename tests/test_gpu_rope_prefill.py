@@ -204,3 +204,27 @@ def test_rope_quantize_pack_parts_across_turns(ops, B, T, Hkv, dtype):
     assert torch.equal(out, two)
     for a, b in zip(got, ops.quantize_pack(two, 1, 0.5)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 2, 1, 0, 1), (3, 37, 2, 5, 20), (2, 33, 8, 0, 7), (2, 30, 3, 9, 21), (5, 19, 4, 0, 0), (2, 8, 2, 0, 8)])
+def test_window_rows(shape, dtype):
+    """Rows around the image block (none before, none after, no block, nothing but the block), keys in padded token rows, values in the projection's
+    block; the same as torch's concatenation, and no row beyond is written.  A layout off 16 bytes is left to the caller."""
+    from calibquant_amd import ops
+    B, N, H, S, T = shape
+    print(f"case window rows {shape} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    k = torch.randn((B, N, H * 128 + 64), generator=g, device="cuda", dtype=dtype)[:, :, :H * 128].unflatten(2, (H, 128))
+    v = torch.randn((B, N, H, 4, 128), generator=g, device="cuda", dtype=dtype)[..., -1, :]
+    R = N - T
+    k_win = torch.full((B, H, R + 3, 128), 7.0, device="cuda", dtype=dtype)
+    v_win = k_win.clone()
+    assert ops.window_rows(k, v, S, T, k_win, v_win)
+    for win, x in ((k_win, k), (v_win, v)):
+        assert torch.equal(win[:, :, :R], torch.cat([x[:, :S], x[:, S + T:]], dim=1).transpose(1, 2))
+        assert (win[:, :, R:] == 7).all()
+    odd = torch.zeros(B * N * H * 128 + 1, device="cuda", dtype=dtype)[1:].view(B, N, H, 128)
+    assert not ops.window_rows(odd, v, S, T, k_win, v_win)
+    with pytest.raises(ops._lib.CalibQuantError):
+        ops.window_rows(k, v, S, T, k_win[:, :, :R - 1] if R else k_win[:, :0], v_win[:, :, :R - 1] if R else v_win[:, :0])
