@@ -171,7 +171,8 @@ def forward_internlm2_calibquant(self, hidden_states: torch.Tensor, attention_ma
     fast = self.__dict__.get("_cq_step")
     if (fast is not None and attention_mask is None and past_key_value is not None and position_ids is not None
             and not kwargs and hidden_states.shape[1] == 1):
-        if hidden_states.shape[0] <= 8 and _plain_products(self.wqkv, self.wo):
+        # (a subclass of torch's tensor may act on the product: it reaches the module)
+        if hidden_states.shape[0] <= 8 and type(hidden_states) is torch.Tensor and _plain_products(self.wqkv, self.wo):
             got = fast[0].step_rows(hidden_states, self.wqkv.weight, self.wo.weight, position_ids, past_key_value[0])
             if got is not None:
                 return got[0], None, ((got[1], got[2]) if use_cache else None)

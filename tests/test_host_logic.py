@@ -328,3 +328,40 @@ def test_plain_products_are_plain():
         torch.func.vmap(lambda x: (seen.append(plain(m)), x)[1])(torch.zeros(2, 8))
         assert seen == [False] and plain(m)
     assert not plain(m)
+
+
+def _stepping(record):
+    """A module as the patched forward meets it in the steady state; what its step object is asked goes to `record`."""
+    class Step:
+        def step_rows(self, hidden, wqkv, wo, pos, past_k):
+            record.append("rows")
+            return hidden, past_k, past_k
+
+        def step(self, qkv, pos, past_k):
+            record.append("step")
+            return qkv, past_k, past_k
+
+    att = torch.nn.Module()
+    att.wqkv, att.wo = torch.nn.Linear(8, 8, bias=False), torch.nn.Linear(8, 8, bias=False)
+    att.__dict__["_cq_step"] = (Step(), None)
+    return att
+
+
+def test_hidden_rows_of_another_type_reach_the_modules():
+    """The decode step goes past the projections for plain tensors only: a subclass that acts on operations is handed to the modules."""
+    from calibquant_amd.patch_internvl import forward_internlm2_calibquant as forward
+    seen = []
+
+    class Watched(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    record, past = [], (torch.zeros(1), torch.zeros(1))
+    att, pos, x = _stepping(record), torch.zeros(1, 1, dtype=torch.long), torch.randn(1, 1, 8)
+    with torch.no_grad():
+        forward(att, x, None, pos, past)
+        assert record == ["rows"]
+        forward(att, x.as_subclass(Watched), None, pos, past)
+    assert record == ["rows", "step"] and torch.nn.functional.linear in seen
