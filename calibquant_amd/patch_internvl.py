@@ -17,12 +17,13 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import types
 import warnings
 from typing import Optional, Tuple
 
 import torch
 from torch.autograd import forward_ad as _forward_ad
-from torch.nn.modules import module as _module
+from torch.nn.modules import linear as _linear, module as _module
 
 from . import _lib, ops
 from ._lib import CalibQuantError
@@ -131,13 +132,25 @@ def _image_token_num(self) -> int:
     return int(n)
 
 
-_LINEAR = (torch.nn.Linear.forward, torch.nn.functional.linear)
+_LINEAR_NAMES, _MODULE_NAMES, _FUNCTION, _BUILTIN = vars(_linear), vars(_module), types.FunctionType, types.BuiltinFunctionType
+
+
+def _calls_are_torchs() -> bool:
+    """Whether calling an `nn.Linear` runs torch's own functions: those have the globals of the torch module that defines them.  A replacement has
+    others, also one that took over the name (functools.wraps) or was there before this file was imported."""
+    nn = torch.nn
+    linear, cls = nn.functional.linear, nn.Linear
+    forward, call, impl = cls.forward, cls.__call__, cls._call_impl
+    return (linear is torch._C._nn.linear and type(linear) is _BUILTIN and type(forward) is type(call) is type(impl) is _FUNCTION
+            and forward.__globals__ is _LINEAR_NAMES and forward.__qualname__ == "Linear.forward"
+            and call.__globals__ is _MODULE_NAMES and call.__qualname__ == "Module._wrapped_call_impl"
+            and impl.__globals__ is _MODULE_NAMES and impl.__qualname__ == "Module._call_impl")
 
 
 def _plain_products(*modules) -> bool:
     """Whether calling the modules would be nothing but a product with their weights: plain `nn.Linear`s without bias, hooks or a
-    replaced `forward`, outside of autograd in either direction, autocast, tracing, compilation, function transforms and tensor modes."""
-    if (torch.is_grad_enabled() or _forward_ad._current_level >= 0 or (torch.nn.Linear.forward, torch.nn.functional.linear) != _LINEAR
+    replaced `forward` or call, outside of autograd in either direction, autocast, tracing, compilation, function transforms and tensor modes."""
+    if (torch.is_grad_enabled() or _forward_ad._current_level >= 0 or not _calls_are_torchs()
             or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None
             or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
             or torch._C._functorch.peek_interpreter_stack() is not None
@@ -147,8 +160,8 @@ def _plain_products(*modules) -> bool:
         if type(m) is not torch.nn.Linear:
             return False
         d = m.__dict__   # (an attribute that is a parameter takes the module's slow look-up)
-        if ("forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]
-                or d["_parameters"].get("bias") is not None or type(d["_parameters"].get("weight")) is not torch.nn.Parameter):
+        if ("forward" in d or "_call_impl" in d or d.get("_compiled_call_impl") is not None or d["_forward_hooks"]
+                or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or d["_parameters"].get("bias") is not None or type(d["_parameters"].get("weight")) is not torch.nn.Parameter):
             return False
     return True
 

@@ -365,3 +365,41 @@ def test_hidden_rows_of_another_type_reach_the_modules():
         assert record == ["rows"]
         forward(att, x.as_subclass(Watched), None, pos, past)
     assert record == ["rows", "step"] and torch.nn.functional.linear in seen
+
+
+def test_replaced_functions_are_seen_whenever_they_were_replaced():
+    """A product, module call or `forward` that was replaced before this package was imported is not taken for torch's own, nor one that is
+    replaced afterwards; nor a module with a call of its own or a compiled one."""
+    import functools
+    import importlib.util
+    from calibquant_amd import patch_internvl
+    nn, F = torch.nn, torch.nn.functional
+
+    def again():   # the module as a program that imports it now gets it
+        spec = importlib.util.spec_from_file_location("calibquant_amd._imported_later", patch_internvl.__file__)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        return mod._plain_products
+
+    def wrapped(f):
+        @functools.wraps(f)
+        def other(*args, **kwargs):
+            return f(*args, **kwargs)
+        return other
+
+    m = nn.Linear(8, 8, bias=False)
+    with torch.no_grad():
+        for owner, name in ((F, "linear"), (nn.Linear, "forward"), (nn.Module, "__call__"), (nn.Module, "_call_impl"), (nn.Linear, "__call__")):
+            own = name in vars(owner)
+            old = getattr(owner, name)
+            setattr(owner, name, wrapped(old))
+            try:
+                assert not again()(m), (owner, name, "before the import")
+                assert not patch_internvl._plain_products(m), (owner, name, "after it")
+            finally:
+                setattr(owner, name, old) if own else delattr(owner, name)
+        for name in ("_call_impl", "_compiled_call_impl"):
+            called = nn.Linear(8, 8, bias=False)
+            setattr(called, name, lambda *a: a)
+            assert not patch_internvl._plain_products(called), name
+        assert again()(m) and patch_internvl._plain_products(m)
