@@ -100,8 +100,10 @@ class LayerStep {
     // one.  The first of the results is wo's output.  (A library product of such rows costs 20 us of host time to launch.)
     py::object step_rows(const at::Tensor& hidden, const at::Tensor& wqkv, const at::Tensor& wo, const at::Tensor& pos, const at::Tensor& past_k) {
         const int64_t B = a_.B, NQ = static_cast<int64_t>(a_.Hq + 2 * a_.Hkv) * a_.D, KO = static_cast<int64_t>(a_.Hq) * a_.D;
+        // (memory that is the tensor's values: not a sparse or other layout, nor one with a sign still to be applied)
         auto ours = [&](const at::Tensor& t) {
-            return t.is_cuda() && t.scalar_type() == dtype_ && t.device() == k_.device() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+            return t.is_cuda() && t.layout() == at::kStrided && !t.is_neg() && t.scalar_type() == dtype_ && t.device() == k_.device() &&
+                   t.has_storage() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
         };
         if (hidden.dim() != 3 || hidden.size(0) != B || hidden.size(1) != 1 || wqkv.dim() != 2 || wo.dim() != 2 || wqkv.size(0) != NQ ||
             wqkv.size(1) != hidden.size(2) || wo.size(1) != KO || hidden.size(2) > INT32_MAX || wo.size(0) > INT32_MAX)

@@ -471,3 +471,73 @@ def test_small_batch_step_takes_its_projections_along():
     assert len(seen) == 7                                     # prefill and six steps
     assert (a - b).norm() / b.norm() < 8e-3                   # two roundings to bf16 (2^-9 each) and the attention between them
     assert (pa[0].float() - pb[0].float()).norm() / pb[0].float().norm() < 4e-3
+
+
+def _stepped_layer(B=3, dtype=torch.bfloat16):
+    """An 8B-shaped attention layer after its prefill and first token: the module with its step object, the next token's hidden row and position, the
+    window."""
+    from calibquant_amd import patch_internvl as pi
+    from calibquant_amd.internlm2 import InternLM2Attention, InternLM2Config
+    cfg = InternLM2Config.internvl2_5_8b()
+    S, T, TXT = 4, 130, 9
+    N = S + T + TXT
+    att = InternLM2Attention(cfg).cuda().to(dtype)
+    att.cq_sprompt_len, att.cq_image_token_num = S, T
+    x = torch.randn(B, N + 2, cfg.hidden_size, device="cuda", dtype=dtype)
+    pos = torch.arange(N + 2, device="cuda")[None].expand(B, N + 2)
+    with torch.no_grad():
+        _, _, past = pi.forward_internlm2_calibquant(att, x[:, :N], None, pos[:, :N], None, False, True)
+        _, _, past = pi.forward_internlm2_calibquant(att, x[:, N:N + 1], None, pos[:, N:N + 1], past, False, True)
+    return att, x[:, N + 1:].contiguous(), pos[:, N + 1:].contiguous(), past
+
+
+def test_step_with_projections_declines_what_it_does_not_read_as_it_is():
+    """Rows and weights whose memory is not what a product would read (a lazy sign, no storage, a layout or type of their own, off 16 bytes), and what is not
+    the next token of the window: None, and nothing has happened."""
+    att, x, pos, past = _stepped_layer()
+    step, wqkv, wo = att._cq_step[0], att.wqkv.weight.detach(), att.wo.weight.detach()
+    K = x.shape[2]
+    off = torch.empty(x.numel() + 1, device="cuda", dtype=x.dtype)[1:].view(x.shape).copy_(x)
+    apart = torch.empty((x.shape[0], 1, K + 4), device="cuda", dtype=x.dtype)[:, :, :K].copy_(x)
+    inner = torch.empty((*x.shape, 2), device="cuda", dtype=x.dtype)[..., 0].copy_(x)
+    turned = lambda w: w.t().contiguous().t()
+    empty = lambda w: torch.sparse_coo_tensor(size=w.shape, dtype=w.dtype, device="cuda")
+    length = step.length
+    cases = {
+        "hidden, lazy sign": (torch._neg_view(x), wqkv, wo, pos, past[0]),
+        "hidden, sparse": (empty(x), wqkv, wo, pos, past[0]),
+        "hidden off 16 bytes": (off, wqkv, wo, pos, past[0]),
+        "hidden rows off 16 bytes": (apart, wqkv, wo, pos, past[0]),
+        "hidden strided": (inner, wqkv, wo, pos, past[0]),
+        "hidden of another type": (x.half(), wqkv, wo, pos, past[0]),
+        "hidden on the host": (x.cpu(), wqkv, wo, pos, past[0]),
+        "wqkv, lazy sign": (x, torch._neg_view(wqkv), wo, pos, past[0]),
+        "wqkv, sparse": (x, empty(wqkv), wo, pos, past[0]),
+        "wqkv turned": (x, turned(wqkv), wo, pos, past[0]),
+        "wo, lazy sign": (x, wqkv, torch._neg_view(wo), pos, past[0]),
+        "wo, sparse": (x, wqkv, empty(wo), pos, past[0]),
+        "wo turned": (x, wqkv, turned(wo), pos, past[0]),
+        "wo of another type": (x, wqkv, wo.half(), pos, past[0]),
+        "positions of another type": (x, wqkv, wo, pos.int(), past[0]),
+        "a position too few": (x, wqkv, wo, pos[1:], past[0]),
+        "a shorter window": (x, wqkv, wo, pos, past[0][:, :, 1:]),
+        "another window": (x, wqkv, wo, pos, past[0].clone()),
+    }
+    for name, args in cases.items():
+        print("case", name, flush=True)
+        assert step.step_rows(*args) is None, name
+        assert step.length == length
+    out, k, v = step.step_rows(x, wqkv, wo, pos, past[0])
+    assert step.length == length + 1 and k.shape[2] == length + 1 and torch.isfinite(out).all()
+
+
+def test_step_of_rows_with_a_lazy_sign():
+    """The step of a hidden row that is held as another tensor and a sign is the step of its values."""
+    from calibquant_amd import patch_internvl as pi
+    att, x, pos, past = _stepped_layer()
+    length = att._cq_step[0].length
+    with torch.no_grad():
+        a, _, pa = pi.forward_internlm2_calibquant(att, torch._neg_view(x.neg()), None, pos, past, False, True)
+        want = torch.nn.functional.linear(x, att.wqkv.weight).view(x.shape[0], 8, 6, 128)[:, :, 5]   # the value row
+    assert att._cq_step[0].length == length + 1
+    assert (pa[1][:, :, -1].float() - want.float()).norm() / want.float().norm() < 4e-3   # (one rounding to bf16 each)
