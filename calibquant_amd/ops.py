@@ -447,7 +447,9 @@ def window_rows(k: torch.Tensor, v: torch.Tensor, sprompt_len: int, image_tokens
     if (v.shape != k.shape or k_win.shape != v_win.shape or k_win.stride() != v_win.stride() or k_win.shape[:2] != (B, H) or k_win.shape[2] < R
             or k_win.shape[3] != D or any(t.dtype != k.dtype or t.device != k.device or t.stride(3) != 1 for t in (v, k_win, v_win)) or k.stride(3) != 1):
         raise _lib.CalibQuantError("window_rows: keys, values and the window buffers do not match")
-    if (D != 128 or B * R * H >= 2 ** 31 or any(t.data_ptr() % 16 or any(s % 8 for s in t.stride()[:3]) for t in (k, v, k_win, v_win))):
+    # (a lazy sign is not in the rows' memory)
+    if (D != 128 or B * R * H >= 2 ** 31 or k.is_neg() or v.is_neg()
+            or any(t.data_ptr() % 16 or any(s % 8 for s in t.stride()[:3]) for t in (k, v, k_win, v_win))):
         return False
     with _on(k.device):
         rc = _lib.load().cq_window_rows(k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), dt,

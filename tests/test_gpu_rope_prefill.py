@@ -210,7 +210,8 @@ def test_rope_quantize_pack_parts_across_turns(ops, B, T, Hkv, dtype):
 @pytest.mark.parametrize("shape", [(1, 2, 1, 0, 1), (3, 37, 2, 5, 20), (2, 33, 8, 0, 7), (2, 30, 3, 9, 21), (5, 19, 4, 0, 0), (2, 8, 2, 0, 8)])
 def test_window_rows(shape, dtype):
     """Rows around the image block (none before, none after, no block, nothing but the block), keys in padded token rows, values in the projection's
-    block; the same as torch's concatenation, and no row beyond is written.  A layout off 16 bytes is left to the caller."""
+    block; the same as torch's concatenation, and no row beyond is written.  A layout off 16 bytes and a sign
+    still to be applied are left to the caller."""
     from calibquant_amd import ops
     B, N, H, S, T = shape
     print(f"case window rows {shape} {dtype}", flush=True)
@@ -226,5 +227,6 @@ def test_window_rows(shape, dtype):
         assert (win[:, :, R:] == 7).all()
     odd = torch.zeros(B * N * H * 128 + 1, device="cuda", dtype=dtype)[1:].view(B, N, H, 128)
     assert not ops.window_rows(odd, v, S, T, k_win, v_win)
+    assert not ops.window_rows(torch._neg_view(k), v, S, T, k_win, v_win) and not ops.window_rows(k, torch._neg_view(v), S, T, k_win, v_win)
     with pytest.raises(ops._lib.CalibQuantError):
         ops.window_rows(k, v, S, T, k_win[:, :, :R - 1] if R else k_win[:, :0], v_win[:, :, :R - 1] if R else v_win[:, :0])
