@@ -214,10 +214,13 @@ __device__ __forceinline__ int virtual_block_id() {
 }
 
 typedef short S4 __attribute__((ext_vector_type(4)));
-// A weight 0 <= p <= 1 in three 16-bit parts, p = part 0 + kPartScale * part 1 + kPartScale^2 * part 2: bf16 holds 8 bits in each, all 24;
-// fp16 11, the lower parts scaled up so that none is lost to its small exponents.
+// A weight 0 <= p <= 1 in three 16-bit parts, p = kPartUnit * (part 0 + kPartScale * part 1 + kPartScale^2 * part 2): bf16 holds 8 bits in each, all
+// 24; fp16 11, the weight and the lower parts scaled up so that none is lost to its small exponents (to 2^-61 of a weight of 1).  Part 0 is 0 only
+// where the weight is, and so infinite times an infinite value (a weight below 2^-39 takes fp16's smallest number, part 1 what that is too much).
 template <typename DT> constexpr float kPartScale = std::is_same<DT, FP16>::value ? 1.f / 4096.f : 1.f;
+template <typename DT> constexpr float kPartUnit = std::is_same<DT, FP16>::value ? 1.f / 16384.f : 1.f;
 template <typename DT> __device__ __forceinline__ void split_weight(float p, uint32_t* o) {
+    if constexpr (std::is_same<DT, FP16>::value) p *= 16384.f;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         if constexpr (std::is_same<DT, BF16>::value) {
@@ -226,6 +229,7 @@ template <typename DT> __device__ __forceinline__ void split_weight(float p, uin
             p -= __uint_as_float(b);
         } else {
             o[i] = Cvt<DT>::from_float(p);
+            if (i == 0) o[0] = max(o[0], min(__float_as_uint(p), 1u));
             p = (p - Cvt<DT>::to_float(o[i])) * 4096.f;
         }
     }
@@ -1352,6 +1356,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
                 o_res = racc[0];
                 // (an infinite sum stays one: 0, a lower part's, times an infinite value would make it a NaN)
                 if (__builtin_fabsf(o_res) != INFINITY) o_res += kPartScale<DT> * (racc[1] + kPartScale<DT> * racc[2]);
+                o_res *= kPartUnit<DT>;
             }
         }
 

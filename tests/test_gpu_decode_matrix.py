@@ -1,5 +1,7 @@
 """The matrix-core form of the decode step at the edges of its tiling: 64-token tiles, 512- and 1 024-token rounds of a
 workgroup, and the fixed-point operands' range."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -284,7 +286,7 @@ def test_window_edges(ops, shape, dtype):
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 def test_window_weights_of_all_sizes(ops, dtype, batch):
     """One row weighs 1, the others 2^-12 to 2^-22 each but have values of 512 times its size, which adds up: the parts a weight is held in
-    keep small ones as exactly as large ones.  An infinite value makes its channel infinite and no other."""
+    keep small ones as exactly as large ones.  An infinite value in the row of weight 1 makes its channel infinite and no other."""
     B, Hq, Hkv, R = batch, 4, 1, 130
     c = _window_case(B, Hq, Hkv, 0, R, dtype, 3)
     c["q"][:] = 0
@@ -300,6 +302,29 @@ def test_window_weights_of_all_sizes(ops, dtype, batch):
     got, want = _run(ops, c, dtype, 0, 1), _oracle(c, 0, 1)
     assert (got[..., 3] == np.inf).all()   # (a weight of 1 on an infinite value, none on any other)
     _close(np.delete(got, 3, -1), np.delete(want, 3, -1), rounding)
+
+
+@pytest.mark.parametrize("form", [(1, 1), (1, 4), (70, 4), (300, 4), (100, 3), (300, 2)])   # (batch, heads): units of 1, 4 (in 1 024 threads, in 512), 3 and 2 heads
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+def test_infinite_value_of_a_row_of_small_weight(ops, dtype, form):
+    """A row whose weight is no zero in 32 bits and whose value is infinite makes the channel infinite, however small the weight, in units of all
+    widths; no other channel notices."""
+    B, Hq = form
+    rounding = 2.0 ** -11 if dtype == "fp16" else 2.0 ** -8
+    for octaves in (13, 24.5, 25.5, 40, 60, 120):
+        print(f"case infinite value {form} {dtype} weight 2^-{octaves}", flush=True)
+        c = _window_case(B, Hq, 1, 0, 130, dtype, 3)
+        c["q"][:], c["kr"][:] = 0, 0
+        c["q"][..., 0] = 8.0
+        c["kr"][:, 0, :, 0] = -140.0                # e^-99 of the largest: adds nothing
+        c["kr"][:, 0, 77, 0] = 0
+        c["kr"][:, 0, 40, 0] = -octaves * math.log(2) * math.sqrt(128) / 8
+        c["kr"] = O.round_to(c["kr"].astype(np.float32), dtype)
+        want = _oracle(c, 0, 1)
+        c["vr"][:, 0, 40, 3], c["vr"][:, 0, 40, 64] = np.inf, -np.inf
+        got = _run(ops, c, dtype, 0, 1)
+        assert (got[..., 3] == np.inf).all() and (got[..., 64] == -np.inf).all()
+        _close(np.delete(got, (3, 64), -1), np.delete(want, (3, 64), -1), rounding)
 
 
 def test_query_and_statistics_on_odd_addresses(ops):
