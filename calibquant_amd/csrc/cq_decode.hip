@@ -179,7 +179,7 @@ static int dispatch(const DecodeGeom& g, const Plan& p, int bits, bool vtok, hip
 #ifdef CQ_PHASE_STOPS
     if (vtok || !std::is_same<DT, BF16>::value || bits != 1 || p.hpb != 4 || p.nh != 4 || p.nt != 512 || g.nsplit > 1)
         return CQ_ERR_UNSUPPORTED;
-    return launch_matrix_one<1, 4, BF16, false, 512, kRegPair, false, false, 4>(gm, units, st);
+    return launch_matrix_one<1, 4, BF16, false, 512, kRegPair, false, kNoExtras, 4>(gm, units, st);
 #else
     return vtok ? launch_matrix_token<DT>(gm, bits, p.hpb, p.nt, units, st)
                 : launch_matrix<DT>(gm, bits, p.hpb, p.nh, p.nt, units, st);

@@ -610,16 +610,21 @@ template <int BITS> __device__ __forceinline__ void matrix_fold_token(const I4* 
     }
 }
 
+enum Extras { kNoExtras, kDeviceRows, kMasked };
+
 // CHUNKED: the launch is one of the two of a chunked step (the min/max launch always is); a single launch carries
-// none of their code.  EXTRAS: an additive mask or a residual row count read from device memory may be present; a
-// call with neither runs an instantiation without their code (the kernel sits at the register limit of its occupancy,
-// and code that never runs still costs registers).
+// none of their code.  EXTRAS: the call has an additive mask (kMasked), or may have a residual row count read from device memory (kDeviceRows;
+// never both); a call with neither runs an instantiation without their code (the kernel sits at the register limit of its occupancy,
+// and code that never runs still costs registers).  The two apart, because a mask's first values are requested ahead: nine loads a lane that
+// a row count, or a chunked launch without a mask, does not need.  Measured, us, one form for both / two: 4 x 733 + 258, per-token values, row count
+// 11.14 / 10.60; 16 x 9 984 + 105, six heads, row count 18.12 / 17.66; fifteen shapes with a row count 4.8 % less.
+// (A chunked launch with a mask gains nothing from the early request and loses nothing: fifty shapes within 0.1 %.)
 // STREAM: the packed rows are read with non-temporal loads (see launch_streams()).
 // NH: query heads a unit serves, at most HPB.  Operands and partials are laid out HPB heads wide either way; with
 // NH = 3 the fourth head's rows are padding - six query heads per kv-head (InternLM2-20B) make two exact units of
 // three instead of two units of four that carry two padding heads between them.
 template <int BITS, int HPB, typename DT, bool MINMAX_ONLY, bool VTOK = false, int NT = 1024, int REGL = 0,
-          bool CHUNKED = MINMAX_ONLY, bool EXTRAS = !MINMAX_ONLY, int NH = HPB, bool STREAM = false>
+          bool CHUNKED = MINMAX_ONLY, Extras EXTRAS = kNoExtras, int NH = HPB, bool STREAM = false>
 // (four waves per SIMD - at most 128 VGPRs - for either workgroup size: two 512-thread workgroups per compute
 // unit are only resident together within that)
 __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
@@ -680,7 +685,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
     const int64_t bh = static_cast<int64_t>(b) * g.Hkv + hkv;
 
     const bool img_unit = split < g.nsplit && g.T > 0;
-    const int R = (EXTRAS && g.r_dev) ? min(*g.r_dev, g.R) : g.R;   // rows in the residual window
+    const int R = (EXTRAS == kDeviceRows && g.r_dev) ? min(*g.r_dev, g.R) : g.R;   // rows in the residual window
     const bool do_res = !MINMAX_ONLY && R > 0 && (!CHUNKED || split == g.nsplit);
     const int t0 = img_unit ? split * g.chunk : 0;
     const int n = img_unit ? min(g.T, t0 + g.chunk) - t0 : 0;
@@ -826,8 +831,8 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         for (int r = 0; r < kVEarly; ++r) request_v(r, r);
     }
     // The mask's values of the first rounds and of the window's first tile, ahead of the phases that add them.  (No mask: q, always mapped.)
-    constexpr int kMaskAhead = EXTRAS ? (REGL < 2 ? REGL : 2) : 0;
-    const bool masked = EXTRAS && g.mask;
+    constexpr int kMaskAhead = EXTRAS == kMasked ? (REGL < 2 ? REGL : 2) : 0;
+    const bool masked = EXTRAS == kMasked && g.mask;
     const float* mask_img = masked && n > 0 ? g.mask + b * g.mask_sb + g.S + t0 : reinterpret_cast<const float*>(g.q);
     const float* mask_win = masked ? g.mask + b * g.mask_sb : reinterpret_cast<const float*>(g.q);
     float mask_v[kMaskAhead ? kMaskAhead : 1][4], mask_w = 0.f;

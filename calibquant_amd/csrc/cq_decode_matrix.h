@@ -6,7 +6,7 @@
 
 namespace cq {
 
-template <int BITS, int HPB, typename DT, bool VTOK, int NT, int REGL, bool CHUNKED, bool EXTRAS, int NH>
+template <int BITS, int HPB, typename DT, bool VTOK, int NT, int REGL, bool CHUNKED, Extras EXTRAS, int NH>
 static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st) {
     constexpr int lds = Lay<BITS, HPB, VTOK, NT>::kLds;
     static_assert(lds <= 64 * 1024, "no raised dynamic-LDS limit needed");
@@ -17,7 +17,7 @@ static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st
         if (!g.fused) {
             const DecodeGeom g1 = minmax_geometry(g);   // (this launch never looks at values)
             constexpr int lds1 = Lay<BITS, HPB, false, NT>::kLds;
-            hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, true, false, NT, REGL, true, false, NH>),
+            hipLaunchKernelGGL((decode_kernel<BITS, HPB, DT, true, false, NT, REGL, true, kNoExtras, NH>),
                                dim3(units * g.nsplit), dim3(NT), lds1, st, g1);
             CQ_LAUNCH_CHECK();
         }
@@ -36,15 +36,18 @@ static int launch_matrix_one(const DecodeGeom& g, unsigned units, hipStream_t st
     return CQ_OK;
 }
 
-// A chunked launch has one instantiation, with the mask and the row count.  All kernels keep within the 128 registers, except those of
-// sixteen rounds with mask and row count (4 to 16 spilled).
+// A chunked launch has two instantiations: with the mask, and with the row count (which may be absent).  All kernels keep within the 128
+// registers, except chunked ones of sixteen rounds with a mask (4 to 32 spilled: two heads, or one at 2 bits) and the fp16 form of per-token values with
+// two heads and eight rounds, chunked without a mask (4).
 // SINGLE: no plan chunks such units.
 template <int BITS, int HPB, typename DT, int NT, int REGL, int NH = HPB, bool VTOK = false, bool SINGLE = false>
 static int launch_matrix_unit(const DecodeGeom& g, unsigned units, hipStream_t st) {
     if constexpr (SINGLE) { if (g.nsplit > 1) return CQ_ERR_UNSUPPORTED; }
-    else if (g.nsplit > 1) return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, true, true, NH>(g, units, st);
-    if (g.mask || g.r_dev) return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, false, true, NH>(g, units, st);
-    return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, false, false, NH>(g, units, st);
+    else if (g.nsplit > 1) return g.mask ? launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, true, kMasked, NH>(g, units, st)
+                                         : launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, true, kDeviceRows, NH>(g, units, st);
+    if (g.mask) return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, false, kMasked, NH>(g, units, st);
+    if (g.r_dev) return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, false, kDeviceRows, NH>(g, units, st);
+    return launch_matrix_one<BITS, HPB, DT, VTOK, NT, REGL, false, kNoExtras, NH>(g, units, st);
 }
 
 template <int BITS, typename DT>

@@ -9,7 +9,7 @@ import torch
 from oracle import cq_oracle as O
 from tests.test_gpu_decode import _oracle, _run
 from tests.test_gpu_token_mode import _token_case
-from tests.util import make_case
+from tests.util import make_case, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -340,3 +340,28 @@ def test_query_and_statistics_on_odd_addresses(ops):
     want = ops.decode_attn(q, ck, cv, sk, zk, sv, zv, None, None, sprompt_len=0, bits=1)
     got = ops.decode_attn(odd(q), ck, cv, odd(sk), odd(zk), odd(sv), odd(zv), None, None, sprompt_len=0, bits=1)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("splits", [0, 2])
+@pytest.mark.parametrize("shape", [(1, 4, 4), (2, 8, 4), (3, 24, 8), (17, 32, 4), (40, 32, 8)])   # units of 1, 2, 3 and 4 heads, the last in 512 threads
+@pytest.mark.parametrize("bits, vals", [(1, "channel"), (2, "channel"), (1, "token"), (2, "token")])
+def test_mask_and_row_count_are_forms_of_one_call(ops, shape, bits, vals, splits):
+    """The call without either, with the window's length on the device and with a mask, whole and in chunks: the row count changes no bit, a mask of
+    zeros only the order in which a logit is put together, and a masked row of the window is as if it were not there."""
+    B, Hq, Hkv = shape
+    T, R, S = 700, 140, 5
+    print(f"case forms {shape} bits={bits} {vals} splits={splits}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(B * bits)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda", dtype=torch.float16)
+    ck, sk, zk = ops.quantize_pack(r(B, T, Hkv, 128), bits, 0.5)
+    cv, sv, zv = ops.quantize_pack_token(r(B, T, Hkv, 128), bits) if vals == "token" else ops.quantize_pack(r(B, T, Hkv, 128), bits, 0.5)
+    q, kr, vr = r(B, Hq, 128), r(B, Hkv, R, 128), r(B, Hkv, R, 128)
+    run = lambda rows, **kw: ops.decode_attn(q, ck, cv, sk, zk, sv, zv, kr[:, :, :rows], vr[:, :, :rows], sprompt_len=S, bits=bits, v_mode=vals,
+                                             force_splits=splits, **kw)
+    plain, shorter = run(R), run(R - 3)
+    assert torch.equal(run(R, r_dev=torch.full((1,), R, dtype=torch.int32, device="cuda")), plain)
+    assert torch.equal(run(R, r_dev=torch.full((1,), R - 3, dtype=torch.int32, device="cuda")), shorter)
+    mask = torch.zeros((B, T + R), device="cuda")
+    _close(to_np(run(R, mask=mask)), to_np(plain), 2.0 ** -10)   # (both results are rounded to fp16: up to half a step, 2^-11 of them, each)
+    mask[:, T + R - 3:] = -1e4
+    _close(to_np(run(R, mask=mask)), to_np(shorter), 2.0 ** -10)
