@@ -20,7 +20,7 @@ SYMBOLS = (
     "cq_lut_vecmat_qk", "cq_lut_vecmat_pv",
     "cq_decode_attn_workspace", "cq_decode_attn", "cq_decode_attn_static", "cq_decode_attn_static_limit",
     "cq_decode_attn_plan", "cq_decode_attn_wait_polls", "cq_decode_attn_gave_up", "cq_quantize_pack_wait_polls", "cq_quantize_pack_plan", "cq_decode_attn_single_launch", "cq_rope_append", "cq_quantize_pack_token",
-    "cq_linear_rows", "cq_linear_rows_takes", "cq_window_rows",
+    "cq_linear_rows", "cq_linear_rows_takes", "cq_linear_rows_pays", "cq_window_rows",
 )
 
 
@@ -128,6 +128,8 @@ def load() -> C.CDLL:
     lib.cq_rope_append.argtypes = [vp, i, i, i, i, i, vp, vp, i64, vp, i64, vp, vp, vp, i64, i64, i64, i, vp, vp]
     lib.cq_linear_rows_takes.restype = i
     lib.cq_linear_rows_takes.argtypes = [i, i, i]
+    lib.cq_linear_rows_pays.restype = i
+    lib.cq_linear_rows_pays.argtypes = [i, i, i]
     lib.cq_linear_rows.restype = i
     lib.cq_linear_rows.argtypes = [vp, i64, i, i, i, vp, i, vp, vp]
     lib.cq_window_rows.restype = i

@@ -172,6 +172,19 @@ int cq_linear_rows_takes(int M, int K, int N) {
     return M >= 1 && M <= cq::kMostRows && K >= 2048 && K % 512 == 0 && N >= 8 && N % 8 == 0;
 }
 
+// Where the product is no slower on the device than the library's, weights from memory (a model's weights do not fit the cache, and from some hundred
+// megabytes of them on the device bounds the step, not the host).  us, this / the library's:
+//   one row 16 384 x 4 096 29.8 / 30.1, two 6 144 x 8 192 20.5 / 23.8, x 6 144 16.8 / 18.1 (7 168 x 7 168 22.2 / 21.4)
+//   three to eight: 4 096 channels are eight pieces a wave, all in flight at once; more come in turns of eight, whose last one is padded with repeats
+//   (eight rows 5 120 x 5 120 24.0 / 14.4, 6 144 x 8 192 26.1 / 23.9, x 6 144 20.2 / 18.1; the 26B-shaped model's step 1.8 % slower); fewer
+//   leave several turns of workgroups too short each (2 048 x 12 288 19.5 / 15.9, 2 560 x 16 384 26.2 / 19.7; x 4 096 7.9 / 10.5, 8.2 / 11.2;
+//   4 096 x 16 384 26.4 / 32.6, at the least 4 096 x 14 336 29.3 / 29.0).
+int cq_linear_rows_pays(int M, int K, int N) {
+    if (!cq_linear_rows_takes(M, K, N)) return 0;
+    if (M <= 2) return K <= (M == 1 ? 16384 : 6144);
+    return K == 4096 || (K < 4096 && N <= 4096);
+}
+
 int cq_linear_rows(const void* x, int64_t ldx, int dtype, int M, int K, const void* w, int N, void* out, cq_stream_t stream) {
     if (!x || !w || !out) return CQ_ERR_NULL;
     if (dtype != CQ_BF16 && dtype != CQ_FP16) return CQ_ERR_DTYPE;

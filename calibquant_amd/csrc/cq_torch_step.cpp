@@ -96,7 +96,7 @@ class LayerStep {
     }
 
     // The same with both projections: hidden (B, 1, K), the weights of wqkv ((Hq + 2 Hkv) D, K) and wo (N, Hq D), no bias.  The projections
-    // of a few rows run in the library (cq_linear_rows); None where those do not take the sizes or the step is not the steady-state
+    // of a few rows run in the library (cq_linear_rows); None where those do not pay at these sizes or the step is not the steady-state
     // one.  The first of the results is wo's output.  (A library product of such rows costs 20 us of host time to launch.)
     py::object step_rows(const at::Tensor& hidden, const at::Tensor& wqkv, const at::Tensor& wo, const at::Tensor& pos, const at::Tensor& past_k) {
         const int64_t B = a_.B, NQ = static_cast<int64_t>(a_.Hq + 2 * a_.Hkv) * a_.D, KO = static_cast<int64_t>(a_.Hq) * a_.D;
@@ -109,7 +109,7 @@ class LayerStep {
             wqkv.size(1) != hidden.size(2) || wo.size(1) != KO || hidden.size(2) > INT32_MAX || wo.size(0) > INT32_MAX)
             return py::none();
         const int K = static_cast<int>(hidden.size(2)), N = static_cast<int>(wo.size(0));
-        if (!cq_linear_rows_takes(a_.B, K, static_cast<int>(NQ)) || !cq_linear_rows_takes(a_.B, static_cast<int>(KO), N) || !ours(hidden) ||
+        if (!cq_linear_rows_pays(a_.B, K, static_cast<int>(NQ)) || !cq_linear_rows_pays(a_.B, static_cast<int>(KO), N) || !ours(hidden) ||
             hidden.stride(2) != 1 || hidden.stride(0) % 8 != 0 || !ours(wqkv) || !wqkv.is_contiguous() || !ours(wo) || !wo.is_contiguous() ||
             !next_token(pos, past_k))
             return py::none();

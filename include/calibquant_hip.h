@@ -378,8 +378,10 @@ int cq_window_rows(const void* k, int64_t k_stride_b, int64_t k_stride_t, int64_
 
 /* Projection of a few rows: out (M, N) = x (M, K) times w (N, K) transposed, storage dtype, fp32 sums, one rounding; out and w
  * contiguous, rows of x ldx elements apart (a multiple of 8).  For the decode step of a small batch (M <= 8, K a multiple of 512 from 2 048 on,
- * N a multiple of 8: cq_linear_rows_takes() is non-zero; else CQ_ERR_UNSUPPORTED).  x and w on 16 bytes. */
+ * N a multiple of 8: cq_linear_rows_takes() is non-zero; else CQ_ERR_UNSUPPORTED).  x and w on 16 bytes.  cq_linear_rows_pays(): non-zero
+ * for the sizes at which the launch is no slower than a library product whose weights come from memory, the ones the decode step takes here. */
 int cq_linear_rows_takes(int M, int K, int N);
+int cq_linear_rows_pays(int M, int K, int N);
 int cq_linear_rows(const void* x, int64_t ldx, int dtype, int M, int K, const void* w, int N, void* out, cq_stream_t stream);
 
 #ifdef __cplusplus

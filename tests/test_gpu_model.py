@@ -473,12 +473,12 @@ def test_small_batch_step_takes_its_projections_along():
     assert (pa[0].float() - pb[0].float()).norm() / pb[0].float().norm() < 4e-3
 
 
-def _stepped_layer(B=3, dtype=torch.bfloat16):
-    """An 8B-shaped attention layer after its prefill and first token: the module with its step object, the next token's hidden row and position, the
+def _stepped_layer(B=3, dtype=torch.bfloat16, cfg=None):
+    """An attention layer (8B-shaped) after its prefill and first token: the module with its step object, the next token's hidden row and position, the
     window."""
     from calibquant_amd import patch_internvl as pi
     from calibquant_amd.internlm2 import InternLM2Attention, InternLM2Config
-    cfg = InternLM2Config.internvl2_5_8b()
+    cfg = cfg or InternLM2Config.internvl2_5_8b()
     S, T, TXT = 4, 130, 9
     N = S + T + TXT
     att = InternLM2Attention(cfg).cuda().to(dtype)
@@ -541,3 +541,12 @@ def test_step_of_rows_with_a_lazy_sign():
         want = torch.nn.functional.linear(x, att.wqkv.weight).view(x.shape[0], 8, 6, 128)[:, :, 5]   # the value row
     assert att._cq_step[0].length == length + 1
     assert (pa[1][:, :, -1].float() - want.float()).norm() / want.float().norm() < 4e-3   # (one rounding to bf16 each)
+
+
+@pytest.mark.parametrize("B", [2, 3, 8])
+def test_step_takes_its_projections_along_only_where_that_pays(B):
+    """The 26B-shaped layer's projections: of two rows they go along, from three on the modules' products are no slower and stay."""
+    from calibquant_amd.internlm2 import InternLM2Config
+    att, x, pos, past = _stepped_layer(B, cfg=InternLM2Config.internvl2_5_26b())
+    got = att._cq_step[0].step_rows(x, att.wqkv.weight.detach(), att.wo.weight.detach(), pos, past[0])
+    assert (got is not None) == (B == 2)

@@ -403,3 +403,16 @@ def test_replaced_functions_are_seen_whenever_they_were_replaced():
             setattr(called, name, lambda *a: a)
             assert not patch_internvl._plain_products(called), name
         assert again()(m) and patch_internvl._plain_products(m)
+
+
+def test_projections_of_a_step_only_where_they_are_no_slower():
+    """Which products of a few rows the decode step launches itself: never one whose launch takes longer than the library's product does."""
+    from calibquant_amd import _lib
+    lib = _lib.load()
+    slower = [(8, 6144, 8192), (8, 6144, 6144), (3, 6144, 6144), (3, 5120, 5120), (8, 4608, 6144), (2, 7168, 7168), (8, 2048, 12288), (8, 3584, 16384)]
+    faster = [(1, 4096, 6144), (8, 4096, 6144), (8, 4096, 4096), (3, 4096, 16384), (1, 6144, 8192), (2, 6144, 6144), (8, 2048, 4096), (1, 2048, 512)]
+    for shape in slower + faster:
+        assert lib.cq_linear_rows_takes(*shape)
+        assert bool(lib.cq_linear_rows_pays(*shape)) == (shape in faster), shape
+    for shape in [(9, 4096, 4096), (0, 4096, 4096), (1, 4096, 4100), (1, 1536, 4096), (1, 4100, 4096)]:
+        assert not lib.cq_linear_rows_takes(*shape) and not lib.cq_linear_rows_pays(*shape)
