@@ -27,7 +27,7 @@ import torch.nn.functional as F
 
 from . import _lib, ops
 from ._lib import CalibQuantError
-from .patch_internvl import CALIB_OFFSET_MAX, CALIB_OFFSET_MIN
+from .patch_internvl import CALIB_OFFSET_MAX, CALIB_OFFSET_MIN, few_rows
 
 
 class _LayerState:
@@ -108,7 +108,11 @@ class StaticDecoder:
             att = layer.attention
             B = self.B
             h = F.rms_norm(x, (x.shape[-1],), layer.attention_norm.weight, layer.attention_norm.eps)
-            torch.matmul(h.view(B, -1), att.wqkv.weight.t(), out=st.qkv)
+            few = self.quantized and few_rows(att, h)   # as the patched forward's own step
+            if few:
+                ops.linear_rows(h, att.wqkv.weight, out=st.qkv)
+            else:
+                torch.matmul(h.view(B, -1), att.wqkv.weight.t(), out=st.qkv)
             st.rope.run()            # st.q <- rotated query heads; window row r_idx <- rotated key, value
             if st.call is not None:
                 st.call.run()
@@ -117,7 +121,8 @@ class StaticDecoder:
                 keep = (self.col < self.r_len.to(torch.long))[None, None, None, :]
                 o = F.scaled_dot_product_attention(st.q[:, :, None, :], st.kbuf, st.vbuf, attn_mask=keep,
                                                    enable_gqa=True)
-            x = x + att.wo(o.reshape(B, 1, att.hidden_size))
+            o = o.reshape(B, 1, att.hidden_size)
+            x = x + (ops.linear_rows(o, att.wo.weight) if few else att.wo(o))
             h = F.rms_norm(x, (x.shape[-1],), layer.ffn_norm.weight, layer.ffn_norm.eps)
             x = x + layer.feed_forward(h)
         x = F.rms_norm(x, (x.shape[-1],), lm.model.norm.weight, lm.model.norm.eps)

@@ -459,6 +459,34 @@ def window_rows(k: torch.Tensor, v: torch.Tensor, sprompt_len: int, image_tokens
     return True
 
 
+def linear_rows_pays(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+    """Whether a decode step's products run as `linear_rows`: hidden rows x (B, 1, K) with the first weight and rows of their own with the others, at sizes where
+    the launch is no slower than the library's product (cq_linear_rows_pays) and from memory that holds the values as they are."""
+    if x.dim() != 3 or x.shape[1] != 1 or x.dtype not in (torch.bfloat16, torch.float16) or not weights or weights[0].shape[-1] != x.shape[2]:
+        return False
+    for t in (x, *weights):
+        if (not t.is_cuda or t.layout is not torch.strided or t.is_neg() or t.dtype != x.dtype or t.device != x.device or t.data_ptr() % 16):
+            return False
+    if x.stride(2) != 1 or x.stride(0) % 8:
+        return False
+    pays = _lib.load().cq_linear_rows_pays
+    return all(w.dim() == 2 and w.is_contiguous() and max(w.shape) < 2 ** 31 and pays(x.shape[0], w.shape[1], w.shape[0]) for w in weights)
+
+
+def linear_rows(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x (B, 1, K) times w (N, K) transposed -> (B, 1, N), 32-bit sums, one rounding; for what `linear_rows_pays` names.  `out`: B * N contiguous elements."""
+    if out is None:
+        out = torch.empty((x.shape[0], 1, w.shape[0]), dtype=x.dtype, device=x.device)
+    elif out.dtype != x.dtype or out.device != x.device or not out.is_contiguous() or out.numel() != x.shape[0] * w.shape[0]:
+        raise _lib.CalibQuantError("linear_rows: out must be B * N contiguous elements like x")
+    if not linear_rows_pays(x, w):
+        raise _lib.CalibQuantError("linear_rows: rows or weight not taken (linear_rows_pays)")
+    with _on(x.device):
+        rc = _lib.load().cq_linear_rows(x.data_ptr(), x.stride(0), _DT[x.dtype], x.shape[0], x.shape[2], w.data_ptr(), w.shape[0], out.data_ptr(), _stream(x))
+    _lib.check(rc, "cq_linear_rows")
+    return out
+
+
 class RopeAppendCall:
     """A prepared `cq_rope_append` launch over fixed buffers: the token's fused projection output
     `qkv` (B, 1, (Hq + 2 Hkv) * D) or (B, Hkv, Hq/Hkv + 2, D), rotary tables (rows, D), device

@@ -166,6 +166,14 @@ def _plain_products(*modules) -> bool:
     return True
 
 
+def few_rows(att, hidden_states: torch.Tensor) -> bool:
+    """Whether the decode step of these hidden rows (B, 1, hidden) takes both projections of the attention module along (`ops.linear_rows`).  Every route of a
+    step asks the same - the host shim, the Python calls, torch's operations, the recorded step -, so that all of them give the same bits."""
+    # (a subclass of torch's tensor may act on the product: it reaches the module)
+    return (hidden_states.shape[0] <= 8 and type(hidden_states) is torch.Tensor and _plain_products(att.wqkv, att.wo)
+            and ops.linear_rows_pays(hidden_states, att.wqkv.weight, att.wo.weight))
+
+
 def forward_internlm2_calibquant(self, hidden_states: torch.Tensor, attention_mask: Optional[torch.Tensor] = None,
                                  position_ids: Optional[torch.LongTensor] = None,
                                  past_key_value: Optional[Tuple[torch.Tensor]] = None,
@@ -216,11 +224,13 @@ def forward_internlm2_calibquant(self, hidden_states: torch.Tensor, attention_ma
     S, T = self.sprompt_len, self.image_token_num
 
     # (h gs d) de-interleave of the fused projection: views only (patch_internvl.py:214-234)
-    qkv = self.wqkv(hidden_states).view(bsz, q_len, Hkv, 2 + G, D)
+    few = q_len == 1 and past_key_value is not None and few_rows(self, hidden_states)
+    product = (lambda m, x: ops.linear_rows(x, m.weight)) if few else (lambda m, x: m(x))
+    qkv = product(self.wqkv, hidden_states).view(bsz, q_len, Hkv, 2 + G, D)
     if (q_len == 1 and past_key_value is not None and position_ids is not None and position_ids.is_cuda
             and position_ids.dtype == torch.int64 and position_ids.numel() == bsz and qkv.is_contiguous()
             and qkv.dtype in (torch.bfloat16, torch.float16)):
-        return _decode_step_fused(self, qkv, position_ids, past_key_value, attention_mask, use_cache)
+        return _decode_step_fused(self, qkv, position_ids, past_key_value, attention_mask, use_cache, product)
     value_states = qkv[..., -1, :].transpose(1, 2)                                 # (B, Hkv, q, D)
     kv_seq_len = q_len
     if past_key_value is not None:
@@ -344,7 +354,7 @@ def forward_internlm2_calibquant(self, hidden_states: torch.Tensor, attention_ma
                              f"but is {attention_mask.size()}")
         mask = attention_mask[:, 0, 0, :]
     out = _attend(self, query_states[:, :, 0, :], k_res, v_res, mask)
-    attn_output = self.wo(out.reshape(bsz, 1, self.hidden_size))
+    attn_output = product(self.wo, out.reshape(bsz, 1, self.hidden_size))
     return attn_output, None, past_key_value
 
 
@@ -372,8 +382,8 @@ def _attend(self, q1, k_res, v_res, mask):
     return out
 
 
-def _decode_step_fused(self, qkv, position_ids, past_key_value, attention_mask, use_cache):
-    """One decode step with the split of the fused projection, the rotary embedding of q and k and
+def _decode_step_fused(self, qkv, position_ids, past_key_value, attention_mask, use_cache, product):
+    """One decode step (`product`: how the step takes a projection) with the split of the fused projection, the rotary embedding of q and k and
     the append of the new key / value row in one launch (`cq_rope_append`, bit-identical to the
     torch ops that run at patch_internvl.py:125-134, 219-266), then the fused attention launch."""
     bsz = qkv.shape[0]
@@ -422,7 +432,7 @@ def _decode_step_fused(self, qkv, position_ids, past_key_value, attention_mask, 
         shim = _lib.load_step_shim()
         self.__dict__["_cq_step"] = (shim.LayerStep(C.addressof(call.args), C.sizeof(call.args), tabs[0], tabs[1],
                                                     win.k, win.v, win.len, rows), call)
-    return self.wo(out.reshape(bsz, 1, self.hidden_size)), None, past_key_value
+    return product(self.wo, out.reshape(bsz, 1, self.hidden_size)), None, past_key_value
 
 
 def _no_qjl(*args, **kwargs):

@@ -494,6 +494,7 @@ def _stepped_layer(B=3, dtype=torch.bfloat16, cfg=None):
 def test_step_with_projections_declines_what_it_does_not_read_as_it_is():
     """Rows and weights whose memory is not what a product would read (a lazy sign, no storage, a layout or type of their own, off 16 bytes), and what is not
     the next token of the window: None, and nothing has happened."""
+    from calibquant_amd import ops
     att, x, pos, past = _stepped_layer()
     step, wqkv, wo = att._cq_step[0], att.wqkv.weight.detach(), att.wo.weight.detach()
     K = x.shape[2]
@@ -527,6 +528,9 @@ def test_step_with_projections_declines_what_it_does_not_read_as_it_is():
         print("case", name, flush=True)
         assert step.step_rows(*args) is None, name
         assert step.length == length
+        if name.startswith(("hidden", "wqkv", "wo")):   # (the other routes of a step ask this)
+            assert not ops.linear_rows_pays(*args[:3]), name
+    assert ops.linear_rows_pays(x, wqkv, wo)
     out, k, v = step.step_rows(x, wqkv, wo, pos, past[0])
     assert step.length == length + 1 and k.shape[2] == length + 1 and torch.isfinite(out).all()
 
@@ -550,3 +554,76 @@ def test_step_takes_its_projections_along_only_where_that_pays(B):
     att, x, pos, past = _stepped_layer(B, cfg=InternLM2Config.internvl2_5_26b())
     got = att._cq_step[0].step_rows(x, att.wqkv.weight.detach(), att.wo.weight.detach(), pos, past[0])
     assert (got is not None) == (B == 2)
+
+
+@pytest.mark.parametrize("B", [1, 3, 8])
+def test_routes_of_a_step_of_few_rows_give_the_same_bits(B):
+    """Steps of an 8B-shaped layer that take the projections along: through the host shim, through the Python call objects and through torch's
+    operations around the kernels (int32 positions)."""
+    from calibquant_amd import patch_internvl as pi
+    from calibquant_amd.internlm2 import InternLM2Attention, InternLM2Config
+    cfg, dtype = InternLM2Config.internvl2_5_8b(), torch.bfloat16
+    S, T, TXT = 4, 130, 9
+    N = S + T + TXT
+    outs, wins = [], []
+    for route in ("shim", "calls", "operations"):
+        print("case route", route, B, flush=True)
+        torch.manual_seed(17)
+        att = InternLM2Attention(cfg).cuda().to(dtype)
+        att.cq_sprompt_len, att.cq_image_token_num, att.cq_no_step_shim = S, T, route != "shim"
+        x = torch.randn(B, N + 5, cfg.hidden_size, device="cuda", dtype=dtype)
+        pos = torch.arange(N + 5, device="cuda")[None].repeat(B, 1)
+        with torch.no_grad():
+            _, _, past = pi.forward_internlm2_calibquant(att, x[:, :N], None, pos[:, :N], None, False, True)
+            steps = []
+            for i in range(N, N + 5):
+                p = pos[:, i:i + 1].int() if route == "operations" else pos[:, i:i + 1]
+                o, _, past = pi.forward_internlm2_calibquant(att, x[:, i:i + 1], None, p, past, False, True)
+                steps.append(o)
+        assert ("_cq_step" in att.__dict__) == (route == "shim")
+        outs.append(torch.stack(steps))
+        wins.append(torch.stack(past))
+    for other in (1, 2):
+        assert torch.equal(outs[0], outs[other]) and torch.equal(wins[0], wins[other])
+
+
+@pytest.mark.parametrize("width, B", [("8b", 1), ("8b", 4), ("8b", 8), ("8b", 9), ("26b", 2), ("26b", 4)])
+def test_recorded_step_of_few_rows_gives_the_eager_steps_bits(width, B):
+    """Two layers of the model's width: the recorded step, replayed, leaves the tokens and the window rows of the model's own eager steps, bit for bit."""
+    import contextlib
+    import io
+    from calibquant_amd import patch_internvl as pi
+    from calibquant_amd.graph_decode import StaticDecoder
+    from calibquant_amd.internlm2 import InternLM2Attention, InternLM2Config, InternVLChatStandIn
+    fp_forward, fp_generate = InternLM2Attention.forward, InternVLChatStandIn.generate
+    hidden, heads = (4096, 32) if width == "8b" else (6144, 48)
+    cfg = InternLM2Config(vocab_size=512, hidden_size=hidden, intermediate_size=1024, num_hidden_layers=2, num_attention_heads=heads,
+                          num_key_value_heads=8, max_position_embeddings=2048)
+    torch.manual_seed(5)
+    m = InternVLChatStandIn(cfg).cuda().to(torch.bfloat16).eval()
+    lm = m.language_model
+    S, T, TXT, NEW = 41, 256, 9, 7
+    N = S + T + TXT
+    try:
+        with contextlib.redirect_stdout(io.StringIO()):
+            pi.patch_model(m, "calibquant")
+        for layer in lm.model.layers:
+            layer.attention.cq_image_token_num = T
+        emb = torch.randn(B, N, hidden, device="cuda", dtype=torch.bfloat16)
+        pos = torch.arange(N, device="cuda")[None].expand(B, N)
+        with torch.no_grad():
+            logits, past = lm.forward_step(emb, pos, None)
+            toks = [logits[:, -1].argmax(-1)]
+            for i in range(NEW - 1):
+                logits, past = lm.forward_step(lm.get_input_embeddings()(toks[-1])[:, None], torch.full((B, 1), N + i, device="cuda"), past)
+                toks.append(logits[:, -1].argmax(-1))
+            want = [torch.stack(p) for p in past]
+            _, past = lm.forward_step(emb, pos, None)
+            dec = StaticDecoder(lm, past, N, NEW)
+            got = dec.generate(toks[0], NEW)
+        assert dec.graph is not None and torch.equal(got, torch.stack(toks, 1))
+        for st, w in zip(dec.state, want):
+            R = w.shape[3]
+            assert torch.equal(st.kbuf[:, :, :R], w[0]) and torch.equal(st.vbuf[:, :, :R], w[1])
+    finally:
+        InternLM2Attention.forward, InternVLChatStandIn.generate = fp_forward, fp_generate
