@@ -156,7 +156,9 @@ def load_step_shim():
         spec = importlib.util.spec_from_file_location("_cq_torch_step", SHIM_PATH)
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
-        if mod.library_version() != load().cq_version():
+        # (what the shim was compiled against: asking it for the library's version would ask the library)
+        built_for = getattr(mod, "header_version", None)
+        if built_for is None or built_for() != load().cq_version():
             raise CalibQuantError("the host shim and the HIP library were built from different sources")
         _shim = mod
     return _shim

@@ -172,5 +172,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def_property_readonly("length", &LayerStep::length)
         .def_property_readonly("steps", &LayerStep::steps)
         .def_property_readonly("capacity", &LayerStep::capacity);
-    m.def("library_version", []() { return cq_version(); });
+    m.def("library_version", []() { return cq_version(); });   // of the library that is loaded
+    m.def("header_version", []() { return CQ_VERSION; });      // this shim was built for
 }

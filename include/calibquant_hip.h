@@ -40,6 +40,10 @@ enum cq_status {
     CQ_ERR_SCRATCH_LIMIT = -8 /* cq_decode_attn_static: the request needs more scratch than the static buffer holds */
 };
 
+/* The interface this header declares; cq_version() is the loaded library's.  106: cq_linear_rows, cq_linear_rows_takes, cq_linear_rows_pays, cq_window_rows;
+ * 105: chunked decode in two launches (merge inside the main launch; the workspace holds min / max, partials and counters); 104:
+ * cq_rope_quantize_pack, cq_rope_rows; 103: cq_decode_attn_static; 102: lut_len argument of the look-up vec-mats, cq_quant_tensor. */
+#define CQ_VERSION 106
 int cq_version(void);
 const char* cq_strerror(int status);
 int cq_last_hip_error(void);

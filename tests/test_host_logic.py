@@ -416,3 +416,20 @@ def test_projections_of_a_step_only_where_they_are_no_slower():
         assert bool(lib.cq_linear_rows_pays(*shape)) == (shape in faster), shape
     for shape in [(9, 4096, 4096), (0, 4096, 4096), (1, 4096, 4100), (1, 1536, 4096), (1, 4100, 4096)]:
         assert not lib.cq_linear_rows_takes(*shape) and not lib.cq_linear_rows_pays(*shape)
+
+
+def test_a_shim_of_other_sources_is_refused(monkeypatch):
+    """The shim says which interface it was compiled against; one from before it said so, or of another interface, is refused whatever the loaded library answers."""
+    import importlib.util
+    from types import SimpleNamespace
+    from calibquant_amd import _lib
+    version = _lib.load().cq_version()
+    assert _lib.load_step_shim().header_version() == version
+    for stale in (SimpleNamespace(library_version=lambda: version), SimpleNamespace(library_version=lambda: version, header_version=lambda: version - 1)):
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "_shim", None)
+            m.setattr(importlib.util, "spec_from_file_location", lambda *a: SimpleNamespace(loader=SimpleNamespace(exec_module=lambda mod: None)))
+            m.setattr(importlib.util, "module_from_spec", lambda spec: stale)
+            with pytest.raises(_lib.CalibQuantError, match="different sources"):
+                _lib.load_step_shim()
+    assert _lib.load_step_shim().LayerStep is not None
