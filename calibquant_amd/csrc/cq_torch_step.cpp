@@ -123,11 +123,13 @@ class LayerStep {
         const at::Tensor att = t[0].cast<at::Tensor>();
         at::Tensor out = at::empty({B, 1, N}, hidden.options());
         check(cq_linear_rows(att.data_ptr(), KO, a_.dtype, a_.B, static_cast<int>(KO), wo.data_ptr(), N, out.data_ptr(), stream), "cq_linear_rows");
+        ++row_steps_;
         return py::make_tuple(out, t[1], t[2]);
     }
 
     int64_t length() const { return len_; }
     int64_t steps() const { return steps_; }
+    int64_t row_steps() const { return row_steps_; }   // of them with their projections
     int64_t capacity() const { return k_.size(2); }
 
   private:
@@ -158,7 +160,7 @@ class LayerStep {
     at::ScalarType dtype_;
     at::Tensor cos_, sin_, k_, v_, ramp_;
     int64_t len_;
-    int64_t steps_ = 0;
+    int64_t steps_ = 0, row_steps_ = 0;
 };
 
 }  // namespace
@@ -171,6 +173,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def("step_rows", &LayerStep::step_rows)
         .def_property_readonly("length", &LayerStep::length)
         .def_property_readonly("steps", &LayerStep::steps)
+        .def_property_readonly("row_steps", &LayerStep::row_steps)
         .def_property_readonly("capacity", &LayerStep::capacity);
     m.def("library_version", []() { return cq_version(); });   // of the library that is loaded
     m.def("header_version", []() { return CQ_VERSION; });      // this shim was built for

@@ -448,7 +448,7 @@ def test_small_batch_step_takes_its_projections_along():
     seen = []
 
     def steps(hook):
-        calls = seen.clear()
+        seen.clear()
         h = att.wqkv.register_forward_hook(lambda *a: seen.append(1)) if hook else None
         outs = []
         with torch.no_grad():
@@ -458,7 +458,8 @@ def test_small_batch_step_takes_its_projections_along():
                 outs.append(o)
         if h:
             h.remove()
-        assert att._cq_step[0].steps == 5
+        step = att._cq_step[0]
+        assert step.steps == 5 and step.row_steps == (0 if hook else 5)
         return torch.stack(outs).float(), past
 
     with torch.no_grad():
