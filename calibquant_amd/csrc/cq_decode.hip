@@ -134,10 +134,10 @@ static int make_plan(const cq_decode_args* a, Plan* p) {
             if (single || chunked) *p = q;
         }
     }
-    // A handful of units leave most compute units idle, and a launch then lasts as long as one unit: fewer
-    // heads per unit make the units cheaper and there are compute units for two or four times as many of them.
-    // (Where the lines lie was measured with the look-up form: 18.8 / 15.5 / 14.2 us for four / two / one head at
-    // 3 328 + 128 tokens.)
+    // A handful of units leave most compute units idle, and a launch then lasts as long as one unit: with one head to a unit
+    // it is a shorter chain, and there are compute units for four times as many.  us from a recorded graph, one / two / four heads a unit, 32 / 8 heads:
+    // 2 x 700 + 60 6.50 / 6.77 / 6.78, 2 x 3 328 + 128 9.50 / 9.63 / 9.60, 8 x 3 328 + 128 10.30 / 9.92 / 9.75, 10 x 3 328 + 128 18.1 / 10.1 / 9.8.
+    // (Two heads from 33 to 64 units of four: within 2 % of four heads either way.  The line is from the look-up form: 15.5 for 18.8.)
     if (a->force_splits == 0 && p->nsplit == 1 && p->hpb == 4) {
         const int64_t u4 = static_cast<int64_t>(a->B) * a->Hkv * ngroups(G, p->nh);
         const int h = u4 <= 32 ? 1 : (u4 <= 64 && G % 2 == 0) ? 2 : 4;

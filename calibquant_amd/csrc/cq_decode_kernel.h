@@ -776,7 +776,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
         *reinterpret_cast<Vec<2>*>(fx + L::F_VSZ + 2 * pair) = Vec<2>{{Cvt<DT>::lo(s_raw), Cvt<DT>::hi(s_raw)}};
         *reinterpret_cast<Vec<2>*>(fx + L::F_VSZ + kD + 2 * pair) = Vec<2>{{Cvt<DT>::lo(z_raw), Cvt<DT>::hi(z_raw)}};
     }
-    if (tid < 3 * HPB) reinterpret_cast<int*>(red)[tid] = static_cast<int>(0x80000000u);   // block_max's meeting words
+    if (tid < 3 * HPB) reinterpret_cast<int*>(red)[tid] = static_cast<int>(0x80000000u);   // the meeting words of the waves' minima and maxima
     // Chunked launch: the chunks' logit min / max, lane s the pair of chunk s for every head (all in flight
     // together; they are folded across the wave where the calibration needs them).
     struct alignas(8) MinMax { float lo, hi; };
@@ -877,7 +877,7 @@ __global__ __launch_bounds__(NT, 4) void decode_kernel(DecodeGeom g) {
 #pragma unroll
             for (int rd = 0; rd < REGL; ++rd) ts[rd] = vsp[min(tid + rd * kNT, n - 1)];
         }
-        // the waves' minima and maxima meet in LDS, as in block_max, from one lane per head
+        // the waves' minima and maxima meet in LDS, from one lane per head
         const int klo = row_max_key(float_key(-lo)), khi = row_max_key(float_key(hi));
         int* redi = reinterpret_cast<int*>(red);
         if ((lane & 15) == 0 && (lane >> 4) < HPB) {

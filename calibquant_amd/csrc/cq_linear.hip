@@ -16,7 +16,7 @@
 //   4 x 6 144 x 8 192 23.5 (20.9) / 23.8 (21.2) / 23.9 (17.4); x 6 144 19.1 (17.0) / 19.4 (16.3) / 18.3 (14.6)
 //   2 x 6 144 x 8 192 21.0 (18.1) / 23.6 (19.8) / 24.1 (17.3); 2 x 4 096 x 6 144 11.7 (8.9) / 11.6 (10.0) / 15.3 (10.9)
 //   1 x 4 096 x 6 144 10.9 (8.2) / 10.7 (9.2) / 14.2 (10.7)
-// Launched one by one, as the eager step does, the library's product takes 20 us of host time, this 3.
+// Launched one by one, as the eager step does, the library's product takes 20 us of host time, this 3.  cq_linear_rows_pays() has the sizes a step takes it for.
 #include "cq_common.h"
 
 namespace cq {

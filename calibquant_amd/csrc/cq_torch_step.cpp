@@ -2,8 +2,8 @@
 // attention layer: the bookkeeping the eager path does per layer and token (allocate the
 // query and output rows, grow the full-precision window, aim the two launches at this step's
 // tensors, take torch's current stream) in one C++ call instead of ~40 lines of Python and two
-// ctypes calls.  It owns no kernels: it calls `cq_rope_append` and `cq_decode_attn` with the
-// same arguments the Python path passes, so the results are the same bits.
+// ctypes calls.  It owns no kernels: it calls `cq_rope_append` and `cq_decode_attn`, and for a few rows
+// `cq_linear_rows` (`step_rows`), with the arguments the Python path passes, so the results are the same bits.
 //
 // What it replaces in the reference is the per-token torch op chain of one layer's decode
 // branch: the (h gs d) split, `apply_rotary_pos_emb`, the `torch.cat` window growth and the
