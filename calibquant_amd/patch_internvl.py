@@ -161,7 +161,8 @@ def _plain_products(*modules) -> bool:
             return False
         d = m.__dict__   # (an attribute that is a parameter takes the module's slow look-up)
         if ("forward" in d or "_call_impl" in d or d.get("_compiled_call_impl") is not None or d["_forward_hooks"]
-                or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or d["_parameters"].get("bias") is not None or type(d["_parameters"].get("weight")) is not torch.nn.Parameter):
+                or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]
+                or d["_parameters"].get("bias") is not None or type(d["_parameters"].get("weight")) is not torch.nn.Parameter):
             return False
     return True
 
